@@ -502,6 +502,11 @@ int mogt_embedding_bwd(const void* grad, int64_t ld_grad, const void* grad2, int
 #define MOGT_CONN_CAYLEY 1
 int mogt_connection_map_fwd(const void* A, void* U, int64_t count, int64_t rank, float scale,
                             float damping, int impl, int out_dtype, void* stream);
+/* Its gradient: dA (fp32 [count, r, r]) from the same skew generators A and the
+ * gradient dU of U (fp32 [count, r, r]); replaces autograd through
+ * torch.matrix_exp / torch.linalg.solve.                                     */
+int mogt_connection_map_bwd(const void* A, const void* dU, void* dA, int64_t count, int64_t rank,
+                            float scale, float damping, int impl, void* stream);
 
 /* ------------------------------------------------------------------------- */
 /* Cross-entropy rows of the chunked tied-head loss, replacing the per-chunk

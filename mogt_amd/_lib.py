@@ -157,6 +157,8 @@ SIGNATURES: dict[str, tuple] = {
                  _c_void_p, _c_void_p, _c_void_p]),
     "mogt_connection_map_fwd": (
         _c_int, [_c_void_p, _c_void_p, _c_i64, _c_i64, _c_float, _c_float, _c_int, _c_int, _c_void_p]),
+    "mogt_connection_map_bwd": (
+        _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_float, _c_float, _c_int, _c_void_p]),
     "mogt_lm_ce_fwd": (
         _c_int, [_c_void_p, _c_i64, _c_int, _c_void_p, _c_i64, _c_i64, _c_i64, _c_void_p, _c_void_p,
                  _c_void_p]),

@@ -1729,18 +1729,6 @@ def silu_mul(y: torch.Tensor) -> torch.Tensor:
 _CONN_IMPL = {"matrix_exp": _lib.MOGT_CONN_EXP, "cayley": _lib.MOGT_CONN_CAYLEY}
 
 
-def _connection_map_reference(A: torch.Tensor, impl: int, scale: float, damping: float) -> torch.Tensor:
-    """The same map with torch's library routines (model_mogt.py:79-102); used
-    to differentiate the HIP forward."""
-    X = A.to(torch.float32) * scale
-    if impl == _lib.MOGT_CONN_EXP:
-        U = torch.matrix_exp(X)
-    else:
-        eye = torch.eye(A.shape[-1], dtype=X.dtype, device=X.device)
-        U = torch.linalg.solve(eye - 0.5 * X, eye + 0.5 * X)
-    return U * damping
-
-
 @torch.library.custom_op("mogt::connection_map", mutates_args=())
 def _connection_map_op(A: torch.Tensor, impl: int, scale: float, damping: float,
                        out_dtype: torch.dtype) -> torch.Tensor:
@@ -1767,13 +1755,32 @@ def _connection_map_setup(ctx, inputs, output):
     ctx.args = (impl, scale, damping)
 
 
+@torch.library.custom_op("mogt::connection_map_bwd", mutates_args=())
+def _connection_map_bwd_op(A: torch.Tensor, grad_u: torch.Tensor, impl: int, scale: float,
+                           damping: float) -> torch.Tensor:
+    """dA of ``connection_map`` (fp32 arithmetic, in A's dtype)."""
+    lib = _lib.load()
+    A32 = A.to(torch.float32).contiguous()
+    g = grad_u.to(torch.float32).contiguous()
+    r = A.shape[-1]
+    dA = torch.empty_like(A32)
+    rc = lib.mogt_connection_map_bwd(A32.data_ptr(), g.data_ptr(), dA.data_ptr(), A32.numel() // (r * r) if r else 0,
+                                     r, float(scale), float(damping), int(impl), _stream_handle(A.device))
+    _lib.check(rc, "mogt_connection_map_bwd")
+    return dA if A.dtype == torch.float32 else dA.to(A.dtype)
+
+
+@_connection_map_bwd_op.register_fake
+def _(A, grad_u, impl, scale, damping):
+    return A.new_empty(A.shape)
+
+
 def _connection_map_backward(ctx, grad_u):
     (A,) = ctx.saved_tensors
-    with torch.enable_grad():
-        Ad = A.detach().requires_grad_()
-        U = _connection_map_reference(Ad, *ctx.args)
-        (gA,) = torch.autograd.grad(U, Ad, grad_u.to(U.dtype))
-    return gA.to(A.dtype), None, None, None, None
+    # a constant for any higher derivative
+    with torch.no_grad():
+        gA = torch.ops.mogt.connection_map_bwd(A, grad_u, *ctx.args)
+    return gA, None, None, None, None
 
 
 torch.library.register_autograd("mogt::connection_map", _connection_map_backward,
@@ -1784,8 +1791,8 @@ def connection_map(A: torch.Tensor, impl: str, *, scale: float = 1.0, damping: f
                    out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
     """``U = damping * f(scale * A)`` for skew-symmetric ``A [..., r, r]`` (r <= 32)
     with ``f`` = ``matrix_exp`` or ``cayley`` (``(I - S/2)^{-1} (I + S/2)``),
-    the transport maps of model_mogt.py:79-102, on the HIP kernels; gradients
-    come from torch's routines on the same inputs."""
+    the transport maps of model_mogt.py:79-102, on the HIP kernels, the
+    gradient included (``mogt_connection_map_bwd``)."""
     require_cuda("connection_map", A)
     if impl not in _CONN_IMPL:
         raise ValueError(f"Unsupported connection_impl: {impl}")

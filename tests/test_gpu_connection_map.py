@@ -3,8 +3,8 @@ matrix exponential and Cayley transform of skew-symmetric generators, against
 float64 library routines (torch.matrix_exp, torch.linalg.solve) on the same
 inputs, plus the orthogonality the maps must produce.  Bar: the fp32 bar 1e-4
 normwise (1e-5 for moderate norms; generators up to ||A||_F ~ 180 are
-included, where 8 squarings amplify fp32 rounding); gradients (torch's
-routines on the same inputs) against float64 autograd <= 1e-4."""
+included, where 8 squarings amplify fp32 rounding); gradients against float64
+autograd: normwise 1e-5 up to norms of about 20, 1e-4 beyond."""
 import numpy as np
 import pytest
 import torch
@@ -74,6 +74,30 @@ def test_connection_map_backward(gpu):
         Ar = A64.clone().requires_grad_()
         ((0.9 * _ref(Ar, impl)) * W).sum().backward()
         assert rel_err(to_np(A.grad), Ar.grad.numpy()) <= 1e-4
+
+
+@pytest.mark.parametrize("impl", ["matrix_exp", "cayley"])
+@pytest.mark.parametrize("n,r,std,scale", [(1, 1, 1.0, 1.0), (5, 2, 0.5, 1.0), (1001, 16, 0.05, 1.0),
+                                           (1001, 16, 2.0, 0.5), (301, 15, 1.0, 1.0), (77, 17, 0.3, 2.0),
+                                           (130, 32, 0.3, 1.0), (64, 16, 8.0, 1.0), (3, 16, 0.0, 1.0)])
+def test_connection_map_gradient_matches_float64(gpu, impl, n, r, std, scale):
+    """Every rank tile edge (r = 1, 15, 16, 17, 32), counts that leave waves of
+    the last work-group idle, the identity (zero generator), several squarings
+    and a permuted (non-contiguous) upstream gradient."""
+    announce(f"connection map gradient {impl} n={n} r={r} std={std}")
+    import mogt_amd
+
+    A64 = _skew(n, r, std, seed=r + n).float().double()
+    W = torch.randn(r, n, r, dtype=torch.float64, generator=torch.Generator().manual_seed(n)).float().double()
+    W = W.permute(1, 2, 0)
+    A = A64.float().to(gpu).requires_grad_()
+    U = mogt_amd.ops.connection_map(A, impl, scale=scale, damping=0.999)
+    (gA,) = torch.autograd.grad(U, A, W.float().to(gpu))
+    torch.cuda.synchronize()
+    Ar = A64.clone().requires_grad_()
+    (ref,) = torch.autograd.grad(0.999 * _ref(scale * Ar, impl), Ar, W)
+    assert gA.dtype == A.dtype and gA.shape == A.shape
+    assert rel_err(to_np(gA), ref.numpy()) <= (1e-5 if std * scale * r <= 20 else 1e-4)
 
 
 def test_connection_map_errors(gpu):
