@@ -530,6 +530,34 @@ int mogt_lm_ce_fwd(const void* logits, int64_t ld, int logits_dtype, const int64
 int mogt_lm_ce_bwd(const void* logits, int64_t ld, int logits_dtype, const int64_t* labels,
                    const float* lse_rows, int64_t rows, int64_t vocab, int64_t ignore_index,
                    const float* scale, void* grad, int64_t ld_grad, int grad_dtype, void* stream);
+/* mogt_lm_ce_bwd with the fp32 gradient written as three bf16 pieces
+ * [3][rows][ld_grad] (their sum is the fp32 value), columns vocab .. ld_grad - 1
+ * zero: an operand of mogt_split_gemm.                                      */
+int mogt_lm_ce_bwd_pieces(const void* logits, int64_t ld, int logits_dtype, const int64_t* labels,
+                          const float* lse_rows, int64_t rows, int64_t vocab, int64_t ignore_index,
+                          const float* scale, void* grad, int64_t ld_grad, void* stream);
+
+/* ------------------------------------------------------------------------- */
+/* fp32 matrix products on the bf16 matrix cores (the tied head's GEMMs,
+ * chunked_lm_loss.py:29-72).
+ * mogt_split_pieces: fp32 src [rows, cols] -> bf16 pieces dst [3][rows][ld_dst]
+ *   with src = dst[0] + dst[1] + dst[2]; columns cols .. ld_dst - 1 zero.
+ * mogt_split_gemm: C[m][n] (+)= sum_k A(m, k) B(n, k).  Each operand is 1 piece
+ *   (bf16 values) or 3 (fp32 values); k_slow 0: element (row, k) at
+ *   row * ld + k, zeros up to a multiple of 32 in memory; k_slow 1: at
+ *   k * ld + row.  plane: elements between pieces.  Built: both k_slow 0 (any
+ *   pieces); A k_slow 0 or 1 in 3 pieces with B k_slow 1.  C fp32 (accumulate
+ *   adds to it) or bf16, row stride ldc >= N rounded up to 4 (those columns are
+ *   written).  Workspace: fp32 partials of the K slices (splits <= 0: chosen),
+ *   mogt_split_gemm_workspace_bytes(... cus <= 0: of the current device).    */
+int mogt_split_pieces(const void* src, int64_t ld_src, void* dst, int64_t ld_dst, int64_t rows, int64_t cols,
+                      void* stream);
+size_t mogt_split_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int pieces_a, int pieces_b, int64_t splits,
+                                       int64_t cus);
+int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int pieces_a, int k_slow_a, const void* B,
+                    int64_t ldb, int64_t plane_b, int pieces_b, int k_slow_b, void* C, int64_t ldc, int64_t M,
+                    int64_t N, int64_t K, int accumulate, int out_dtype, int64_t splits, void* workspace,
+                    size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -19,6 +19,10 @@ How it runs here:
   forward ran under (recorded at forward time), so they match the forward's
   logits, whose log-sum-exp it reuses.  The two gradient GEMMs run in fp32
   with autocast off, as the reference's backward does.
+* fp32 GEMMs of blocks large enough (``_split_ok``) run on the bf16 matrix
+  cores from exact three-piece splits of their fp32 operands
+  (``csrc/split_gemm.hip``); the gradient block is then written as its pieces.
+  The rest go to the BLAS library.
 * Labels equal to -100 (F.cross_entropy's default ``ignore_index``) add zero
   loss, as in the reference's forward, and a zero gradient row; the
   reference's backward subtracts 1 at column ``vocab - 100`` for them.
@@ -59,6 +63,90 @@ def _block_logits(rows: torch.Tensor, w32: torch.Tensor) -> torch.Tensor:
     return rows.float().matmul(w32.t())
 
 
+# Where a block's fp32 GEMMs take the split form, in multiply-adds of one of
+# them (rows x vocab x D).  Below, both forms take the host time of their
+# launches, of which the split form has more (2048 x 4000 x 512, 2^32: 471 us a
+# forward and backward against the library's 452; fp32 hidden states 513
+# against 435); above, the matrix units decide (256 x 32000 x 768, 2^32.6: 481
+# against 690 us; 1024 rows: 896 against 2017; fp32 hidden states 1202 against
+# 2027).
+SPLIT_MIN_MACS = 6_000_000_000
+
+
+def _split_ok(rows: torch.Tensor, weight: torch.Tensor, chunk: int) -> bool:
+    """Whether this head's fp32 GEMMs run from bf16 pieces: tensors on the GPU,
+    a contraction of whole stages, a first block large enough to gain and
+    gradient rows within the kernel's 32-bit offsets."""
+    n, D = min(rows.shape[0], chunk), rows.shape[1]
+    V = weight.shape[0]
+    return (rows.is_cuda and weight.is_cuda and rows.device == weight.device and D % ops.SPLIT_K == 0
+            and n * V * D >= SPLIT_MIN_MACS
+            and (ops.split_pad(n) + ops.SPLIT_K) * ops.split_pad(V) * 2 < 1 << 31
+            and (ops.split_pad(V) + ops.SPLIT_K) * D * 2 < 1 << 31)
+
+
+def _pieces(x: torch.Tensor) -> torch.Tensor:
+    """``x [rows, D]`` as the bf16 pieces of its fp32 value (one where it is
+    bf16 already)."""
+    if x.dtype != torch.bfloat16:
+        return ops.split_pieces(x.float())
+    if x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < x.shape[1] or x.data_ptr() % 16 != 0:
+        x = x.contiguous()
+    return x.unsqueeze(0)
+
+
+class _Head:
+    """The tied head's GEMMs for one call: logits of a block of rows, and a
+    block's share of the two gradients."""
+
+    def __init__(self, rows: torch.Tensor, weight: torch.Tensor, chunk: int):
+        self.weight = weight
+        self.split = _split_ok(rows, weight, chunk)
+        self._w32 = self._pieces = None
+
+    @property
+    def w32(self) -> torch.Tensor:
+        if self._w32 is None:
+            self._w32 = self.weight.float()
+        return self._w32
+
+    @property
+    def pieces(self) -> torch.Tensor:
+        if self._pieces is None:
+            self._pieces = _pieces(self.weight)
+        return self._pieces
+
+    def logits(self, block: torch.Tensor, autocast: bool) -> torch.Tensor:
+        if autocast or not self.split:
+            return _block_logits(block, self.w32)
+        V, D = self.weight.shape
+        out = torch.empty((block.shape[0], ops.split_pad(V)), dtype=torch.float32, device=block.device)[:, :V]
+        return ops.split_gemm_(out, _pieces(block), self.pieces, D)
+
+    def new_weight_grad(self) -> torch.Tensor:
+        # the split form writes it with the first block
+        make = torch.empty if self.split else torch.zeros
+        return make(self.weight.shape, dtype=torch.float32, device=self.weight.device)
+
+    def backward(self, logits, targets, lse, scale, block, d_rows, d_w32, first: bool) -> None:
+        """d_rows = g @ weight and d_w32 += g^T @ block for the block's fp32
+        gradient g, in fp32."""
+        if not self.split:
+            # fp32 gradient block, whatever the logits' dtype
+            g = ops.lm_ce_grad(logits, targets, lse, scale, ignore_index=IGNORE_INDEX)
+            d_rows.copy_(g.matmul(self.w32))
+            d_w32.addmm_(g.t(), block.float())
+            return
+        V, D = self.weight.shape
+        g = ops.lm_ce_grad_pieces(logits, targets, lse, scale, ignore_index=IGNORE_INDEX)
+        direct = d_rows.dtype in (torch.float32, torch.bfloat16) and d_rows.is_contiguous()
+        dh = d_rows if direct else torch.empty(d_rows.shape, dtype=torch.float32, device=d_rows.device)
+        ops.split_gemm_(dh, g, self.pieces, V, k_slow_b=True)
+        if not direct:
+            d_rows.copy_(dh)
+        ops.split_gemm_(d_w32, g, _pieces(block), block.shape[0], k_slow_a=True, k_slow_b=True, accumulate=not first)
+
+
 class _ChunkedLinearCrossEntropy(torch.autograd.Function):
     """chunked_lm_loss.py:5-72 on the HIP cross-entropy rows."""
 
@@ -77,18 +165,18 @@ class _ChunkedLinearCrossEntropy(torch.autograd.Function):
         n_tok = labels.numel()
         rows = hidden_states.reshape(n_tok, hidden_states.shape[-1])
         targets = labels.reshape(n_tok).to(torch.int64).contiguous()
-        w32 = weight.float()
+        ctx.autocast = _AutocastState()
+        head = _Head(rows, weight, chunk_size)
         per_row = torch.empty(n_tok, dtype=torch.float32, device=hidden_states.device)
         lse = torch.empty(n_tok, dtype=torch.float32, device=hidden_states.device)
         with torch.no_grad():
             for sl in _token_blocks(n_tok, chunk_size):
-                loss_rows, lse_rows = ops.lm_ce_forward(_block_logits(rows[sl], w32), targets[sl],
-                                                        ignore_index=IGNORE_INDEX)
+                logits = head.logits(rows[sl], ctx.autocast.enabled)
+                loss_rows, lse_rows = ops.lm_ce_forward(logits, targets[sl], ignore_index=IGNORE_INDEX)
                 per_row[sl] = loss_rows
                 lse[sl] = lse_rows
         ctx.save_for_backward(hidden_states, weight, targets, lse)
         ctx.chunk_size = chunk_size
-        ctx.autocast = _AutocastState()
         return per_row.sum() / n_tok
 
     @staticmethod
@@ -96,19 +184,16 @@ class _ChunkedLinearCrossEntropy(torch.autograd.Function):
         hidden_states, weight, targets, lse = ctx.saved_tensors
         n_tok = targets.numel()
         rows = hidden_states.reshape(n_tok, hidden_states.shape[-1])
-        w32 = weight.float()
         scale = (grad_output.float() / n_tok).reshape(1)
+        head = _Head(rows, weight, ctx.chunk_size)
         d_rows = torch.empty_like(rows)
-        d_w32 = torch.zeros_like(w32)
-        for sl in _token_blocks(n_tok, ctx.chunk_size):
+        d_w32 = head.new_weight_grad()
+        for i, sl in enumerate(_token_blocks(n_tok, ctx.chunk_size)):
             block = rows[sl]
             with ctx.autocast():
-                logits = _block_logits(block, w32)
-            # fp32 gradient block, whatever the logits' dtype
-            g = ops.lm_ce_grad(logits, targets[sl], lse[sl], scale, ignore_index=IGNORE_INDEX)
+                logits = head.logits(block, ctx.autocast.enabled)
             with torch.autocast("cuda", enabled=False):
-                d_rows[sl] = g.matmul(w32).to(d_rows.dtype)
-                d_w32.addmm_(g.t(), block.float())
+                head.backward(logits, targets[sl], lse[sl], scale, block, d_rows[sl], d_w32, first=i == 0)
         return d_rows.view_as(hidden_states), d_w32.to(weight.dtype), None, None
 
 

@@ -17,7 +17,7 @@
 // in base 2 on the hardware unit (v_exp_f32): exp(x - m) = 2^((x - m) log2 e),
 // the difference taken first so the row maximum's term is exactly 1; terms
 // below 2^-126 of the row maximum flush to zero.
-#include "common.h"
+#include "bf16_pieces.h"
 
 #include <math.h>
 
@@ -160,6 +160,42 @@ __global__ __launch_bounds__(CE_THREADS) void ce_bwd_kernel(const TL* logits, in
     }
 }
 
+// The gradient block as three bf16 pieces [3][rows][ldg] (split_gemm.hip's
+// operand), columns vocab .. ldg - 1 zero: the same values as ce_bwd_kernel's
+// fp32 block, split in registers, so no fp32 block is written and read back.
+template <typename TL>
+__global__ __launch_bounds__(CE_THREADS) void ce_bwd_pieces_kernel(const TL* __restrict__ logits, int64_t ld,
+                                                                   const int64_t* __restrict__ labels,
+                                                                   const float* __restrict__ lse, int64_t vocab,
+                                                                   int64_t ignore, const float* __restrict__ scale,
+                                                                   bf16_t* __restrict__ grad, int64_t ldg,
+                                                                   int64_t plane) {
+    const int64_t row = blockIdx.x;
+    const TL* x = logits + row * ld;
+    bf16_t* g = grad + row * ldg;
+    const int64_t lab = labels[row];
+    const bool skip = lab == ignore;
+    const float bad = (!skip && (lab < 0 || lab >= vocab)) ? __builtin_nanf("") : 0.0f;
+    const float lr = lse[row];
+    const float sc = *scale;
+    const bool vec = reinterpret_cast<uintptr_t>(x) % (4 * sizeof(TL)) == 0;
+    for (int64_t j = threadIdx.x * 4; j < ldg; j += CE_THREADS * 4) {
+        float v[4];
+        if (vec && j + 4 <= vocab) {
+            load_vec<TL, 4>(x + j, v);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = j + e < vocab ? IO<TL>::ld(x[j + e]) : 0.0f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float p = __builtin_amdgcn_exp2f((v[e] - lr) * CE_LOG2E) - (j + e == lab ? 1.0f : 0.0f);
+            v[e] = (skip || j + e >= vocab) ? 0.0f : p * sc + bad;
+        }
+        store_pieces4(v, g + j, plane);
+    }
+}
+
 namespace {
 
 bool ce_dt(int d) { return d == MOGT_F32 || d == MOGT_BF16; }
@@ -221,4 +257,31 @@ extern "C" int mogt_lm_ce_bwd(const void* logits, int64_t ld, int logits_dtype, 
     else MOGT_CE_BWD(bf16_t, bf16_t);
 #undef MOGT_CE_BWD
     return check_launch("ce_bwd_kernel");
+}
+
+extern "C" int mogt_lm_ce_bwd_pieces(const void* logits, int64_t ld, int logits_dtype, const int64_t* labels,
+                                     const float* lse_rows, int64_t rows, int64_t vocab, int64_t ignore_index,
+                                     const float* scale, void* grad, int64_t ld_grad, void* stream) {
+    clear_error();
+    int rc = ce_check(rows, vocab, ld, "lm_ce_bwd_pieces");
+    if (rc) return rc;
+    if (ld_grad < vocab || ld_grad % 8 != 0)
+        return set_error(MOGT_E_INVALID, "lm_ce_bwd_pieces: gradient row stride must cover the vocab, a multiple of 8");
+    if (!ce_dt(logits_dtype)) return set_error(MOGT_E_INVALID, "lm_ce_bwd_pieces: dtype");
+    if (rows == 0) return MOGT_OK;
+    if (!logits || !labels || !lse_rows || !scale || !grad)
+        return set_error(MOGT_E_INVALID, "lm_ce_bwd_pieces: null pointer");
+    if (reinterpret_cast<uintptr_t>(grad) & 15)
+        return set_error(MOGT_E_INVALID, "lm_ce_bwd_pieces: gradient needs 16-byte alignment");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const dim3 grid(static_cast<unsigned>(rows));
+    if (logits_dtype == MOGT_F32)
+        hipLaunchKernelGGL((ce_bwd_pieces_kernel<float>), grid, dim3(CE_THREADS), 0, st,
+                           static_cast<const float*>(logits), ld, labels, lse_rows, vocab, ignore_index, scale,
+                           static_cast<bf16_t*>(grad), ld_grad, rows * ld_grad);
+    else
+        hipLaunchKernelGGL((ce_bwd_pieces_kernel<bf16_t>), grid, dim3(CE_THREADS), 0, st,
+                           static_cast<const bf16_t*>(logits), ld, labels, lse_rows, vocab, ignore_index, scale,
+                           static_cast<bf16_t*>(grad), ld_grad, rows * ld_grad);
+    return check_launch("ce_bwd_pieces_kernel");
 }

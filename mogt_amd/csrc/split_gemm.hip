@@ -1,0 +1,550 @@
+// fp32 matrix products on the bf16 matrix cores, for the tied head's loss
+// (chunked_lm_loss.py:29-72: logits, and the gradients of hidden states and
+// weight):
+//   C[m][n] (+)= sum_k A(m, k) B(n, k)
+// Each fp32 operand comes as three bf16 pieces x = x1 + x2 + x3 (each the
+// rounded remainder of the ones before: 3 x 8 significant bits hold all 24 of
+// x), a bf16 operand as one.  A product of two bf16 pieces is exact in fp32
+// and the MFMA accumulates in fp32, so
+//   1 x 3 pieces  x1 (y1 + y2 + y3)                              exact products
+//   3 x 3 pieces  x1 y1 + x1 y2 + x1 y3 + x2 y1 + x2 y2 + x3 y1  (the terms left
+//                 out are below 2^-26 of |x y|, under fp32's own rounding 2^-24)
+// at 3 or 6 bf16 products instead of one fp32 product: the bf16 matrix rate is
+// 16 times the fp32 one (155 TFLOP/s reached by the BLAS library's fp32 GEMM,
+// which is that unit's peak).  Elements that are not finite go whole into the
+// first piece.
+//
+// Operand layouts, per operand:
+//   K_FAST  element (row, k) at row * ld + k   (K padded with zeros in memory
+//           to a multiple of 32)
+//   K_SLOW  element (row, k) at k * ld + row   (k past K loads zero)
+// K_SLOW fragments come out of LDS through the transposing read
+// ds_read_b64_tr_b16 (wgrad_gemm.hip describes it), its 4 x 16 blocks chosen so
+// that the K-slots agree with K_FAST's: lane half h, slot q <-> k = 8 h + q.
+//
+// Tile: 256 rows of A x 64 TNF rows of B (TNF = 4, or 2 for 3 x 3 pieces),
+// 4 waves of 128 x 32 TNF, v_mfma_f32_32x32x16_bf16 with B as the MFMA's A
+// operand (a lane's results are 4 consecutive n of one m: 16-byte stores).
+// A stage is 32 of K for every piece of both operands: a fragment is read from
+// LDS once and multiplied with every piece of the other operand it meets, so
+// the LDS moves 1/2 (1 x 3) to 3/8 (3 x 3) of what separate bf16 GEMMs per
+// piece pair would: 96 MFMAs (3072 cycles) a stage and wave against 16 - 18 KB
+// of fragment reads and loads each.  That is what bounds the bf16 GEMMs of this
+// library (swiglu_gemm.hip); here the MFMA does.  Two stages of 64 - 72 KB in LDS:
+// stage s + 2 is loaded (direct to LDS) into stage s's buffer from the middle
+// of stage s on, one barrier a stage.
+//
+// Split K: the stages are cut into slices so that tiles x slices fill the CUs
+// (plan_split); each slice's fp32 partial goes to the workspace and a second
+// kernel adds them in slice order, so results do not depend on scheduling.
+//
+// Measured (4096 rows, D = 768, vocabulary 32000; the library's fp32 GEMM before
+// -> here; error of the result against 64 bits, normwise):
+//   logits, bf16 x fp32        1536 -> 590 us (1.02 PFLOP/s bf16)  5.0e-7 -> 3.0e-7
+//   logits, fp32 x fp32        1518 -> 998 us (1.21)               5.0e-7 -> 4.3e-7
+//   d hidden, fp32 x fp32      1458 -> 1064 us (1.14)              3.2e-6 -> 1.4e-6
+//   d weight, fp32 x bf16      1448 -> 568 us (1.06)               1.1e-6 -> 7.0e-7
+//   d weight, fp32 x fp32      1417 -> 957 us (1.26)               1.1e-6 -> 1.0e-6
+#include <type_traits>
+
+#include "bf16_pieces.h"
+#include "lds_dma.h"
+
+namespace mogt {
+namespace {
+
+typedef __bf16 sp_bf16x8 __attribute__((ext_vector_type(8)));
+typedef short sp_i16x4 __attribute__((ext_vector_type(4)));
+typedef short sp_i16x8 __attribute__((ext_vector_type(8)));
+typedef float sp_f32x16 __attribute__((ext_vector_type(16)));
+typedef float sp_f32x4 __attribute__((ext_vector_type(4)));
+typedef float sp_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 sp_bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t sp_u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int SP_BM = 256;        // rows of A per work-group
+constexpr int SP_BK = 32;         // contraction per stage
+constexpr int SP_THREADS = 256;   // 4 waves, 2 x 2
+constexpr int SP_GROUP_M = 8;     // row blocks walked together per XCD
+
+struct SplitParams {
+    const bf16_t* a;
+    const bf16_t* b;
+    float* out;                // C (one slice) or the partials [slices][M][N]
+    int64_t lda, ldb, ldo;     // elements
+    int64_t pa, pb;            // elements between pieces
+    int64_t po;                // elements between slices of out
+    int M, N, K;               // N: multiple of 4 within ldo
+    int nb_valid;              // rows of B that exist (K_FAST loads clamp to them)
+    int n_mb, n_nb;            // tiles
+    int stages, per_slice;     // in all, per slice
+    int accumulate;            // out += (one slice)
+};
+
+// block id -> (row block, column block, slice): each XCD (ids mod 8) a
+// contiguous run, 8 row blocks walked together so that its L2 keeps them
+__device__ __forceinline__ void sp_tile(const SplitParams& p, int& mb, int& nb, int& s) {
+    const int tiles = p.n_mb * p.n_nb;
+    const int n = static_cast<int>(gridDim.x);
+    const int bid = blockIdx.x;
+    const int q = n >> 3, rem = n & 7;
+    const int xcd = bid & 7, loc = bid >> 3;
+    const int v = xcd < rem ? xcd * (q + 1) + loc : rem * (q + 1) + (xcd - rem) * q + loc;
+    s = v / tiles;
+    const int t = v - s * tiles;
+    const int group = SP_GROUP_M * p.n_nb;
+    const int g = t / group, first = g * SP_GROUP_M;
+    const int gm = (p.n_mb - first) < SP_GROUP_M ? (p.n_mb - first) : SP_GROUP_M;
+    const int w = t - g * group;
+    mb = first + w % gm;
+    nb = w / gm;
+}
+
+__device__ __forceinline__ sp_i16x4 sp_read_tr(const char* p) {
+    typedef __attribute__((address_space(3))) sp_i16x4 lds_i16x4;
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_i16x4*)((__attribute__((address_space(3))) char*)(const_cast<char*>(p))));
+}
+
+// One operand's side of the tile: ROWS = 64 F rows, F 32-row fragments per wave.
+template <bool KS, int F>
+struct Operand {
+    static constexpr int ROWS = 64 * F;
+    static constexpr int BYTES = ROWS * 64;          // one piece of a stage
+    static constexpr int LOADS = BYTES / 4096;       // 1 KB load instructions per wave and piece
+    static constexpr int CMASK = 2 * F - 1;          // K_SLOW: 64-byte chunks per LDS row - 1
+    int vo[LOADS];       // per-lane global byte offsets
+    int fo[F];           // per-lane LDS byte offsets of the fragments (K_FAST: of the row)
+    int swz;             // K_FAST: chunk swizzle of the lane's row
+
+    // valid: rows of this block that exist (K_FAST); side: the wave's half
+    __device__ __forceinline__ void init(int wave, int side, int lane, int64_t ld, int valid) {
+        const int l32 = lane & 31;
+        if constexpr (KS) {
+            // an LDS row is one k: 2 F chunks of 32 rows' values (64 B), chunk c
+            // of row r at position c ^ (r mod 2 F)
+            constexpr int LPR = ROWS / 8;            // lanes per LDS row
+            constexpr int RPI = 64 / LPR;            // LDS rows per instruction
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                const int r = (wave * LOADS + i) * RPI + lane / LPR, q = lane % LPR;
+                vo[i] = static_cast<int>((r * ld + (((q >> 2) ^ (r & CMASK)) << 5) + ((q & 3) << 3)) * 2);
+            }
+            const int G = lane >> 4, j = lane & 15, r = 8 * (lane >> 5) + (j >> 2);
+#pragma unroll
+            for (int f = 0; f < F; ++f)
+                fo[f] = r * (ROWS * 2) + (((F * side + f) ^ (r & CMASK)) << 6) + 32 * (G & 1) + 8 * (j & 3);
+            swz = 0;
+        } else {
+            const int lc = (lane & 3) ^ (((lane >> 3) ^ (lane >> 4)) & 3);
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                const int r = 16 * (wave * LOADS + i) + (lane >> 2);
+                vo[i] = static_cast<int>((r < valid ? r : valid - 1) * ld * 2) + lc * 16;
+            }
+#pragma unroll
+            for (int f = 0; f < F; ++f) fo[f] = (32 * F * side + 32 * f + l32) * 64;
+            swz = ((l32 >> 1) ^ (l32 >> 2)) & 3;
+        }
+    }
+    // instruction i of the wave's loads of stage s into LDS `dst` (the piece's base)
+    __device__ __forceinline__ void load(lds_i32x4 rsrc, int i, int s, int64_t ld, uint32_t dst, int wave) const {
+        const uint32_t at = dst + (wave * LOADS + i) * 1024;
+        if constexpr (KS) lds_dma16(rsrc, vo[i] + s * static_cast<int>(SP_BK * ld * 2), 0, at);
+        else lds_dma16(rsrc, vo[i], s * (SP_BK * 2), at);
+    }
+    // fragment f of K-step ks (16 of K) from the piece at `st`
+    __device__ __forceinline__ sp_bf16x8 read(const char* st, int ks, int f, int hb) const {
+        if constexpr (KS) {
+            // rows 8 h + j / 4 and 4 further: the swizzle's bit 2 flips (F = 4)
+            const int o0 = fo[f] + ks * (16 * ROWS * 2);
+            const int o1 = (CMASK >= 4 ? o0 ^ 256 : o0) + 4 * (ROWS * 2);
+            const sp_i16x8 v = __builtin_shufflevector(sp_read_tr(st + o0), sp_read_tr(st + o1), 0, 1, 2, 3, 4, 5, 6, 7);
+            return __builtin_bit_cast(sp_bf16x8, v);
+        } else {
+            return *reinterpret_cast<const sp_bf16x8*>(st + fo[f] + (((2 * ks + hb) ^ swz) << 4));
+        }
+    }
+};
+
+template <int NA, int NB, bool KSA, bool KSB, int TNF>
+__global__ __launch_bounds__(SP_THREADS) void split_gemm_kernel(SplitParams p) {
+    using OA = Operand<KSA, 4>;
+    using OB = Operand<KSB, TNF>;
+    constexpr int STB = NA * OA::BYTES + NB * OB::BYTES;
+    constexpr int NP = NA == 3 && NB == 3 ? 6 : NA * NB;   // piece pairs
+    constexpr int NM = NP * 4 * TNF;                       // MFMAs per K-step and wave
+    constexpr int NR = NA * 4 + NB * TNF;                  // fragments per K-step
+    constexpr int NL = NA * OA::LOADS + NB * OB::LOADS;    // loads per stage and wave
+    static_assert(2 * NR <= NM && 2 * NL <= NM + 1, "reads and loads interleave with the MFMAs");
+    __shared__ __attribute__((aligned(1024))) char smem[2 * STB];
+    int mb, nb, sl;
+    sp_tile(p, mb, nb, sl);
+    const int m0 = mb * SP_BM, n0 = nb * OB::ROWS;
+    const int s0 = sl * p.per_slice;
+    const int T = min(p.per_slice, p.stages - s0);   // >= 1 (host)
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int l32 = lane & 31, hb = lane >> 5;
+    const uint32_t lds0 = lds_addr(smem);
+
+    OA oa;
+    OB ob;
+    oa.init(wave, wm, lane, p.lda, p.M - m0);
+    ob.init(wave, wn, lane, p.ldb, p.nb_valid - n0);
+    lds_i32x4 ra[NA], rb[NB];
+    // K_FAST: from the block's first row to the block's last element; K_SLOW:
+    // from (slice start, block's first row) to the last k's row end, in whole
+    // 16-byte pieces (a dword partly past the range would load zero)
+    const int kv = p.K - s0 * SP_BK;
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        if constexpr (KSA)
+            ra[i] = lds_rsrc(p.a + i * p.pa + static_cast<int64_t>(s0) * SP_BK * p.lda + m0,
+                             static_cast<uint32_t>(((kv - 1) * p.lda + ((p.M - m0 + 7) & ~7)) * 2));
+        else
+            ra[i] = lds_rsrc(p.a + i * p.pa + m0 * p.lda + s0 * SP_BK,
+                             static_cast<uint32_t>((min(p.M - m0, SP_BM) * p.lda - s0 * SP_BK) * 2));
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        if constexpr (KSB)
+            rb[i] = lds_rsrc(p.b + i * p.pb + static_cast<int64_t>(s0) * SP_BK * p.ldb + n0,
+                             static_cast<uint32_t>(((kv - 1) * p.ldb + ((p.nb_valid - n0 + 7) & ~7)) * 2));
+        else
+            rb[i] = lds_rsrc(p.b + i * p.pb + n0 * p.ldb + s0 * SP_BK,
+                             static_cast<uint32_t>((min(p.nb_valid - n0, OB::ROWS) * p.ldb - s0 * SP_BK) * 2));
+    }
+    // load t of stage s (t = 0 .. NL - 1: A's pieces, then B's)
+    auto load = [&](int t, int s) {
+        const uint32_t st = lds0 + (s & 1) * STB;
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+            if (t >= i * OA::LOADS && t < (i + 1) * OA::LOADS)
+                oa.load(ra[i], t - i * OA::LOADS, s, p.lda, st + i * OA::BYTES, wave);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int u = t - NA * OA::LOADS;
+            if (u >= i * OB::LOADS && u < (i + 1) * OB::LOADS)
+                ob.load(rb[i], u - i * OB::LOADS, s, p.ldb, st + NA * OA::BYTES + i * OB::BYTES, wave);
+        }
+    };
+
+    sp_f32x16 acc[TNF][4];
+#pragma unroll
+    for (int j = 0; j < TNF; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.0f;
+
+    struct Frags {
+        sp_bf16x8 a[NA][4], b[NB][TNF];
+    };
+    // fragment r of a K-step in order of first use: a1, b1, then b2, b3, a2, a3
+    auto read = [&](Frags& f, int r, int s, int ks) {
+        const char* st = smem + (s & 1) * STB;
+        if (r < 4) {
+            f.a[0][r] = oa.read(st, ks, r, hb);
+        } else if (r < 4 + NB * TNF) {
+            const int u = r - 4;
+            f.b[u / TNF][u % TNF] = ob.read(st + NA * OA::BYTES + (u / TNF) * OB::BYTES, ks, u % TNF, hb);
+        } else {
+            const int u = r - 4 - NB * TNF;
+            f.a[1 + u / 4][u % 4] = oa.read(st + (1 + u / 4) * OA::BYTES, ks, u % 4, hb);
+        }
+    };
+    // pair q of the piece pairs, A's piece slowest: for 3 x 3 (0,0) (0,1) (0,2)
+    // (1,0) (1,1) (2,0)
+    auto pair_a = [](int q) { return NP == 6 ? (q < 3 ? 0 : q < 5 ? 1 : 2) : NB == 1 ? q : 0; };
+    auto pair_b = [](int q) { return NP == 6 ? (q < 3 ? q : q < 5 ? q - 3 : 0) : NB == 1 ? 0 : q; };
+    // One K-step's MFMAs on `cur`, with one fragment read of `next` (K-step kn of
+    // stage sn) and one load of stage sld every other MFMA.
+    auto kstep = [&](const Frags& cur, Frags& next, int sn, int kn, int sld, auto reads, auto loads) {
+        int t = 0;
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+            for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.b[pair_b(q)][j], cur.a[pair_a(q)][i],
+                                                                        acc[j][i], 0, 0, 0);
+                    if constexpr (decltype(reads)::value)
+                        if (t % 2 == 0 && t / 2 < NR) read(next, t / 2, sn, kn);
+                    if constexpr (decltype(loads)::value)
+                        if (t % 2 == 1 && t / 2 < NL) load(t / 2, sld);
+                    __builtin_amdgcn_sched_barrier(0);
+                    ++t;
+                }
+    };
+    constexpr std::true_type YES{};
+    constexpr std::false_type NO{};
+
+    // stages are numbered within the slice (the descriptors start at it)
+#pragma unroll
+    for (int t = 0; t < NL; ++t) load(t, 0);
+    if (T > 1) {
+#pragma unroll
+        for (int t = 0; t < NL; ++t) load(t, 1);
+        lds_wait_vm<NL>();
+    } else {
+        lds_wait_vm<0>();
+    }
+    __syncthreads();
+    Frags f0, f1;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) read(f0, r, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    // Stage s: its first K-step reads its second's fragments; then stage s + 1
+    // has landed for every wave and stage s's buffer is free (every wave's
+    // reads of it are complete before the barrier).
+    int s = 0;
+    for (; s + 2 < T; ++s) {
+        kstep(f0, f1, s, 1, 0, YES, NO);
+        lds_wait_vm<0>();
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        kstep(f1, f0, s + 1, 0, s + 2, YES, YES);
+    }
+    for (; s + 1 < T; ++s) {
+        kstep(f0, f1, s, 1, 0, YES, NO);
+        lds_wait_vm<0>();
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        kstep(f1, f0, s + 1, 0, 0, YES, NO);
+    }
+    kstep(f0, f1, s, 1, 0, YES, NO);
+    kstep(f1, f0, 0, 0, 0, NO, NO);
+
+    // lane (l32, hb), register group q of acc[j][i]: row m0 + 128 wm + 32 i +
+    // l32, columns n0 + 32 TNF wn + 32 j + 8 q + 4 hb .. + 3
+    float* out = p.out + sl * p.po;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = m0 + 128 * wm + 32 * i + l32;
+        if (m >= p.M) continue;
+        float* row = out + m * p.ldo;
+#pragma unroll
+        for (int j = 0; j < TNF; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int n = n0 + 32 * TNF * wn + 32 * j + 8 * q + 4 * hb;
+                if (n >= p.N) continue;
+                sp_f32x4 v = {acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
+                if (p.accumulate) v += *reinterpret_cast<const sp_f32x4*>(row + n);
+                *reinterpret_cast<sp_f32x4*>(row + n) = v;
+            }
+    }
+}
+
+// C (+)= sum over slices of the partials, in slice order
+template <bool BF16OUT>
+__global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ part, void* __restrict__ out,
+                                                           int64_t ldo, int slices, int M, int N, int accumulate) {
+    const int per_row = N >> 2;
+    const int64_t n = static_cast<int64_t>(M) * per_row, plane = static_cast<int64_t>(M) * N;
+    for (int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; g < n;
+         g += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+        const int64_t m = g / per_row;
+        const int c = static_cast<int>(g - m * per_row) << 2;
+        const float* src = part + m * N + c;
+        sp_f32x4 v = *reinterpret_cast<const sp_f32x4*>(src);
+        for (int k = 1; k < slices; ++k) v += *reinterpret_cast<const sp_f32x4*>(src + k * plane);
+        if constexpr (BF16OUT) {
+            const sp_u32x2 w = {
+                __builtin_bit_cast(uint32_t, __builtin_convertvector((sp_f32x2{v[0], v[1]}), sp_bf16x2)),
+                __builtin_bit_cast(uint32_t, __builtin_convertvector((sp_f32x2{v[2], v[3]}), sp_bf16x2))};
+            *reinterpret_cast<sp_u32x2*>(static_cast<bf16_t*>(out) + m * ldo + c) = w;
+        } else {
+            float* dst = static_cast<float*>(out) + m * ldo + c;
+            if (accumulate) v += *reinterpret_cast<const sp_f32x4*>(dst);
+            *reinterpret_cast<sp_f32x4*>(dst) = v;
+        }
+    }
+}
+
+// fp32 [rows, cols] -> three bf16 pieces [3][rows][ldd], columns cols .. ldd - 1
+// zero; 4 elements per thread
+__global__ __launch_bounds__(256) void split_pieces_kernel(const float* __restrict__ src, int64_t lds,
+                                                           bf16_t* __restrict__ dst, int64_t ldd, int64_t plane,
+                                                           int64_t rows, int64_t cols) {
+    const int64_t per_row = ldd >> 2, n = rows * per_row;
+    for (int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; g < n;
+         g += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+        const int64_t r = g / per_row, c = (g - r * per_row) << 2;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = c + e < cols ? src[r * lds + c + e] : 0.0f;
+        store_pieces4(v, dst + r * ldd + c, plane);
+    }
+}
+
+struct SplitPlan {
+    int64_t stages, per_slice, slices, n_mb, n_nb;
+};
+
+// Slices: the count that makes rounds of work-groups (one per CU) times their
+// length, in MFMA cycles, plus the partials' traffic the least.
+SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int na, int nb, int64_t splits, int64_t cus) {
+    SplitPlan pl{};
+    const int np = na == 3 && nb == 3 ? 6 : na * nb;
+    const int tnf = np == 6 ? 2 : 4;
+    pl.n_mb = (M + SP_BM - 1) / SP_BM;
+    pl.n_nb = (N + 64 * tnf - 1) / (64 * tnf);
+    pl.stages = (K + SP_BK - 1) / SP_BK;
+    const int64_t tiles = pl.n_mb * pl.n_nb;
+    int64_t best = splits > 0 ? splits : 1;
+    if (splits <= 0) {
+        const double stage = np * 4 * tnf * 2 * 32 / 1.9e3;   // us
+        double least = 1e30;
+        for (int64_t s = 1; s <= 64 && s <= pl.stages; ++s) {
+            const int64_t per = (pl.stages + s - 1) / s;
+            const int64_t rounds = (tiles * s + cus - 1) / cus;
+            double us = static_cast<double>(rounds) * (per * stage + 8.0);
+            if (s > 1) us += 4.0 + static_cast<double>(s + 1) * M * N * 8 / 4.0e6;
+            if (us < least * 0.98) {
+                least = us;
+                best = s;
+            }
+        }
+    }
+    if (best > pl.stages) best = pl.stages;
+    pl.per_slice = (pl.stages + best - 1) / best;
+    pl.slices = (pl.stages + pl.per_slice - 1) / pl.per_slice;
+    return pl;
+}
+
+template <int NA, int NB, bool KSA, bool KSB>
+void launch_split(const SplitParams& p, int64_t blocks, hipStream_t st) {
+    constexpr int TNF = NA == 3 && NB == 3 ? 2 : 4;
+    hipLaunchKernelGGL((split_gemm_kernel<NA, NB, KSA, KSB, TNF>), dim3(static_cast<unsigned>(blocks)),
+                       dim3(SP_THREADS), 0, st, p);
+}
+
+// the head's products: logits (K_FAST, any pieces), hidden states' gradient
+// (K_FAST gradient x K_SLOW weight) and weight's (both K_SLOW), A in 3 pieces
+template <bool KSA, bool KSB>
+void launch_split_pieces(const SplitParams& p, int na, int nb, int64_t blocks, hipStream_t st) {
+    if (na == 3 && nb == 3) launch_split<3, 3, KSA, KSB>(p, blocks, st);
+    else if (na == 3) launch_split<3, 1, KSA, KSB>(p, blocks, st);
+    else if constexpr (!KSB) {
+        if (nb == 3) launch_split<1, 3, KSA, KSB>(p, blocks, st);
+        else launch_split<1, 1, KSA, KSB>(p, blocks, st);
+    }
+}
+
+int check_split_shape(int64_t M, int64_t N, int64_t K, int na, int nb) {
+    if (M < 0 || N < 0 || K < 0) return set_error(MOGT_E_INVALID, "split_gemm: negative size");
+    if (M > 0x3fffffff || N > 0x3fffffff || K > 0x3fffffff) return set_error(MOGT_E_INVALID, "split_gemm: size");
+    if ((na != 1 && na != 3) || (nb != 1 && nb != 3)) return set_error(MOGT_E_INVALID, "split_gemm: 1 or 3 pieces");
+    return MOGT_OK;
+}
+
+}  // namespace
+}  // namespace mogt
+
+using namespace mogt;
+
+extern "C" int mogt_split_pieces(const void* src, int64_t ld_src, void* dst, int64_t ld_dst, int64_t rows,
+                                 int64_t cols, void* stream) {
+    clear_error();
+    if (rows < 0 || cols < 0 || ld_src < cols || ld_dst < cols || ld_dst % 8 != 0)
+        return set_error(MOGT_E_INVALID, "split_pieces: bad shape or row stride");
+    if (rows == 0 || ld_dst == 0) return MOGT_OK;
+    if (!src || !dst) return set_error(MOGT_E_INVALID, "split_pieces: null pointer");
+    if (reinterpret_cast<uintptr_t>(dst) & 15) return set_error(MOGT_E_INVALID, "split_pieces: dst needs 16-byte alignment");
+    const int64_t groups = rows * (ld_dst / 4);
+    const int64_t blocks = (groups + 255) / 256 < 8192 ? (groups + 255) / 256 : 8192;
+    hipLaunchKernelGGL(split_pieces_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const float*>(src), ld_src,
+                       static_cast<bf16_t*>(dst), ld_dst, rows * ld_dst, rows, cols);
+    return check_launch("split_pieces_kernel");
+}
+
+extern "C" size_t mogt_split_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int pieces_a, int pieces_b,
+                                                  int64_t splits, int64_t cus) {
+    if (check_split_shape(M, N, K, pieces_a, pieces_b) != MOGT_OK || M == 0 || N == 0 || K == 0) return 0;
+    if (cus <= 0) {
+        int n = 0;
+        if (device_cu_count(n) != MOGT_OK) return 0;
+        cus = n;
+    }
+    // at most this many bytes whatever the output type (a bf16 output always
+    // goes through the partials)
+    return static_cast<size_t>(plan_split(M, N, K, pieces_a, pieces_b, splits, cus).slices) * M * ((N + 3) / 4 * 4) *
+           sizeof(float);
+}
+
+extern "C" int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int pieces_a, int k_slow_a, const void* B,
+                               int64_t ldb, int64_t plane_b, int pieces_b, int k_slow_b, void* C, int64_t ldc,
+                               int64_t M, int64_t N, int64_t K, int accumulate, int out_dtype, int64_t splits,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+    clear_error();
+    if (int rc = check_split_shape(M, N, K, pieces_a, pieces_b)) return rc;
+    if (out_dtype != MOGT_F32 && (out_dtype != MOGT_BF16 || accumulate))
+        return set_error(MOGT_E_INVALID, "split_gemm: fp32 output, or bf16 without accumulation");
+    if ((k_slow_a && !k_slow_b) || (k_slow_b && pieces_a != 3)) return set_error(MOGT_E_INVALID, "split_gemm: layout pair not built");
+    const int64_t Kp = (K + SP_BK - 1) / SP_BK * SP_BK, Np = (N + 3) / 4 * 4;
+    if (lda % 8 != 0 || ldb % 8 != 0 || plane_a % 8 != 0 || plane_b % 8 != 0 || ldc % 4 != 0 || ldc < Np ||
+        lda < (k_slow_a ? M : Kp) || ldb < (k_slow_b ? N : Kp))
+        return set_error(MOGT_E_INVALID, "split_gemm: row strides must cover the (padded) rows, multiples of 8 (C: 4)");
+    if (M == 0 || N == 0) return MOGT_OK;
+    if (K == 0) return set_error(MOGT_E_INVALID, "split_gemm: empty contraction");
+    if (!A || !B || !C) return set_error(MOGT_E_INVALID, "split_gemm: null pointer");
+    if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) & 15)
+        return set_error(MOGT_E_INVALID, "split_gemm: A, B and C need 16-byte alignment");
+    // byte offsets within a block's descriptor are 32-bit
+    const int64_t spanA = (k_slow_a ? (Kp + SP_BK) : SP_BM) * lda * 2, spanB = (k_slow_b ? (Kp + SP_BK) : 256) * ldb * 2;
+    if (spanA >= (int64_t(1) << 31) || spanB >= (int64_t(1) << 31))
+        return set_error(MOGT_E_INVALID, "split_gemm: operand block exceeds 2 GiB");
+    int cus = 0;
+    if (int rc = device_cu_count(cus)) return rc;
+    const SplitPlan pl = plan_split(M, N, K, pieces_a, pieces_b, splits, cus);
+    const int64_t blocks = pl.n_mb * pl.n_nb * pl.slices;
+    if (blocks > 0x7fffffff) return set_error(MOGT_E_INVALID, "split_gemm: too many tiles");
+    const bool parts = pl.slices > 1 || out_dtype == MOGT_BF16;
+    if (parts) {
+        const size_t need = static_cast<size_t>(pl.slices) * M * Np * sizeof(float);
+        if (!workspace || workspace_bytes < need)
+            return set_error(MOGT_E_WORKSPACE, "split_gemm: workspace of %zu bytes needed, %zu given", need,
+                             workspace_bytes);
+        if (reinterpret_cast<uintptr_t>(workspace) & 15)
+            return set_error(MOGT_E_INVALID, "split_gemm: workspace needs 16-byte alignment");
+    }
+    SplitParams p{};
+    p.a = static_cast<const bf16_t*>(A);
+    p.b = static_cast<const bf16_t*>(B);
+    p.out = static_cast<float*>(parts ? workspace : C);
+    p.lda = lda;
+    p.ldb = ldb;
+    p.ldo = parts ? Np : ldc;
+    p.pa = plane_a;
+    p.pb = plane_b;
+    p.po = M * Np;
+    p.M = static_cast<int>(M);
+    p.N = static_cast<int>(Np);
+    p.K = static_cast<int>(K);
+    p.nb_valid = static_cast<int>(N);
+    p.n_mb = static_cast<int>(pl.n_mb);
+    p.n_nb = static_cast<int>(pl.n_nb);
+    p.stages = static_cast<int>(pl.stages);
+    p.per_slice = static_cast<int>(pl.per_slice);
+    p.accumulate = !parts && accumulate;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (k_slow_a) launch_split_pieces<true, true>(p, pieces_a, pieces_b, blocks, st);
+    else if (k_slow_b) launch_split_pieces<false, true>(p, pieces_a, pieces_b, blocks, st);
+    else launch_split_pieces<false, false>(p, pieces_a, pieces_b, blocks, st);
+    int rc = check_launch("split_gemm_kernel");
+    if (rc != MOGT_OK || !parts) return rc;
+    const int64_t groups = M * (Np / 4);
+    const dim3 rb(static_cast<unsigned>((groups + 255) / 256 < 8192 ? (groups + 255) / 256 : 8192));
+    if (out_dtype == MOGT_BF16)
+        hipLaunchKernelGGL(split_reduce_kernel<true>, rb, dim3(256), 0, st, static_cast<const float*>(workspace), C, ldc,
+                           static_cast<int>(pl.slices), p.M, p.N, 0);
+    else
+        hipLaunchKernelGGL(split_reduce_kernel<false>, rb, dim3(256), 0, st, static_cast<const float*>(workspace), C,
+                           ldc, static_cast<int>(pl.slices), p.M, p.N, accumulate);
+    return check_launch("split_reduce_kernel");
+}

@@ -2000,3 +2000,119 @@ def lm_ce_backward_(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Tenso
         raise ValueError("lm_ce_backward_: scale must be a one-element float32 tensor on the logits' device")
     torch.ops.mogt.lm_ce_bwd_(logits, labels, lse, scale.reshape(1).contiguous(), int(ignore_index))
     return logits
+
+
+def _lm_ce_grad_pieces_impl(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Tensor, scale: torch.Tensor,
+                          ignore_index: int) -> torch.Tensor:
+    lib = _lib.load()
+    labels = labels.contiguous()
+    lse = lse.contiguous()
+    rows, vocab = logits.shape
+    grad = torch.empty((3, rows, split_pad(vocab)), dtype=torch.bfloat16, device=logits.device)
+    rc = lib.mogt_lm_ce_bwd_pieces(logits.data_ptr(), logits.stride(0), dtype_code(logits.dtype, "lm_ce_grad_pieces"),
+                                   labels.data_ptr(), lse.data_ptr(), rows, vocab, int(ignore_index),
+                                   scale.data_ptr(), grad.data_ptr(), grad.stride(1), _stream_handle(logits.device))
+    _lib.check(rc, "mogt_lm_ce_bwd_pieces")
+    return grad
+
+
+_lm_ce_grad_pieces_op = torch.library.custom_op("mogt::lm_ce_grad_pieces", _lm_ce_grad_pieces_impl, mutates_args=())
+
+
+@_lm_ce_grad_pieces_op.register_fake
+def _(logits, labels, lse, scale, ignore_index):
+    return logits.new_empty((3, logits.shape[0], split_pad(logits.shape[1])), dtype=torch.bfloat16)
+
+
+def lm_ce_grad_pieces(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Tensor, scale: torch.Tensor, *,
+                      ignore_index: int = -100) -> torch.Tensor:
+    """``lm_ce_grad``'s fp32 block as three bf16 pieces ``[3, rows, vocab padded
+    to a multiple of 32]`` (``split_gemm``'s operand; the padding is zero)."""
+    _check_ce_rows(logits, labels, "lm_ce_grad_pieces")
+    if lse.shape != labels.shape or lse.dtype != torch.float32:
+        raise ValueError("lm_ce_grad_pieces: lse must be float32 [rows]")
+    if scale.numel() != 1 or scale.dtype != torch.float32 or scale.device != logits.device:
+        raise ValueError("lm_ce_grad_pieces: scale must be a one-element float32 tensor on the logits' device")
+    scale = scale.reshape(1).contiguous()
+    if _direct(logits, labels, lse, scale):
+        return _lm_ce_grad_pieces_impl(logits, labels, lse, scale, int(ignore_index))
+    return torch.ops.mogt.lm_ce_grad_pieces(logits, labels, lse, scale, int(ignore_index))
+
+
+# ---------------------------------------------------------------------------
+# fp32 products from bf16 pieces (csrc/split_gemm.hip)
+# ---------------------------------------------------------------------------
+SPLIT_K = 32   # the contraction is padded to whole stages of this many
+
+
+def split_pad(n: int) -> int:
+    return -(-n // SPLIT_K) * SPLIT_K
+
+
+def _split_pieces_impl(x: torch.Tensor) -> torch.Tensor:
+    lib = _lib.load()
+    x = x if x.stride(1) == 1 else x.contiguous()
+    rows, cols = x.shape
+    out = torch.empty((3, rows, split_pad(cols)), dtype=torch.bfloat16, device=x.device)
+    rc = lib.mogt_split_pieces(x.data_ptr(), x.stride(0) if rows > 1 else cols, out.data_ptr(), out.stride(1), rows,
+                               cols, _stream_handle(x.device))
+    _lib.check(rc, "mogt_split_pieces")
+    return out
+
+
+_split_pieces_op = torch.library.custom_op("mogt::split_pieces", _split_pieces_impl, mutates_args=())
+
+
+@_split_pieces_op.register_fake
+def _(x):
+    return x.new_empty((3, x.shape[0], split_pad(x.shape[1])), dtype=torch.bfloat16)
+
+
+def split_pieces(x: torch.Tensor) -> torch.Tensor:
+    """fp32 ``x [rows, cols]`` as bf16 pieces ``[3, rows, cols padded to a
+    multiple of 32]`` whose sum is ``x`` (zero padding)."""
+    require_cuda("split_pieces", x)
+    if x.ndim != 2 or x.dtype != torch.float32:
+        raise ValueError("split_pieces: x must be float32 [rows, cols]")
+    return _split_pieces_impl(x) if _direct(x) else torch.ops.mogt.split_pieces(x)
+
+
+def _split_gemm_impl(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, k: int, k_slow_a: bool, k_slow_b: bool,
+                   accumulate: bool) -> None:
+    lib = _lib.load()
+    M, N = out.shape
+    nbytes = int(lib.mogt_split_gemm_workspace_bytes(M, N, k, a.shape[0], b.shape[0], 0, 0))
+    ws = workspace(nbytes, out.device)
+    rc = lib.mogt_split_gemm(a.data_ptr(), a.stride(1), a.stride(0), a.shape[0], int(k_slow_a), b.data_ptr(),
+                             b.stride(1), b.stride(0), b.shape[0], int(k_slow_b), out.data_ptr(), out.stride(0), M, N,
+                             k, int(accumulate), dtype_code(out.dtype, "split_gemm"), 0, ws.data_ptr(), ws.numel(),
+                             _stream_handle(out.device))
+    _lib.check(rc, "mogt_split_gemm")
+
+
+_split_gemm_op = torch.library.custom_op("mogt::split_gemm_", _split_gemm_impl, mutates_args=("out",))
+
+
+@_split_gemm_op.register_fake
+def _(out, a, b, k, k_slow_a, k_slow_b, accumulate):
+    return None
+
+
+def split_gemm_(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, k: int, *, k_slow_a: bool = False,
+                k_slow_b: bool = False, accumulate: bool = False) -> torch.Tensor:
+    """``out[m, n] (+)= sum_k A(m, k) B(n, k)`` with fp32 accumulation, each
+    operand the sum of its bf16 pieces: ``[pieces, rows, K padded to 32]`` or,
+    ``k_slow``, ``[pieces, K, rows]`` (1 or 3 pieces).  ``out`` float32, or
+    bfloat16 without ``accumulate``; its row stride covers N rounded up to 4."""
+    require_cuda("split_gemm", out, a, b)
+    for t, slow, rows in ((a, k_slow_a, out.shape[0]), (b, k_slow_b, out.shape[1])):
+        shape_ok = t.ndim == 3 and t.dtype == torch.bfloat16 and t.stride(2) == 1 and t.shape[0] in (1, 3)
+        if not shape_ok or (t.shape[1:] != (k, rows) if slow else t.shape[1] != rows or t.shape[2] != split_pad(k)):
+            if not (shape_ok and slow and t.shape[1] == k and t.shape[2] >= rows):
+                raise ValueError("split_gemm: operands must be bf16 pieces [1 or 3, rows, K padded to 32] or "
+                                 "[1 or 3, K, rows]")
+    if out.ndim != 2 or out.stride(1) != 1:
+        raise ValueError("split_gemm: out must be [M, N] with contiguous rows")
+    run = _split_gemm_impl if _direct(out, a, b) else torch.ops.mogt.split_gemm_
+    run(out, a, b, int(k), bool(k_slow_a), bool(k_slow_b), bool(accumulate))
+    return out

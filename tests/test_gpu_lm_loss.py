@@ -189,3 +189,131 @@ def test_model_chunked_loss_paths(gpu):
     for k, p in model.named_parameters():
         if k in g0:
             assert rel_err(to_np(p.grad), to_np(g0[k])) <= E2E_TOL, k
+
+
+def _bf16_or_f32(shape, dtype, seed, std=1.0):
+    return (torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * std).to(dtype)
+
+
+def _pieces_of(x):
+    from mogt_amd import ops
+
+    return x.unsqueeze(0).contiguous() if x.dtype == torch.bfloat16 else ops.split_pieces(x)
+
+
+def test_split_pieces_sum_is_exact(gpu):
+    """x1 + x2 + x3 == x for every exponent that leaves the last piece normal,
+    zero padding, strided rows; non-finite values and the largest floats whole
+    in the first piece."""
+    announce("split pieces")
+    from mogt_amd import ops
+
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(37, 70, generator=g) * torch.exp2(torch.randint(-60, 60, (37, 70), generator=g).float())
+    x[0, :6] = torch.tensor([0.0, -0.0, 3.4028235e38, -3.4028235e38, 1.0, 2.0 ** -30])
+    p = ops.split_pieces(x.to(gpu)[:, 1:66])
+    assert p.shape == (3, 37, 96) and float(p[:, :, 65:].float().abs().sum()) == 0.0
+    assert torch.equal(p.double().sum(0)[:, :65].cpu(), x[:, 1:66].double())
+    bad = torch.tensor([[float("inf"), float("-inf"), float("nan"), 1.0]], device=gpu)
+    q = ops.split_pieces(bad).float().cpu()
+    assert torch.equal(q[0, 0, :2], bad[0, :2].cpu()) and torch.isnan(q[0, 0, 2])
+    assert float(q[1:, 0, :4].abs().sum()) == 0.0
+
+
+SPLIT_DT = [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16),
+            (torch.float32, torch.float32)]
+
+
+@pytest.mark.parametrize("da,db", SPLIT_DT)
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (255, 257, 64), (256, 256, 96), (300, 129, 160), (513, 1001, 768)])
+def test_split_gemm_logits_form(gpu, M, N, K, da, db):
+    """One to 24 stages, ragged row and column tiles, every piece pair, and the
+    accumulating output: within the elementwise bound (K + 8) 2^-24 sum |a b|
+    that an fp32 sum of the products has in any order."""
+    announce(f"split gemm nt {M} {N} {K} {da} {db}")
+    from mogt_amd import ops
+
+    a, b = _bf16_or_f32((M, K), da, 1).to(gpu), _bf16_or_f32((N, K), db, 2).to(gpu)
+    out = torch.full((M, -(-N // 4) * 4), 7.0, device=gpu)[:, :N]
+    ops.split_gemm_(out, _pieces_of(a), _pieces_of(b), K)
+    ref = a.double() @ b.double().t()
+    bound = (K + 8) * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t())
+    assert bool(((out.double() - ref).abs() <= bound).all())
+    ops.split_gemm_(out, _pieces_of(a), _pieces_of(b), K, accumulate=True)
+    assert bool(((out.double() - 2 * ref).abs() <= 3 * bound).all())
+
+
+@pytest.mark.parametrize("db", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,V,D", [(1, 33, 32), (37, 1001, 64), (300, 4096, 96), (257, 10007, 256)])
+def test_split_gemm_gradient_forms(gpu, n, V, D, db):
+    """The hidden states' gradient (contraction over the vocabulary, ragged, the
+    weight K-slow, K slices) and the weight's (both K-slow, contraction over
+    the rows), odd sizes included (the last column of a K-slow row is a half
+    dword); fp32 and bf16 outputs, run to run equal."""
+    announce(f"split gemm gradients {n} {V} {D} {db}")
+    from mogt_amd import ops
+
+    g = _bf16_or_f32((n, V), torch.float32, 5).to(gpu)
+    x = _bf16_or_f32((V, D), db, 6).to(gpu)
+    gp = ops.split_pieces(g)
+    dh = torch.empty(n, D, device=gpu)
+    ops.split_gemm_(dh, gp, _pieces_of(x), V, k_slow_b=True)
+    ref = g.double() @ x.double()
+    bound = (V + 8) * 2.0 ** -24 * (g.double().abs() @ x.double().abs())
+    assert bool(((dh.double() - ref).abs() <= bound).all())
+    half = torch.empty(n, D, device=gpu, dtype=torch.bfloat16)
+    ops.split_gemm_(half, gp, _pieces_of(x), V, k_slow_b=True)
+    assert torch.equal(half, dh.to(torch.bfloat16))
+    h = _bf16_or_f32((n, D), db, 7).to(gpu)
+    dw = torch.zeros(V, D, device=gpu)
+    ops.split_gemm_(dw, gp, _pieces_of(h), n, k_slow_a=True, k_slow_b=True, accumulate=True)
+    ref = g.double().t() @ h.double()
+    bound = (n + 8) * 2.0 ** -24 * (g.double().abs().t() @ h.double().abs())
+    assert bool(((dw.double() - ref).abs() <= bound).all())
+    again = torch.empty(V, D, device=gpu)
+    ops.split_gemm_(again, gp, _pieces_of(h), n, k_slow_a=True, k_slow_b=True)
+    assert torch.equal(again, dw)
+
+
+@pytest.mark.parametrize("rows,vocab,dtype,pad", [(3, 7, torch.float32, 0), (64, 129, torch.float32, 3),
+                                                  (40, 50257, torch.bfloat16, 5), (33, 4000, torch.bfloat16, 0)])
+def test_ce_gradient_pieces_equal_the_block(gpu, rows, vocab, dtype, pad):
+    """The pieces sum to lm_ce_grad's fp32 block bit for bit, padding zero."""
+    announce(f"ce gradient pieces {rows} {vocab} {dtype} {pad}")
+    from mogt_amd import ops
+
+    x = _logits(rows, vocab, dtype, gpu, seed=vocab, pad=pad)
+    lab = _labels(rows, vocab, gpu, seed=rows, ignore_every=5)
+    _, lse = ops.lm_ce_forward(x, lab)
+    scale = torch.tensor([0.37], device=gpu)
+    g = ops.lm_ce_grad(x, lab, lse, scale)
+    p = ops.lm_ce_grad_pieces(x, lab, lse, scale)
+    total = p.double().sum(0)
+    # below 2^-110 the last piece leaves bf16's normal range
+    assert bool(((total[:, :vocab] - g.double()).abs() <= 2.0 ** -133).all())
+    assert float(p[:, :, vocab:].float().abs().sum()) == 0.0
+
+
+@pytest.mark.parametrize("hd,wd,autocast", [(torch.float32, torch.float32, False), (torch.bfloat16, torch.float32, False),
+                                            (torch.float32, torch.bfloat16, False), (torch.float32, torch.float32, True)])
+def test_chunked_linear_ce_split_form_matches_library_form(gpu, monkeypatch, hd, wd, autocast):
+    """Loss and gradients of the split form against the library form of the same
+    call: ragged last chunk, odd vocabulary, ignored labels."""
+    announce(f"chunked CE split form {hd} {wd} {autocast}")
+    from mogt_amd import chunked_lm_loss as cl
+
+    h = _bf16_or_f32((2, 150, 64), hd, 11).to(gpu).requires_grad_()
+    w = _bf16_or_f32((1003, 64), wd, 12, 0.3).to(gpu).requires_grad_()
+    lab = _labels(300, 1003, gpu, seed=13, ignore_every=7).view(2, 150)
+
+    def call():
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            loss = cl.chunked_linear_cross_entropy(h, w, lab, chunk_size=128)
+        return [loss.detach(), *torch.autograd.grad(loss, [h, w])]
+
+    lib = call()
+    monkeypatch.setattr(cl, "SPLIT_MIN_MACS", 0)
+    for got, ref, what in zip(call(), lib, ("loss", "dh", "dw")):
+        assert got.dtype == ref.dtype and got.shape == ref.shape
+        # both fp32 sums in other orders; bf16 gradients one rounding apart
+        assert rel_err(to_np(got), to_np(ref)) <= (1e-5 if got.dtype == torch.float32 else 2.0 ** -8), what

@@ -352,7 +352,7 @@ def test_checked_mode_reports_each_give_up_once(monkeypatch):
         ops._checked(ws, "scan")                  # one more
 
 
-@pytest.mark.parametrize("source", ["swiglu_gemm.hip", "wgrad_gemm.hip", "rank1_scan.hip"])
+@pytest.mark.parametrize("source", ["swiglu_gemm.hip", "wgrad_gemm.hip", "rank1_scan.hip", "split_gemm.hip"])
 def test_gemm_m0_only_feeds_lds_dma(tmp_path, source):
     """The bf16 GEMMs (fused SwiGLU, split-K weight gradient) and the rank-1
     scan's carry exchange set m0 in inline assembly for their direct-to-LDS
