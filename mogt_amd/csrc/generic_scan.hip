@@ -3,28 +3,30 @@
 // state_dtype argument, affine_scan.py:14-62, :127-172, :175-278).
 //
 // The MFMA pipeline of dense_scan.hip covers the model's shapes (R <= 32, fp32 state).
-// This kernel covers everything else the reference's functions accept: a float64 state
+// This file covers everything else the reference's functions accept: a float64 state
 // (the reference's own sanity check runs in float64, sanity_affine_scan.py:19-61), ranks
-// above 32, fp16 / fp64 inputs and outputs.  It is a latency-bound scalar kernel, not a
-// matrix-core one: every state element is one thread's running dot product over the R
-// rows of the previous state, with the state in LDS.
+// above 32, fp16 / fp64 inputs and outputs.  Ranks up to 64 run on the matrix-core chunk
+// kernel of generic_mfma.h; above (or where a step's block exceeds its 32-bit offsets) on
+// the scalar kernel below: every state element is one thread's running dot product over
+// the R rows of the previous state, with the state in LDS.
 //
 // The prefix product U_prefix_t = U_t ... U_1 (return_prefix=True, affine_scan.py:43-55)
 // is the same recurrence applied to R extra state columns that start at the identity and
 // take no input, so one augmented state [H | U_prefix] of width C + R serves both.
 //
-// Three passes over chunks of `seg` steps (seg ~ sqrt(L)):
+// Three passes over chunks of `seg` steps (generic_geometry):
 //   LOCAL   per chunk, from [0 | I]: the chunk's end state [E_j | P_j] (E_j: the
 //           chunk's own contribution, P_j: the product of its transitions);
-//   CARRY   per batch row, sequentially over chunks: M_in(j+1) = P_j M_in(j) + [E_j | 0],
-//           M_in(0) = [0 | I] (the carry recursion of affine_scan.py:175-278);
+//   CARRY   M_in(j+1) = P_j M_in(j) + [E_j | 0], M_in(0) = [0 | I] (the carry recursion of
+//           affine_scan.py:175-278): the same scan over the chunk summaries, in one pass or,
+//           where that would be the longer chain, through these three passes once more;
 //   OUTPUT  per chunk, from M_in(j): every step's state, written as H and U_prefix.
 // One pass (OUTPUT from [0 | I]) when the whole sequence is one chunk.
 //
 // Reverse mode (the backward's total-gradient recursion, affine_scan.py:110-118):
 // G_t = X_t + U_{t+1}^T G_{t+1}: position q of the scan is time L-1-q, its transition is
 // U_{L-q}^T (the identity at q = 0, where the state is still zero).
-#include "common.h"
+#include "generic_mfma.h"
 
 namespace mogt {
 namespace {
@@ -33,65 +35,6 @@ constexpr int GS_THREADS = 256;
 constexpr int GS_EPT = 4;                          // state elements per thread
 constexpr int GS_MAX_ELEMS = GS_THREADS * GS_EPT;  // R * column-tile width
 constexpr int GS_MAX_R = 1024;
-constexpr int GS_ULDS_MAX_R = 64;                  // transitions staged in LDS up to this rank
-
-// A [batch][sequence][rows][cols] view of a device buffer (strides in elements).
-struct GView {
-    void* p;
-    int64_t bs, ss, rs;
-    int code;
-};
-
-struct GParams {
-    GView tr;        // transitions, state dtype; column offset tr_c0
-    GView in;        // inputs, columns [0, cin)
-    GView init;      // initial state per (batch, chunk), state dtype; p == nullptr: [0 | I]
-    GView out_h;     // state columns [0, csplit)
-    GView out_p;     // state columns [csplit, W), written at column c - csplit (p may be null)
-    int64_t L;       // positions in the scanned sequence
-    int64_t seg;     // positions per chunk (one work-group's run)
-    int nseg, ntile;
-    int R, W, Cb;    // rank, state width, column-tile width
-    int tr_c0, cin, cid, csplit;  // cid: first identity column of the [0 | I] start
-    int every;       // 1: write the state after every step; 0: the final state at the chunk index
-    int shift;       // 1: step q is written at index q + 1 and the initial state at index 0
-    int rev;         // reverse, transposed transitions (see the file comment)
-};
-
-__device__ __forceinline__ int64_t at(const GView& v, int64_t b, int64_t s, int64_t r, int64_t c) {
-    return b * v.bs + s * v.ss + r * v.rs + c;
-}
-
-template <typename TS>
-__device__ __forceinline__ TS ld_code(const void* p, int64_t i, int code) {
-    if (code == MOGT_F64) return static_cast<TS>(static_cast<const double*>(p)[i]);
-    if (code == MOGT_BF16) return static_cast<TS>(bf16_to_f32(static_cast<const bf16_t*>(p)[i]));
-    if (code == MOGT_F16) return static_cast<TS>(static_cast<float>(static_cast<const _Float16*>(p)[i]));
-    return static_cast<TS>(static_cast<const float*>(p)[i]);
-}
-
-// Narrow outputs round from the state through fp32 (round to nearest even at each step),
-// as a torch float64 -> bfloat16 / float16 conversion does.
-template <typename TS>
-__device__ __forceinline__ void st_code(void* p, int64_t i, int code, TS x) {
-    if (code == MOGT_F64) {
-        static_cast<double*>(p)[i] = static_cast<double>(x);
-        return;
-    }
-    const float f = static_cast<float>(x);
-    if (code == MOGT_BF16) static_cast<bf16_t*>(p)[i] = f32_to_bf16(f);
-    else if (code == MOGT_F16) static_cast<_Float16*>(p)[i] = static_cast<_Float16>(f);
-    else static_cast<float*>(p)[i] = f;
-}
-
-template <typename TS>
-__device__ __forceinline__ void put(const GParams& p, int64_t b, int64_t idx, int i, int c, TS x) {
-    if (c < p.csplit) {
-        st_code<TS>(p.out_h.p, at(p.out_h, b, idx, i, c), p.out_h.code, x);
-    } else if (p.out_p.p) {
-        st_code<TS>(p.out_p.p, at(p.out_p, b, idx, i, c - p.csplit), p.out_p.code, x);
-    }
-}
 
 // Row length in LDS of the staged transition and of a state column: R rounded
 // up to 16 bytes, plus 16 bytes of skew between rows.
@@ -101,22 +44,17 @@ __host__ __device__ constexpr int gs_ld(int R) {
                static_cast<int>(16 / sizeof(TS)) + static_cast<int>(16 / sizeof(TS));
 }
 
-// ULDS: the step's transition staged through LDS (R <= 64), UPT of its values
-// per thread; PD: steps of operands in flight.
-template <typename TS, bool ULDS, int UPT, int PD, int RM = 0>
+// PD: steps of inputs in flight; the threads read their rows of U_t from memory.
+template <typename TS, int PD>
 __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_scan_kernel(GParams p) {
     extern __shared__ __align__(16) unsigned char gs_smem[];
-    // LDS: the step's transition U [R][ld] (staged variant) then two state
-    // buffers stored column-major, [Cb][ld]; ld = R rounded up to 16 bytes plus
-    // 16 bytes of skew, so a thread reads 16 bytes of a U row or of its state
-    // column per instruction.  Padding columns / rows stay zero.
-    constexpr int VE = 16 / sizeof(TS);
+    // LDS: two state buffers stored column-major, [Cb][ld]; ld = R rounded up to
+    // 16 bytes plus 16 bytes of skew.  Padding columns / rows stay zero.
     const int R = p.R, Cb = p.Cb, RCb = R * Cb;
     const int ld = gs_ld<TS>(R);
-    TS* sU = reinterpret_cast<TS*>(gs_smem);
-    TS* sS = sU + (ULDS ? R * ld : 0);
-    const int lds_elems = (ULDS ? R * ld : 0) + 2 * Cb * ld;
-    for (int e = threadIdx.x; e < lds_elems; e += GS_THREADS) sU[e] = TS(0);
+    TS* sS = reinterpret_cast<TS*>(gs_smem);
+    const int lds_elems = 2 * Cb * ld;
+    for (int e = threadIdx.x; e < lds_elems; e += GS_THREADS) sS[e] = TS(0);
     __syncthreads();
 
     const int tid = threadIdx.x;
@@ -148,7 +86,7 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
         if (ok[m]) {
             if (p.init.p) v0 = ld_code<TS>(p.init.p, at(p.init, b, j, oi[m], oc[m]), p.init.code);
             else if (oc[m] >= p.cid) v0 = (oi[m] == oc[m] - p.cid) ? TS(1) : TS(0);
-            if (p.shift) put<TS>(p, b, 0, oi[m], oc[m], v0);
+            if (p.shift && j == 0) put<TS>(p, b, 0, oi[m], oc[m], v0);
         }
         acc[m] = v0;
         if (own[m]) sS[ocl[m] * ld + oi[m]] = v0;
@@ -157,22 +95,8 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
     // Operands of the next PD steps are in flight: slot pp of the ring holds
     // step s0 + pp of the current round and is refilled with step s0 + pp + PD
     // once its values have been consumed.
-    TS ureg[PD][ULDS ? UPT : 1];
     TS vreg[PD][GS_EPT];
-    auto fetch = [&](int64_t q, TS (&u)[ULDS ? UPT : 1], TS (&v)[GS_EPT]) {
-        if constexpr (ULDS) {
-            const bool ident = p.rev && q == 0;
-            const int64_t tt = p.rev ? p.L - q : q;
-#pragma unroll
-            for (int m = 0; m < UPT; ++m) {
-                const int idx = tid + m * GS_THREADS;
-                if (idx < R * R) {
-                    const int rr = idx / R, cc = idx - rr * R;
-                    u[m] = ident ? TS(rr == cc ? 1 : 0)
-                                 : static_cast<const TS*>(p.tr.p)[at(p.tr, b, tt, rr, p.tr_c0 + cc)];
-                }
-            }
-        }
+    auto fetch = [&](int64_t q, TS (&v)[GS_EPT]) {
         const int64_t ti = p.rev ? p.L - 1 - q : q;
 #pragma unroll
         for (int m = 0; m < GS_EPT; ++m)
@@ -182,29 +106,16 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
 
 #pragma unroll
     for (int pp = 0; pp < PD; ++pp)
-        if (pp < n) fetch(q0 + pp, ureg[pp], vreg[pp]);
+        if (pp < n) fetch(q0 + pp, vreg[pp]);
     __syncthreads();
     int cur = 0;
-    // one step: slot (u, v) holds step s; refilled with step s + PD
-    auto step = [&](int64_t s, TS (&u)[ULDS ? UPT : 1], TS (&v)[GS_EPT]) {
+    // one step: slot v holds step s; refilled with step s + PD
+    auto step = [&](int64_t s, TS (&v)[GS_EPT]) {
         const int64_t q = q0 + s;
-        if constexpr (ULDS) {
-#pragma unroll
-            for (int m = 0; m < UPT; ++m) {
-                const int idx = tid + m * GS_THREADS;
-                if (idx < R * R) {
-                    const int rr = idx / R, cc = idx - rr * R;
-                    // stored as the transition itself: row i, column k
-                    if (p.rev) sU[cc * ld + rr] = u[m];
-                    else sU[rr * ld + cc] = u[m];
-                }
-            }
-        }
         TS vin[GS_EPT];
 #pragma unroll
         for (int m = 0; m < GS_EPT; ++m) vin[m] = v[m];
-        if (s + PD < n) fetch(q + PD, u, v);   // later steps' loads overlap this step's arithmetic
-        if constexpr (ULDS) __syncthreads();
+        if (s + PD < n) fetch(q + PD, v);   // later steps' loads overlap this step's arithmetic
 
         const TS* Sc = sS + cur * Cb * ld;
         TS* Sn = sS + (cur ^ 1) * Cb * ld;
@@ -220,27 +131,6 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
         if (ident) {
 #pragma unroll
             for (int m = 0; m < GS_EPT; ++m) a[m] += scol[oi[m]];
-        } else if constexpr (ULDS) {
-            typedef TS vec_t __attribute__((ext_vector_type(VE)));
-            auto kstep = [&](int k) {
-                const vec_t sv = *reinterpret_cast<const vec_t*>(scol + k);
-#pragma unroll
-                for (int m = 0; m < GS_EPT; ++m) {
-                    const vec_t uv = *reinterpret_cast<const vec_t*>(sU + oi[m] * ld + k);
-#pragma unroll
-                    for (int e = 0; e < VE; ++e) a[m] += uv[e] * sv[e];
-                }
-            };
-            if constexpr (RM > 0) {
-                // rank bounded at compile time: the whole contraction unrolled,
-                // its LDS reads issued together
-#pragma unroll
-                for (int k = 0; k < RM; k += VE)
-                    if (k < R) kstep(k);
-            } else {
-#pragma unroll 2
-                for (int k = 0; k < R; k += VE) kstep(k);
-            }
         } else {
             const TS* ut = static_cast<const TS*>(p.tr.p);
             for (int k = 0; k < R; ++k) {
@@ -263,15 +153,11 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
         __syncthreads();
         cur ^= 1;
     };
-    if constexpr (PD == 1) {
-        for (int64_t s = 0; s < n; ++s) step(s, ureg[0], vreg[0]);
-    } else {
-        for (int64_t s0 = 0; s0 < n; s0 += PD) {
+    for (int64_t s0 = 0; s0 < n; s0 += PD) {
 #pragma unroll
-            for (int pp = 0; pp < PD; ++pp) {
-                if (s0 + pp >= n) break;   // uniform over the work-group
-                step(s0 + pp, ureg[pp], vreg[pp]);
-            }
+        for (int pp = 0; pp < PD; ++pp) {
+            if (s0 + pp >= n) break;   // uniform over the work-group
+            step(s0 + pp, vreg[pp]);
         }
     }
     if (!p.every) {
@@ -281,29 +167,43 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
     }
 }
 
+// Level 0 is the sequence itself; a level above scans the chunk summaries of
+// the one below (the carries).  Two levels above at most: the top one is one
+// chunk per sequence.
+constexpr int GS_LEVELS = 2;
+
 struct GGeo {
-    int64_t seg, nch;
+    int64_t seg[GS_LEVELS], nch[GS_LEVELS];   // steps per chunk, chunks
+    int levels;                               // levels cut into more than one chunk
     int Wl, Wo;          // LOCAL state width (C + R), OUTPUT / CARRY width (C + R if prefix)
-    size_t s_off, m_off, bytes;
+    size_t s_off[GS_LEVELS], m_off[GS_LEVELS], bytes;
 };
 
 size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 GGeo generic_geometry(int64_t B, int64_t L, int64_t R, int64_t C, int with_prefix, int state_code) {
     GGeo g{};
-    g.seg = 16;
-    while (g.seg * g.seg < L && g.seg < 1024) g.seg *= 2;
-    g.nch = (L + g.seg - 1) / g.seg;
     g.Wl = static_cast<int>(C + R);
     g.Wo = static_cast<int>(C + (with_prefix ? R : 0));
     const size_t ts = state_code == MOGT_F64 ? 8 : 4;
-    g.s_off = 0;
-    g.m_off = 0;
+    const bool mfma = gm_fits(R, C);
     g.bytes = WS_HDR_BYTES;
-    if (g.nch > 1) {
-        g.s_off = WS_HDR_BYTES;
-        g.m_off = g.s_off + align256(static_cast<size_t>(B * g.nch * R * g.Wl) * ts);
-        g.bytes = g.m_off + align256(static_cast<size_t>(B * g.nch * R * g.Wo) * ts);
+    int64_t len = L;
+    for (int l = 0; l < GS_LEVELS; ++l) {
+        if (mfma) {
+            g.seg[l] = gm_segment(B, len, R, C, g.Wo, state_code == MOGT_F64);
+        } else {
+            if (l > 0) break;   // the scalar kernel's carries: one pass
+            g.seg[l] = 16;
+            while (g.seg[l] * g.seg[l] < len && g.seg[l] < 1024) g.seg[l] *= 2;
+        }
+        g.nch[l] = (len + g.seg[l] - 1) / g.seg[l];
+        if (g.nch[l] <= 1) break;
+        g.levels = l + 1;
+        g.s_off[l] = g.bytes;
+        g.m_off[l] = g.s_off[l] + align256(static_cast<size_t>(B * g.nch[l] * R * g.Wl) * ts);
+        g.bytes = g.m_off[l] + align256(static_cast<size_t>(B * g.nch[l] * R * g.Wo) * ts);
+        len = g.nch[l] - 1;   // the last chunk's summary is not needed
     }
     return g;
 }
@@ -318,30 +218,54 @@ int tile_width(int R, int W) {
 
 template <typename TS>
 int launch_generic(GParams p, int64_t batch, hipStream_t st, const char* what) {
+    if (gm_fits(p.R, p.W - p.R > 0 ? p.W - p.R : 0) && p.tr.rs * p.R * 8 <= GM_MAX_BLOCK)
+        return generic_mfma_launch<TS>(p, batch, st);   // rank <= 64
     p.Cb = tile_width(p.R, p.W);
     p.ntile = (p.W + p.Cb - 1) / p.Cb;
     const int64_t blocks = batch * p.nseg * p.ntile;
     if (blocks <= 0) return MOGT_OK;
     if (blocks > 0x7fffffffLL) return set_error(MOGT_E_INVALID, "%s: problem too large for one launch", what);
-    const bool ulds = p.R <= GS_ULDS_MAX_R;
-    const int ld = gs_ld<TS>(p.R);
-    const size_t lds = (static_cast<size_t>(ulds ? p.R * ld : 0) + 2 * static_cast<size_t>(p.Cb) * ld) * sizeof(TS);
-    const dim3 grid(static_cast<unsigned>(blocks)), block(GS_THREADS);
-    // transitions staged per thread: R^2 / 256 values (1, 4 or 16); the
-    // shallower the stash, the more steps in flight
-    if (p.R <= 16)
-        hipLaunchKernelGGL((generic_scan_kernel<TS, true, 1, 4, 16>), grid, block, lds, st, p);
-    else if (p.R <= 32)
-        hipLaunchKernelGGL((generic_scan_kernel<TS, true, 4, 4>), grid, block, lds, st, p);
-    else if (ulds)
-        hipLaunchKernelGGL((generic_scan_kernel<TS, true, GS_ULDS_MAX_R * GS_ULDS_MAX_R / GS_THREADS, 1>), grid,
-                           block, lds, st, p);
-    else
-        hipLaunchKernelGGL((generic_scan_kernel<TS, false, 1, 2>), grid, block, lds, st, p);
+    const size_t lds = 2 * static_cast<size_t>(p.Cb) * gs_ld<TS>(p.R) * sizeof(TS);
+    hipLaunchKernelGGL((generic_scan_kernel<TS, 2>), dim3(static_cast<unsigned>(blocks)), dim3(GS_THREADS), lds, st, p);
     return check_launch(what);
 }
 
 bool io_code(int c) { return c == MOGT_F32 || c == MOGT_BF16 || c == MOGT_F64 || c == MOGT_F16; }
+
+// The scan `out` describes, at level l of the geometry: in one pass, or LOCAL
+// over its chunks (state [H | P], the summaries), the carries as the exclusive
+// scan of the summaries (one level up), then `out` from each chunk's carry.
+template <typename TS>
+int scan_level(GParams out, int64_t B, const GGeo& g, int l, unsigned char* base, int state_code, hipStream_t st) {
+    if (l >= g.levels) {
+        out.seg = out.L; out.nseg = 1;
+        return launch_generic<TS>(out, B, st, "generic_scan output");
+    }
+    const int64_t R = out.R, nch = g.nch[l];
+    const GView vS{base + g.s_off[l], nch * R * g.Wl, R * g.Wl, g.Wl, state_code};   // [B][nch][R][C+R]
+    const GView vM{base + g.m_off[l], nch * R * g.Wo, R * g.Wo, g.Wo, state_code};   // [B][nch][R][Wo]
+    const GView none{nullptr, 0, 0, 0, state_code};
+    const int iC = out.cid;
+
+    GParams loc = out;
+    loc.seg = g.seg[l]; loc.nseg = static_cast<int>(nch);
+    loc.init = none; loc.out_h = vS; loc.out_p = none;
+    loc.W = g.Wl; loc.csplit = g.Wl; loc.every = 0; loc.shift = 0; loc.stream = 0;
+    int rc = launch_generic<TS>(loc, B, st, "generic_scan local");
+    if (rc) return rc;
+
+    GParams car{};
+    car.tr = vS; car.in = vS; car.init = none; car.out_h = vM; car.out_p = none;
+    car.L = nch - 1;
+    car.R = out.R; car.W = g.Wo; car.tr_c0 = iC; car.cin = iC; car.cid = iC; car.csplit = g.Wo;
+    car.every = 1; car.shift = 1; car.rev = 0;
+    rc = scan_level<TS>(car, B, g, l + 1, base, state_code, st);
+    if (rc) return rc;
+
+    out.seg = g.seg[l]; out.nseg = static_cast<int>(nch);
+    out.init = vM;
+    return launch_generic<TS>(out, B, st, "generic_scan output");
+}
 
 template <typename TS>
 int run_generic(const void* U, const void* V, void* H, void* P, int64_t B, int64_t L, int64_t R, int64_t C,
@@ -354,34 +278,13 @@ int run_generic(const void* U, const void* V, void* H, void* P, int64_t B, int64
     const GView vH{H, L * R * C, R * C, C, out_code};
     const GView vP{P, L * R * R, R * R, R, out_code};
     const GView none{nullptr, 0, 0, 0, state_code};
-
     unsigned char* base = static_cast<unsigned char*>(ws);
-    const GView vS{base + g.s_off, g.nch * R * g.Wl, R * g.Wl, g.Wl, state_code};   // [B][nch][R][C+R]
-    const GView vM{base + g.m_off, g.nch * R * g.Wo, R * g.Wo, g.Wo, state_code};   // [B][nch][R][Wo]
 
-    if (g.nch > 1) {
-        GParams loc{};
-        loc.tr = vU; loc.in = vV; loc.init = none; loc.out_h = vS; loc.out_p = none;
-        loc.L = L; loc.seg = g.seg; loc.nseg = static_cast<int>(g.nch);
-        loc.R = iR; loc.W = g.Wl; loc.tr_c0 = 0; loc.cin = iC; loc.cid = iC; loc.csplit = g.Wl;
-        loc.every = 0; loc.shift = 0; loc.rev = reverse;
-        int rc = launch_generic<TS>(loc, B, st, "generic_scan local");
-        if (rc) return rc;
-
-        GParams car{};
-        car.tr = vS; car.in = vS; car.init = none; car.out_h = vM; car.out_p = none;
-        car.L = g.nch - 1; car.seg = g.nch - 1; car.nseg = 1;
-        car.R = iR; car.W = g.Wo; car.tr_c0 = iC; car.cin = iC; car.cid = iC; car.csplit = g.Wo;
-        car.every = 1; car.shift = 1; car.rev = 0;
-        rc = launch_generic<TS>(car, B, st, "generic_scan carry");
-        if (rc) return rc;
-    }
-    GParams out{};
-    out.tr = vU; out.in = vV; out.init = g.nch > 1 ? vM : none; out.out_h = vH; out.out_p = vP;
-    out.L = L; out.seg = g.seg; out.nseg = static_cast<int>(g.nch);
-    out.R = iR; out.W = g.Wo; out.tr_c0 = 0; out.cin = iC; out.cid = iC; out.csplit = iC;
-    out.every = 1; out.shift = 0; out.rev = reverse;
-    return launch_generic<TS>(out, B, st, "generic_scan output");
+    GParams out{};   // the sequence's OUTPUT pass
+    out.tr = vU; out.in = vV; out.init = none; out.out_h = vH; out.out_p = vP;
+    out.L = L; out.R = iR; out.W = g.Wo; out.tr_c0 = 0; out.cin = iC; out.cid = iC; out.csplit = iC;
+    out.every = 1; out.shift = 0; out.rev = reverse; out.stream = 1;
+    return scan_level<TS>(out, B, g, 0, base, state_code, st);
 }
 
 int check_generic(int64_t B, int64_t L, int64_t R, int64_t C, int v_code, int state_code, int out_code,
@@ -419,7 +322,7 @@ extern "C" int mogt_affine_scan_generic_fwd(const void* U, const void* V, void* 
     if (batch == 0 || length == 0 || (channels == 0 && !U_prefix)) return MOGT_OK;
     if (!U || (channels > 0 && (!V || !H))) return set_error(MOGT_E_INVALID, "null tensor pointer");
     const GGeo g = generic_geometry(batch, length, rank, channels, U_prefix != nullptr, state_dtype);
-    if (g.nch > 1 && (!workspace || workspace_bytes < g.bytes))
+    if (g.levels > 0 && (!workspace || workspace_bytes < g.bytes))
         return set_error(MOGT_E_WORKSPACE, "workspace of %zu bytes needed", g.bytes);
     hipStream_t st = static_cast<hipStream_t>(stream);
     return state_dtype == MOGT_F64

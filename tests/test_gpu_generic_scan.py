@@ -334,3 +334,86 @@ def test_hand_backward_rank_above_64(gpu, sdt, tol):
     assert gU.dtype == tdt and gV.dtype == tdt
     assert rel_err(np64(gV), gV_ref) <= tol
     assert rel_err(np64(gU), gU_ref) <= tol
+
+
+def _loop64(U, V, rev=False):
+    """H_t = U_t H_{t-1} + V_t (rev: H_t = V_t + U_{t+1}^T H_{t+1}) step by step
+    in float64 on the host, and the prefix products."""
+    U, V = U.double().cpu(), V.double().cpu()
+    B, L, R, C = V.shape
+    H, P = torch.empty_like(V), torch.empty_like(U)
+    h = torch.zeros(B, R, C, dtype=torch.float64)
+    pr = torch.eye(R, dtype=torch.float64).expand(B, R, R)
+    for s in range(L):
+        t = L - 1 - s if rev else s
+        if not rev:
+            h = U[:, t] @ h + V[:, t]
+            pr = U[:, t] @ pr
+            P[:, t] = pr
+        else:
+            h = V[:, t] + (U[:, t + 1].transpose(-1, -2) @ h if s > 0 else 0)
+        H[:, t] = h
+    return P, H
+
+
+@pytest.mark.parametrize("state", [torch.float32, torch.float64])
+@pytest.mark.parametrize("B,L,R,C", [(1, 1, 1, 1), (2, 7, 15, 16), (1, 16, 16, 17), (3, 17, 17, 5), (1, 300, 32, 33),
+                                     (2, 130, 33, 1), (1, 65, 48, 48), (1, 70, 49, 20), (2, 90, 64, 64),
+                                     (1, 2100, 4, 3), (40, 33, 64, 40)])
+def test_matrix_core_ranks_match_the_loop(gpu, state, B, L, R, C):
+    """Ranks up to 64 on the matrix-core chunk kernel: every row-tile edge (with
+    and without 16-byte rows of U), ragged column tiles that hold state and
+    prefix columns, one step to several chunks of carries, two tiles per wave
+    (40 sequences of 64), forward with prefix, forward alone, and reversed."""
+    announce(f"generic mfma {state} {B} {L} {R} {C}")
+    from mogt_amd import ops
+
+    g = torch.Generator().manual_seed(L + R)
+    U = (0.9 * torch.eye(R, dtype=torch.float64) + 0.3 / R * torch.randn(B, L, R, R, generator=g, dtype=torch.float64))
+    V = torch.randn(B, L, R, C, generator=g, dtype=torch.float64)
+    Ug, Vg = U.to(state).to(gpu), V.to(state).to(gpu)
+    Pr, Hr = _loop64(Ug, Vg)
+    tol = 2e-6 if state == torch.float32 else 1e-13
+    P, H = torch.ops.mogt.affine_scan_generic(Ug, Vg, state, state, True, False)
+    assert rel_err(H.double().cpu().numpy(), Hr.numpy()) <= tol
+    assert rel_err(P.double().cpu().numpy(), Pr.numpy()) <= tol
+    _, H = torch.ops.mogt.affine_scan_generic(Ug, Vg, state, state, False, False)
+    assert rel_err(H.double().cpu().numpy(), Hr.numpy()) <= tol
+    _, G = torch.ops.mogt.affine_scan_generic(Ug, Vg, state, state, False, True)
+    assert rel_err(G.double().cpu().numpy(), _loop64(Ug, Vg, rev=True)[1].numpy()) <= tol
+
+
+@pytest.mark.parametrize("state", [torch.float32, torch.float64])
+@pytest.mark.parametrize("vdt", [torch.float16, torch.bfloat16, torch.float32, torch.float64])
+@pytest.mark.parametrize("odt", [torch.float16, torch.bfloat16, torch.float32, torch.float64])
+def test_matrix_core_io_dtypes(gpu, state, vdt, odt):
+    """Every input and output type of the general form (ragged last chunk), each
+    output rounded once from the state through fp32."""
+    announce(f"generic mfma io {state} {vdt} {odt}")
+    from mogt_amd import ops
+
+    g = torch.Generator().manual_seed(4)
+    B, L, R, C = 2, 45, 20, 18
+    U = 0.9 * torch.eye(R) + 0.02 * torch.randn(B, L, R, R, generator=g)
+    V = torch.randn(B, L, R, C, generator=g).to(vdt)
+    P, H = torch.ops.mogt.affine_scan_generic(U.to(gpu), V.to(gpu), state, odt, True, False)
+    Pr, Hr = _loop64(U, V)
+    tol = {torch.float16: 2e-3, torch.bfloat16: 1e-2, torch.float32: 1e-6, torch.float64: 1e-6}[odt]
+    assert H.dtype == odt and P.dtype == odt
+    assert rel_err(H.double().cpu().numpy(), Hr.numpy()) <= tol
+    assert rel_err(P.double().cpu().numpy(), Pr.numpy()) <= tol
+    wide = torch.ops.mogt.affine_scan_generic(U.to(gpu), V.to(gpu), state, state, True, False)
+    assert torch.equal(H, wide[1].float().to(odt) if odt != torch.float64 else wide[1].double())
+
+
+def test_matrix_core_workspace_covers_both_levels():
+    """The workspace the C entry asks for grows with the chunks of both levels
+    and is the header alone for one pass (host arithmetic only)."""
+    from mogt_amd import _lib
+
+    lib = _lib.load()
+    one = lib.mogt_affine_scan_generic_workspace_bytes(1, 16, 16, 48, 0, 2)
+    assert one == 256
+    n = lib.mogt_affine_scan_generic_workspace_bytes(1, 32768, 16, 48, 0, 2)
+    assert n > 256 + 8 * 16 * (64 + 48) * 128
+    assert lib.mogt_affine_scan_generic_workspace_bytes(1, 32768, 16, 48, 1, 2) > n
