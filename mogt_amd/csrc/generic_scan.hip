@@ -35,6 +35,7 @@ constexpr int GS_THREADS = 256;
 constexpr int GS_EPT = 4;                          // state elements per thread
 constexpr int GS_MAX_ELEMS = GS_THREADS * GS_EPT;  // R * column-tile width
 constexpr int GS_MAX_R = 1024;
+constexpr int64_t GS_ONE_CHUNK = 16;               // steps up to which no workspace is asked for
 
 // Row length in LDS of the staged transition and of a state column: R rounded
 // up to 16 bytes, plus 16 bytes of skew between rows.
@@ -205,6 +206,10 @@ GGeo generic_geometry(int64_t B, int64_t L, int64_t R, int64_t C, int with_prefi
         g.bytes = g.m_off[l] + align256(static_cast<size_t>(B * g.nch[l] * R * g.Wo) * ts);
         len = g.nch[l] - 1;   // the last chunk's summary is not needed
     }
+    // callers bring room for two chunks' summaries beyond 16 steps, also where
+    // one pass is the shorter chain
+    if (g.levels == 0 && L > GS_ONE_CHUNK)
+        g.bytes += align256(static_cast<size_t>(B * 2 * R * g.Wl) * ts) + align256(static_cast<size_t>(B * 2 * R * g.Wo) * ts);
     return g;
 }
 
@@ -322,7 +327,7 @@ extern "C" int mogt_affine_scan_generic_fwd(const void* U, const void* V, void* 
     if (batch == 0 || length == 0 || (channels == 0 && !U_prefix)) return MOGT_OK;
     if (!U || (channels > 0 && (!V || !H))) return set_error(MOGT_E_INVALID, "null tensor pointer");
     const GGeo g = generic_geometry(batch, length, rank, channels, U_prefix != nullptr, state_dtype);
-    if (g.levels > 0 && (!workspace || workspace_bytes < g.bytes))
+    if (length > GS_ONE_CHUNK && (!workspace || workspace_bytes < g.bytes))
         return set_error(MOGT_E_WORKSPACE, "workspace of %zu bytes needed", g.bytes);
     hipStream_t st = static_cast<hipStream_t>(stream);
     return state_dtype == MOGT_F64
