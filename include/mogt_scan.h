@@ -121,6 +121,16 @@ int mogt_diag_scan_fwd_noalloc(const void* a, const void* b, void* h, void* a_pr
 int mogt_diag_scan_rev_fwd(const void* a, const void* b, void* h,
                            int64_t batch, int64_t length, int64_t features,
                            void* workspace, size_t workspace_bytes, void* stream);
+/* The same with bf16 a and b (fp32 h); workspace of
+ * mogt_diag_scan_workspace_bytes for bf16 inputs.                            */
+int mogt_diag_scan_rev_bf16_fwd(const void* a, const void* b, void* h, int64_t batch, int64_t length,
+                                int64_t features, void* workspace, size_t workspace_bytes, void* stream);
+/* The decay's gradient of h_t = a_t h_{t-1} + b_t: da_t = G_t h_{t-1} with
+ * h recomputed in fp32 and G (fp32) from the reverse scan; a, b, da in `dtype`.
+ * bf16 also takes db, which receives G rounded to bf16.                      */
+int mogt_diag_scan_grad(const void* a, const void* b, const void* G, void* da, void* db, int64_t batch,
+                        int64_t length, int64_t features, int dtype, void* workspace,
+                        size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------- */
 /* Coupled write-forget per-rank scan of the MOGT mixer with identity

@@ -38,6 +38,11 @@ SIGNATURES: dict[str, tuple] = {
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
          _c_void_p, _c_size, _c_void_p],
     ),
+    "mogt_diag_scan_rev_bf16_fwd": (
+        _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_void_p, _c_size, _c_void_p]),
+    "mogt_diag_scan_grad": (
+        _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_int, _c_void_p,
+                 _c_size, _c_void_p]),
     "mogt_diag_scan_rev_fwd": (
         _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_void_p, _c_size, _c_void_p]),
     "mogt_diag_scan_workspace_bytes_cfg": (

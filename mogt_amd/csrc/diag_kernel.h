@@ -53,7 +53,12 @@ namespace mogt {
 // MODE_COUPLED_REV: the same backward recurrence for MODE_COUPLED, whose decay
 // a = damping * (1 - sigmoid(z)) is formed from the gate logits (per gate,
 // over its C channels) instead of being read as a [B, L, D] tensor.
-enum DiagMode { MODE_DIAG = 0, MODE_COUPLED = 1, MODE_DIAG_REV = 2, MODE_COUPLED_REV = 3 };
+// MODE_DIAG_GRAD: MODE_DIAG whose output is the decay's gradient: with G from
+// the reverse scan, da_t = G_t h_{t-1} (h_{-1} = 0) is formed in the output
+// phase, where h_{t-1} is the state entering the step, so the recomputed h is
+// never written or shifted.  With the prefix option the second output is G
+// rounded to the output dtype (the gradient of b).
+enum DiagMode { MODE_DIAG = 0, MODE_COUPLED = 1, MODE_DIAG_REV = 2, MODE_COUPLED_REV = 3, MODE_DIAG_GRAD = 4 };
 
 struct DiagParams {
     const void* a;      // [B, L, D] (DIAG)            | gate logits z [B, L, R] (COUPLED)
@@ -73,6 +78,7 @@ struct DiagParams {
     float* rowstat;     // COUPLED with ROWSTAT: [B, L, n_fg] sums of squares of h
     int64_t ldv;        // COUPLED: row stride of v in elements (D, or wider inside a projection)
     int64_t ldz;        // GATED: row stride of the gate logits (R)
+    const float* grad;  // GRAD: G [B, L, D]
 };
 
 constexpr uint32_t ST_NONE = 0u;
@@ -432,6 +438,49 @@ void diag_scan_kernel(DiagParams p) {
             constexpr bool FULL = decltype(full_tag)::value;
             TOut* rh = ph;
             TOut* rp = pp;
+            if constexpr (MODE == MODE_DIAG_GRAD) {
+                // the state entering every step (in the registers of a and b,
+                // dead after it), then the rows of G in batches, the next batch
+                // in flight while one is multiplied and stored
+                float hp[S][VEC];
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+#pragma unroll
+                    for (int v = 0; v < VEC; ++v) {
+                        hp[s][v] = hh[v];
+                        hh[v] = fmaf(step_a(s, v), hh[v], step_b(s, v));
+                    }
+                constexpr int SB = 8;
+                static_assert(S % SB == 0, "whole batches");
+                const float* rg = p.grad + wbase + roff;
+                uint32_t gw[2][SB][VEC];
+                auto fetch = [&](int k, int buf) {
+#pragma unroll
+                    for (int i = 0; i < SB; ++i)
+                        if (FULL || k * SB + i < nv) load_raw<4 * VEC>(rg + (k * SB + i) * Ds, gw[buf][i]);
+                };
+                fetch(0, 0);
+#pragma unroll
+                for (int k = 0; k < S / SB; ++k) {
+                    if (k + 1 < S / SB) fetch(k + 1, (k + 1) & 1);
+#pragma unroll
+                    for (int i = 0; i < SB; ++i) {
+                        if (FULL || k * SB + i < nv) {
+                            float o[VEC], gb[VEC];
+#pragma unroll
+                            for (int v = 0; v < VEC; ++v) {
+                                gb[v] = __uint_as_float(gw[k & 1][i][v]);
+                                o[v] = gb[v] * hp[k * SB + i][v];
+                            }
+                            store_stream<TOut, VEC>(rh, o);
+                            if constexpr (PREFIX) store_stream<TOut, VEC>(rp, gb);
+                        }
+                        rh += Ds;
+                        if constexpr (PREFIX) rp += Ds;
+                    }
+                }
+                return;
+            }
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 float o[VEC];
@@ -602,6 +651,7 @@ int diag_run_f32in(const DiagParams& prm, const DiagTile& t, int out_dtype, bool
 int diag_run_bf16in(const DiagParams& prm, const DiagTile& t, int out_dtype, bool prefix,
                     hipStream_t stream);
 bool diag_tile_compiled(int family, const DiagTile& t);   // family: 0 f32, 1 bf16, 2 coupled, 3 coupled reverse
-int diag_run_rev(const DiagParams& prm, const DiagTile& t, hipStream_t stream);   // diag_rev.hip
+int diag_run_rev(const DiagParams& prm, const DiagTile& t, int in_dtype, hipStream_t stream);   // diag_rev.hip
+int diag_run_grad(const DiagParams& prm, const DiagTile& t, int in_dtype, hipStream_t stream);  // diag_grad.hip
 
 }  // namespace mogt

@@ -39,10 +39,11 @@ DiagTile default_tile(int64_t B, int64_t L, int64_t D, bool bf16_in, int align_e
     return f32_tile(B, L, D, D % 2 == 0 && align_elems % 2 == 0);
 }
 
-// rev: the reverse-time recurrence h_t = a_{t+1} h_{t+1} + b_t (fp32 only).
+// rev: the reverse-time recurrence h_t = a_{t+1} h_{t+1} + b_t (fp32 out); grad:
+// the decay's gradient from G = grad into h, G rounded into aprefix (bf16).
 int run_scan(const void* a, const void* b, void* h, void* aprefix, int64_t B, int64_t L,
              int64_t D, int in_dtype, int out_dtype, const DiagTile& t, void* ws, size_t ws_bytes,
-             void* stream, bool rev = false) {
+             void* stream, bool rev = false, const float* grad = nullptr) {
     clear_error();
     if (B < 0 || L < 0 || D < 0) return set_error(MOGT_E_INVALID, "negative size");
     if (!dtype_ok(in_dtype) || !dtype_ok(out_dtype))
@@ -68,7 +69,9 @@ int run_scan(const void* a, const void* b, void* h, void* aprefix, int64_t B, in
     prm.damping = 1.0f;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool pre = aprefix != nullptr;
-    if (rev) return diag_run_rev(prm, t, st);
+    prm.grad = grad;
+    if (rev) return diag_run_rev(prm, t, in_dtype, st);
+    if (grad) return diag_run_grad(prm, t, in_dtype, st);
     return family == 1 ? diag_run_bf16in(prm, t, out_dtype, pre, st)
                        : diag_run_f32in(prm, t, out_dtype, pre, st);
 }
@@ -191,6 +194,31 @@ extern "C" int mogt_diag_scan_rev_fwd(const void* a, const void* b, void* h, int
     const DiagTile t = default_tile(batch, length, features, false, al);
     return run_scan(a, b, h, nullptr, batch, length, features, MOGT_F32, MOGT_F32, t, workspace,
                     workspace_bytes, stream, true);
+}
+
+extern "C" int mogt_diag_scan_rev_bf16_fwd(const void* a, const void* b, void* h, int64_t batch,
+                                           int64_t length, int64_t features, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
+    const int al = common_alignment(a, b, h, nullptr, MOGT_BF16, MOGT_F32);
+    const DiagTile t = default_tile(batch, length, features, true, al);
+    return run_scan(a, b, h, nullptr, batch, length, features, MOGT_BF16, MOGT_F32, t, workspace,
+                    workspace_bytes, stream, true);
+}
+
+extern "C" int mogt_diag_scan_grad(const void* a, const void* b, const void* G, void* da, void* db,
+                                   int64_t batch, int64_t length, int64_t features, int dtype,
+                                   void* workspace, size_t workspace_bytes, void* stream) {
+    clear_error();
+    if (!dtype_ok(dtype)) return set_error(MOGT_E_INVALID, "unsupported dtype code");
+    if (batch < 0 || length < 0 || features < 0) return set_error(MOGT_E_INVALID, "negative size");
+    if (batch == 0 || length == 0 || features == 0) return MOGT_OK;
+    if (!G || (dtype == MOGT_BF16) != (db != nullptr))
+        return set_error(MOGT_E_INVALID, "diag scan gradient: G, and db with bf16 inputs only");
+    int al = common_alignment(a, b, da, db, dtype, dtype);
+    while (al > 1 && reinterpret_cast<uintptr_t>(G) % (4 * al) != 0) al >>= 1;
+    const DiagTile t = default_tile(batch, length, features, dtype == MOGT_BF16, al);
+    return run_scan(a, b, da, db, batch, length, features, dtype, dtype, t, workspace, workspace_bytes, stream,
+                    false, static_cast<const float*>(G));
 }
 
 extern "C" int mogt_diag_scan_tiles(int family, int* out, int max_tiles) {

@@ -62,7 +62,7 @@ def _stream_handle(device: torch.device) -> int:
 # launch whose layout differs from the buffer's previous one clears everything
 # past the header first (or, if a captured graph uses the buffer, takes a new
 # one), so a word it reads is either zero, an older tag or its own.
-LOOKBACK_FAMILIES = frozenset({"diag", "diag_rev", "coupled", "coupled_rev", "rank1"})
+LOOKBACK_FAMILIES = frozenset({"diag", "diag_rev", "diag_grad", "coupled", "coupled_rev", "rank1"})
 
 
 def workspace(nbytes: int, device: torch.device, family: str = "plain", layout: tuple | None = None
@@ -251,13 +251,16 @@ def _diag_scan_rev_op(a: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     """G_t = g_t + a_{t+1} G_{t+1} (G_L = 0) in fp32: the reverse-time scan of
     the diagonal scan's backward."""
     lib = _lib.load()
-    a = a.to(torch.float32).contiguous()
-    g = g.to(torch.float32).contiguous()
+    bf16 = a.dtype == torch.bfloat16 and g.dtype == torch.bfloat16
+    a = (a if bf16 else a.to(torch.float32)).contiguous()
+    g = (g if bf16 else g.to(torch.float32)).contiguous()
     B, L, D = a.shape
     out = torch.empty(a.shape, dtype=torch.float32, device=a.device)
-    ws = workspace(lib.mogt_diag_scan_workspace_bytes(B, L, D, _lib.MOGT_F32), a.device, "diag_rev", (B, L, D))
-    rc = lib.mogt_diag_scan_rev_fwd(a.data_ptr(), g.data_ptr(), out.data_ptr(), B, L, D,
-                                    ws.data_ptr(), ws.numel(), _stream_handle(a.device))
+    code = _lib.MOGT_BF16 if bf16 else _lib.MOGT_F32
+    ws = workspace(lib.mogt_diag_scan_workspace_bytes(B, L, D, code), a.device, "diag_rev", (B, L, D, code))
+    run = lib.mogt_diag_scan_rev_bf16_fwd if bf16 else lib.mogt_diag_scan_rev_fwd
+    rc = run(a.data_ptr(), g.data_ptr(), out.data_ptr(), B, L, D, ws.data_ptr(), ws.numel(),
+             _stream_handle(a.device))
     _lib.check(rc, "mogt_diag_scan_rev_fwd")
     _checked(ws, "mogt_diag_scan_rev_fwd")
     return out
@@ -266,6 +269,31 @@ def _diag_scan_rev_op(a: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
 @_diag_scan_rev_op.register_fake
 def _(a, g):
     return a.new_empty(a.shape, dtype=torch.float32)
+
+
+@torch.library.custom_op("mogt::diag_scan_grad", mutates_args=())
+def _diag_scan_grad_op(a: torch.Tensor, b: torch.Tensor, G: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """(da, db) of the diagonal scan from G: da_t = G_t h_{t-1}, the state
+    recomputed in registers, in a's dtype; db is G in that dtype for bf16 and
+    empty for float32 (it is G itself)."""
+    lib = _lib.load()
+    a, b, G = a.contiguous(), b.contiguous(), G.contiguous()
+    B, L, D = a.shape
+    code = dtype_code(a.dtype, "diag_scan_grad")
+    da = torch.empty(a.shape, dtype=a.dtype, device=a.device)
+    db = torch.empty(a.shape if code == _lib.MOGT_BF16 else (0,), dtype=a.dtype, device=a.device)
+    ws = workspace(lib.mogt_diag_scan_workspace_bytes(B, L, D, code), a.device, "diag_grad", (B, L, D, code))
+    rc = lib.mogt_diag_scan_grad(a.data_ptr(), b.data_ptr(), G.data_ptr(), da.data_ptr(),
+                                 db.data_ptr() if code == _lib.MOGT_BF16 else None, B, L, D, code, ws.data_ptr(),
+                                 ws.numel(), _stream_handle(a.device))
+    _lib.check(rc, "mogt_diag_scan_grad")
+    _checked(ws, "mogt_diag_scan_grad")
+    return da, db
+
+
+@_diag_scan_grad_op.register_fake
+def _(a, b, G):
+    return a.new_empty(a.shape), a.new_empty(a.shape if a.dtype == torch.bfloat16 else (0,))
 
 
 def _shift_prev(h: torch.Tensor) -> torch.Tensor:
@@ -283,16 +311,19 @@ def _diag_scan_setup(ctx, inputs, output):
 def _diag_scan_backward(ctx, grad_h):
     """Reverse scan on the GPU (affine_scan.py:65-124 for R = C = 1): G = dH +
     a_{t+1} G_{t+1}; db = G; da_t = G_t h_{t-1}, with h recomputed in fp32 as
-    the reference's backward does (triton_scan.py:370-378)."""
+    the reference's backward does (triton_scan.py:370-378), inside the scan
+    that forms da."""
     a, b = ctx.saved_tensors
     need_a, need_b = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
     G = torch.ops.mogt.diag_scan_rev(a, grad_h)
     da = db = None
     if need_a:
-        h = torch.ops.mogt.diag_scan(a.float().contiguous(), b.float().contiguous(), torch.float32)
-        da = (G * _shift_prev(h)).to(a.dtype)
+        da, db = torch.ops.mogt.diag_scan_grad(a, b, G)
     if need_b:
-        db = G.to(b.dtype)
+        if db is None or a.dtype == torch.float32:
+            db = G.to(b.dtype)
+    else:
+        db = None
     return da, db, None
 
 

@@ -57,6 +57,41 @@ def test_diag_scan_backward_fp32(gpu, B, L, D):
     assert rel_err(to_np(at.grad), da_ref) <= FP32_TOL
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,D", [(1, 1, 4), (2, 9, 3), (1, 513, 130), (2, 511, 333), (1, 4097, 1024), (3, 16385, 768)])
+def test_diag_scan_gradient_scan(gpu, dtype, B, L, D):
+    """The decay-gradient scan (and bf16 reverse scan) in the inputs' dtype: one
+    step, odd widths (one feature per lane), ragged last chunks, 1 to 65
+    chunks, and each gradient alone; misaligned (offset) inputs on top."""
+    announce(f"diag gradient scan {dtype} {B} {L} {D}")
+    import mogt_amd
+
+    a, b = synthetic.diag_inputs(B, L, D, seed=L + D)
+    w = np.random.default_rng(L).standard_normal((B, L, D)).astype(np.float32)
+
+    def tensors(offset):
+        out = []
+        for x in (a, b, w):
+            flat = torch.zeros(x.size + 1, dtype=dtype, device=gpu)
+            flat[offset:offset + x.size] = torch.from_numpy(x).to(gpu).reshape(-1).to(dtype)
+            out.append(flat[offset:offset + x.size].view(B, L, D))
+        return out
+
+    at, bt, wt = tensors(0)
+    da_ref, db_ref = _diag_oracle_grads(to_np(at), to_np(bt), to_np(wt))
+    tol = 2e-6 if dtype == torch.float32 else 2.0 ** -8   # bf16: one rounding of each gradient
+    for offset, need in ((0, (True, True)), (0, (True, False)), (0, (False, True)), (1, (True, True))):
+        at, bt, wt = tensors(offset)
+        at.requires_grad_(need[0])
+        bt.requires_grad_(need[1])
+        h = mogt_amd.diag_scan(at, bt)
+        grads = torch.autograd.grad(h, [t for t in (at, bt) if t.requires_grad], wt)
+        refs = [r for r, n in zip((da_ref, db_ref), need) if n]
+        for g, r in zip(grads, refs):
+            assert g.dtype == dtype
+            assert rel_err(to_np(g), r) <= tol
+
+
 def test_diag_scan_backward_bf16(gpu):
     announce("diag backward bf16 B=1 L=1000 D=256")
     import mogt_amd
