@@ -326,6 +326,12 @@ int mogt_affine_scan_rev_fwd(const void* U, const void* X, void* G, int64_t batc
  * all fp32, R <= 32.  No workspace.                                        */
 int mogt_affine_scan_grad_u(const void* G, const void* H, const void* P, void* dU, int64_t batch,
                             int64_t length, int64_t rank, int64_t channels, void* stream);
+/* The same without P, the forward state recomputed from U and V (fp32 or bf16)
+ * inside the pass that forms dU, never written: C a multiple of 8 up to 64, V
+ * and G 16-byte aligned.  Workspace of mogt_affine_scan_workspace_bytes.    */
+int mogt_affine_scan_recompute_grad_u(const void* U, const void* V, const void* G, void* dU, int64_t batch,
+                                      int64_t length, int64_t rank, int64_t channels, int v_dtype,
+                                      void* workspace, size_t workspace_bytes, void* stream);
 
 /* Block-local affine scan: per block of `block_size` steps, the local prefixes
  * U_prefix/H_prefix [B, L, ...] and the per-block summaries U_summary

@@ -18,8 +18,13 @@
 //   EXCL     X_0 = the chunk's carry (or [I | 0]); writes the state *before*
 //            every step, i.e. exclusive prefixes.
 //   OUTPUT   X_0 = the chunk's carry; writes H_t (and P_t) after every step.
-// SUMMARY, EXCL and OUTPUT run chunks of exactly kDenseChunk steps (the last
-// one ragged), which fixes the trip count of the step loop at compile time.
+//   GRADU    X_0 = the chunk's carry; writes dU_t = G_t H_{t-1}^T (the gradient
+//            of U, affine_scan.py:119-124) instead of H_t: the state entering
+//            the step goes through a small LDS tile into the B operand of
+//            RT x RT more tiles, so the recomputed H is never written and read
+//            back.  One column block (C <= 64, a multiple of 8).
+// SUMMARY, EXCL, OUTPUT and GRADU run chunks of exactly kDenseChunk steps (the
+// last one ragged), which fixes the trip count of the step loop at compile time.
 //
 // REV (level-0 SUMMARY and OUTPUT): the reverse-time recurrence of the
 // backward, G_t = X_t + U_{t+1}^T G_{t+1} (affine_scan.py:110-118), run as a
@@ -38,7 +43,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 
-enum ChunkMode { CM_SUMMARY = 0, CM_LOCAL = 1, CM_EXCL = 2, CM_OUTPUT = 3 };
+enum ChunkMode { CM_SUMMARY = 0, CM_LOCAL = 1, CM_EXCL = 2, CM_OUTPUT = 3, CM_GRADU = 4 };
 
 // Steps per chunk of the SUMMARY / EXCL / OUTPUT passes at every level.
 constexpr int kDenseChunk = 32;
@@ -54,6 +59,8 @@ struct ChunkParams {
     void* outH;          // per-step H: LOCAL fp32 / EXCL fp32 / OUTPUT TO
     float* sumP;         // [B, nb, R, R] chunk products (SUMMARY / LOCAL)
     float* sumH;         // [B, nb, R, C]
+    const float* G;      // GRADU: [B, L, R, C] total gradients of H
+    float* dU;           // GRADU: [B, L, R, R]
     int64_t L;           // steps of this level
     int R, C, T, nb;
     int withP;           // carry / write the P columns (column block 0 only)
@@ -88,11 +95,13 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
     static_assert(!REV || (!U4 && !VK && (MODE == CM_SUMMARY || MODE == CM_OUTPUT)),
                   "the reverse form reads U transposed, level 0 only");
     constexpr bool FIXED = MODE != CM_LOCAL;   // trip count kDenseChunk
+    constexpr bool GRADU = MODE == CM_GRADU;
+    static_assert(!GRADU || (W16 && !WITHP && !VK && !REV), "the gradient form: whole 16-byte pieces, H only");
     // OUTPUT passes write H (and P) non-temporally: lines left dirty in the
     // caches are otherwise written back while the next pass streams its
     // operands (measured: level-0 summary after an OUTPUT pass 37-39 -> 23 us
     // at R = 16, C = 48; configs[3] 540 -> 519 us).
-    constexpr int kOutPolicy = MODE == CM_OUTPUT ? 2 : 0;
+    constexpr int kOutPolicy = MODE == CM_OUTPUT || MODE == CM_GRADU ? 2 : 0;
     constexpr int NT = RT + CTW;               // column tiles: RT of P, then CTW of H
     constexpr int D = RT == 1 ? 8 : 4;         // steps of operands in flight
     static_assert(!FIXED || kDenseChunk % D == 0, "chunk must be a multiple of the prefetch depth");
@@ -120,7 +129,7 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
 
     // ---- initial state ------------------------------------------------------
     f32x4 X[RT][NT];
-    const bool fromCarry = (MODE == CM_EXCL || MODE == CM_OUTPUT) && p.carH != nullptr;
+    const bool fromCarry = (MODE == CM_EXCL || MODE == CM_OUTPUT || GRADU) && p.carH != nullptr;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -163,7 +172,7 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
     constexpr int OE = 16 / static_cast<int>(sizeof(TO));     // output elements per piece
     constexpr bool VBLOCK = W16 && !VK;                       // V_t block through LDS
     constexpr int NV = VBLOCK ? (ROWS * VW / VE + 63) / 64 : 1;
-    constexpr bool STORES = MODE != CM_SUMMARY;
+    constexpr bool STORES = MODE != CM_SUMMARY && !GRADU;
     constexpr bool STAGE_OUT = W16 && STORES;
     constexpr int NO = STAGE_OUT ? (ROWS * VW / OE + 63) / 64 : 1;
     constexpr int ES = MODE == CM_OUTPUT ? static_cast<int>(sizeof(TO)) : 4;   // stored element bytes
@@ -243,6 +252,29 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
                 offP[rt][ct][i] = (hasP && r < R && c < R) ? (r * R + c) * ES : kOOB;
             }
 
+    // GRADU: G_t as an A operand (row 16 rt + n, columns 16 h + 4 g .. + 3) and
+    // dU stores (element i of tile (rt, ct), columns below R)
+    uint32_t offG[GRADU ? RT : 1][GRADU ? CTW : 1];
+    uint32_t offD[GRADU ? RT : 1][GRADU ? RT : 1][4];
+    if constexpr (GRADU) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+            for (int h = 0; h < CTW; ++h) {
+                const int r = 16 * rt + n, c = 16 * h + 4 * g;
+                offG[rt][h] = (r < R && c < C) ? (r * C + c) * 4 : kOOB;
+            }
+#pragma unroll
+            for (int ct = 0; ct < RT; ++ct)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int r = trow(rt, i), c = pcol(ct);
+                    offD[rt][ct][i] = (r < R && c < R) ? (r * R + c) * 4 : kOOB;
+                }
+        }
+    }
+
+    __shared__ __align__(16) float s_h[GRADU ? ROWS : 1][GRADU ? VS : 4];
     __shared__ __align__(16) float s_v[VBLOCK ? ROWS : 1][VBLOCK ? VS : 4];
     __shared__ __align__(16) float s_o[STAGE_OUT ? ROWS : 1][STAGE_OUT ? VS : 4];
     // Orders this wave's LDS writes before its reads of other lanes' data and
@@ -257,6 +289,7 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
         u32x4 raw[NV];
         f32x4 vv[VK ? RT : 1];   // VK: v rows of the tile row groups
         float kk[VK ? CTW : 1];  // VK: k columns of the column tiles
+        f32x4 Gv[GRADU ? RT : 1][GRADU ? CTW : 1];
     };
     const int64_t seqStep = static_cast<int64_t>(b) * p.L;
     // memory step of the operands / outputs of step t (REV: reversed time)
@@ -277,6 +310,15 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
                         o.A[rt][kt][kk] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ru, offA[rt][kt][kk], 0, 0));
                 }
             }
+        if constexpr (GRADU) {
+            const auto rg = rsrc(p.G + (seqStep + t) * R * static_cast<int64_t>(C),
+                                 valid ? static_cast<uint32_t>(R * C * 4) : 0u);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int h = 0; h < CTW; ++h)
+                    o.Gv[rt][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rg, offG[rt][h], 0, 0));
+        }
         if (!VBLOCK && !Vg) return;   // C == 0: no V (VBLOCK implies V)
         const auto rv = rsrc(static_cast<const char*>(p.V) + (seqStep + vrow(t)) * vBytes, valid ? vBytes : 0u);
         auto ld1 = [](__amdgpu_buffer_rsrc_t r, int off) {   // one element as fp32 bits (bf16: raw)
@@ -436,6 +478,53 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
         }
     };
 
+    // GRADU: dU_t = G_t X^T from the state X before step t.  Two accumulators
+    // per tile (K-steps alternating) shorten the dependent MFMA chain.
+    auto grad_step = [&](const Ops& o, int64_t t, bool valid) {
+        if constexpr (GRADU) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int h = 0; h < CTW; ++h)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s_h[trow(rt, i)][16 * h + n] = X[rt][RT + h][i];
+            lds_order();
+            f32x4 hb[RT][CTW];
+#pragma unroll
+            for (int ct = 0; ct < RT; ++ct)
+#pragma unroll
+                for (int h = 0; h < CTW; ++h)
+                    hb[ct][h] = *reinterpret_cast<const f32x4*>(&s_h[16 * ct + n][16 * h + 4 * g]);
+            lds_order();
+            f32x4 d[2][RT][RT];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int ct = 0; ct < RT; ++ct) d[q][rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int h = 0; h < CTW; ++h)
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                        for (int ct = 0; ct < RT; ++ct)
+                            d[kk & 1][rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.Gv[rt][h][kk], hb[ct][h][kk],
+                                                                                     d[kk & 1][rt][ct], 0, 0, 0);
+            const auto rd = rsrc(p.dU + (seqStep + t) * RR, valid ? uBytes : 0u);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int ct = 0; ct < RT; ++ct)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(d[0][rt][ct][i] + d[1][rt][ct][i]), rd,
+                                                              offD[rt][ct][i], 0, kOutPolicy);
+        }
+    };
+
     // ---- the recurrence, operands D steps ahead ---------------------------
     Ops buf[D];
     if constexpr (FIXED) {
@@ -452,6 +541,7 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
             for (int i = 0; i < D; ++i) {
                 const int s = s0 + i;
                 if constexpr (MODE == CM_EXCL) store_state(t0 + min(s, last), s < nv);
+                if constexpr (GRADU) grad_step(buf[i], t0 + min(s, last), s < nv);
                 step(buf[i]);
                 if constexpr (MODE == CM_OUTPUT) store_state(t0 + min(s, last), s < nv);
                 // refill this slot, then convert the next step's operands
@@ -550,6 +640,29 @@ int dense_launch_pass(const ChunkParams& c, int64_t B, hipStream_t st) {
         return u4 ? dense_launch_c<2, true, TV, TO, MODE, VK, false>(c, B, st) : dense_launch_c<2, false, TV, TO, MODE, VK, false>(c, B, st);
     }
 }
+
+// The gradient pass (level 0, one column block): the caller checked C and the
+// alignment of V and G.
+template <typename TV, int RT, bool U4>
+int dense_launch_gradu_c(const ChunkParams& c, int64_t B, hipStream_t st) {
+    const dim3 grid(c.nb, 1, static_cast<unsigned>(B));
+    switch (dense_col_tiles(c.C)) {
+        case 1: hipLaunchKernelGGL((dense_chunk_kernel<RT, 1, false, U4, true, TV, float, CM_GRADU, false, false>), grid, dim3(64), 0, st, c); break;
+        case 2: hipLaunchKernelGGL((dense_chunk_kernel<RT, 2, false, U4, true, TV, float, CM_GRADU, false, false>), grid, dim3(64), 0, st, c); break;
+        case 3: hipLaunchKernelGGL((dense_chunk_kernel<RT, 3, false, U4, true, TV, float, CM_GRADU, false, false>), grid, dim3(64), 0, st, c); break;
+        default: hipLaunchKernelGGL((dense_chunk_kernel<RT, 4, false, U4, true, TV, float, CM_GRADU, false, false>), grid, dim3(64), 0, st, c);
+    }
+    return check_launch("dense_chunk_kernel");
+}
+
+template <typename TV>
+int dense_launch_gradu(const ChunkParams& c, int64_t B, hipStream_t st) {
+    const bool u4 = c.R % 4 == 0 && reinterpret_cast<uintptr_t>(c.U) % 16 == 0;
+    if (c.R <= 16) return u4 ? dense_launch_gradu_c<TV, 1, true>(c, B, st) : dense_launch_gradu_c<TV, 1, false>(c, B, st);
+    return u4 ? dense_launch_gradu_c<TV, 2, true>(c, B, st) : dense_launch_gradu_c<TV, 2, false>(c, B, st);
+}
+extern template int dense_launch_gradu<float>(const ChunkParams&, int64_t, hipStream_t);
+extern template int dense_launch_gradu<bf16_t>(const ChunkParams&, int64_t, hipStream_t);
 
 // Instantiated once each in dense_pass_*.hip (parallel compilation).
 #define MOGT_DENSE_PASSES(X)                 \

@@ -137,6 +137,30 @@ int run_rev(const float* U, const float* X, float* G, int64_t B, int64_t L, int6
     return dense_launch_pass<float, float, CM_OUTPUT, false, true>(c, B, st);
 }
 
+// dU_t = G_t H_{t-1}^T with H recomputed: the forward's summaries and carries,
+// then one pass that forms dU from the state it carries (CM_GRADU).
+template <typename TV>
+int run_gradu(const float* U, const void* V, const float* G, float* dU, int64_t B, int64_t L, int64_t R, int64_t C,
+              char* ws, const DenseGeo& geo, hipStream_t st) {
+    ChunkParams c{};
+    c.U = U; c.V = V; c.G = G; c.dU = dU;
+    c.L = L; c.R = static_cast<int>(R); c.C = static_cast<int>(C); c.T = kDenseChunk;
+    c.nb = static_cast<int>((L + c.T - 1) / c.T);
+    if (c.nb > 1) {
+        const Level& v = geo.lv[0];
+        ChunkParams s = c;
+        s.sumP = reinterpret_cast<float*>(ws + v.sumP);
+        s.sumH = reinterpret_cast<float*>(ws + v.sumH);
+        int rc = dense_launch_pass<TV, float, CM_SUMMARY>(s, B, st);
+        if (rc) return rc;
+        rc = excl_scan<float>(s.sumP, s.sumH, c.nb, reinterpret_cast<float*>(ws + v.carP),
+                              reinterpret_cast<float*>(ws + v.carH), B, R, C, false, ws, geo, 1, st);
+        if (rc) return rc;
+        c.carH = reinterpret_cast<float*>(ws + v.carH);
+    }
+    return dense_launch_gradu<TV>(c, B, st);
+}
+
 // dU_t = G_t M_{t-1}^T for the augmented state M = [H | P] of the forward
 // scan (P: the prefix products, only when their gradient is part of G), with
 // M_{-1} = [0 | I]: the dU of affine_scan_sequential_backward
@@ -334,4 +358,31 @@ extern "C" int mogt_affine_scan_grad_u(const void* G, const void* H, const void*
                        static_cast<const float*>(H), static_cast<const float*>(P), static_cast<float*>(dU),
                        length, static_cast<int>(rank), static_cast<int>(channels), CG);
     return check_launch("dense_grad_u_kernel");
+}
+
+extern "C" int mogt_affine_scan_recompute_grad_u(const void* U, const void* V, const void* G, void* dU, int64_t batch,
+                                                 int64_t length, int64_t rank, int64_t channels, int v_dtype,
+                                                 void* workspace, size_t workspace_bytes, void* stream) {
+    clear_error();
+    int rc = check_dense_shapes(batch, length, rank, channels);
+    if (rc) return rc;
+    if (v_dtype != MOGT_F32 && v_dtype != MOGT_BF16) return set_error(MOGT_E_INVALID, "unsupported V dtype");
+    if (channels < 8 || channels > 64 || channels % 8 != 0)
+        return set_error(MOGT_E_INVALID, "the recomputing gradient takes C = 8 .. 64, a multiple of 8");
+    if (batch == 0 || length == 0) return MOGT_OK;
+    if (!U || !V || !G || !dU) return set_error(MOGT_E_INVALID, "null tensor pointer");
+    if ((reinterpret_cast<uintptr_t>(V) | reinterpret_cast<uintptr_t>(G)) % 16)
+        return set_error(MOGT_E_INVALID, "V and G need 16-byte alignment");
+    if (batch > 65535 || (length + kDenseChunk - 1) / kDenseChunk > 0x7fffffffLL)
+        return set_error(MOGT_E_INVALID, "problem too large for one launch");
+    const DenseGeo g = dense_geometry(batch, length, rank, channels);
+    if (!workspace || workspace_bytes < g.bytes)
+        return set_error(MOGT_E_WORKSPACE, "workspace of %zu bytes required, got %zu", g.bytes, workspace_bytes);
+    const float* u = static_cast<const float*>(U);
+    const float* gp = static_cast<const float*>(G);
+    float* d = static_cast<float*>(dU);
+    char* base = static_cast<char*>(workspace);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return v_dtype == MOGT_F32 ? run_gradu<float>(u, V, gp, d, batch, length, rank, channels, base, g, st)
+                               : run_gradu<bf16_t>(u, V, gp, d, batch, length, rank, channels, base, g, st);
 }

@@ -874,6 +874,35 @@ def _(G, H, P):
     return H.new_empty(B, L, R, R)
 
 
+GRADU_MAX_CHANNELS = 64   # one column block of the recomputing gradient pass
+
+
+@torch.library.custom_op("mogt::affine_scan_recompute_grad_u", mutates_args=())
+def _affine_scan_recompute_grad_u_op(U: torch.Tensor, V: torch.Tensor, G: torch.Tensor) -> torch.Tensor:
+    """dU_t = G_t H_{t-1}^T (fp32), H recomputed from U and V: inside the pass
+    that forms dU where its layout allows, else written and read back."""
+    lib = _lib.load()
+    U, V = _prep_uv(U, V)
+    G = G.contiguous()
+    B, L, R, C = V.shape
+    if C % 8 != 0 or not 0 < C <= GRADU_MAX_CHANNELS or (V.data_ptr() | G.data_ptr()) % 16 != 0:
+        H = torch.empty(V.shape, dtype=torch.float32, device=V.device)
+        _affine_launch(U, V, H, None)
+        return torch.ops.mogt.affine_scan_grad_u(G, H, None)
+    dU = torch.empty(B, L, R, R, dtype=torch.float32, device=G.device)
+    ws = workspace(lib.mogt_affine_scan_workspace_bytes(B, L, R, C), G.device)
+    rc = lib.mogt_affine_scan_recompute_grad_u(U.data_ptr(), V.data_ptr(), G.data_ptr(), dU.data_ptr(), B, L, R, C,
+                                               dtype_code(V.dtype, "affine_scan_grad"), ws.data_ptr(), ws.numel(),
+                                               _stream_handle(G.device))
+    _lib.check(rc, "mogt_affine_scan_recompute_grad_u")
+    return dU
+
+
+@_affine_scan_recompute_grad_u_op.register_fake
+def _(U, V, G):
+    return U.new_empty(U.shape, dtype=torch.float32)
+
+
 def _reverse_scan(U: torch.Tensor, X: torch.Tensor, state_dtype: torch.dtype) -> torch.Tensor:
     """G_t = X_t + U_{t+1}^T G_{t+1}, G_{L-1} = X_{L-1}, in the state dtype
     (the carry recursion of affine_scan.py:110-118): the matrix-core
@@ -909,7 +938,7 @@ def affine_scan_grad(U: torch.Tensor, V: torch.Tensor, grad_H: torch.Tensor | No
                 P, H = _forward_state(U, V, state_dtype, True)
                 grad_u = torch.ops.mogt.affine_scan_grad_u(G, H, P)
             else:
-                grad_u = torch.ops.mogt.affine_scan_grad_u(G, _forward_state(U, V, state_dtype, False), None)
+                grad_u = torch.ops.mogt.affine_scan_recompute_grad_u(U, V, G)
             return grad_u.to(U.dtype), grad_v
         zeros = torch.zeros(B, 1, R, C, dtype=state_dtype, device=V.device)
         if grad_P is not None:

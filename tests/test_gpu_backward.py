@@ -297,3 +297,28 @@ def test_projection_fed_scan_gradients(gpu, B, L, r, c, dt, prev, with_const):
         assert np.all(gp[:, -1, D + r:] == 0)
     if gc is not None:
         assert rel_err(to_np(gct.grad), g64.grad.numpy()) <= tol
+
+
+@pytest.mark.parametrize("vdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,R,C", [(1, 1, 4, 8), (2, 31, 7, 16), (1, 33, 16, 40), (2, 300, 16, 48), (1, 70, 17, 24),
+                                     (1, 129, 32, 64), (1, 1100, 32, 48), (1, 40, 5, 12), (1, 40, 16, 72)])
+def test_recomputed_grad_u(gpu, vdt, B, L, R, C):
+    """dU from the pass that recomputes H: rank tiles with and without 16-byte
+    rows of U, every column-tile count (1 to 4, ragged), one chunk to two
+    levels of carries, and the shapes that keep the written state (C not a
+    multiple of 8, C above 64); a misaligned G too."""
+    announce(f"recomputed dU {vdt} {B} {L} {R} {C}")
+    rng = np.random.default_rng(R + C)
+    U = (0.9 * np.eye(R) + 0.2 / R * rng.standard_normal((B, L, R, R))).astype(np.float32)
+    V = torch.from_numpy(rng.standard_normal((B, L, R, C)).astype(np.float32)).to(gpu).to(vdt)
+    G = rng.standard_normal((B, L, R, C)).astype(np.float32)
+    H = np.zeros((B, L + 1, R, C))
+    for t in range(L):
+        H[:, t + 1] = U[:, t].astype(np.float64) @ H[:, t] + to_np(V[:, t])
+    ref = G.astype(np.float64) @ np.swapaxes(H[:, :-1], -1, -2)
+    flat = torch.zeros(G.size + 1, device=gpu)
+    for off in (0, 1):
+        Gt = flat[off:off + G.size].view(G.shape)
+        Gt.copy_(torch.from_numpy(G))
+        dU = torch.ops.mogt.affine_scan_recompute_grad_u(torch.from_numpy(U).to(gpu), V, Gt)
+        assert rel_err(to_np(dU), ref) <= 3e-6
