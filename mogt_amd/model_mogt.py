@@ -24,6 +24,7 @@ Tensors must be on the GPU; there is no CPU execution path.
 """
 from __future__ import annotations
 
+import contextlib
 from dataclasses import dataclass
 
 import torch
@@ -41,6 +42,13 @@ def _autocast_dtype() -> torch.dtype | None:
     return None
 
 
+def _range(name: str):
+    """A profiler range while a profiler runs (entering one costs about 5 us of
+    host time, a dozen times per layer)."""
+    return torch.autograd.profiler.record_function(name) if torch.autograd._profiler_enabled() else _NO_RANGE
+
+
+_NO_RANGE = contextlib.nullcontext()
 _CACHE_ATTR = "_gemm_weight_cache"
 
 
@@ -164,6 +172,17 @@ def _gate_input_parts(mode: str) -> tuple[str, ...]:
     return ("cur",) + (("prev",) if "prev" in mode else ()) + (("prefix",) if "prefix" in mode else ())
 
 
+def _attr(block: nn.Module, name: str, default):
+    """``getattr(block, name, default)`` without the exception nn.Module raises
+    and getattr swallows for every attribute a block does not set."""
+    for table in (block.__dict__, block._modules, block._parameters, block._buffers):
+        if name in table:
+            return table[name]
+    if type(block).__getattr__ is nn.Module.__getattr__ and not hasattr(type(block), name):
+        return default
+    return getattr(block, name, default)
+
+
 @dataclass(frozen=True)
 class MixerSpec:
     """A block's duck-typed configuration, resolved for one call."""
@@ -182,24 +201,24 @@ class MixerSpec:
 
     @staticmethod
     def of(block: "MOGTBlock") -> "MixerSpec":
-        scan = "transport_triton" if getattr(block, "fast_throughput_mode", False) else \
-            getattr(block, "scan_impl", "sequential")
-        gate_logit = getattr(block, "mogt_residual_gate_logit", None)
-        if not getattr(block, "mogt_residual_gate_enabled", False):
+        scan = "transport_triton" if _attr(block, "fast_throughput_mode", False) else \
+            _attr(block, "scan_impl", "sequential")
+        gate_logit = _attr(block, "mogt_residual_gate_logit", None)
+        if not _attr(block, "mogt_residual_gate_enabled", False):
             gate_logit = None
         return MixerSpec(
-            connection=getattr(block, "connection_impl", "matrix_exp"),
-            damping=float(getattr(block, "connection_damping", 0.999)),
-            transport_gate=getattr(block, "phi_transport_gate", None),
-            transport_mode=getattr(block, "transport_gate_mode", "multiply"),
-            transport_scale=float(getattr(block, "transport_gate_scale", 1.0)),
-            value_gate=getattr(block, "phi_value_gate", None),
-            gate_parts=_gate_input_parts(getattr(block, "value_gate_input_mode", "current")),
-            coupled=bool(getattr(block, "couple_forget_to_value_gate", False)),
+            connection=_attr(block, "connection_impl", "matrix_exp"),
+            damping=float(_attr(block, "connection_damping", 0.999)),
+            transport_gate=_attr(block, "phi_transport_gate", None),
+            transport_mode=_attr(block, "transport_gate_mode", "multiply"),
+            transport_scale=float(_attr(block, "transport_gate_scale", 1.0)),
+            value_gate=_attr(block, "phi_value_gate", None),
+            gate_parts=_gate_input_parts(_attr(block, "value_gate_input_mode", "current")),
+            coupled=bool(_attr(block, "couple_forget_to_value_gate", False)),
             scan=scan,
-            residual_scale=float(getattr(block, "mogt_residual_scale", 1.0)),
+            residual_scale=float(_attr(block, "mogt_residual_scale", 1.0)),
             residual_gate_logit=gate_logit,
-            ffn_scale=float(getattr(block, "mogt_ffn_residual_scale", 1.0)),
+            ffn_scale=float(_attr(block, "mogt_ffn_residual_scale", 1.0)),
         )
 
     def validate(self) -> None:
@@ -265,6 +284,8 @@ class MOGTBlock(_WeightCacheOwner):
         return MixerSpec.of(self).connection
 
     def _residual_scale(self, like: torch.Tensor) -> float:
+        if not _attr(self, "mogt_residual_gate_enabled", False):
+            return float(_attr(self, "mogt_residual_scale", 1.0))
         return float(MixerSpec.of(self).residual_factor(like))
 
     def fused_path_ok(self) -> bool:
@@ -297,7 +318,7 @@ class MOGTBlock(_WeightCacheOwner):
         if spec.connection not in _CONNECTIONS:
             raise ValueError(f"Unsupported connection_impl: {spec.connection}")
         label = "mogt.matrix_exp" if spec.connection == "matrix_exp" else "mogt.cayley_solve"
-        with torch.autograd.profiler.record_function(label):
+        with _range(label):
             mapped = ops.connection_map((A / self.r).to(torch.float32), spec.connection)
         return (mapped * spec.damping).to(output_dtype)
 
@@ -329,7 +350,7 @@ class MOGTBlock(_WeightCacheOwner):
         B, L, D = xn.shape
         r, c = self.r, self.c
         diagonal = spec.connection == "identity" and spec.scan != "transport_triton"
-        with torch.autograd.profiler.record_function("mogt.connection_map"):
+        with _range("mogt.connection_map"):
             if diagonal:
                 # per-rank factor of U = factor * I: starts as the damping
                 factor = torch.full((1, 1, 1, 1), spec.damping, dtype=torch.float32,
@@ -339,7 +360,7 @@ class MOGTBlock(_WeightCacheOwner):
                 if spec.connection == "identity":
                     A = xn.new_zeros(B, L, r, r)   # the identity map ignores A
                 else:
-                    with torch.autograd.profiler.record_function("mogt.connection"):
+                    with _range("mogt.connection"):
                         A_raw = self.phi_conn(xn).view(B, L, r, r)
                         A = A_raw - A_raw.transpose(-2, -1)
                 U = self._build_transport(A, xn.dtype)
@@ -349,7 +370,7 @@ class MOGTBlock(_WeightCacheOwner):
                     factor = factor * tg.to(factor.dtype)
                 else:
                     U = U * tg.to(U.dtype)
-        with torch.autograd.profiler.record_function("mogt.value_projection"):
+        with _range("mogt.value_projection"):
             values = self.phi_val(xn).view(B, L, r, c)
             if spec.value_gate is not None:
                 vg = self._value_gate_probs(spec, xn, prefix_condition)
@@ -361,7 +382,7 @@ class MOGTBlock(_WeightCacheOwner):
                     else:
                         U = U * keep.to(U.dtype)
         out_dtype = xn.dtype   # the scan's output dtype is U's (model_mogt.py:202)
-        with torch.autograd.profiler.record_function("mogt.affine_scan"):
+        with _range("mogt.affine_scan"):
             if diagonal:
                 decay = factor.float().expand(B, L, r, c).reshape(B, L, D)
                 h = ops.diag_scan(decay, values.float().reshape(B, L, D), out_dtype=out_dtype)
@@ -375,10 +396,10 @@ class MOGTBlock(_WeightCacheOwner):
                     U, values, block_size=getattr(self, "scan_block_size", 256),
                     block_c=getattr(self, "scan_block_c", 32), carry_scan=carry,
                     output_dtype=out_dtype).reshape(B, L, D)
-        with torch.autograd.profiler.record_function("mogt.readout"):
+        with _range("mogt.readout"):
             z = self.theta_read(self.norm_out(h))
         x = x + spec.residual_factor(z) * z
-        with torch.autograd.profiler.record_function("mogt.ffn"):
+        with _range("mogt.ffn"):
             x = x + spec.ffn_scale * self.ffn(self.norm_ffn(x))
         return x
 
@@ -465,12 +486,12 @@ class MOGTBlock(_WeightCacheOwner):
         writes h in the GEMM's dtype plus per-row sums of squares, the GEMM runs
         against theta_read * norm_out.weight, and the next RMSNorm applies each
         row's factor rsqrt(mean(h^2) + eps) as it reads Z."""
-        with torch.autograd.profiler.record_function("mogt.affine_scan"):
+        with _range("mogt.affine_scan"):
             proj, gate_prev, gconst = self._value_and_gate_projection(xn, prefix_condition, gate_const,
                                                                       const_given=gate_const is not None)
             h, stats = ops.coupled_rank_scan_proj(proj, self.d_model, rank=self.r, gate_prev=gate_prev,
                                                   gate_const=gconst, damping=damping)
-        with torch.autograd.profiler.record_function("mogt.readout"):
+        with _range("mogt.readout"):
             Zr = F.linear(h, _gemm_weight(self, "theta_read_folded", (self.theta_read.weight, self.norm_out.weight),
                                           lambda: self.theta_read.weight * self.norm_out.weight))
         return ops.add_rmsnorm_rowscale(x, Zr, stats, self._residual_scale(Zr), self.norm_ffn.weight,
@@ -484,20 +505,20 @@ class MOGTBlock(_WeightCacheOwner):
         weights); otherwise by separately computed gate logits."""
         parts = _gate_input_parts(getattr(self, "value_gate_input_mode", "current"))
         if ops.coupled_proj_scan_supported(self.d_model, self.r, "prev" in parts):
-            with torch.autograd.profiler.record_function("mogt.affine_scan"):
+            with _range("mogt.affine_scan"):
                 proj, gate_prev, gconst = self._value_and_gate_projection(xn, prefix_condition, packed=packed)
                 if gconst is not None:
                     gconst = gconst.expand(xn.size(0), self.r).contiguous()
                 h = ops.coupled_proj_scan(proj, self.d_model, rank=self.r, gate_prev=gate_prev, gate_const=gconst,
                                           damping=damping)
         else:
-            with torch.autograd.profiler.record_function("mogt.value_projection"):
+            with _range("mogt.value_projection"):
                 v_raw = F.linear(xn, _gemm_weight(self, "phi_val", (self.phi_val.weight,),
                                                   lambda: self.phi_val.weight))
                 z = self._gate_logits(xn, prefix_condition)
-            with torch.autograd.profiler.record_function("mogt.affine_scan"):
+            with _range("mogt.affine_scan"):
                 h = ops.coupled_rank_scan(z, v_raw, damping=damping, out_dtype=torch.float32)
-        with torch.autograd.profiler.record_function("mogt.readout"):
+        with _range("mogt.readout"):
             hn = ops.rmsnorm(h, self.norm_out.weight, self.norm_out.eps, out_dtype=gemm_dtype)
             Wr = packed["theta"] if packed is not None else _gemm_weight(self, "theta_read", (self.theta_read.weight,),
                                                                            lambda: self.theta_read.weight)
@@ -543,7 +564,7 @@ class MOGTBlock(_WeightCacheOwner):
             x, xn2 = self._mixer_training(x, xn, prefix_condition, damping, gemm_dtype, packed)
         else:
             x, xn2 = self._mixer_inference(x, xn, prefix_condition, damping, gemm_dtype, gate_const)
-        with torch.autograd.profiler.record_function("mogt.ffn"):
+        with _range("mogt.ffn"):
             f = self.ffn(xn2) if packed is None else self.ffn.forward_with(xn2, packed["w12"], packed["w3"])
         return x, (f, float(getattr(self, "mogt_ffn_residual_scale", 1.0)))
 
@@ -567,8 +588,10 @@ class MOGTModel(_WeightCacheOwner):
         in one), instead of a cast kernel per weight and the fp32
         concatenations; a list of None otherwise."""
         ad = _autocast_dtype()
+        if not torch.is_grad_enabled() or ad is None:
+            return [None] * len(self.blocks)
         groups = [blk.training_weight_groups() for blk in self.blocks]
-        if not torch.is_grad_enabled() or ad is None or any(g is None for g in groups):
+        if any(g is None for g in groups):
             return [None] * len(self.blocks)
         outs = ops.cast_groups([grp for g in groups for grp in g], ad)
         packed, i = [], 0
@@ -678,6 +701,17 @@ class MOGTForCausalLM(_WeightCacheOwner):
             blk.theta_read.weight.zero_()
             blk.ffn.w3.weight.zero_()
 
+    def _lm_logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        """``lm_head(hidden)``; without gradients the head's autocast weight (a
+        cast of the whole table, 27 us at 32000 x 768) is kept until the weight
+        changes, like the blocks' GEMM operands."""
+        head = self.lm_head
+        plain = type(head) is nn.Linear and not (head._forward_hooks or head._forward_pre_hooks or
+                                                 head._backward_hooks or head._backward_pre_hooks)
+        if not plain or head.bias is not None or torch.is_grad_enabled() or _autocast_dtype() is None:
+            return head(hidden)
+        return F.linear(hidden, _gemm_weight(self, "lm_head", (head.weight,), lambda: head.weight))
+
     def forward(self, input_ids, labels=None, *, return_logits=True, loss_chunk_size=0):
         """model_mogt.py:350-380.  Without labels: logits.  With labels and
         ``loss_chunk_size <= 0``: F.cross_entropy over the full logits (mean
@@ -687,11 +721,11 @@ class MOGTForCausalLM(_WeightCacheOwner):
         logits through chunked_linear_cross_entropy."""
         hidden = self.mogt(input_ids)
         chunk = int(loss_chunk_size or 0)
-        with torch.autograd.profiler.record_function("mogt.lm_head_loss"):
+        with _range("mogt.lm_head_loss"):
             if labels is not None and chunk > 0 and not return_logits:
                 return None, chunked_linear_cross_entropy(hidden, self.lm_head.weight, labels,
                                                           chunk_size=chunk)
-            logits = self.lm_head(hidden)
+            logits = self._lm_logits(hidden)
             loss = None
             if labels is not None:
                 flat_logits = logits.reshape(-1, logits.size(-1))

@@ -1,7 +1,8 @@
 """PyTorch custom ops (``torch.ops.mogt.*``) over the HIP C-ABI library.
 
 Each op validates its inputs with the reference's ``ValueError`` conditions,
-allocates outputs through the PyTorch caching allocator, and enqueues the HIP
+runs directly on plain eager tensors and through the dispatcher otherwise
+(``_Op``), allocates outputs through the PyTorch caching allocator, and enqueues the HIP
 kernel on the current stream.  The native library never allocates: single-pass
 scans get a persistent, zero-initialised workspace per (device, stream) that
 the kernels leave reusable after every launch.
@@ -9,6 +10,7 @@ the kernels leave reusable after every launch.
 from __future__ import annotations
 
 import ctypes
+import inspect
 import os
 import threading
 import warnings
@@ -51,7 +53,8 @@ def dtype_code(dt: torch.dtype, what: str) -> int:
 
 
 def _stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 # Workspace families.  "plain" holds data that the kernels read back only in
@@ -155,16 +158,79 @@ def _checked(ws: torch.Tensor, what: str) -> None:
             raise WorkspaceFault(f"{what}: {n} look-back wait(s) gave up; the output is invalid (NaN)")
 
 
-def _direct(*tensors: torch.Tensor) -> bool:
-    """Whether a public op may call its implementation directly: a plain eager
-    call on real tensors with no autograd recording and no compiler tracing,
-    where the custom-op dispatch would only add host time (about 13 us per
-    call, more than a short scan's kernel).  Everything else goes through
-    ``torch.ops.mogt.*`` (autograd, fake tensors, torch.compile)."""
-    if torch.compiler.is_compiling():
+def _plain(args: tuple) -> bool:
+    """Whether an op's arguments make a plain eager call: ordinary tensors, no
+    compiler or tracer, no functorch transform, no dispatch or function mode,
+    no forward-mode level, nothing left to materialise (negation bit)."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None):
         return False
-    grad = torch.is_grad_enabled()
-    return all(type(t) is torch.Tensor and not (grad and t.requires_grad) for t in tensors)
+    for a in args:
+        if isinstance(a, torch.Tensor) and ((type(a) is not torch.Tensor and type(a) is not torch.nn.Parameter)
+                                            or a.is_neg()):
+            return False
+    return True
+
+
+class _Op:
+    """A custom op (``torch.ops.mogt.<name>``) and its direct call.
+
+    The Python custom-op dispatch costs about 13 us of host time per call, and
+    its generated autograd wrapper about 40 -- more than most of these kernels
+    at short lengths (a 4-layer forward of 256 tokens has 30 such calls).  A
+    plain eager call (``_plain``) therefore runs the implementation directly or,
+    where a gradient is recorded, through an autograd function of the op's own
+    setup and backward (what the generated wrapper contains).  Every other call
+    goes through the dispatcher."""
+
+    def __init__(self, qualname: str, impl, mutates: tuple):
+        self.impl = impl
+        self.mutates = mutates
+        self.custom = torch.library.custom_op(qualname, impl, mutates_args=mutates)
+        self.dispatched = getattr(torch.ops.mogt, qualname.split("::")[1])
+        self.function = None
+        self.register_fake = self.custom.register_fake
+
+    def register_autograd(self, backward, setup_context) -> None:
+        self.custom.register_autograd(backward, setup_context=setup_context)
+        impl = self.impl
+
+        # the setup runs inside forward: with a setup_context of its own, apply()
+        # binds the arguments to forward's signature anew on every call (20 us)
+        class Function(torch.autograd.Function):
+            @staticmethod
+            def forward(ctx, *args):
+                out = impl(*args)
+                setup_context(ctx, args, out)
+                return out
+
+        Function.backward = staticmethod(backward)
+        Function.__name__ = Function.__qualname__ = self.custom._name
+        self.function = Function
+
+    def __call__(self, *args):
+        if not _plain(args):
+            return self.dispatched(*args)
+        if torch.is_grad_enabled():
+            for a in args:
+                if isinstance(a, torch.Tensor) and a.requires_grad:
+                    return self.dispatched(*args) if self.function is None else self.function.apply(*args)
+        out = self.impl(*args)
+        for i in self.mutates:   # what the dispatcher records for a written argument
+            if not args[i].is_inference():
+                torch.autograd.graph.increment_version(args[i])
+        return out
+
+
+def _op(qualname: str, mutates: tuple = ()):
+    """Decorator: the function as an ``_Op``; ``mutates`` names written arguments."""
+    def wrap(impl):
+        order = list(inspect.signature(impl).parameters)
+        op = _Op(qualname, impl, mutates)
+        op.mutates = tuple(order.index(m) for m in mutates)
+        return op
+    return wrap
 
 
 def require_cuda(what: str, *tensors: torch.Tensor) -> None:
@@ -220,7 +286,7 @@ def _diag_scan_impl(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype) ->
     return h
 
 
-_diag_scan_op = torch.library.custom_op("mogt::diag_scan", _diag_scan_impl, mutates_args=())
+_diag_scan_op = _op("mogt::diag_scan")(_diag_scan_impl)
 
 
 @_diag_scan_op.register_fake
@@ -238,7 +304,7 @@ def _diag_scan_prefix_impl(a: torch.Tensor, b: torch.Tensor,
     return pre, h
 
 
-_diag_scan_prefix_op = torch.library.custom_op("mogt::diag_scan_prefix", _diag_scan_prefix_impl, mutates_args=())
+_diag_scan_prefix_op = _op("mogt::diag_scan_prefix")(_diag_scan_prefix_impl)
 
 
 @_diag_scan_prefix_op.register_fake
@@ -246,7 +312,7 @@ def _(a, b, out_dtype):
     return a.new_empty(a.shape, dtype=out_dtype), a.new_empty(a.shape, dtype=out_dtype)
 
 
-@torch.library.custom_op("mogt::diag_scan_rev", mutates_args=())
+@_op("mogt::diag_scan_rev")
 def _diag_scan_rev_op(a: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     """G_t = g_t + a_{t+1} G_{t+1} (G_L = 0) in fp32: the reverse-time scan of
     the diagonal scan's backward."""
@@ -271,7 +337,7 @@ def _(a, g):
     return a.new_empty(a.shape, dtype=torch.float32)
 
 
-@torch.library.custom_op("mogt::diag_scan_grad", mutates_args=())
+@_op("mogt::diag_scan_grad")
 def _diag_scan_grad_op(a: torch.Tensor, b: torch.Tensor, G: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """(da, db) of the diagonal scan from G: da_t = G_t h_{t-1}, the state
     recomputed in registers, in a's dtype; db is G in that dtype for bf16 and
@@ -315,10 +381,10 @@ def _diag_scan_backward(ctx, grad_h):
     that forms da."""
     a, b = ctx.saved_tensors
     need_a, need_b = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-    G = torch.ops.mogt.diag_scan_rev(a, grad_h)
+    G = _diag_scan_rev_op(a, grad_h)
     da = db = None
     if need_a:
-        da, db = torch.ops.mogt.diag_scan_grad(a, b, G)
+        da, db = _diag_scan_grad_op(a, b, G)
     if need_b:
         if db is None or a.dtype == torch.float32:
             db = G.to(b.dtype)
@@ -327,7 +393,7 @@ def _diag_scan_backward(ctx, grad_h):
     return da, db, None
 
 
-torch.library.register_autograd("mogt::diag_scan", _diag_scan_backward, setup_context=_diag_scan_setup)
+_diag_scan_op.register_autograd(_diag_scan_backward, _diag_scan_setup)
 
 
 def diag_scan(a: torch.Tensor, b: torch.Tensor, *, out_dtype: torch.dtype | None = None,
@@ -342,11 +408,9 @@ def diag_scan(a: torch.Tensor, b: torch.Tensor, *, out_dtype: torch.dtype | None
     _check_diag_inputs(a, b)
     out_dtype = out_dtype or b.dtype
     dtype_code(out_dtype, "diag_scan")
-    if _direct(a, b):
-        return _diag_scan_prefix_impl(a, b, out_dtype) if return_prefix else _diag_scan_impl(a, b, out_dtype)
     if return_prefix:
-        return torch.ops.mogt.diag_scan_prefix(a, b, out_dtype)
-    return torch.ops.mogt.diag_scan(a, b, out_dtype)
+        return _diag_scan_prefix_op(a, b, out_dtype)
+    return _diag_scan_op(a, b, out_dtype)
 
 
 # ---------------------------------------------------------------------------
@@ -373,8 +437,7 @@ def _coupled_rank_scan_impl(z: torch.Tensor, v: torch.Tensor, rank: int, damping
     return h
 
 
-_coupled_rank_scan_op = torch.library.custom_op("mogt::coupled_rank_scan", _coupled_rank_scan_impl,
-                                                mutates_args=())
+_coupled_rank_scan_op = _op("mogt::coupled_rank_scan")(_coupled_rank_scan_impl)
 
 
 @_coupled_rank_scan_op.register_fake
@@ -382,7 +445,7 @@ def _(z, v, rank, damping, out_dtype):
     return v.new_empty(v.shape, dtype=out_dtype)
 
 
-@torch.library.custom_op("mogt::coupled_scan_rev", mutates_args=())
+@_op("mogt::coupled_scan_rev")
 def _coupled_scan_rev_op(z: torch.Tensor, grad_h: torch.Tensor, rank: int, damping: float) -> torch.Tensor:
     """G_t = dH_t + a_{t+1} G_{t+1} with a = damping (1 - sigmoid(z)) per rank,
     the decay formed from the gate logits inside the reverse scan."""
@@ -406,7 +469,7 @@ def _(z, grad_h, rank, damping):
     return grad_h.new_empty(grad_h.shape, dtype=torch.float32)
 
 
-@torch.library.custom_op("mogt::coupled_grad", mutates_args=())
+@_op("mogt::coupled_grad")
 def _coupled_grad_op(G: torch.Tensor, z: torch.Tensor, v: torch.Tensor, h: torch.Tensor, rank: int,
                      damping: float) -> tuple[torch.Tensor, torch.Tensor]:
     lib = _lib.load()
@@ -451,11 +514,11 @@ def _coupled_backward(ctx, grad_h):
     r, damping = ctx.rank, ctx.damping
     B, L, D = v.shape
     c = D // r
-    G = torch.ops.mogt.coupled_scan_rev(z, grad_h, r, damping)    # fp32 [B, L, D]
+    G = _coupled_scan_rev_op(z, grad_h, r, damping)    # fp32 [B, L, D]
     if c % 4 == 0 and D <= 4096:
         if h is None:   # the forward returned a rounded h: recompute the fp32 state
-            h = torch.ops.mogt.coupled_rank_scan(z, v, r, damping, torch.float32)
-        dv, dz = torch.ops.mogt.coupled_grad(G, z, v, h, r, damping)
+            h = _coupled_rank_scan_op(z, v, r, damping, torch.float32)
+        dv, dz = _coupled_grad_op(G, z, v, h, r, damping)
         return (dz.to(z.dtype) if ctx.needs_input_grad[0] else None,
                 dv if ctx.needs_input_grad[1] else None, None, None, None)
     g = torch.sigmoid(z.float())                                   # [B, L, r]
@@ -466,20 +529,20 @@ def _coupled_backward(ctx, grad_h):
         dv = (Gr * g_io.unsqueeze(-1)).reshape(B, L, D).to(v.dtype)
     if ctx.needs_input_grad[0]:
         if h is None:
-            h = torch.ops.mogt.coupled_rank_scan(z, v, r, damping, torch.float32)
+            h = _coupled_rank_scan_op(z, v, r, damping, torch.float32)
         hp = _shift_prev(h).view(B, L, r, c)
         dg = (Gr * v.float().view(B, L, r, c)).sum(-1) - damping * (Gr * hp).sum(-1)
         dz = (dg * g * (1.0 - g)).to(z.dtype)
     return dz, dv, None, None, None
 
 
-torch.library.register_autograd("mogt::coupled_rank_scan", _coupled_backward, setup_context=_coupled_setup)
+_coupled_rank_scan_op.register_autograd(_coupled_backward, _coupled_setup)
 
 
 STAT_GROUP = 64   # features per column of the coupled scan's row statistics
 
 
-@torch.library.custom_op("mogt::coupled_rank_scan_stats", mutates_args=())
+@_op("mogt::coupled_rank_scan_stats")
 def _coupled_rank_scan_stats_op(z: torch.Tensor, v: torch.Tensor, rank: int, damping: float,
                                 out_dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
     lib = _lib.load()
@@ -519,10 +582,10 @@ def coupled_rank_scan_stats(gate_logits: torch.Tensor, v_raw: torch.Tensor, *, d
     B, L, r = gate_logits.shape
     if v_raw.shape[:2] != (B, L) or v_raw.shape[2] % r != 0:
         raise ValueError("gate_logits must be [B, L, r] and v_raw [B, L, r*c]")
-    return torch.ops.mogt.coupled_rank_scan_stats(gate_logits, v_raw, r, float(damping), out_dtype)
+    return _coupled_rank_scan_stats_op(gate_logits, v_raw, r, float(damping), out_dtype)
 
 
-@torch.library.custom_op("mogt::coupled_rank_scan_proj", mutates_args=())
+@_op("mogt::coupled_rank_scan_proj")
 def _coupled_rank_scan_proj_op(proj: torch.Tensor, features: int, gate_prev: bool, gate_const: torch.Tensor | None,
                                rank: int, damping: float) -> tuple[torch.Tensor, torch.Tensor]:
     lib = _lib.load()
@@ -569,11 +632,11 @@ def coupled_rank_scan_proj(proj: torch.Tensor, features: int, *, rank: int, gate
         require_cuda("coupled_rank_scan_proj", gate_const)
         if gate_const.shape[-1] != rank or gate_const.ndim > 2:
             raise ValueError("gate_const must be [rank] or [B, rank]")
-    return torch.ops.mogt.coupled_rank_scan_proj(proj, int(features), bool(gate_prev), gate_const, int(rank),
+    return _coupled_rank_scan_proj_op(proj, int(features), bool(gate_prev), gate_const, int(rank),
                                                  float(damping))
 
 
-@torch.library.custom_op("mogt::coupled_proj_scan", mutates_args=())
+@_op("mogt::coupled_proj_scan")
 def _coupled_proj_scan_op(proj: torch.Tensor, gate_const: torch.Tensor | None, features: int, rank: int,
                           gate_prev: bool, damping: float) -> tuple[torch.Tensor, torch.Tensor]:
     """Training form of the projection-fed scan: fp32 h and the assembled
@@ -605,7 +668,7 @@ def _(proj, gate_const, features, rank, gate_prev, damping):
             proj.new_empty((B, L, rank), dtype=torch.float32))
 
 
-@torch.library.custom_op("mogt::coupled_proj_grad", mutates_args=())
+@_op("mogt::coupled_proj_grad")
 def _coupled_proj_grad_op(G: torch.Tensor, z: torch.Tensor, proj: torch.Tensor, h: torch.Tensor, features: int,
                           rank: int, gate_prev: bool, damping: float) -> tuple[torch.Tensor, torch.Tensor]:
     lib = _lib.load()
@@ -646,13 +709,13 @@ def _coupled_proj_backward(ctx, grad_h, grad_z):
     features, rank, gate_prev, damping = ctx.args
     if grad_h is None:
         return None, None, None, None, None, None
-    G = torch.ops.mogt.coupled_scan_rev(z, grad_h, rank, damping)
-    dproj, dz = torch.ops.mogt.coupled_proj_grad(G, z, proj, h, features, rank, gate_prev, damping)
+    G = _coupled_scan_rev_op(z, grad_h, rank, damping)
+    dproj, dz = _coupled_proj_grad_op(G, z, proj, h, features, rank, gate_prev, damping)
     dconst = dz.sum(1) if ctx.needs_input_grad[1] else None
     return dproj, dconst, None, None, None, None
 
 
-torch.library.register_autograd("mogt::coupled_proj_scan", _coupled_proj_backward, setup_context=_coupled_proj_setup)
+_coupled_proj_scan_op.register_autograd(_coupled_proj_backward, _coupled_proj_setup)
 
 
 def coupled_proj_scan(proj: torch.Tensor, features: int, *, rank: int, gate_prev: bool,
@@ -668,7 +731,7 @@ def coupled_proj_scan(proj: torch.Tensor, features: int, *, rank: int, gate_prev
         raise ValueError("proj must be [B, L, features + rank * (1 + gate_prev)]")
     if gate_const is not None and tuple(gate_const.shape) != (B, rank):
         raise ValueError("gate_const must be [B, rank]")
-    h, _ = torch.ops.mogt.coupled_proj_scan(proj, gate_const, int(features), int(rank), bool(gate_prev),
+    h, _ = _coupled_proj_scan_op(proj, gate_const, int(features), int(rank), bool(gate_prev),
                                             float(damping))
     return h
 
@@ -695,9 +758,7 @@ def coupled_rank_scan(gate_logits: torch.Tensor, v_raw: torch.Tensor, *, damping
     B, L, r = gate_logits.shape
     if v_raw.shape[:2] != (B, L) or v_raw.shape[2] % r != 0:
         raise ValueError("gate_logits must be [B, L, r] and v_raw [B, L, r*c]")
-    if _direct(gate_logits, v_raw):
-        return _coupled_rank_scan_impl(gate_logits, v_raw, r, float(damping), out_dtype)
-    return torch.ops.mogt.coupled_rank_scan(gate_logits, v_raw, r, float(damping), out_dtype)
+    return _coupled_rank_scan_op(gate_logits, v_raw, r, float(damping), out_dtype)
 
 
 # ---------------------------------------------------------------------------
@@ -762,7 +823,7 @@ def _prep_uv(U: torch.Tensor, V: torch.Tensor) -> tuple[torch.Tensor, torch.Tens
     return U, V
 
 
-@torch.library.custom_op("mogt::affine_scan", mutates_args=())
+@_op("mogt::affine_scan")
 def _affine_scan_op(U: torch.Tensor, V: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     U, V = _prep_uv(U, V)
     H = torch.empty(V.shape, dtype=out_dtype, device=V.device)
@@ -775,7 +836,7 @@ def _(U, V, out_dtype):
     return V.new_empty(V.shape, dtype=out_dtype)
 
 
-@torch.library.custom_op("mogt::affine_scan_prefix", mutates_args=())
+@_op("mogt::affine_scan_prefix")
 def _affine_scan_prefix_op(U: torch.Tensor, V: torch.Tensor,
                            out_dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
     U, V = _prep_uv(U, V)
@@ -790,7 +851,7 @@ def _(U, V, out_dtype):
     return U.new_empty(U.shape, dtype=out_dtype), V.new_empty(V.shape, dtype=out_dtype)
 
 
-@torch.library.custom_op("mogt::affine_scan_generic", mutates_args=())
+@_op("mogt::affine_scan_generic")
 def _affine_scan_generic_op(U: torch.Tensor, V: torch.Tensor, state_dtype: torch.dtype,
                             out_dtype: torch.dtype, with_prefix: bool,
                             reverse: bool) -> tuple[torch.Tensor, torch.Tensor]:
@@ -828,13 +889,13 @@ def _forward_state(U: torch.Tensor, V: torch.Tensor, state_dtype: torch.dtype, p
     """H (and U_prefix) kept in the state dtype, as the backward needs them."""
     if _use_mfma(U.shape[-1], state_dtype, state_dtype):
         if prefix:
-            return torch.ops.mogt.affine_scan_prefix(U, V, state_dtype)
-        return torch.ops.mogt.affine_scan(U, V, state_dtype)
-    P, H = torch.ops.mogt.affine_scan_generic(U, V, state_dtype, state_dtype, prefix, False)
+            return _affine_scan_prefix_op(U, V, state_dtype)
+        return _affine_scan_op(U, V, state_dtype)
+    P, H = _affine_scan_generic_op(U, V, state_dtype, state_dtype, prefix, False)
     return (P, H) if prefix else H
 
 
-@torch.library.custom_op("mogt::affine_scan_rev", mutates_args=())
+@_op("mogt::affine_scan_rev")
 def _affine_scan_rev_op(U: torch.Tensor, X: torch.Tensor) -> torch.Tensor:
     """G_t = X_t + U_{t+1}^T G_{t+1} on the matrix-core pipeline (fp32, R <= 32):
     time walked backwards and U_{t+1} read transposed inside the kernels."""
@@ -854,7 +915,7 @@ def _(U, X):
     return torch.empty_like(X)
 
 
-@torch.library.custom_op("mogt::affine_scan_grad_u", mutates_args=())
+@_op("mogt::affine_scan_grad_u")
 def _affine_scan_grad_u_op(G: torch.Tensor, H: torch.Tensor, P: torch.Tensor | None) -> torch.Tensor:
     """dU_t = G_t M_{t-1}^T with M = H or [H | P], M_{-1} = [0 | I] (fp32)."""
     lib = _lib.load()
@@ -877,7 +938,7 @@ def _(G, H, P):
 GRADU_MAX_CHANNELS = 64   # one column block of the recomputing gradient pass
 
 
-@torch.library.custom_op("mogt::affine_scan_recompute_grad_u", mutates_args=())
+@_op("mogt::affine_scan_recompute_grad_u")
 def _affine_scan_recompute_grad_u_op(U: torch.Tensor, V: torch.Tensor, G: torch.Tensor) -> torch.Tensor:
     """dU_t = G_t H_{t-1}^T (fp32), H recomputed from U and V: inside the pass
     that forms dU where its layout allows, else written and read back."""
@@ -888,7 +949,7 @@ def _affine_scan_recompute_grad_u_op(U: torch.Tensor, V: torch.Tensor, G: torch.
     if C % 8 != 0 or not 0 < C <= GRADU_MAX_CHANNELS or (V.data_ptr() | G.data_ptr()) % 16 != 0:
         H = torch.empty(V.shape, dtype=torch.float32, device=V.device)
         _affine_launch(U, V, H, None)
-        return torch.ops.mogt.affine_scan_grad_u(G, H, None)
+        return _affine_scan_grad_u_op(G, H, None)
     dU = torch.empty(B, L, R, R, dtype=torch.float32, device=G.device)
     ws = workspace(lib.mogt_affine_scan_workspace_bytes(B, L, R, C), G.device)
     rc = lib.mogt_affine_scan_recompute_grad_u(U.data_ptr(), V.data_ptr(), G.data_ptr(), dU.data_ptr(), B, L, R, C,
@@ -910,8 +971,8 @@ def _reverse_scan(U: torch.Tensor, X: torch.Tensor, state_dtype: torch.dtype) ->
     otherwise."""
     R = U.shape[-1]
     if _use_mfma(R, state_dtype, state_dtype):
-        return torch.ops.mogt.affine_scan_rev(U.to(torch.float32), X.to(torch.float32))
-    _, G = torch.ops.mogt.affine_scan_generic(U, X, state_dtype, state_dtype, False, True)
+        return _affine_scan_rev_op(U.to(torch.float32), X.to(torch.float32))
+    _, G = _affine_scan_generic_op(U, X, state_dtype, state_dtype, False, True)
     return G
 
 
@@ -936,9 +997,9 @@ def affine_scan_grad(U: torch.Tensor, V: torch.Tensor, grad_H: torch.Tensor | No
             # dU from the recomputed forward state read in place (shifted by a step)
             if grad_P is not None:
                 P, H = _forward_state(U, V, state_dtype, True)
-                grad_u = torch.ops.mogt.affine_scan_grad_u(G, H, P)
+                grad_u = _affine_scan_grad_u_op(G, H, P)
             else:
-                grad_u = torch.ops.mogt.affine_scan_recompute_grad_u(U, V, G)
+                grad_u = _affine_scan_recompute_grad_u_op(U, V, G)
             return grad_u.to(U.dtype), grad_v
         zeros = torch.zeros(B, 1, R, C, dtype=state_dtype, device=V.device)
         if grad_P is not None:
@@ -990,11 +1051,9 @@ def _generic_backward(ctx, grad_P, grad_H):
     return gu, gv, None, None, None, None
 
 
-torch.library.register_autograd("mogt::affine_scan", _affine_backward, setup_context=_affine_setup)
-torch.library.register_autograd("mogt::affine_scan_prefix", _affine_prefix_backward,
-                                setup_context=_affine_setup)
-torch.library.register_autograd("mogt::affine_scan_generic", _generic_backward,
-                                setup_context=_generic_setup)
+_affine_scan_op.register_autograd(_affine_backward, _affine_setup)
+_affine_scan_prefix_op.register_autograd(_affine_prefix_backward, _affine_setup)
+_affine_scan_generic_op.register_autograd(_generic_backward, _generic_setup)
 
 
 def affine_scan(U: torch.Tensor, V: torch.Tensor, *, output_dtype: torch.dtype | None = None,
@@ -1014,9 +1073,9 @@ def affine_scan(U: torch.Tensor, V: torch.Tensor, *, output_dtype: torch.dtype |
         raise ValueError(f"output dtype {output_dtype} not supported (float32, bfloat16, float16, float64)")
     if _use_mfma(R, state_dtype, output_dtype):
         if return_prefix:
-            return torch.ops.mogt.affine_scan_prefix(U, V, output_dtype)
-        return torch.ops.mogt.affine_scan(U, V, output_dtype)
-    P, H = torch.ops.mogt.affine_scan_generic(U, V, state_dtype, output_dtype, return_prefix, False)
+            return _affine_scan_prefix_op(U, V, output_dtype)
+        return _affine_scan_op(U, V, output_dtype)
+    P, H = _affine_scan_generic_op(U, V, state_dtype, output_dtype, return_prefix, False)
     return (P, H) if return_prefix else H
 
 
@@ -1034,7 +1093,7 @@ def check_vk_shapes(U: torch.Tensor, v: torch.Tensor, k: torch.Tensor) -> tuple[
     return B, L, R, k.shape[-1]
 
 
-@torch.library.custom_op("mogt::affine_scan_vk", mutates_args=())
+@_op("mogt::affine_scan_vk")
 def _affine_scan_vk_op(U: torch.Tensor, v: torch.Tensor, k: torch.Tensor,
                        out_dtype: torch.dtype) -> torch.Tensor:
     B, L, R, C = check_vk_shapes(U, v, k)
@@ -1082,10 +1141,10 @@ def dense_scan(A: torch.Tensor, Bm: torch.Tensor | None = None, *, v: torch.Tens
         # products (as the in-register form does) and scanned by the generic kernel
         Bm = v.to(torch.float32).unsqueeze(-1) * k.to(torch.float32).unsqueeze(-2)
         return affine_scan(A, Bm, output_dtype=output_dtype)
-    return torch.ops.mogt.affine_scan_vk(A, v, k, output_dtype)
+    return _affine_scan_vk_op(A, v, k, output_dtype)
 
 
-@torch.library.custom_op("mogt::fused_scan", mutates_args=())
+@_op("mogt::fused_scan")
 def _fused_scan_op(U: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     Uf = U.contiguous().to(torch.float32)
     Y = torch.empty(U.shape, dtype=out_dtype, device=U.device)
@@ -1110,14 +1169,14 @@ def fused_scan(U: torch.Tensor, *, output_dtype: torch.dtype | None = None) -> t
     if output_dtype not in _GENERIC_CODE:
         raise ValueError(f"output dtype {output_dtype} not supported (float32, bfloat16, float16, float64)")
     if R <= MFMA_MAX_RANK and output_dtype in _DTYPE_CODE:
-        return torch.ops.mogt.fused_scan(U, output_dtype)
+        return _fused_scan_op(U, output_dtype)
     # the generic scan's prefix columns with no channels: Y_t = U_t Y_{t-1}, Y_0 = I
-    Y, _ = torch.ops.mogt.affine_scan_generic(U, U.new_empty((B, L, R, 0), dtype=torch.float32),
+    Y, _ = _affine_scan_generic_op(U, U.new_empty((B, L, R, 0), dtype=torch.float32),
                                               torch.float32, output_dtype, True, False)
     return Y
 
 
-@torch.library.custom_op("mogt::affine_local_scan", mutates_args=())
+@_op("mogt::affine_local_scan")
 def _affine_local_scan_op(U: torch.Tensor, V: torch.Tensor, block_size: int
                           ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     lib = _lib.load()
@@ -1148,7 +1207,7 @@ def _(U, V, block_size):
             U.new_empty((B, nb, R, R), **f), V.new_empty((B, nb, R, C), **f))
 
 
-@torch.library.custom_op("mogt::affine_local_scan_generic", mutates_args=())
+@_op("mogt::affine_local_scan_generic")
 def _affine_local_scan_generic_op(U: torch.Tensor, V: torch.Tensor, block_size: int
                                   ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """The block-local scan on the generic kernel (R > 32), fp32 like the
@@ -1188,14 +1247,14 @@ def affine_local_scan(U: torch.Tensor, V: torch.Tensor, *, block_size: int = 256
     if block_size <= 0:
         raise ValueError("block_size must be positive")
     if R > MFMA_MAX_RANK:
-        return torch.ops.mogt.affine_local_scan_generic(U, V, int(block_size))
-    return torch.ops.mogt.affine_local_scan(U, V, int(block_size))
+        return _affine_local_scan_generic_op(U, V, int(block_size))
+    return _affine_local_scan_op(U, V, int(block_size))
 
 
 # ---------------------------------------------------------------------------
 # row-wise block kernels: rmsnorm, residual-add + rmsnorm, silu-mul
 # ---------------------------------------------------------------------------
-@torch.library.custom_op("mogt::rmsnorm", mutates_args=())
+@_op("mogt::rmsnorm")
 def _rmsnorm_op(x: torch.Tensor, weight: torch.Tensor, eps: float,
                 out_dtype: torch.dtype) -> torch.Tensor:
     lib = _lib.load()
@@ -1220,10 +1279,10 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6,
     """RMSNorm.forward (model_mogt.py:15-20) in one pass; ``out_dtype`` defaults
     to float32 (the dtype of ``normalised.type_as(x) * fp32 weight``)."""
     require_cuda("rmsnorm", x, weight)
-    return torch.ops.mogt.rmsnorm(x, weight, float(eps), out_dtype or torch.float32)
+    return _rmsnorm_op(x, weight, float(eps), out_dtype or torch.float32)
 
 
-@torch.library.custom_op("mogt::add_rmsnorm", mutates_args=())
+@_op("mogt::add_rmsnorm")
 def _add_rmsnorm_op(x: torch.Tensor, z: torch.Tensor, scale: float, weight: torch.Tensor, eps: float,
                     out_dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
     lib = _lib.load()
@@ -1254,10 +1313,10 @@ def add_rmsnorm(x: torch.Tensor, z: torch.Tensor, scale: float, weight: torch.Te
         raise ValueError("add_rmsnorm keeps the residual stream in float32")
     if x.shape != z.shape:
         raise ValueError("x and z must have the same shape")
-    return torch.ops.mogt.add_rmsnorm(x, z, float(scale), weight, float(eps), out_dtype)
+    return _add_rmsnorm_op(x, z, float(scale), weight, float(eps), out_dtype)
 
 
-@torch.library.custom_op("mogt::add_rmsnorm_final", mutates_args=())
+@_op("mogt::add_rmsnorm_final")
 def _add_rmsnorm_final_op(x: torch.Tensor, z: torch.Tensor, scale: float, weight: torch.Tensor, eps: float,
                           out_dtype: torch.dtype) -> torch.Tensor:
     lib = _lib.load()
@@ -1285,10 +1344,10 @@ def add_rmsnorm_final(x: torch.Tensor, z: torch.Tensor, scale: float, weight: to
     require_cuda("add_rmsnorm_final", x, z, weight)
     if x.dtype != torch.float32 or x.shape != z.shape:
         raise ValueError("add_rmsnorm_final: x float32 and z of the same shape")
-    return torch.ops.mogt.add_rmsnorm_final(x, z, float(scale), weight, float(eps), out_dtype)
+    return _add_rmsnorm_final_op(x, z, float(scale), weight, float(eps), out_dtype)
 
 
-@torch.library.custom_op("mogt::add_rmsnorm_rowscale", mutates_args=())
+@_op("mogt::add_rmsnorm_rowscale")
 def _add_rmsnorm_rowscale_op(x: torch.Tensor, z: torch.Tensor, stats: torch.Tensor, stat_eps: float, scale: float,
                              weight: torch.Tensor, eps: float, out_dtype: torch.dtype
                              ) -> tuple[torch.Tensor, torch.Tensor]:
@@ -1328,11 +1387,11 @@ def add_rmsnorm_rowscale(x: torch.Tensor, z: torch.Tensor, stats: torch.Tensor, 
         raise ValueError("add_rmsnorm_rowscale keeps the residual stream in float32")
     if x.shape != z.shape or stats.shape[:-1] != x.shape[:-1] or stats.dtype != torch.float32:
         raise ValueError("x and z must have the same shape and stats must be float32 [..., n_stats]")
-    return torch.ops.mogt.add_rmsnorm_rowscale(x, z, stats, float(stat_eps), float(scale), weight, float(eps),
+    return _add_rmsnorm_rowscale_op(x, z, stats, float(stat_eps), float(scale), weight, float(eps),
                                                out_dtype)
 
 
-@torch.library.custom_op("mogt::silu_mul", mutates_args=())
+@_op("mogt::silu_mul")
 def _silu_mul_op(y: torch.Tensor) -> torch.Tensor:
     lib = _lib.load()
     y = y.contiguous()
@@ -1349,7 +1408,7 @@ def _(y):
     return y.new_empty((*y.shape[:-1], y.shape[-1] // 2))
 
 
-@torch.library.custom_op("mogt::swiglu_gate", mutates_args=())
+@_op("mogt::swiglu_gate")
 def _swiglu_gate_op(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:
     lib = _lib.load()
     x = x if x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 else x.contiguous()
@@ -1391,7 +1450,7 @@ def swiglu_gate(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor) -> to
     if not swiglu_gate_supported(x, w_gate, w_up):
         raise ValueError("swiglu_gate needs bf16 x [..., K] and weights [H, K] with K % 32 == 0, H % 128 == 0")
     lead = x.shape[:-1]
-    y = torch.ops.mogt.swiglu_gate(x.reshape(-1, x.shape[-1]), w_gate, w_up)
+    y = _swiglu_gate_op(x.reshape(-1, x.shape[-1]), w_gate, w_up)
     return y.reshape(*lead, w_gate.shape[0])
 
 
@@ -1423,7 +1482,7 @@ def _linear_wgrad_impl(dy: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype
     return dw
 
 
-@torch.library.custom_op("mogt::linear_wgrad", mutates_args=())
+@_op("mogt::linear_wgrad")
 def _linear_wgrad_op(dy: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype, splits: int = 0) -> torch.Tensor:
     """dW = dY^T X over the flattened leading dimensions."""
     return _linear_wgrad_impl(dy, x, out_dtype, splits)
@@ -1453,9 +1512,7 @@ def linear_wgrad(dy: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype = tor
     if not linear_wgrad_supported(dy, x):
         raise ValueError("linear_wgrad needs bf16 dy [..., O] and x [..., I] with equal leading shapes and "
                          "O % 8 == 0, I % 8 == 0")
-    if _direct(dy, x):
-        return _linear_wgrad_impl(dy, x, out_dtype, int(splits))
-    return torch.ops.mogt.linear_wgrad(dy, x, out_dtype, int(splits))
+    return _linear_wgrad_op(dy, x, out_dtype, int(splits))
 
 
 class _Linear(torch.autograd.Function):
@@ -1474,7 +1531,7 @@ class _Linear(torch.autograd.Function):
         dx = g.matmul(w) if ctx.needs_input_grad[0] else None
         dw = None
         if ctx.needs_input_grad[1]:
-            dw = torch.ops.mogt.linear_wgrad(g, x, w.dtype, 0) if linear_wgrad_supported(g, x) \
+            dw = _linear_wgrad_op(g, x, w.dtype, 0) if linear_wgrad_supported(g, x) \
                 else g.reshape(-1, g.shape[-1]).t().mm(x.reshape(-1, x.shape[-1]))
         return dx, dw
 
@@ -1502,7 +1559,7 @@ def _rows_for_embedding_bwd(grad: torch.Tensor, D: int) -> torch.Tensor:
     return g
 
 
-@torch.library.custom_op("mogt::embedding_bwd", mutates_args=())
+@_op("mogt::embedding_bwd")
 def _embedding_bwd_op(grad: torch.Tensor, ids: torch.Tensor, vocab: int, grad2: torch.Tensor | None = None,
                       ids2: torch.Tensor | None = None) -> torch.Tensor:
     """fp32 [vocab, D] gradient of the table from the rows of ``grad`` at
@@ -1555,7 +1612,7 @@ class _Embedding(torch.autograd.Function):
             grad_out2 = None
         if grad_out is None:
             return None, None, None
-        dw = torch.ops.mogt.embedding_bwd(grad_out, ids, ctx.vocab, grad_out2, ids2 if grad_out2 is not None else None)
+        dw = _embedding_bwd_op(grad_out, ids, ctx.vocab, grad_out2, ids2 if grad_out2 is not None else None)
         return dw.to(ctx.wdtype), None, None
 
 
@@ -1674,7 +1731,7 @@ def _rmsnorm_bwd_launch(x: torch.Tensor, weight: torch.Tensor, dy: torch.Tensor,
     return dx, dw
 
 
-@torch.library.custom_op("mogt::rmsnorm_bwd", mutates_args=())
+@_op("mogt::rmsnorm_bwd")
 def _rmsnorm_bwd_op(x: torch.Tensor, weight: torch.Tensor, dy: torch.Tensor, dres: torch.Tensor | None,
                     eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     return _rmsnorm_bwd_launch(x, weight, dy, dres, eps, None, 0.0)
@@ -1685,7 +1742,7 @@ def _(x, weight, dy, dres, eps):
     return torch.empty_like(x), x.new_empty(x.shape[-1], dtype=torch.float32)
 
 
-@torch.library.custom_op("mogt::add_rmsnorm_bwd", mutates_args=())
+@_op("mogt::add_rmsnorm_bwd")
 def _add_rmsnorm_bwd_op(x_out: torch.Tensor, weight: torch.Tensor, dy: torch.Tensor, dres: torch.Tensor | None,
                         eps: float, scale: float, z_dtype: torch.dtype
                         ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -1710,11 +1767,11 @@ def _rmsnorm_setup(ctx, inputs, output):
 
 def _rmsnorm_backward(ctx, g):
     x, weight = ctx.saved_tensors
-    dx, dw = torch.ops.mogt.rmsnorm_bwd(x, weight, g, None, ctx.eps)
+    dx, dw = _rmsnorm_bwd_op(x, weight, g, None, ctx.eps)
     return dx, dw.to(weight.dtype), None, None
 
 
-torch.library.register_autograd("mogt::rmsnorm", _rmsnorm_backward, setup_context=_rmsnorm_setup)
+_rmsnorm_op.register_autograd(_rmsnorm_backward, _rmsnorm_setup)
 
 
 def _add_rmsnorm_setup(ctx, inputs, output):
@@ -1737,15 +1794,15 @@ def _add_rmsnorm_backward(ctx, g_xout, g_out):
         dz = (dx * float(ctx.scale)).to(ctx.z_dtype)
         dw = torch.zeros(x_out.shape[-1], dtype=weight.dtype, device=x_out.device)
         return dx, dz, None, dw, None, None
-    dx, dz, dw = torch.ops.mogt.add_rmsnorm_bwd(x_out, weight, g_out, g_xout, ctx.eps, float(ctx.scale),
+    dx, dz, dw = _add_rmsnorm_bwd_op(x_out, weight, g_out, g_xout, ctx.eps, float(ctx.scale),
                                                 ctx.z_dtype)
     return dx, dz, None, dw.to(weight.dtype), None, None
 
 
-torch.library.register_autograd("mogt::add_rmsnorm", _add_rmsnorm_backward, setup_context=_add_rmsnorm_setup)
+_add_rmsnorm_op.register_autograd(_add_rmsnorm_backward, _add_rmsnorm_setup)
 
 
-@torch.library.custom_op("mogt::silu_mul_bwd", mutates_args=())
+@_op("mogt::silu_mul_bwd")
 def _silu_mul_bwd_op(y: torch.Tensor, dout: torch.Tensor) -> torch.Tensor:
     lib = _lib.load()
     y = y.contiguous()
@@ -1769,10 +1826,10 @@ def _silu_mul_setup(ctx, inputs, output):
 
 def _silu_mul_backward(ctx, g):
     (y,) = ctx.saved_tensors
-    return torch.ops.mogt.silu_mul_bwd(y, g)
+    return _silu_mul_bwd_op(y, g)
 
 
-torch.library.register_autograd("mogt::silu_mul", _silu_mul_backward, setup_context=_silu_mul_setup)
+_silu_mul_op.register_autograd(_silu_mul_backward, _silu_mul_setup)
 
 
 def silu_mul(y: torch.Tensor) -> torch.Tensor:
@@ -1780,7 +1837,7 @@ def silu_mul(y: torch.Tensor) -> torch.Tensor:
     require_cuda("silu_mul", y)
     if y.shape[-1] % 8 != 0:
         raise ValueError("silu_mul needs an even hidden size that is a multiple of 4")
-    return torch.ops.mogt.silu_mul(y)
+    return _silu_mul_op(y)
 
 
 # ---------------------------------------------------------------------------
@@ -1789,7 +1846,7 @@ def silu_mul(y: torch.Tensor) -> torch.Tensor:
 _CONN_IMPL = {"matrix_exp": _lib.MOGT_CONN_EXP, "cayley": _lib.MOGT_CONN_CAYLEY}
 
 
-@torch.library.custom_op("mogt::connection_map", mutates_args=())
+@_op("mogt::connection_map")
 def _connection_map_op(A: torch.Tensor, impl: int, scale: float, damping: float,
                        out_dtype: torch.dtype) -> torch.Tensor:
     lib = _lib.load()
@@ -1815,7 +1872,7 @@ def _connection_map_setup(ctx, inputs, output):
     ctx.args = (impl, scale, damping)
 
 
-@torch.library.custom_op("mogt::connection_map_bwd", mutates_args=())
+@_op("mogt::connection_map_bwd")
 def _connection_map_bwd_op(A: torch.Tensor, grad_u: torch.Tensor, impl: int, scale: float,
                            damping: float) -> torch.Tensor:
     """dA of ``connection_map`` (fp32 arithmetic, in A's dtype)."""
@@ -1839,12 +1896,11 @@ def _connection_map_backward(ctx, grad_u):
     (A,) = ctx.saved_tensors
     # a constant for any higher derivative
     with torch.no_grad():
-        gA = torch.ops.mogt.connection_map_bwd(A, grad_u, *ctx.args)
+        gA = _connection_map_bwd_op(A, grad_u, *ctx.args)
     return gA, None, None, None, None
 
 
-torch.library.register_autograd("mogt::connection_map", _connection_map_backward,
-                                setup_context=_connection_map_setup)
+_connection_map_op.register_autograd(_connection_map_backward, _connection_map_setup)
 
 
 def connection_map(A: torch.Tensor, impl: str, *, scale: float = 1.0, damping: float = 1.0,
@@ -1860,7 +1916,7 @@ def connection_map(A: torch.Tensor, impl: str, *, scale: float = 1.0, damping: f
         raise ValueError("A must be [..., r, r]")
     if A.shape[-1] > 32:
         raise ValueError(f"r = {A.shape[-1]} not supported by the MI355X connection map (r <= 32)")
-    return torch.ops.mogt.connection_map(A, _CONN_IMPL[impl], float(scale), float(damping), out_dtype)
+    return _connection_map_op(A, _CONN_IMPL[impl], float(scale), float(damping), out_dtype)
 
 
 # ---------------------------------------------------------------------------
@@ -1923,7 +1979,7 @@ def _rank1_impl(f: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q: torch.Tens
     return y
 
 
-_rank1_op = torch.library.custom_op("mogt::rank1_coupled_scan", _rank1_impl, mutates_args=())
+_rank1_op = _op("mogt::rank1_coupled_scan")(_rank1_impl)
 
 
 @_rank1_op.register_fake
@@ -1951,9 +2007,7 @@ def rank1_coupled_scan(f: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q: tor
         raise ValueError("k, v and q must share a dtype")
     if k.shape[-1] != 64:
         raise ValueError(f"head dim {k.shape[-1]} not supported (64)")
-    if _direct(f, k, v, q):
-        return _rank1_impl(f, k, v, q, out_dtype or q.dtype, RANK1_PATHS[path])
-    return torch.ops.mogt.rank1_coupled_scan(f, k, v, q, out_dtype or q.dtype, RANK1_PATHS[path])
+    return _rank1_op(f, k, v, q, out_dtype or q.dtype, RANK1_PATHS[path])
 
 
 # ---------------------------------------------------------------------------
@@ -1968,7 +2022,7 @@ def _check_ce_rows(logits: torch.Tensor, labels: torch.Tensor, what: str) -> Non
     dtype_code(logits.dtype, what)
 
 
-@torch.library.custom_op("mogt::lm_ce_fwd", mutates_args=())
+@_op("mogt::lm_ce_fwd")
 def _lm_ce_fwd_op(logits: torch.Tensor, labels: torch.Tensor,
                   ignore_index: int) -> tuple[torch.Tensor, torch.Tensor]:
     lib = _lib.load()
@@ -1994,10 +2048,10 @@ def lm_ce_forward(logits: torch.Tensor, labels: torch.Tensor, *, ignore_index: i
     fp32 [rows]; ``loss = logsumexp(logits) - logits[label]`` (0 where the label
     is ``ignore_index``), as F.cross_entropy(..., reduction="none")."""
     _check_ce_rows(logits, labels, "lm_ce_forward")
-    return torch.ops.mogt.lm_ce_fwd(logits, labels, int(ignore_index))
+    return _lm_ce_fwd_op(logits, labels, int(ignore_index))
 
 
-@torch.library.custom_op("mogt::lm_ce_bwd_", mutates_args=("logits",))
+@_op("mogt::lm_ce_bwd_", mutates=("logits",))
 def _lm_ce_bwd_op(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Tensor, scale: torch.Tensor,
                   ignore_index: int) -> None:
     lib = _lib.load()
@@ -2016,7 +2070,7 @@ def _(logits, labels, lse, scale, ignore_index):
     return None
 
 
-@torch.library.custom_op("mogt::lm_ce_grad", mutates_args=())
+@_op("mogt::lm_ce_grad")
 def _lm_ce_grad_op(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Tensor, scale: torch.Tensor,
                    ignore_index: int) -> torch.Tensor:
     lib = _lib.load()
@@ -2045,7 +2099,7 @@ def lm_ce_grad(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Tensor, sc
         raise ValueError("lm_ce_grad: lse must be float32 [rows]")
     if scale.numel() != 1 or scale.dtype != torch.float32 or scale.device != logits.device:
         raise ValueError("lm_ce_grad: scale must be a one-element float32 tensor on the logits' device")
-    return torch.ops.mogt.lm_ce_grad(logits, labels, lse, scale.reshape(1).contiguous(), int(ignore_index))
+    return _lm_ce_grad_op(logits, labels, lse, scale.reshape(1).contiguous(), int(ignore_index))
 
 
 def lm_ce_backward_(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Tensor,
@@ -2058,7 +2112,7 @@ def lm_ce_backward_(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Tenso
         raise ValueError("lm_ce_backward_: lse must be float32 [rows]")
     if scale.numel() != 1 or scale.dtype != torch.float32 or scale.device != logits.device:
         raise ValueError("lm_ce_backward_: scale must be a one-element float32 tensor on the logits' device")
-    torch.ops.mogt.lm_ce_bwd_(logits, labels, lse, scale.reshape(1).contiguous(), int(ignore_index))
+    _lm_ce_bwd_op(logits, labels, lse, scale.reshape(1).contiguous(), int(ignore_index))
     return logits
 
 
@@ -2076,7 +2130,7 @@ def _lm_ce_grad_pieces_impl(logits: torch.Tensor, labels: torch.Tensor, lse: tor
     return grad
 
 
-_lm_ce_grad_pieces_op = torch.library.custom_op("mogt::lm_ce_grad_pieces", _lm_ce_grad_pieces_impl, mutates_args=())
+_lm_ce_grad_pieces_op = _op("mogt::lm_ce_grad_pieces")(_lm_ce_grad_pieces_impl)
 
 
 @_lm_ce_grad_pieces_op.register_fake
@@ -2093,10 +2147,7 @@ def lm_ce_grad_pieces(logits: torch.Tensor, labels: torch.Tensor, lse: torch.Ten
         raise ValueError("lm_ce_grad_pieces: lse must be float32 [rows]")
     if scale.numel() != 1 or scale.dtype != torch.float32 or scale.device != logits.device:
         raise ValueError("lm_ce_grad_pieces: scale must be a one-element float32 tensor on the logits' device")
-    scale = scale.reshape(1).contiguous()
-    if _direct(logits, labels, lse, scale):
-        return _lm_ce_grad_pieces_impl(logits, labels, lse, scale, int(ignore_index))
-    return torch.ops.mogt.lm_ce_grad_pieces(logits, labels, lse, scale, int(ignore_index))
+    return _lm_ce_grad_pieces_op(logits, labels, lse, scale.reshape(1).contiguous(), int(ignore_index))
 
 
 # ---------------------------------------------------------------------------
@@ -2120,7 +2171,7 @@ def _split_pieces_impl(x: torch.Tensor) -> torch.Tensor:
     return out
 
 
-_split_pieces_op = torch.library.custom_op("mogt::split_pieces", _split_pieces_impl, mutates_args=())
+_split_pieces_op = _op("mogt::split_pieces")(_split_pieces_impl)
 
 
 @_split_pieces_op.register_fake
@@ -2134,7 +2185,7 @@ def split_pieces(x: torch.Tensor) -> torch.Tensor:
     require_cuda("split_pieces", x)
     if x.ndim != 2 or x.dtype != torch.float32:
         raise ValueError("split_pieces: x must be float32 [rows, cols]")
-    return _split_pieces_impl(x) if _direct(x) else torch.ops.mogt.split_pieces(x)
+    return _split_pieces_op(x)
 
 
 def _split_gemm_impl(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, k: int, k_slow_a: bool, k_slow_b: bool,
@@ -2150,7 +2201,7 @@ def _split_gemm_impl(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, k: int
     _lib.check(rc, "mogt_split_gemm")
 
 
-_split_gemm_op = torch.library.custom_op("mogt::split_gemm_", _split_gemm_impl, mutates_args=("out",))
+_split_gemm_op = _op("mogt::split_gemm_", mutates=("out",))(_split_gemm_impl)
 
 
 @_split_gemm_op.register_fake
@@ -2173,6 +2224,5 @@ def split_gemm_(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, k: int, *, 
                                  "[1 or 3, K, rows]")
     if out.ndim != 2 or out.stride(1) != 1:
         raise ValueError("split_gemm: out must be [M, N] with contiguous rows")
-    run = _split_gemm_impl if _direct(out, a, b) else torch.ops.mogt.split_gemm_
-    run(out, a, b, int(k), bool(k_slow_a), bool(k_slow_b), bool(accumulate))
+    _split_gemm_op(out, a, b, int(k), bool(k_slow_a), bool(k_slow_b), bool(accumulate))
     return out
