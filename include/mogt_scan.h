@@ -574,6 +574,23 @@ int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int pieces_a, i
                     int64_t ldb, int64_t plane_b, int pieces_b, int k_slow_b, void* C, int64_t ldc, int64_t M,
                     int64_t N, int64_t K, int accumulate, int out_dtype, int64_t splits, void* workspace,
                     size_t workspace_bytes, void* stream);
+/* K slices mogt_split_gemm would choose (cus <= 0: the current device's). */
+int64_t mogt_split_gemm_slices(int64_t M, int64_t N, int64_t K, int pieces_a, int pieces_b, int64_t cus);
+/* The logits product of rows A [M, K] against the vocabulary B [N, K] (both
+ * k_slow 0) with the cross-entropy rows in its epilogue, in one K slice:
+ *   fwd  loss_rows, lse_rows as mogt_lm_ce_fwd on those logits, which are not
+ *        written (workspace: mogt_split_ce_workspace_bytes);
+ *   bwd  the gradient pieces as mogt_lm_ce_bwd_pieces on them ([3][M][ld_grad],
+ *        ld_grad a multiple of 8, N <= ld_grad <= N rounded up to 128).       */
+size_t mogt_split_ce_workspace_bytes(int64_t M, int64_t N, int pieces_a, int pieces_b);
+int mogt_split_ce_fwd(const void* A, int64_t lda, int64_t plane_a, int pieces_a, const void* B, int64_t ldb,
+                      int64_t plane_b, int pieces_b, const int64_t* labels, int64_t M, int64_t N, int64_t K,
+                      int64_t ignore_index, float* loss_rows, float* lse_rows, void* workspace,
+                      size_t workspace_bytes, void* stream);
+int mogt_split_ce_bwd(const void* A, int64_t lda, int64_t plane_a, int pieces_a, const void* B, int64_t ldb,
+                      int64_t plane_b, int pieces_b, const int64_t* labels, const float* lse_rows, int64_t M,
+                      int64_t N, int64_t K, int64_t ignore_index, const float* scale, void* grad,
+                      int64_t ld_grad, void* stream);
 
 #ifdef __cplusplus
 }

@@ -181,6 +181,14 @@ SIGNATURES: dict[str, tuple] = {
     "mogt_split_gemm": (
         _c_int, [_c_void_p, _c_i64, _c_i64, _c_int, _c_int, _c_void_p, _c_i64, _c_i64, _c_int, _c_int, _c_void_p,
                  _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_i64, _c_void_p, _c_size, _c_void_p]),
+    "mogt_split_gemm_slices": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_i64]),
+    "mogt_split_ce_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_int, _c_int]),
+    "mogt_split_ce_fwd": (
+        _c_int, [_c_void_p, _c_i64, _c_i64, _c_int, _c_void_p, _c_i64, _c_i64, _c_int, _c_void_p, _c_i64, _c_i64,
+                 _c_i64, _c_i64, _c_void_p, _c_void_p, _c_void_p, _c_size, _c_void_p]),
+    "mogt_split_ce_bwd": (
+        _c_int, [_c_void_p, _c_i64, _c_i64, _c_int, _c_void_p, _c_i64, _c_i64, _c_int, _c_void_p, _c_void_p, _c_i64,
+                 _c_i64, _c_i64, _c_i64, _c_void_p, _c_void_p, _c_i64, _c_void_p]),
     "mogt_rank1_coupled_scan_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "mogt_rank1_coupled_scan_fwd": (
         _c_int,

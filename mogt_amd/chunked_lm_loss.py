@@ -21,8 +21,10 @@ How it runs here:
   with autocast off, as the reference's backward does.
 * fp32 GEMMs of blocks large enough (``_split_ok``) run on the bf16 matrix
   cores from exact three-piece splits of their fp32 operands
-  (``csrc/split_gemm.hip``); the gradient block is then written as its pieces.
-  The rest go to the BLAS library.
+  (``csrc/split_gemm.hip``), the cross-entropy rows in the logits product's
+  epilogue where one slice of it fills the GPU: the logits are then not
+  written, and the gradient block only as its pieces.  The rest go to the BLAS
+  library.
 * Labels equal to -100 (F.cross_entropy's default ``ignore_index``) add zero
   loss, as in the reference's forward, and a zero gradient row; the
   reference's backward subtracts 1 at column ``vocab - 100`` for them.
@@ -64,23 +66,26 @@ def _block_logits(rows: torch.Tensor, w32: torch.Tensor) -> torch.Tensor:
 
 
 # Where a block's fp32 GEMMs take the split form, in multiply-adds of one of
-# them (rows x vocab x D).  Below, both forms take the host time of their
-# launches, of which the split form has more (2048 x 4000 x 512, 2^32: 471 us a
-# forward and backward against the library's 452; fp32 hidden states 513
-# against 435); above, the matrix units decide (256 x 32000 x 768, 2^32.6: 481
-# against 690 us; 1024 rows: 896 against 2017; fp32 hidden states 1202 against
-# 2027).
-SPLIT_MIN_MACS = 6_000_000_000
+# them (rows x vocab x D).  Small heads take the host time of their launches in
+# both forms, of which the split form has fewer with its cross-entropy
+# epilogues (1024 x 4000 x 256, 2^30: 305 us a forward and backward against the
+# library's 344 - 374; below 2^30 the two cross) and more under autocast, whose
+# logits stay with the library (2048 x 4000 x 512, 2^32: 428 against 424).
+# Above, the matrix units decide (256 x 32000 x 768, 2^32.6: 355 against 682 us,
+# autocast 434 against 603; 1024 rows: 788 against 2023, autocast 803 against
+# 1555).
+SPLIT_MIN_MACS = 1 << 30
+SPLIT_MIN_MACS_AUTOCAST = 6_000_000_000
 
 
-def _split_ok(rows: torch.Tensor, weight: torch.Tensor, chunk: int) -> bool:
+def _split_ok(rows: torch.Tensor, weight: torch.Tensor, chunk: int, autocast: bool) -> bool:
     """Whether this head's fp32 GEMMs run from bf16 pieces: tensors on the GPU,
     a contraction of whole stages, a first block large enough to gain and
     gradient rows within the kernel's 32-bit offsets."""
     n, D = min(rows.shape[0], chunk), rows.shape[1]
     V = weight.shape[0]
     return (rows.is_cuda and weight.is_cuda and rows.device == weight.device and D % ops.SPLIT_K == 0
-            and n * V * D >= SPLIT_MIN_MACS
+            and n * V * D >= (SPLIT_MIN_MACS_AUTOCAST if autocast else SPLIT_MIN_MACS)
             and (ops.split_pad(n) + ops.SPLIT_K) * ops.split_pad(V) * 2 < 1 << 31
             and (ops.split_pad(V) + ops.SPLIT_K) * D * 2 < 1 << 31)
 
@@ -99,9 +104,10 @@ class _Head:
     """The tied head's GEMMs for one call: logits of a block of rows, and a
     block's share of the two gradients."""
 
-    def __init__(self, rows: torch.Tensor, weight: torch.Tensor, chunk: int):
+    def __init__(self, rows: torch.Tensor, weight: torch.Tensor, chunk: int, autocast: _AutocastState):
         self.weight = weight
-        self.split = _split_ok(rows, weight, chunk)
+        self.autocast = autocast
+        self.split = _split_ok(rows, weight, chunk, autocast.enabled)
         self._w32 = self._pieces = None
 
     @property
@@ -116,21 +122,40 @@ class _Head:
             self._pieces = _pieces(self.weight)
         return self._pieces
 
-    def logits(self, block: torch.Tensor, autocast: bool) -> torch.Tensor:
-        if autocast or not self.split:
+    def logits(self, block: torch.Tensor) -> torch.Tensor:
+        if self.autocast.enabled or not self.split:
             return _block_logits(block, self.w32)
         V, D = self.weight.shape
         out = torch.empty((block.shape[0], ops.split_pad(V)), dtype=torch.float32, device=block.device)[:, :V]
         return ops.split_gemm_(out, _pieces(block), self.pieces, D)
+
+    def fused(self, block: torch.Tensor) -> bool:
+        """Whether the cross-entropy rows run in the logits product's epilogue:
+        the split form, where one K slice already fills the compute units."""
+        V, D = self.weight.shape
+        return (self.split and not self.autocast.enabled
+                and ops.split_logits_slices(block.shape[0], V, D, 1 if block.dtype == torch.bfloat16 else 3,
+                                            self.pieces.shape[0]) == 1)
+
+    def loss_rows(self, block: torch.Tensor, targets: torch.Tensor):
+        """The block's per-row loss and log-sum-exp."""
+        if self.fused(block):
+            return ops.split_ce_forward(_pieces(block), self.pieces, self.weight.shape[1], targets,
+                                        ignore_index=IGNORE_INDEX)
+        return ops.lm_ce_forward(self.logits(block), targets, ignore_index=IGNORE_INDEX)
 
     def new_weight_grad(self) -> torch.Tensor:
         # the split form writes it with the first block
         make = torch.empty if self.split else torch.zeros
         return make(self.weight.shape, dtype=torch.float32, device=self.weight.device)
 
-    def backward(self, logits, targets, lse, scale, block, d_rows, d_w32, first: bool) -> None:
-        """d_rows = g @ weight and d_w32 += g^T @ block for the block's fp32
-        gradient g, in fp32."""
+    def backward(self, targets, lse, scale, block, d_rows, d_w32, first: bool) -> None:
+        """d_rows = g @ weight and d_w32 += g^T @ block in fp32, for the gradient
+        g of the block's logits, recomputed under the forward's autocast state."""
+        logits = None
+        if not self.fused(block):
+            with self.autocast():
+                logits = self.logits(block)
         if not self.split:
             # fp32 gradient block, whatever the logits' dtype
             g = ops.lm_ce_grad(logits, targets, lse, scale, ignore_index=IGNORE_INDEX)
@@ -138,13 +163,17 @@ class _Head:
             d_w32.addmm_(g.t(), block.float())
             return
         V, D = self.weight.shape
-        g = ops.lm_ce_grad_pieces(logits, targets, lse, scale, ignore_index=IGNORE_INDEX)
+        rows = _pieces(block)
+        if logits is None:
+            g = ops.split_ce_grad_pieces(rows, self.pieces, D, targets, lse, scale, ignore_index=IGNORE_INDEX)
+        else:
+            g = ops.lm_ce_grad_pieces(logits, targets, lse, scale, ignore_index=IGNORE_INDEX)
         direct = d_rows.dtype in (torch.float32, torch.bfloat16) and d_rows.is_contiguous()
         dh = d_rows if direct else torch.empty(d_rows.shape, dtype=torch.float32, device=d_rows.device)
         ops.split_gemm_(dh, g, self.pieces, V, k_slow_b=True)
         if not direct:
             d_rows.copy_(dh)
-        ops.split_gemm_(d_w32, g, _pieces(block), block.shape[0], k_slow_a=True, k_slow_b=True, accumulate=not first)
+        ops.split_gemm_(d_w32, g, rows, block.shape[0], k_slow_a=True, k_slow_b=True, accumulate=not first)
 
 
 class _ChunkedLinearCrossEntropy(torch.autograd.Function):
@@ -166,13 +195,12 @@ class _ChunkedLinearCrossEntropy(torch.autograd.Function):
         rows = hidden_states.reshape(n_tok, hidden_states.shape[-1])
         targets = labels.reshape(n_tok).to(torch.int64).contiguous()
         ctx.autocast = _AutocastState()
-        head = _Head(rows, weight, chunk_size)
+        head = _Head(rows, weight, chunk_size, ctx.autocast)
         per_row = torch.empty(n_tok, dtype=torch.float32, device=hidden_states.device)
         lse = torch.empty(n_tok, dtype=torch.float32, device=hidden_states.device)
         with torch.no_grad():
             for sl in _token_blocks(n_tok, chunk_size):
-                logits = head.logits(rows[sl], ctx.autocast.enabled)
-                loss_rows, lse_rows = ops.lm_ce_forward(logits, targets[sl], ignore_index=IGNORE_INDEX)
+                loss_rows, lse_rows = head.loss_rows(rows[sl], targets[sl])
                 per_row[sl] = loss_rows
                 lse[sl] = lse_rows
         ctx.save_for_backward(hidden_states, weight, targets, lse)
@@ -185,15 +213,12 @@ class _ChunkedLinearCrossEntropy(torch.autograd.Function):
         n_tok = targets.numel()
         rows = hidden_states.reshape(n_tok, hidden_states.shape[-1])
         scale = (grad_output.float() / n_tok).reshape(1)
-        head = _Head(rows, weight, ctx.chunk_size)
+        head = _Head(rows, weight, ctx.chunk_size, ctx.autocast)
         d_rows = torch.empty_like(rows)
         d_w32 = head.new_weight_grad()
         for i, sl in enumerate(_token_blocks(n_tok, ctx.chunk_size)):
-            block = rows[sl]
-            with ctx.autocast():
-                logits = head.logits(block, ctx.autocast.enabled)
             with torch.autocast("cuda", enabled=False):
-                head.backward(logits, targets[sl], lse[sl], scale, block, d_rows[sl], d_w32, first=i == 0)
+                head.backward(targets[sl], lse[sl], scale, rows[sl], d_rows[sl], d_w32, first=i == 0)
         return d_rows.view_as(hidden_states), d_w32.to(weight.dtype), None, None
 
 

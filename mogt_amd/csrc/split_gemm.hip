@@ -22,17 +22,25 @@
 // ds_read_b64_tr_b16 (wgrad_gemm.hip describes it), its 4 x 16 blocks chosen so
 // that the K-slots agree with K_FAST's: lane half h, slot q <-> k = 8 h + q.
 //
-// Tile: 256 rows of A x 64 TNF rows of B (TNF = 4, or 2 for 3 x 3 pieces),
-// 4 waves of 128 x 32 TNF, v_mfma_f32_32x32x16_bf16 with B as the MFMA's A
+// Tile: 256 rows of A x 64 TNF rows of B (TNF = 2 for B in three pieces, else
+// 4), 4 waves of 128 x 32 TNF, v_mfma_f32_32x32x16_bf16 with B as the MFMA's A
 // operand (a lane's results are 4 consecutive n of one m: 16-byte stores).
 // A stage is 32 of K for every piece of both operands: a fragment is read from
 // LDS once and multiplied with every piece of the other operand it meets, so
-// the LDS moves 1/2 (1 x 3) to 3/8 (3 x 3) of what separate bf16 GEMMs per
-// piece pair would: 96 MFMAs (3072 cycles) a stage and wave against 16 - 18 KB
-// of fragment reads and loads each.  That is what bounds the bf16 GEMMs of this
-// library (swiglu_gemm.hip); here the MFMA does.  Two stages of 64 - 72 KB in LDS:
-// stage s + 2 is loaded (direct to LDS) into stage s's buffer from the middle
-// of stage s on, one barrier a stage.
+// the LDS moves 5/8 (1 x 3) to 3/8 (3 x 3) of what separate bf16 GEMMs per
+// piece pair would.  LDS traffic is what bounds the bf16 GEMMs of this library
+// (swiglu_gemm.hip); here the MFMA does (48 or 96 of 32 cycles a stage and
+// wave).  Two stages of 40 - 72 KB in LDS: stage s + 2 is loaded (direct to LDS)
+// into stage s's buffer from the middle of stage s on, one barrier a stage.
+//
+// Epilogues (EPI) of the logits form, one slice only:
+//   STORE    C in fp32 (above).
+//   CE_FWD   per row and wave (32 TNF columns) the maximum of the logits and the sum
+//            of exp(x - max), and the label's logit: the logits are not written.
+//            ce_merge_kernel merges a row's pairs into its log-sum-exp and loss.
+//   CE_BWD   the gradient block scale * (exp(x - lse) - onehot) as its three bf16
+//            pieces (the operand of the two gradient products), from the
+//            accumulators: neither the logits nor an fp32 gradient are written.
 //
 // Split K: the stages are cut into slices so that tiles x slices fill the CUs
 // (plan_split); each slice's fp32 partial goes to the workspace and a second
@@ -40,11 +48,15 @@
 //
 // Measured (4096 rows, D = 768, vocabulary 32000; the library's fp32 GEMM before
 // -> here; error of the result against 64 bits, normwise):
-//   logits, bf16 x fp32        1536 -> 590 us (1.02 PFLOP/s bf16)  5.0e-7 -> 3.0e-7
+//   logits, bf16 x fp32        1536 -> 589 us (1.02 PFLOP/s bf16)  5.0e-7 -> 3.0e-7
+//     with the loss rows       1650 -> 481 us (1.26)
+//     with the gradient block  1720 -> 660 us (786 MB of pieces written)
 //   logits, fp32 x fp32        1518 -> 998 us (1.21)               5.0e-7 -> 4.3e-7
 //   d hidden, fp32 x fp32      1458 -> 1064 us (1.14)              3.2e-6 -> 1.4e-6
 //   d weight, fp32 x bf16      1448 -> 568 us (1.06)               1.1e-6 -> 7.0e-7
 //   d weight, fp32 x fp32      1417 -> 957 us (1.26)               1.1e-6 -> 1.0e-6
+#include <math.h>
+
 #include <type_traits>
 
 #include "bf16_pieces.h"
@@ -79,7 +91,25 @@ struct SplitParams {
     int n_mb, n_nb;            // tiles
     int stages, per_slice;     // in all, per slice
     int accumulate;            // out += (one slice)
+    // CE_FWD / CE_BWD
+    const int64_t* labels;     // [M]
+    int64_t ignore;
+    float* pairs;              // CE_FWD: [M][2 n_nb][2] (max, sum)
+    float* xlab;               // CE_FWD: [M] the label's logit
+    const float* lse;          // CE_BWD: [M]
+    const float* scale;        // CE_BWD: one value
+    bf16_t* grad;              // CE_BWD: [3][M][ldo]
 };
+
+enum SplitEpi { EPI_STORE = 0, EPI_CE_FWD = 1, EPI_CE_BWD = 2 };
+constexpr float SP_LOG2E = 1.4426950408889634f;
+
+// B's fragments per wave: 2 where B comes in three pieces.  1 x 3 pieces then
+// need 80 KB of LDS and 256 registers, so two work-groups share a CU and one's
+// epilogue runs beside the other's products: logits with the cross-entropy
+// epilogue 566 -> 481 us, with the gradient epilogue 850 -> 660 us (one
+// work-group of 256 columns before), the written logits unchanged (589 us).
+__host__ __device__ constexpr int sp_tnf(int nb) { return nb == 3 ? 2 : 4; }
 
 // block id -> (row block, column block, slice): each XCD (ids mod 8) a
 // contiguous run, 8 row blocks walked together so that its L2 keeps them
@@ -167,8 +197,9 @@ struct Operand {
     }
 };
 
-template <int NA, int NB, bool KSA, bool KSB, int TNF>
-__global__ __launch_bounds__(SP_THREADS) void split_gemm_kernel(SplitParams p) {
+template <int NA, int NB, bool KSA, bool KSB, int TNF, int EPI>
+__global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split_gemm_kernel(SplitParams p) {
+    static_assert(EPI == EPI_STORE || (!KSA && !KSB), "cross-entropy epilogues: the logits form");
     using OA = Operand<KSA, 4>;
     using OB = Operand<KSB, TNF>;
     constexpr int STB = NA * OA::BYTES + NB * OB::BYTES;
@@ -320,6 +351,105 @@ __global__ __launch_bounds__(SP_THREADS) void split_gemm_kernel(SplitParams p) {
 
     // lane (l32, hb), register group q of acc[j][i]: row m0 + 128 wm + 32 i +
     // l32, columns n0 + 32 TNF wn + 32 j + 8 q + 4 hb .. + 3
+    if constexpr (EPI == EPI_CE_FWD) {
+        const int c0 = n0 + 32 * TNF * wn + 4 * hb;   // column of (j, q, e): c0 + 32 j + 8 q + e
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = m0 + 128 * wm + 32 * i + l32;
+            const int64_t lab = m < p.M ? p.labels[m] : -1;
+            // the label's place among this lane's columns (no match: outside)
+            const int at = lab >= 0 && lab < p.nb_valid ? static_cast<int>(lab) - c0 : -1;
+            float mx = -INFINITY, xl = 0.0f;
+            bool has = false;
+#pragma unroll
+            for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int o = 32 * j + 8 * q + e;
+                        float x = acc[j][i][4 * q + e];
+                        if (at == o) {
+                            xl = x;
+                            has = true;
+                        }
+                        if (c0 + o >= p.nb_valid) x = -INFINITY;
+                        acc[j][i][4 * q + e] = x;
+                        mx = fmaxf(mx, x);
+                    }
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float mm = mx == -INFINITY ? 0.0f : mx;   // nothing but -inf: every term is 0
+            float sum = 0.0f;
+#pragma unroll
+            for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sum += __builtin_amdgcn_exp2f((acc[j][i][r] - mm) * SP_LOG2E);
+            sum += __shfl_xor(sum, 32, 64);
+            if (m < p.M) {
+                if (hb == 0) {
+                    sp_f32x2* pr = reinterpret_cast<sp_f32x2*>(p.pairs) + (static_cast<int64_t>(m) * p.n_nb + nb) * 2 + wn;
+                    *pr = sp_f32x2{mx, sum};
+                }
+                if (has) p.xlab[m] = xl;   // one lane of the grid per row
+            }
+        }
+        return;
+    }
+    if constexpr (EPI == EPI_CE_BWD) {
+        // 32 rows x the wave's columns of one piece at a time through a wave-private
+        // LDS tile (rows padded by 16 bytes), so that every store instruction
+        // covers whole rows of the wave's columns: with 8-byte stores into 32 rows
+        // the kernel ran 897 us at 4096 x 32000 x 768, with the rows
+        // staged 850 us, and with two work-groups per CU (below) 660 us.
+        constexpr int CW = 32 * TNF;              // the wave's columns
+        constexpr int RS = CW * 2 + 16;           // LDS row stride
+        constexpr int LPR = CW / 8;               // lanes per row of 16-byte stores
+        static_assert(4 * 32 * RS <= 2 * STB, "four waves' tiles");
+        __syncthreads();                          // every wave's fragment reads are done
+        char* tile = smem + wave * (32 * RS);
+        const float sc = *p.scale;
+        const int64_t plane = static_cast<int64_t>(p.M) * p.ldo;
+        const int cw0 = n0 + CW * wn;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int mb0 = m0 + 128 * wm + 32 * i;
+            const int m = mb0 + l32;
+            const int64_t lab = m < p.M ? p.labels[m] : p.ignore;
+            const bool skip = lab == p.ignore;
+            const float bad = (!skip && (lab < 0 || lab >= p.nb_valid)) ? __builtin_nanf("") : 0.0f;
+            const float lr = m < p.M ? p.lse[m] : 0.0f;
+            Pack<bf16_t, 4> pc[3][TNF * 4];
+#pragma unroll
+            for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int n = cw0 + 32 * j + 8 * q + 4 * hb;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float pr = __builtin_amdgcn_exp2f((acc[j][i][4 * q + e] - lr) * SP_LOG2E) -
+                                         (n + e == lab ? 1.0f : 0.0f);
+                        const float v = (skip || n + e >= p.nb_valid) ? 0.0f : pr * sc + bad;
+                        bf16_pieces(v, pc[0][4 * j + q].v[e], pc[1][4 * j + q].v[e], pc[2][4 * j + q].v[e]);
+                    }
+                }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+#pragma unroll
+                for (int t = 0; t < TNF * 4; ++t)
+                    *reinterpret_cast<Pack<bf16_t, 4>*>(tile + l32 * RS + (8 * t + 4 * hb) * 2) = pc[k][t];
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+                for (int t = 0; t < 32 * LPR / 64; ++t) {
+                    const int r = t * (64 / LPR) + lane / LPR, c = (lane % LPR) * 8;
+                    const Pack<bf16_t, 8> w = *reinterpret_cast<const Pack<bf16_t, 8>*>(tile + r * RS + c * 2);
+                    if (mb0 + r < p.M && cw0 + c < p.N)   // N: the padded width here, a multiple of 8
+                        *reinterpret_cast<Pack<bf16_t, 8>*>(p.grad + k * plane + static_cast<int64_t>(mb0 + r) * p.ldo + cw0 + c) = w;
+                }
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            }
+        }
+        return;
+    }
     float* out = p.out + sl * p.po;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -336,6 +466,35 @@ __global__ __launch_bounds__(SP_THREADS) void split_gemm_kernel(SplitParams p) {
                 if (p.accumulate) v += *reinterpret_cast<const sp_f32x4*>(row + n);
                 *reinterpret_cast<sp_f32x4*>(row + n) = v;
             }
+    }
+}
+
+// Per-row log-sum-exp and loss from the row's (max, sum) pairs: one wave per
+// row.  Labels: ignore_index gives loss 0, others outside the vocabulary NaN.
+__global__ __launch_bounds__(256) void ce_merge_kernel(const float* __restrict__ pairs, const float* __restrict__ xlab,
+                                                       const int64_t* __restrict__ labels, int64_t ignore, int M,
+                                                       int npair, int64_t vocab, float* __restrict__ loss,
+                                                       float* __restrict__ lse) {
+    const int m = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (m >= M) return;
+    const sp_f32x2* pr = reinterpret_cast<const sp_f32x2*>(pairs) + static_cast<int64_t>(m) * npair;
+    float mx = -INFINITY;
+    for (int k = lane; k < npair; k += 64) mx = fmaxf(mx, pr[k][0]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    const float mm = mx == -INFINITY ? 0.0f : mx;
+    float sum = 0.0f;
+    for (int k = lane; k < npair; k += 64) {
+        const sp_f32x2 v = pr[k];
+        sum += v[1] * __builtin_amdgcn_exp2f((v[0] - mm) * SP_LOG2E);   // v[0] = -inf: 0 (its sum is 0)
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    if (lane == 0) {
+        const float l = mx + logf(sum);
+        const int64_t lab = labels[m];
+        loss[m] = lab == ignore ? 0.0f : (lab < 0 || lab >= vocab) ? __builtin_nanf("") : l - xlab[m];
+        lse[m] = l;
     }
 }
 
@@ -390,7 +549,7 @@ struct SplitPlan {
 SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int na, int nb, int64_t splits, int64_t cus) {
     SplitPlan pl{};
     const int np = na == 3 && nb == 3 ? 6 : na * nb;
-    const int tnf = np == 6 ? 2 : 4;
+    const int tnf = sp_tnf(nb);
     pl.n_mb = (M + SP_BM - 1) / SP_BM;
     pl.n_nb = (N + 64 * tnf - 1) / (64 * tnf);
     pl.stages = (K + SP_BK - 1) / SP_BK;
@@ -416,10 +575,10 @@ SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int na, int nb, int64_t sp
     return pl;
 }
 
-template <int NA, int NB, bool KSA, bool KSB>
+template <int NA, int NB, bool KSA, bool KSB, int EPI = EPI_STORE>
 void launch_split(const SplitParams& p, int64_t blocks, hipStream_t st) {
-    constexpr int TNF = NA == 3 && NB == 3 ? 2 : 4;
-    hipLaunchKernelGGL((split_gemm_kernel<NA, NB, KSA, KSB, TNF>), dim3(static_cast<unsigned>(blocks)),
+    constexpr int TNF = sp_tnf(NB);
+    hipLaunchKernelGGL((split_gemm_kernel<NA, NB, KSA, KSB, TNF, EPI>), dim3(static_cast<unsigned>(blocks)),
                        dim3(SP_THREADS), 0, st, p);
 }
 
@@ -433,6 +592,14 @@ void launch_split_pieces(const SplitParams& p, int na, int nb, int64_t blocks, h
         if (nb == 3) launch_split<1, 3, KSA, KSB>(p, blocks, st);
         else launch_split<1, 1, KSA, KSB>(p, blocks, st);
     }
+}
+
+template <int EPI>
+void launch_split_ce(const SplitParams& p, int na, int nb, int64_t blocks, hipStream_t st) {
+    if (na == 3 && nb == 3) launch_split<3, 3, false, false, EPI>(p, blocks, st);
+    else if (na == 3) launch_split<3, 1, false, false, EPI>(p, blocks, st);
+    else if (nb == 3) launch_split<1, 3, false, false, EPI>(p, blocks, st);
+    else launch_split<1, 1, false, false, EPI>(p, blocks, st);
 }
 
 int check_split_shape(int64_t M, int64_t N, int64_t K, int na, int nb) {
@@ -547,4 +714,114 @@ extern "C" int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int 
         hipLaunchKernelGGL(split_reduce_kernel<false>, rb, dim3(256), 0, st, static_cast<const float*>(workspace), C,
                            ldc, static_cast<int>(pl.slices), p.M, p.N, accumulate);
     return check_launch("split_reduce_kernel");
+}
+
+namespace {
+
+// Checks and fills the parameters the logits form's cross-entropy entries share;
+// out: blocks of the launch.
+int prepare_split_ce(SplitParams& p, const void* A, int64_t lda, int64_t plane_a, int na, const void* B, int64_t ldb,
+                     int64_t plane_b, int nb, const int64_t* labels, int64_t M, int64_t N, int64_t K, int64_t ignore,
+                     int64_t& blocks) {
+    if (int rc = check_split_shape(M, N, K, na, nb)) return rc;
+    const int64_t Kp = (K + SP_BK - 1) / SP_BK * SP_BK;
+    if (N == 0 || K == 0) return set_error(MOGT_E_INVALID, "split_ce: empty vocabulary or contraction");
+    if (lda % 8 != 0 || ldb % 8 != 0 || plane_a % 8 != 0 || plane_b % 8 != 0 || lda < Kp || ldb < Kp)
+        return set_error(MOGT_E_INVALID, "split_ce: row strides must cover the padded rows, multiples of 8");
+    if (M > 0 && (!A || !B || !labels)) return set_error(MOGT_E_INVALID, "split_ce: null pointer");
+    if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15)
+        return set_error(MOGT_E_INVALID, "split_ce: A and B need 16-byte alignment");
+    if (SP_BM * lda * 2 >= (int64_t(1) << 31) || 256 * ldb * 2 >= (int64_t(1) << 31))
+        return set_error(MOGT_E_INVALID, "split_ce: operand block exceeds 2 GiB");
+    const SplitPlan pl = plan_split(M, N, K, na, nb, 1, 1);
+    blocks = pl.n_mb * pl.n_nb;
+    if (blocks > 0x7fffffff) return set_error(MOGT_E_INVALID, "split_ce: too many tiles");
+    p.a = static_cast<const bf16_t*>(A);
+    p.b = static_cast<const bf16_t*>(B);
+    p.lda = lda;
+    p.ldb = ldb;
+    p.pa = plane_a;
+    p.pb = plane_b;
+    p.M = static_cast<int>(M);
+    p.N = static_cast<int>(N);
+    p.K = static_cast<int>(K);
+    p.nb_valid = static_cast<int>(N);
+    p.n_mb = static_cast<int>(pl.n_mb);
+    p.n_nb = static_cast<int>(pl.n_nb);
+    p.stages = p.per_slice = static_cast<int>(pl.stages);
+    p.labels = labels;
+    p.ignore = ignore;
+    return MOGT_OK;
+}
+
+int64_t split_ce_pairs(int64_t N, int na, int nb) {
+    const int64_t cols = 64 * sp_tnf(nb);
+    return 2 * ((N + cols - 1) / cols);
+}
+
+}  // namespace
+
+extern "C" int64_t mogt_split_gemm_slices(int64_t M, int64_t N, int64_t K, int pieces_a, int pieces_b, int64_t cus) {
+    if (check_split_shape(M, N, K, pieces_a, pieces_b) != MOGT_OK || M == 0 || N == 0 || K == 0) return 0;
+    if (cus <= 0) {
+        int n = 0;
+        if (device_cu_count(n) != MOGT_OK) return 0;
+        cus = n;
+    }
+    return plan_split(M, N, K, pieces_a, pieces_b, 0, cus).slices;
+}
+
+extern "C" size_t mogt_split_ce_workspace_bytes(int64_t M, int64_t N, int pieces_a, int pieces_b) {
+    if (M <= 0 || N <= 0) return 0;
+    return static_cast<size_t>(M) * (split_ce_pairs(N, pieces_a, pieces_b) * 2 + 1) * sizeof(float);
+}
+
+extern "C" int mogt_split_ce_fwd(const void* A, int64_t lda, int64_t plane_a, int pieces_a, const void* B, int64_t ldb,
+                                 int64_t plane_b, int pieces_b, const int64_t* labels, int64_t M, int64_t N, int64_t K,
+                                 int64_t ignore_index, float* loss_rows, float* lse_rows, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
+    clear_error();
+    SplitParams p{};
+    int64_t blocks = 0;
+    int rc = prepare_split_ce(p, A, lda, plane_a, pieces_a, B, ldb, plane_b, pieces_b, labels, M, N, K, ignore_index, blocks);
+    if (rc) return rc;
+    if (M == 0) return MOGT_OK;
+    if (!loss_rows || !lse_rows) return set_error(MOGT_E_INVALID, "split_ce_fwd: null pointer");
+    const size_t need = mogt_split_ce_workspace_bytes(M, N, pieces_a, pieces_b);
+    if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15))
+        return set_error(MOGT_E_WORKSPACE, "split_ce_fwd: 16-byte aligned workspace of %zu bytes needed, %zu given", need,
+                         workspace_bytes);
+    const int npair = static_cast<int>(split_ce_pairs(N, pieces_a, pieces_b));
+    p.pairs = static_cast<float*>(workspace);
+    p.xlab = p.pairs + M * npair * 2;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    launch_split_ce<EPI_CE_FWD>(p, pieces_a, pieces_b, blocks, st);
+    rc = check_launch("split_gemm_kernel");
+    if (rc) return rc;
+    hipLaunchKernelGGL(ce_merge_kernel, dim3(static_cast<unsigned>((M + 3) / 4)), dim3(256), 0, st, p.pairs, p.xlab, labels,
+                       ignore_index, p.M, npair, N, loss_rows, lse_rows);
+    return check_launch("ce_merge_kernel");
+}
+
+extern "C" int mogt_split_ce_bwd(const void* A, int64_t lda, int64_t plane_a, int pieces_a, const void* B, int64_t ldb,
+                                 int64_t plane_b, int pieces_b, const int64_t* labels, const float* lse_rows, int64_t M,
+                                 int64_t N, int64_t K, int64_t ignore_index, const float* scale, void* grad,
+                                 int64_t ld_grad, void* stream) {
+    clear_error();
+    SplitParams p{};
+    int64_t blocks = 0;
+    int rc = prepare_split_ce(p, A, lda, plane_a, pieces_a, B, ldb, plane_b, pieces_b, labels, M, N, K, ignore_index, blocks);
+    if (rc) return rc;
+    if (M == 0) return MOGT_OK;
+    if (!lse_rows || !scale || !grad) return set_error(MOGT_E_INVALID, "split_ce_bwd: null pointer");
+    // the zero padding is written by the tiles, which end at a multiple of 128
+    if (ld_grad < N || ld_grad % 8 != 0 || ld_grad > (N + 127) / 128 * 128 || (reinterpret_cast<uintptr_t>(grad) & 15))
+        return set_error(MOGT_E_INVALID, "split_ce_bwd: gradient row stride or alignment");
+    p.lse = lse_rows;
+    p.scale = scale;
+    p.grad = static_cast<bf16_t*>(grad);
+    p.ldo = ld_grad;
+    p.N = static_cast<int>(ld_grad);
+    launch_split_ce<EPI_CE_BWD>(p, pieces_a, pieces_b, blocks, static_cast<hipStream_t>(stream));
+    return check_launch("split_gemm_kernel");
 }

@@ -2226,3 +2226,78 @@ def split_gemm_(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, k: int, *, 
         raise ValueError("split_gemm: out must be [M, N] with contiguous rows")
     _split_gemm_op(out, a, b, int(k), bool(k_slow_a), bool(k_slow_b), bool(accumulate))
     return out
+
+
+def split_logits_slices(rows: int, vocab: int, k: int, pieces_a: int, pieces_b: int) -> int:
+    """K slices the logits product of these sizes is cut into (1: its
+    cross-entropy epilogues apply without leaving compute units idle)."""
+    return int(_lib.load().mogt_split_gemm_slices(rows, vocab, k, pieces_a, pieces_b, 0))
+
+
+def _check_split_ce(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor, what: str) -> None:
+    require_cuda(what, a, b, labels)
+    for t in (a, b):
+        if t.ndim != 3 or t.dtype != torch.bfloat16 or t.stride(2) != 1 or t.shape[0] not in (1, 3) or \
+                t.shape[2] != split_pad(k):
+            raise ValueError(f"{what}: operands must be bf16 pieces [1 or 3, rows, K padded to 32]")
+    if labels.dim() != 1 or labels.shape[0] != a.shape[1] or labels.dtype != torch.int64:
+        raise ValueError(f"{what}: labels must be int64 [rows]")
+
+
+@_op("mogt::split_ce_fwd")
+def _split_ce_fwd_op(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor,
+                     ignore_index: int) -> tuple[torch.Tensor, torch.Tensor]:
+    lib = _lib.load()
+    labels = labels.contiguous()
+    M, V = a.shape[1], b.shape[1]
+    loss = torch.empty(M, dtype=torch.float32, device=a.device)
+    lse = torch.empty(M, dtype=torch.float32, device=a.device)
+    ws = workspace(int(lib.mogt_split_ce_workspace_bytes(M, V, a.shape[0], b.shape[0])), a.device)
+    rc = lib.mogt_split_ce_fwd(a.data_ptr(), a.stride(1), a.stride(0), a.shape[0], b.data_ptr(), b.stride(1),
+                               b.stride(0), b.shape[0], labels.data_ptr(), M, V, k, int(ignore_index),
+                               loss.data_ptr(), lse.data_ptr(), ws.data_ptr(), ws.numel(), _stream_handle(a.device))
+    _lib.check(rc, "mogt_split_ce_fwd")
+    return loss, lse
+
+
+@_split_ce_fwd_op.register_fake
+def _(a, b, k, labels, ignore_index):
+    return a.new_empty(a.shape[1], dtype=torch.float32), a.new_empty(a.shape[1], dtype=torch.float32)
+
+
+def split_ce_forward(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor, *, ignore_index: int = -100):
+    """``lm_ce_forward`` of the logits ``a @ b^T`` (``split_gemm_``'s operands:
+    rows and vocabulary) without writing them: ``(loss_rows, lse_rows)``."""
+    _check_split_ce(a, b, k, labels, "split_ce_forward")
+    return _split_ce_fwd_op(a, b, int(k), labels, int(ignore_index))
+
+
+@_op("mogt::split_ce_bwd")
+def _split_ce_bwd_op(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor, lse: torch.Tensor,
+                     scale: torch.Tensor, ignore_index: int) -> torch.Tensor:
+    lib = _lib.load()
+    labels, lse = labels.contiguous(), lse.contiguous()
+    M, V = a.shape[1], b.shape[1]
+    grad = torch.empty((3, M, split_pad(V)), dtype=torch.bfloat16, device=a.device)
+    rc = lib.mogt_split_ce_bwd(a.data_ptr(), a.stride(1), a.stride(0), a.shape[0], b.data_ptr(), b.stride(1),
+                               b.stride(0), b.shape[0], labels.data_ptr(), lse.data_ptr(), M, V, k,
+                               int(ignore_index), scale.data_ptr(), grad.data_ptr(), grad.stride(1),
+                               _stream_handle(a.device))
+    _lib.check(rc, "mogt_split_ce_bwd")
+    return grad
+
+
+@_split_ce_bwd_op.register_fake
+def _(a, b, k, labels, lse, scale, ignore_index):
+    return a.new_empty((3, a.shape[1], split_pad(b.shape[1])))
+
+
+def split_ce_grad_pieces(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor, lse: torch.Tensor,
+                         scale: torch.Tensor, *, ignore_index: int = -100) -> torch.Tensor:
+    """``lm_ce_grad_pieces`` of the logits ``a @ b^T`` without writing them."""
+    _check_split_ce(a, b, k, labels, "split_ce_grad_pieces")
+    if lse.shape != labels.shape or lse.dtype != torch.float32:
+        raise ValueError("split_ce_grad_pieces: lse must be float32 [rows]")
+    if scale.numel() != 1 or scale.dtype != torch.float32 or scale.device != a.device:
+        raise ValueError("split_ce_grad_pieces: scale must be a one-element float32 tensor on the operands' device")
+    return _split_ce_bwd_op(a, b, int(k), labels, lse, scale.reshape(1).contiguous(), int(ignore_index))

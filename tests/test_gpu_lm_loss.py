@@ -313,7 +313,74 @@ def test_chunked_linear_ce_split_form_matches_library_form(gpu, monkeypatch, hd,
 
     lib = call()
     monkeypatch.setattr(cl, "SPLIT_MIN_MACS", 0)
+    monkeypatch.setattr(cl, "SPLIT_MIN_MACS_AUTOCAST", 0)
     for got, ref, what in zip(call(), lib, ("loss", "dh", "dw")):
         assert got.dtype == ref.dtype and got.shape == ref.shape
         # both fp32 sums in other orders; bf16 gradients one rounding apart
         assert rel_err(to_np(got), to_np(ref)) <= (1e-5 if got.dtype == torch.float32 else 2.0 ** -8), what
+
+
+@pytest.mark.parametrize("da,db", SPLIT_DT)
+@pytest.mark.parametrize("M,V,K", [(1, 3, 32), (5, 129, 64), (257, 1000, 96), (300, 513, 32), (64, 4099, 160)])
+def test_split_ce_epilogues_match_the_row_kernels(gpu, da, db, M, V, K):
+    """The cross-entropy epilogues against the row kernels on the same product's
+    written logits: ragged row and column tiles, a label in every column group
+    and at the edges, ignored and bad labels, a row of equal logits and rows
+    with -inf / NaN."""
+    announce(f"split ce {M} {V} {K} {da} {db}")
+    from mogt_amd import ops
+
+    a, b = _bf16_or_f32((M, K), da, 21), _bf16_or_f32((V, K), db, 22)
+    a[0] = 0.0
+    if M > 4:
+        a[3, 0] = float("nan")
+    a, b = a.to(gpu), b.to(gpu)
+    lab = torch.randint(0, V, (M,), generator=torch.Generator().manual_seed(M))
+    lab[-1] = V - 1
+    if M > 8:
+        lab[1], lab[2], lab[4], lab[5], lab[6] = 0, -100, V, -7, V - 1
+    lab = lab.to(gpu)
+    ap, bp = _pieces_of(a), _pieces_of(b)
+    logits = torch.empty(M, ops.split_pad(V), device=gpu)[:, :V]
+    ops.split_gemm_(logits, ap, bp, K)
+    loss, lse = ops.lm_ce_forward(logits, lab)
+    loss2, lse2 = ops.split_ce_forward(ap, bp, K, lab)
+    torch.cuda.synchronize()
+    # fp32 sums of exponentials in another order: a few ulp of the log-sum-exp
+    eps = 4 * 2.0 ** -23 * (1 + lse.abs().nan_to_num(0).max())
+    assert torch.equal(torch.isnan(lse), torch.isnan(lse2)) and torch.equal(torch.isnan(loss), torch.isnan(loss2))
+    assert bool(((lse - lse2).nan_to_num(0).abs() <= eps).all())
+    assert bool(((loss - loss2).nan_to_num(0).abs() <= 2 * eps).all())
+    scale = torch.tensor([0.37], device=gpu)
+    g = ops.lm_ce_grad_pieces(logits, lab, lse, scale).double().sum(0)
+    g2 = ops.split_ce_grad_pieces(ap, bp, K, lab, lse, scale)
+    assert float(g2[:, :, V:].float().nan_to_num(1).abs().sum()) == 0.0
+    g2 = g2.double().sum(0)
+    assert torch.equal(torch.isnan(g), torch.isnan(g2))
+    assert bool(((g - g2).nan_to_num(0).abs() <= 2.0 ** -22 * g.nan_to_num(0).abs() + 1e-37).all())
+
+
+def test_chunked_linear_ce_fused_epilogue_end_to_end(gpu):
+    """A head whose logits product fills the GPU (the epilogues are taken), with
+    a ragged last chunk that takes the written logits: loss and gradients
+    against the library form."""
+    announce("chunked CE fused epilogues")
+    from mogt_amd import chunked_lm_loss as cl
+    from mogt_amd import ops
+
+    N, D, V = 2100, 64, 33000
+    assert ops.split_logits_slices(2048, V, D, 1, 3) == 1
+    h = _bf16_or_f32((1, N, D), torch.bfloat16, 31).to(gpu).requires_grad_()
+    w = _bf16_or_f32((V, D), torch.float32, 32, 0.1).to(gpu).requires_grad_()
+    lab = _labels(N, V, gpu, seed=33, ignore_every=9).view(1, N)
+
+    def call(min_macs):
+        cl_min, cl.SPLIT_MIN_MACS = cl.SPLIT_MIN_MACS, min_macs
+        try:
+            loss = cl.chunked_linear_cross_entropy(h, w, lab, chunk_size=2048)
+            return [loss.detach(), *torch.autograd.grad(loss, [h, w])]
+        finally:
+            cl.SPLIT_MIN_MACS = cl_min
+
+    for got, ref in zip(call(0), call(1 << 62)):
+        assert rel_err(to_np(got), to_np(ref)) <= (1e-5 if got.dtype == torch.float32 else 2.0 ** -8)
