@@ -329,9 +329,17 @@ int mogt_affine_scan_grad_u(const void* G, const void* H, const void* P, void* d
 /* The same without P, the forward state recomputed from U and V (fp32 or bf16)
  * inside the pass that forms dU, never written: C a multiple of 8 up to 64, V
  * and G 16-byte aligned.  Workspace of mogt_affine_scan_workspace_bytes.    */
-int mogt_affine_scan_recompute_grad_u(const void* U, const void* V, const void* G, void* dU, int64_t batch,
-                                      int64_t length, int64_t rank, int64_t channels, int v_dtype,
+int mogt_affine_scan_recompute_grad_u(const void* U, const void* V, const void* G, const void* carry, void* dU,
+                                      int64_t batch, int64_t length, int64_t rank, int64_t channels, int v_dtype,
                                       void* workspace, size_t workspace_bytes, void* stream);
+/* mogt_affine_scan_fwd that also leaves the state entering every 32-step chunk
+ * in carry (fp32, mogt_affine_scan_carry_floats of them; none up to 32 steps):
+ * with it (else null) the recomputing gradient starts its chunks directly and
+ * needs no workspace.                                                        */
+int64_t mogt_affine_scan_carry_floats(int64_t batch, int64_t length, int64_t rank, int64_t channels);
+int mogt_affine_scan_fwd_carry(const void* U, const void* V, void* H, void* carry, int64_t batch, int64_t length,
+                               int64_t rank, int64_t channels, int v_dtype, int out_dtype, void* workspace,
+                               size_t workspace_bytes, void* stream);
 
 /* Block-local affine scan: per block of `block_size` steps, the local prefixes
  * U_prefix/H_prefix [B, L, ...] and the per-block summaries U_summary

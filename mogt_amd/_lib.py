@@ -111,8 +111,14 @@ SIGNATURES: dict[str, tuple] = {
         _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_void_p, _c_size, _c_void_p]),
     "mogt_affine_scan_grad_u": (
         _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_void_p]),
+    "mogt_affine_scan_carry_floats": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64]),
+    "mogt_affine_scan_fwd_carry": (
+        _c_int,
+        [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
+         _c_void_p, _c_size, _c_void_p],
+    ),
     "mogt_affine_scan_recompute_grad_u": (
-        _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_void_p,
+        _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_void_p,
                  _c_size, _c_void_p]),
     "mogt_affine_scan_generic_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int]),
     "mogt_affine_scan_generic_fwd": (

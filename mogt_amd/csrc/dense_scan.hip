@@ -84,8 +84,9 @@ int excl_scan(const float* U, const void* V, int64_t len, float* outP, float* ou
 }
 
 // Level 0 (VK: V_t = v_t k_t^T from V = v, K = k), then the carries, then H.
+// carry: where to leave the level-0 carries of H (null: the workspace).
 template <typename TV, typename TO, bool VK>
-int run_levels(const float* U, const void* V, const void* K, void* H, void* P, int64_t B, int64_t L,
+int run_levels(const float* U, const void* V, const void* K, void* H, void* P, float* carry, int64_t B, int64_t L,
                int64_t R, int64_t C, char* ws, const DenseGeo& geo, hipStream_t st) {
     const bool withP = P != nullptr;
     ChunkParams c{};
@@ -101,11 +102,12 @@ int run_levels(const float* U, const void* V, const void* K, void* H, void* P, i
         s.sumH = reinterpret_cast<float*>(ws + v.sumH);
         int rc = dense_launch_pass<TV, float, CM_SUMMARY, VK>(s, B, st);
         if (rc) return rc;
-        rc = excl_scan<float>(s.sumP, s.sumH, c.nb, reinterpret_cast<float*>(ws + v.carP),
-                              reinterpret_cast<float*>(ws + v.carH), B, R, C, withP, ws, geo, 1, st);
+        float* carH = carry ? carry : reinterpret_cast<float*>(ws + v.carH);
+        rc = excl_scan<float>(s.sumP, s.sumH, c.nb, reinterpret_cast<float*>(ws + v.carP), carH, B, R, C, withP, ws,
+                              geo, 1, st);
         if (rc) return rc;
         c.carP = withP ? reinterpret_cast<float*>(ws + v.carP) : nullptr;
-        c.carH = reinterpret_cast<float*>(ws + v.carH);
+        c.carH = carH;
     }
     return dense_launch_pass<TV, TO, CM_OUTPUT, VK>(c, B, st);
 }
@@ -138,15 +140,18 @@ int run_rev(const float* U, const float* X, float* G, int64_t B, int64_t L, int6
 }
 
 // dU_t = G_t H_{t-1}^T with H recomputed: the forward's summaries and carries,
-// then one pass that forms dU from the state it carries (CM_GRADU).
+// then one pass that forms dU from the state it carries (CM_GRADU).  carry: the
+// carries the forward left (then that pass alone).
 template <typename TV>
-int run_gradu(const float* U, const void* V, const float* G, float* dU, int64_t B, int64_t L, int64_t R, int64_t C,
-              char* ws, const DenseGeo& geo, hipStream_t st) {
+int run_gradu(const float* U, const void* V, const float* G, const float* carry, float* dU, int64_t B, int64_t L,
+              int64_t R, int64_t C, char* ws, const DenseGeo& geo, hipStream_t st) {
     ChunkParams c{};
     c.U = U; c.V = V; c.G = G; c.dU = dU;
     c.L = L; c.R = static_cast<int>(R); c.C = static_cast<int>(C); c.T = kDenseChunk;
     c.nb = static_cast<int>((L + c.T - 1) / c.T);
-    if (c.nb > 1) {
+    if (c.nb > 1 && carry) {
+        c.carH = carry;
+    } else if (c.nb > 1) {
         const Level& v = geo.lv[0];
         ChunkParams s = c;
         s.sumP = reinterpret_cast<float*>(ws + v.sumP);
@@ -222,7 +227,7 @@ int check_dense_shapes(int64_t B, int64_t L, int64_t R, int64_t C) {
 }
 
 // K != nullptr: the rank-1 form, V holds v [B, L, R] and K holds k [B, L, C].
-int run_dense(const float* U, const void* V, const void* K, void* H, void* P, int64_t B, int64_t L,
+int run_dense(const float* U, const void* V, const void* K, void* H, void* P, float* carry, int64_t B, int64_t L,
               int64_t R, int64_t C, int v_dtype, int out_dtype, void* ws, size_t ws_bytes, void* stream) {
     clear_error();
     int rc = check_dense_shapes(B, L, R, C);
@@ -240,15 +245,15 @@ int run_dense(const float* U, const void* V, const void* K, void* H, void* P, in
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool vf = v_dtype == MOGT_F32, of = out_dtype == MOGT_F32;
     if (K) {
-        if (vf && of) return run_levels<float, float, true>(U, V, K, H, P, B, L, R, C, base, g, st);
-        if (vf) return run_levels<float, bf16_t, true>(U, V, K, H, P, B, L, R, C, base, g, st);
-        if (of) return run_levels<bf16_t, float, true>(U, V, K, H, P, B, L, R, C, base, g, st);
-        return run_levels<bf16_t, bf16_t, true>(U, V, K, H, P, B, L, R, C, base, g, st);
+        if (vf && of) return run_levels<float, float, true>(U, V, K, H, P, carry, B, L, R, C, base, g, st);
+        if (vf) return run_levels<float, bf16_t, true>(U, V, K, H, P, carry, B, L, R, C, base, g, st);
+        if (of) return run_levels<bf16_t, float, true>(U, V, K, H, P, carry, B, L, R, C, base, g, st);
+        return run_levels<bf16_t, bf16_t, true>(U, V, K, H, P, carry, B, L, R, C, base, g, st);
     }
-    if (vf && of) return run_levels<float, float, false>(U, V, K, H, P, B, L, R, C, base, g, st);
-    if (vf) return run_levels<float, bf16_t, false>(U, V, K, H, P, B, L, R, C, base, g, st);
-    if (of) return run_levels<bf16_t, float, false>(U, V, K, H, P, B, L, R, C, base, g, st);
-    return run_levels<bf16_t, bf16_t, false>(U, V, K, H, P, B, L, R, C, base, g, st);
+    if (vf && of) return run_levels<float, float, false>(U, V, K, H, P, carry, B, L, R, C, base, g, st);
+    if (vf) return run_levels<float, bf16_t, false>(U, V, K, H, P, carry, B, L, R, C, base, g, st);
+    if (of) return run_levels<bf16_t, float, false>(U, V, K, H, P, carry, B, L, R, C, base, g, st);
+    return run_levels<bf16_t, bf16_t, false>(U, V, K, H, P, carry, B, L, R, C, base, g, st);
 }
 
 }  // namespace
@@ -266,8 +271,24 @@ extern "C" int mogt_affine_scan_fwd(const void* U, const void* V, void* H, void*
                                     int64_t length, int64_t rank, int64_t channels, int v_dtype,
                                     int out_dtype, void* workspace, size_t workspace_bytes,
                                     void* stream) {
-    return run_dense(static_cast<const float*>(U), V, nullptr, H, U_prefix, batch, length, rank, channels,
+    return run_dense(static_cast<const float*>(U), V, nullptr, H, U_prefix, nullptr, batch, length, rank, channels,
                      v_dtype, out_dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int64_t mogt_affine_scan_carry_floats(int64_t batch, int64_t length, int64_t rank, int64_t channels) {
+    if (batch <= 0 || length <= kDenseChunk || rank <= 0 || channels <= 0) return 0;
+    return batch * ((length + kDenseChunk - 1) / kDenseChunk) * rank * channels;
+}
+
+extern "C" int mogt_affine_scan_fwd_carry(const void* U, const void* V, void* H, void* carry, int64_t batch,
+                                          int64_t length, int64_t rank, int64_t channels, int v_dtype, int out_dtype,
+                                          void* workspace, size_t workspace_bytes, void* stream) {
+    if (!carry && mogt_affine_scan_carry_floats(batch, length, rank, channels) > 0) {
+        clear_error();
+        return set_error(MOGT_E_INVALID, "null carry pointer");
+    }
+    return run_dense(static_cast<const float*>(U), V, nullptr, H, nullptr, static_cast<float*>(carry), batch, length,
+                     rank, channels, v_dtype, out_dtype, workspace, workspace_bytes, stream);
 }
 
 extern "C" int mogt_affine_scan_vk_fwd(const void* U, const void* v, const void* k, void* H, void* U_prefix,
@@ -279,7 +300,7 @@ extern "C" int mogt_affine_scan_vk_fwd(const void* U, const void* v, const void*
         clear_error();
         return set_error(MOGT_E_INVALID, "null tensor pointer");
     }
-    return run_dense(static_cast<const float*>(U), v, channels > 0 ? k : nullptr, H, U_prefix, batch, length,
+    return run_dense(static_cast<const float*>(U), v, channels > 0 ? k : nullptr, H, U_prefix, nullptr, batch, length,
                      rank, channels, vk_dtype, out_dtype, workspace, workspace_bytes, stream);
 }
 
@@ -290,7 +311,7 @@ extern "C" size_t mogt_fused_scan_workspace_bytes(int64_t batch, int64_t length,
 extern "C" int mogt_fused_scan_fwd(const void* U, void* Y, int64_t batch, int64_t length, int64_t rank,
                                    int out_dtype, void* workspace, size_t workspace_bytes,
                                    void* stream) {
-    return run_dense(static_cast<const float*>(U), nullptr, nullptr, nullptr, Y, batch, length, rank, 0,
+    return run_dense(static_cast<const float*>(U), nullptr, nullptr, nullptr, Y, nullptr, batch, length, rank, 0,
                      MOGT_F32, out_dtype, workspace, workspace_bytes, stream);
 }
 
@@ -360,8 +381,8 @@ extern "C" int mogt_affine_scan_grad_u(const void* G, const void* H, const void*
     return check_launch("dense_grad_u_kernel");
 }
 
-extern "C" int mogt_affine_scan_recompute_grad_u(const void* U, const void* V, const void* G, void* dU, int64_t batch,
-                                                 int64_t length, int64_t rank, int64_t channels, int v_dtype,
+extern "C" int mogt_affine_scan_recompute_grad_u(const void* U, const void* V, const void* G, const void* carry, void* dU,
+                                                 int64_t batch, int64_t length, int64_t rank, int64_t channels, int v_dtype,
                                                  void* workspace, size_t workspace_bytes, void* stream) {
     clear_error();
     int rc = check_dense_shapes(batch, length, rank, channels);
@@ -376,13 +397,14 @@ extern "C" int mogt_affine_scan_recompute_grad_u(const void* U, const void* V, c
     if (batch > 65535 || (length + kDenseChunk - 1) / kDenseChunk > 0x7fffffffLL)
         return set_error(MOGT_E_INVALID, "problem too large for one launch");
     const DenseGeo g = dense_geometry(batch, length, rank, channels);
-    if (!workspace || workspace_bytes < g.bytes)
+    if (!carry && (!workspace || workspace_bytes < g.bytes))
         return set_error(MOGT_E_WORKSPACE, "workspace of %zu bytes required, got %zu", g.bytes, workspace_bytes);
     const float* u = static_cast<const float*>(U);
     const float* gp = static_cast<const float*>(G);
+    const float* cp = static_cast<const float*>(carry);
     float* d = static_cast<float*>(dU);
     char* base = static_cast<char*>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return v_dtype == MOGT_F32 ? run_gradu<float>(u, V, gp, d, batch, length, rank, channels, base, g, st)
-                               : run_gradu<bf16_t>(u, V, gp, d, batch, length, rank, channels, base, g, st);
+    return v_dtype == MOGT_F32 ? run_gradu<float>(u, V, gp, cp, d, batch, length, rank, channels, base, g, st)
+                               : run_gradu<bf16_t>(u, V, gp, cp, d, batch, length, rank, channels, base, g, st);
 }

@@ -24,7 +24,6 @@ Tensors must be on the GPU; there is no CPU execution path.
 """
 from __future__ import annotations
 
-import contextlib
 from dataclasses import dataclass
 
 import torch
@@ -42,13 +41,6 @@ def _autocast_dtype() -> torch.dtype | None:
     return None
 
 
-def _range(name: str):
-    """A profiler range while a profiler runs (entering one costs about 5 us of
-    host time, a dozen times per layer)."""
-    return torch.autograd.profiler.record_function(name) if torch.autograd._profiler_enabled() else _NO_RANGE
-
-
-_NO_RANGE = contextlib.nullcontext()
 _CACHE_ATTR = "_gemm_weight_cache"
 
 
@@ -318,7 +310,7 @@ class MOGTBlock(_WeightCacheOwner):
         if spec.connection not in _CONNECTIONS:
             raise ValueError(f"Unsupported connection_impl: {spec.connection}")
         label = "mogt.matrix_exp" if spec.connection == "matrix_exp" else "mogt.cayley_solve"
-        with _range(label):
+        with ops.profiler_range(label):
             mapped = ops.connection_map((A / self.r).to(torch.float32), spec.connection)
         return (mapped * spec.damping).to(output_dtype)
 
@@ -350,7 +342,7 @@ class MOGTBlock(_WeightCacheOwner):
         B, L, D = xn.shape
         r, c = self.r, self.c
         diagonal = spec.connection == "identity" and spec.scan != "transport_triton"
-        with _range("mogt.connection_map"):
+        with ops.profiler_range("mogt.connection_map"):
             if diagonal:
                 # per-rank factor of U = factor * I: starts as the damping
                 factor = torch.full((1, 1, 1, 1), spec.damping, dtype=torch.float32,
@@ -360,7 +352,7 @@ class MOGTBlock(_WeightCacheOwner):
                 if spec.connection == "identity":
                     A = xn.new_zeros(B, L, r, r)   # the identity map ignores A
                 else:
-                    with _range("mogt.connection"):
+                    with ops.profiler_range("mogt.connection"):
                         A_raw = self.phi_conn(xn).view(B, L, r, r)
                         A = A_raw - A_raw.transpose(-2, -1)
                 U = self._build_transport(A, xn.dtype)
@@ -370,7 +362,7 @@ class MOGTBlock(_WeightCacheOwner):
                     factor = factor * tg.to(factor.dtype)
                 else:
                     U = U * tg.to(U.dtype)
-        with _range("mogt.value_projection"):
+        with ops.profiler_range("mogt.value_projection"):
             values = self.phi_val(xn).view(B, L, r, c)
             if spec.value_gate is not None:
                 vg = self._value_gate_probs(spec, xn, prefix_condition)
@@ -382,7 +374,7 @@ class MOGTBlock(_WeightCacheOwner):
                     else:
                         U = U * keep.to(U.dtype)
         out_dtype = xn.dtype   # the scan's output dtype is U's (model_mogt.py:202)
-        with _range("mogt.affine_scan"):
+        with ops.profiler_range("mogt.affine_scan"):
             if diagonal:
                 decay = factor.float().expand(B, L, r, c).reshape(B, L, D)
                 h = ops.diag_scan(decay, values.float().reshape(B, L, D), out_dtype=out_dtype)
@@ -396,10 +388,10 @@ class MOGTBlock(_WeightCacheOwner):
                     U, values, block_size=getattr(self, "scan_block_size", 256),
                     block_c=getattr(self, "scan_block_c", 32), carry_scan=carry,
                     output_dtype=out_dtype).reshape(B, L, D)
-        with _range("mogt.readout"):
+        with ops.profiler_range("mogt.readout"):
             z = self.theta_read(self.norm_out(h))
         x = x + spec.residual_factor(z) * z
-        with _range("mogt.ffn"):
+        with ops.profiler_range("mogt.ffn"):
             x = x + spec.ffn_scale * self.ffn(self.norm_ffn(x))
         return x
 
@@ -486,12 +478,12 @@ class MOGTBlock(_WeightCacheOwner):
         writes h in the GEMM's dtype plus per-row sums of squares, the GEMM runs
         against theta_read * norm_out.weight, and the next RMSNorm applies each
         row's factor rsqrt(mean(h^2) + eps) as it reads Z."""
-        with _range("mogt.affine_scan"):
+        with ops.profiler_range("mogt.affine_scan"):
             proj, gate_prev, gconst = self._value_and_gate_projection(xn, prefix_condition, gate_const,
                                                                       const_given=gate_const is not None)
             h, stats = ops.coupled_rank_scan_proj(proj, self.d_model, rank=self.r, gate_prev=gate_prev,
                                                   gate_const=gconst, damping=damping)
-        with _range("mogt.readout"):
+        with ops.profiler_range("mogt.readout"):
             Zr = F.linear(h, _gemm_weight(self, "theta_read_folded", (self.theta_read.weight, self.norm_out.weight),
                                           lambda: self.theta_read.weight * self.norm_out.weight))
         return ops.add_rmsnorm_rowscale(x, Zr, stats, self._residual_scale(Zr), self.norm_ffn.weight,
@@ -505,20 +497,20 @@ class MOGTBlock(_WeightCacheOwner):
         weights); otherwise by separately computed gate logits."""
         parts = _gate_input_parts(getattr(self, "value_gate_input_mode", "current"))
         if ops.coupled_proj_scan_supported(self.d_model, self.r, "prev" in parts):
-            with _range("mogt.affine_scan"):
+            with ops.profiler_range("mogt.affine_scan"):
                 proj, gate_prev, gconst = self._value_and_gate_projection(xn, prefix_condition, packed=packed)
                 if gconst is not None:
                     gconst = gconst.expand(xn.size(0), self.r).contiguous()
                 h = ops.coupled_proj_scan(proj, self.d_model, rank=self.r, gate_prev=gate_prev, gate_const=gconst,
                                           damping=damping)
         else:
-            with _range("mogt.value_projection"):
+            with ops.profiler_range("mogt.value_projection"):
                 v_raw = F.linear(xn, _gemm_weight(self, "phi_val", (self.phi_val.weight,),
                                                   lambda: self.phi_val.weight))
                 z = self._gate_logits(xn, prefix_condition)
-            with _range("mogt.affine_scan"):
+            with ops.profiler_range("mogt.affine_scan"):
                 h = ops.coupled_rank_scan(z, v_raw, damping=damping, out_dtype=torch.float32)
-        with _range("mogt.readout"):
+        with ops.profiler_range("mogt.readout"):
             hn = ops.rmsnorm(h, self.norm_out.weight, self.norm_out.eps, out_dtype=gemm_dtype)
             Wr = packed["theta"] if packed is not None else _gemm_weight(self, "theta_read", (self.theta_read.weight,),
                                                                            lambda: self.theta_read.weight)
@@ -564,7 +556,7 @@ class MOGTBlock(_WeightCacheOwner):
             x, xn2 = self._mixer_training(x, xn, prefix_condition, damping, gemm_dtype, packed)
         else:
             x, xn2 = self._mixer_inference(x, xn, prefix_condition, damping, gemm_dtype, gate_const)
-        with _range("mogt.ffn"):
+        with ops.profiler_range("mogt.ffn"):
             f = self.ffn(xn2) if packed is None else self.ffn.forward_with(xn2, packed["w12"], packed["w3"])
         return x, (f, float(getattr(self, "mogt_ffn_residual_scale", 1.0)))
 
@@ -721,7 +713,7 @@ class MOGTForCausalLM(_WeightCacheOwner):
         logits through chunked_linear_cross_entropy."""
         hidden = self.mogt(input_ids)
         chunk = int(loss_chunk_size or 0)
-        with _range("mogt.lm_head_loss"):
+        with ops.profiler_range("mogt.lm_head_loss"):
             if labels is not None and chunk > 0 and not return_logits:
                 return None, chunked_linear_cross_entropy(hidden, self.lm_head.weight, labels,
                                                           chunk_size=chunk)

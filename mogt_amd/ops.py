@@ -9,6 +9,7 @@ the kernels leave reusable after every launch.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import inspect
 import os
@@ -231,6 +232,15 @@ def _op(qualname: str, mutates: tuple = ()):
         op.mutates = tuple(order.index(m) for m in mutates)
         return op
     return wrap
+
+
+_NO_RANGE = contextlib.nullcontext()
+
+
+def profiler_range(name: str):
+    """A profiler range while a profiler runs (entering one costs about 5 us of
+    host time, several times per layer)."""
+    return torch.autograd.profiler.record_function(name) if torch.autograd._profiler_enabled() else _NO_RANGE
 
 
 def require_cuda(what: str, *tensors: torch.Tensor) -> None:
@@ -939,9 +949,11 @@ GRADU_MAX_CHANNELS = 64   # one column block of the recomputing gradient pass
 
 
 @_op("mogt::affine_scan_recompute_grad_u")
-def _affine_scan_recompute_grad_u_op(U: torch.Tensor, V: torch.Tensor, G: torch.Tensor) -> torch.Tensor:
+def _affine_scan_recompute_grad_u_op(U: torch.Tensor, V: torch.Tensor, G: torch.Tensor,
+                                     carry: torch.Tensor | None = None) -> torch.Tensor:
     """dU_t = G_t H_{t-1}^T (fp32), H recomputed from U and V: inside the pass
-    that forms dU where its layout allows, else written and read back."""
+    that forms dU where its layout allows (from the forward's carries if they
+    were kept), else written and read back."""
     lib = _lib.load()
     U, V = _prep_uv(U, V)
     G = G.contiguous()
@@ -951,17 +963,62 @@ def _affine_scan_recompute_grad_u_op(U: torch.Tensor, V: torch.Tensor, G: torch.
         _affine_launch(U, V, H, None)
         return _affine_scan_grad_u_op(G, H, None)
     dU = torch.empty(B, L, R, R, dtype=torch.float32, device=G.device)
-    ws = workspace(lib.mogt_affine_scan_workspace_bytes(B, L, R, C), G.device)
-    rc = lib.mogt_affine_scan_recompute_grad_u(U.data_ptr(), V.data_ptr(), G.data_ptr(), dU.data_ptr(), B, L, R, C,
-                                               dtype_code(V.dtype, "affine_scan_grad"), ws.data_ptr(), ws.numel(),
+    kept = carry is not None and carry.numel() > 0
+    ws = None if kept else workspace(lib.mogt_affine_scan_workspace_bytes(B, L, R, C), G.device)
+    rc = lib.mogt_affine_scan_recompute_grad_u(U.data_ptr(), V.data_ptr(), G.data_ptr(),
+                                               carry.data_ptr() if kept else None, dU.data_ptr(), B, L, R, C,
+                                               dtype_code(V.dtype, "affine_scan_grad"),
+                                               None if kept else ws.data_ptr(), 0 if kept else ws.numel(),
                                                _stream_handle(G.device))
     _lib.check(rc, "mogt_affine_scan_recompute_grad_u")
     return dU
 
 
 @_affine_scan_recompute_grad_u_op.register_fake
-def _(U, V, G):
+def _(U, V, G, carry=None):
     return U.new_empty(U.shape, dtype=torch.float32)
+
+
+@_op("mogt::affine_scan_carry")
+def _affine_scan_carry_op(U: torch.Tensor, V: torch.Tensor,
+                          out_dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
+    """``affine_scan`` and the fp32 state entering each of its chunks (flat)."""
+    lib = _lib.load()
+    U, V = _prep_uv(U, V)
+    B, L, R, C = V.shape
+    H = torch.empty(V.shape, dtype=out_dtype, device=V.device)
+    carry = torch.empty(lib.mogt_affine_scan_carry_floats(B, L, R, C), dtype=torch.float32, device=V.device)
+    ws = workspace(lib.mogt_affine_scan_workspace_bytes(B, L, R, C), U.device)
+    rc = lib.mogt_affine_scan_fwd_carry(U.data_ptr(), V.data_ptr(), H.data_ptr(),
+                                        carry.data_ptr() if carry.numel() else None, B, L, R, C,
+                                        dtype_code(V.dtype, "affine_scan"), dtype_code(out_dtype, "affine_scan"),
+                                        ws.data_ptr(), ws.numel(), _stream_handle(U.device))
+    _lib.check(rc, "mogt_affine_scan_fwd_carry")
+    return H, carry
+
+
+@_affine_scan_carry_op.register_fake
+def _(U, V, out_dtype):
+    B, L, R, C = V.shape
+    n = B * -(-L // DENSE_CHUNK) * R * C if L > DENSE_CHUNK else 0
+    return V.new_empty(V.shape, dtype=out_dtype), V.new_empty((n,), dtype=torch.float32)
+
+
+DENSE_CHUNK = 32   # steps per chunk of the matrix-core pipeline (dense_kernel.h)
+
+
+def affine_scan_carry_supported(V: torch.Tensor, output_dtype: torch.dtype) -> bool:
+    """Whether the gradient can use the carries ``affine_scan_carry`` keeps."""
+    R, C = V.shape[-2:]
+    return _use_mfma(R, torch.float32, output_dtype) and C % 8 == 0 and 0 < C <= GRADU_MAX_CHANNELS
+
+
+def affine_scan_carry(U: torch.Tensor, V: torch.Tensor, output_dtype: torch.dtype):
+    """``(affine_scan(U, V), carry)`` in fp32 state, no autograd; ``carry`` (1/32 of
+    H) lets ``affine_scan_grad`` skip the recomputation of the chunk carries."""
+    require_cuda("affine_scan", U, V)
+    check_affine_shapes(U, V)
+    return _affine_scan_carry_op(U, V, output_dtype)
 
 
 def _reverse_scan(U: torch.Tensor, X: torch.Tensor, state_dtype: torch.dtype) -> torch.Tensor:
@@ -978,7 +1035,7 @@ def _reverse_scan(U: torch.Tensor, X: torch.Tensor, state_dtype: torch.dtype) ->
 
 def affine_scan_grad(U: torch.Tensor, V: torch.Tensor, grad_H: torch.Tensor | None,
                      grad_P: torch.Tensor | None = None, *, state_dtype: torch.dtype = torch.float32,
-                     need_grad_u: bool = True, need_grad_v: bool = True):
+                     need_grad_u: bool = True, need_grad_v: bool = True, carry: torch.Tensor | None = None):
     """Gradients of H_t = U_t H_{t-1} + V_t (affine_scan_sequential_backward,
     affine_scan.py:65-124) and, with ``grad_P``, of U_prefix_t = U_t U_prefix_{t-1}:
     the augmented state M = [H | U_prefix] gets G = [dH | dP] + U_{t+1}^T G_{t+1}
@@ -999,7 +1056,7 @@ def affine_scan_grad(U: torch.Tensor, V: torch.Tensor, grad_H: torch.Tensor | No
                 P, H = _forward_state(U, V, state_dtype, True)
                 grad_u = _affine_scan_grad_u_op(G, H, P)
             else:
-                grad_u = _affine_scan_recompute_grad_u_op(U, V, G)
+                grad_u = _affine_scan_recompute_grad_u_op(U, V, G, carry)
             return grad_u.to(U.dtype), grad_v
         zeros = torch.zeros(B, 1, R, C, dtype=state_dtype, device=V.device)
         if grad_P is not None:

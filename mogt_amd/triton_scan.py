@@ -57,13 +57,7 @@ def triton_affine_local_scan(U: torch.Tensor, V: torch.Tensor, *, block_size: in
     return ops.affine_local_scan(U, V, block_size=block_size)
 
 
-def _triton_affine_scan_hybrid_forward(U: torch.Tensor, V: torch.Tensor, *, block_size: int = 256,
-                                       block_c: int = 32, carry_scan: str = "sequential",
-                                       output_dtype: torch.dtype | None = None,
-                                       return_prefix: bool = False):
-    """Forward of the hybrid scan (triton_scan.py:232-311) as one HIP pipeline:
-    chunk summaries, carries, output in registers -- no L-sized carry-apply
-    pass.  ``output_dtype`` defaults to ``V.dtype`` (triton_scan.py:251)."""
+def _check_hybrid(U, V, block_size: int, block_c: int, carry_scan: str) -> None:
     if carry_scan not in {"sequential", "doubling"}:
         raise ValueError("carry_scan must be 'sequential' or 'doubling'")
     _check_cuda("triton_affine_local_scan", U, V)
@@ -71,18 +65,28 @@ def _triton_affine_scan_hybrid_forward(U: torch.Tensor, V: torch.Tensor, *, bloc
     _next_power_of_two(block_c)
     if block_size <= 0:
         raise ValueError("block_size must be positive")
+
+
+def _triton_affine_scan_hybrid_forward(U: torch.Tensor, V: torch.Tensor, *, block_size: int = 256,
+                                       block_c: int = 32, carry_scan: str = "sequential",
+                                       output_dtype: torch.dtype | None = None,
+                                       return_prefix: bool = False):
+    """Forward of the hybrid scan (triton_scan.py:232-311) as one HIP pipeline:
+    chunk summaries, carries, output in registers -- no L-sized carry-apply
+    pass.  ``output_dtype`` defaults to ``V.dtype`` (triton_scan.py:251)."""
+    _check_hybrid(U, V, block_size, block_c, carry_scan)
     output_dtype = output_dtype or V.dtype
     return ops.affine_scan(U, V, output_dtype=output_dtype, return_prefix=return_prefix)
 
 
 def _triton_affine_scan_hybrid_backward(U: torch.Tensor, V: torch.Tensor, grad_H: torch.Tensor, *,
                                         block_size: int, block_c: int, carry_scan: str,
-                                        need_grad_u: bool, need_grad_v: bool):
+                                        need_grad_u: bool, need_grad_v: bool, carry=None):
     """dV = G (reverse scan G_t = dH_t + U_{t+1}^T G_{t+1}), dU_t = G_t H_{t-1}^T
-    (triton_scan.py:359-426) in fp32; H is recomputed with the forward scan,
-    the outer products use a batched GEMM."""
+    (triton_scan.py:359-426) in fp32; H is recomputed, from the forward's chunk
+    carries where they were kept."""
     return ops.affine_scan_grad(U, V, grad_H, None, state_dtype=torch.float32,
-                                need_grad_u=need_grad_u, need_grad_v=need_grad_v)
+                                need_grad_u=need_grad_u, need_grad_v=need_grad_v, carry=carry)
 
 
 class _TritonAffineScanHybridAutograd(torch.autograd.Function):
@@ -90,24 +94,30 @@ class _TritonAffineScanHybridAutograd(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, U, V, block_size, block_c, carry_scan, output_dtype):
-        with torch.autograd.profiler.record_function("triton_hybrid.forward"):
+        with ops.profiler_range("triton_hybrid.forward"):
             ctx.block_size = block_size
             ctx.block_c = block_c
             ctx.carry_scan = carry_scan
             ctx.output_dtype = output_dtype or V.dtype
-            ctx.save_for_backward(U, V)
+            if ctx.needs_input_grad[0] and U.is_cuda and V.is_cuda and U.ndim == 4 and V.ndim == 4 \
+                    and ops.affine_scan_carry_supported(V, ctx.output_dtype):
+                _check_hybrid(U, V, block_size, block_c, carry_scan)
+                H, carry = ops.affine_scan_carry(U, V, ctx.output_dtype)
+                ctx.save_for_backward(U, V, carry)
+                return H
+            ctx.save_for_backward(U, V, None)
             return _triton_affine_scan_hybrid_forward(
                 U, V, block_size=block_size, block_c=block_c, carry_scan=carry_scan,
                 output_dtype=ctx.output_dtype, return_prefix=False)
 
     @staticmethod
     def backward(ctx, grad_output):
-        U_saved, V_saved = ctx.saved_tensors
-        with torch.autograd.profiler.record_function("triton_hybrid.backward_recompute"):
+        U_saved, V_saved, carry = ctx.saved_tensors
+        with ops.profiler_range("triton_hybrid.backward_recompute"):
             grad_u, grad_v = _triton_affine_scan_hybrid_backward(
                 U_saved, V_saved, grad_output, block_size=ctx.block_size, block_c=ctx.block_c,
                 carry_scan=ctx.carry_scan, need_grad_u=ctx.needs_input_grad[0],
-                need_grad_v=ctx.needs_input_grad[1])
+                need_grad_v=ctx.needs_input_grad[1], carry=carry)
         return grad_u, grad_v, None, None, None, None
 
 

@@ -322,3 +322,31 @@ def test_recomputed_grad_u(gpu, vdt, B, L, R, C):
         Gt.copy_(torch.from_numpy(G))
         dU = torch.ops.mogt.affine_scan_recompute_grad_u(torch.from_numpy(U).to(gpu), V, Gt)
         assert rel_err(to_np(dU), ref) <= 3e-6
+
+
+@pytest.mark.parametrize("vdt,odt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("B,L,R,C", [(1, 32, 16, 16), (2, 33, 7, 8), (1, 1500, 16, 48), (3, 65, 32, 64)])
+def test_kept_carries_give_the_same_scan_and_gradient(gpu, vdt, odt, B, L, R, C):
+    """The forward that keeps its chunk carries (none for one chunk) writes the
+    same H, and dU from the kept carries is the recomputed one bit for bit;
+    through the public function both gradients follow."""
+    announce(f"kept carries {vdt} {B} {L} {R} {C}")
+    from mogt_amd import ops, triton_scan
+
+    g = torch.Generator().manual_seed(L + C)
+    U = (0.9 * torch.eye(R) + 0.1 / R * torch.randn(B, L, R, R, generator=g)).to(gpu)
+    V = torch.randn(B, L, R, C, generator=g).to(gpu).to(vdt)
+    G = torch.randn(B, L, R, C, generator=g).to(gpu)
+    H, carry = ops.affine_scan_carry(U, V, odt)
+    assert torch.equal(H, ops.affine_scan(U, V, output_dtype=odt))
+    assert carry.numel() == (B * -(-L // 32) * R * C if L > 32 else 0)
+    kept = torch.ops.mogt.affine_scan_recompute_grad_u(U, V, G, carry)
+    assert torch.equal(kept, torch.ops.mogt.affine_scan_recompute_grad_u(U, V, G))
+    Ur, Vr = U.clone().requires_grad_(), V.clone().requires_grad_()
+    h = triton_scan.triton_affine_scan_hybrid(Ur, Vr, output_dtype=odt)
+    gu, gv = torch.autograd.grad(h, [Ur, Vr], G.to(odt))
+    ru, rv = ops.affine_scan_grad(U, V, G.to(odt))
+    assert torch.equal(h, H) and torch.equal(gu, ru) and torch.equal(gv, rv)
+    Vr = V.clone().requires_grad_()   # no gradient of U: no carries kept
+    (gv,) = torch.autograd.grad(triton_scan.triton_affine_scan_hybrid(U, Vr, output_dtype=odt), Vr, G.to(odt))
+    assert torch.equal(gv, rv)
