@@ -53,7 +53,7 @@
 //     with the gradient block  1720 -> 660 us (786 MB of pieces written)
 //   logits, fp32 x fp32        1518 -> 998 us (1.21)               5.0e-7 -> 4.3e-7
 //   d hidden, fp32 x fp32      1458 -> 1064 us (1.14)              3.2e-6 -> 1.4e-6
-//   d weight, fp32 x bf16      1448 -> 568 us (1.06)               1.1e-6 -> 7.0e-7
+//   d weight, fp32 x bf16      1448 -> 469 us (1.29)               1.1e-6 -> 7.0e-7
 //   d weight, fp32 x fp32      1417 -> 957 us (1.26)               1.1e-6 -> 1.0e-6
 #include <math.h>
 
@@ -197,9 +197,9 @@ struct Operand {
     }
 };
 
-template <int NA, int NB, bool KSA, bool KSB, int TNF, int EPI>
+template <int NA, int NB, bool KSA, bool KSB, int TNF, int EPI, bool TR>
 __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split_gemm_kernel(SplitParams p) {
-    static_assert(EPI == EPI_STORE || (!KSA && !KSB), "cross-entropy epilogues: the logits form");
+    static_assert(EPI == EPI_STORE || (!KSA && !KSB && !TR), "cross-entropy epilogues: the logits form");
     using OA = Operand<KSA, 4>;
     using OB = Operand<KSB, TNF>;
     constexpr int STB = NA * OA::BYTES + NB * OB::BYTES;
@@ -300,8 +300,8 @@ __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split
             for (int j = 0; j < TNF; ++j)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.b[pair_b(q)][j], cur.a[pair_a(q)][i],
-                                                                        acc[j][i], 0, 0, 0);
+                    const sp_bf16x8 fa = cur.a[pair_a(q)][i], fb = cur.b[pair_b(q)][j];
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(TR ? fa : fb, TR ? fb : fa, acc[j][i], 0, 0, 0);
                     if constexpr (decltype(reads)::value)
                         if (t % 2 == 0 && t / 2 < NR) read(next, t / 2, sn, kn);
                     if constexpr (decltype(loads)::value)
@@ -451,6 +451,27 @@ __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split
         return;
     }
     float* out = p.out + sl * p.po;
+    if constexpr (TR) {
+        // A was the MFMA's A operand: a lane's results are 4 consecutive m of one
+        // n, and C is stored transposed, out[n][m]
+#pragma unroll
+        for (int j = 0; j < TNF; ++j) {
+            const int n = n0 + 32 * TNF * wn + 32 * j + l32;
+            if (n >= p.nb_valid) continue;
+            float* row = out + n * p.ldo;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int m = m0 + 128 * wm + 32 * i + 8 * q + 4 * hb;
+                    if (m >= p.M) continue;
+                    sp_f32x4 v = {acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
+                    if (p.accumulate) v += *reinterpret_cast<const sp_f32x4*>(row + m);
+                    *reinterpret_cast<sp_f32x4*>(row + m) = v;
+                }
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int m = m0 + 128 * wm + 32 * i + l32;
@@ -575,24 +596,33 @@ SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int na, int nb, int64_t sp
     return pl;
 }
 
-template <int NA, int NB, bool KSA, bool KSB, int EPI = EPI_STORE>
+template <int NA, int NB, bool KSA, bool KSB, int EPI = EPI_STORE, bool TR = false>
 void launch_split(const SplitParams& p, int64_t blocks, hipStream_t st) {
     constexpr int TNF = sp_tnf(NB);
-    hipLaunchKernelGGL((split_gemm_kernel<NA, NB, KSA, KSB, TNF, EPI>), dim3(static_cast<unsigned>(blocks)),
+    hipLaunchKernelGGL((split_gemm_kernel<NA, NB, KSA, KSB, TNF, EPI, TR>), dim3(static_cast<unsigned>(blocks)),
                        dim3(SP_THREADS), 0, st, p);
 }
 
 // the head's products: logits (K_FAST, any pieces), hidden states' gradient
 // (K_FAST gradient x K_SLOW weight) and weight's (both K_SLOW), A in 3 pieces
-template <bool KSA, bool KSB>
+template <bool KSB>
 void launch_split_pieces(const SplitParams& p, int na, int nb, int64_t blocks, hipStream_t st) {
-    if (na == 3 && nb == 3) launch_split<3, 3, KSA, KSB>(p, blocks, st);
-    else if (na == 3) launch_split<3, 1, KSA, KSB>(p, blocks, st);
+    if (na == 3 && nb == 3) launch_split<3, 3, false, KSB>(p, blocks, st);
+    else if (na == 3) launch_split<3, 1, false, KSB>(p, blocks, st);
     else if constexpr (!KSB) {
-        if (nb == 3) launch_split<1, 3, KSA, KSB>(p, blocks, st);
-        else launch_split<1, 1, KSA, KSB>(p, blocks, st);
+        if (nb == 3) launch_split<1, 3, false, KSB>(p, blocks, st);
+        else launch_split<1, 1, false, KSB>(p, blocks, st);
     }
 }
+
+// Both operands K_SLOW, 3 x 1 pieces (the weight gradient of a bf16 hidden
+// state): the operands swap places and the result is stored transposed, which
+// is the 1 x 3 form with its smaller tiles and two work-groups per CU.  At 32000 x
+// 768 over 4096 rows that is 750 tiles for 256 CUs (2.9 rounds) where the tiles of
+// the 3 x 1 form, one work-group per CU, are 375 (1.5 rounds, run as 2): 552 -> 469
+// us; over 1024 rows 184 -> 156, 256 rows 77 -> 56; 4000 x 256 over 1024 rows 30 ->
+// 21; 16000 x 1024 over 4096 rows, where both fill their rounds, 305 in both.
+bool swap_operands(int na, int nb, bool k_slow_a) { return k_slow_a && na == 3 && nb == 1; }
 
 template <int EPI>
 void launch_split_ce(const SplitParams& p, int na, int nb, int64_t blocks, hipStream_t st) {
@@ -639,9 +669,13 @@ extern "C" size_t mogt_split_gemm_workspace_bytes(int64_t M, int64_t N, int64_t 
         cus = n;
     }
     // at most this many bytes whatever the output type (a bf16 output always
-    // goes through the partials)
-    return static_cast<size_t>(plan_split(M, N, K, pieces_a, pieces_b, splits, cus).slices) * M * ((N + 3) / 4 * 4) *
-           sizeof(float);
+    // goes through the partials) and the layouts (swap_operands)
+    int64_t slices = plan_split(M, N, K, pieces_a, pieces_b, splits, cus).slices;
+    if (swap_operands(pieces_a, pieces_b, true)) {
+        const int64_t swapped = plan_split(N, M, K, pieces_b, pieces_a, splits, cus).slices;
+        if (swapped > slices) slices = swapped;
+    }
+    return static_cast<size_t>(slices) * M * ((N + 3) / 4 * 4) * sizeof(float);
 }
 
 extern "C" int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int pieces_a, int k_slow_a, const void* B,
@@ -668,7 +702,9 @@ extern "C" int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int 
         return set_error(MOGT_E_INVALID, "split_gemm: operand block exceeds 2 GiB");
     int cus = 0;
     if (int rc = device_cu_count(cus)) return rc;
-    const SplitPlan pl = plan_split(M, N, K, pieces_a, pieces_b, splits, cus);
+    const bool swap = swap_operands(pieces_a, pieces_b, k_slow_a);
+    const SplitPlan pl = swap ? plan_split(N, M, K, pieces_b, pieces_a, splits, cus)
+                              : plan_split(M, N, K, pieces_a, pieces_b, splits, cus);
     const int64_t blocks = pl.n_mb * pl.n_nb * pl.slices;
     if (blocks > 0x7fffffff) return set_error(MOGT_E_INVALID, "split_gemm: too many tiles");
     const bool parts = pl.slices > 1 || out_dtype == MOGT_BF16;
@@ -681,38 +717,39 @@ extern "C" int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int 
             return set_error(MOGT_E_INVALID, "split_gemm: workspace needs 16-byte alignment");
     }
     SplitParams p{};
-    p.a = static_cast<const bf16_t*>(A);
-    p.b = static_cast<const bf16_t*>(B);
+    p.a = static_cast<const bf16_t*>(swap ? B : A);
+    p.b = static_cast<const bf16_t*>(swap ? A : B);
     p.out = static_cast<float*>(parts ? workspace : C);
-    p.lda = lda;
-    p.ldb = ldb;
+    p.lda = swap ? ldb : lda;
+    p.ldb = swap ? lda : ldb;
     p.ldo = parts ? Np : ldc;
-    p.pa = plane_a;
-    p.pb = plane_b;
+    p.pa = swap ? plane_b : plane_a;
+    p.pb = swap ? plane_a : plane_b;
     p.po = M * Np;
-    p.M = static_cast<int>(M);
+    p.M = static_cast<int>(swap ? N : M);
     p.N = static_cast<int>(Np);
     p.K = static_cast<int>(K);
-    p.nb_valid = static_cast<int>(N);
+    p.nb_valid = static_cast<int>(swap ? M : N);
     p.n_mb = static_cast<int>(pl.n_mb);
     p.n_nb = static_cast<int>(pl.n_nb);
     p.stages = static_cast<int>(pl.stages);
     p.per_slice = static_cast<int>(pl.per_slice);
     p.accumulate = !parts && accumulate;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (k_slow_a) launch_split_pieces<true, true>(p, pieces_a, pieces_b, blocks, st);
-    else if (k_slow_b) launch_split_pieces<false, true>(p, pieces_a, pieces_b, blocks, st);
-    else launch_split_pieces<false, false>(p, pieces_a, pieces_b, blocks, st);
+    if (swap) launch_split<1, 3, true, true, EPI_STORE, true>(p, blocks, st);
+    else if (k_slow_a) launch_split<3, 3, true, true>(p, blocks, st);
+    else if (k_slow_b) launch_split_pieces<true>(p, pieces_a, pieces_b, blocks, st);
+    else launch_split_pieces<false>(p, pieces_a, pieces_b, blocks, st);
     int rc = check_launch("split_gemm_kernel");
     if (rc != MOGT_OK || !parts) return rc;
     const int64_t groups = M * (Np / 4);
     const dim3 rb(static_cast<unsigned>((groups + 255) / 256 < 8192 ? (groups + 255) / 256 : 8192));
     if (out_dtype == MOGT_BF16)
         hipLaunchKernelGGL(split_reduce_kernel<true>, rb, dim3(256), 0, st, static_cast<const float*>(workspace), C, ldc,
-                           static_cast<int>(pl.slices), p.M, p.N, 0);
+                           static_cast<int>(pl.slices), static_cast<int>(M), p.N, 0);
     else
         hipLaunchKernelGGL(split_reduce_kernel<false>, rb, dim3(256), 0, st, static_cast<const float*>(workspace), C,
-                           ldc, static_cast<int>(pl.slices), p.M, p.N, accumulate);
+                           ldc, static_cast<int>(pl.slices), static_cast<int>(M), p.N, accumulate);
     return check_launch("split_reduce_kernel");
 }
 
