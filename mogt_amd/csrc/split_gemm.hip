@@ -50,7 +50,7 @@
 // -> here; error of the result against 64 bits, normwise):
 //   logits, bf16 x fp32        1536 -> 589 us (1.02 PFLOP/s bf16)  5.0e-7 -> 3.0e-7
 //     with the loss rows       1650 -> 481 us (1.26)
-//     with the gradient block  1720 -> 660 us (786 MB of pieces written)
+//     with the gradient block  1720 -> 620 us (786 MB of pieces written)
 //   logits, fp32 x fp32        1518 -> 998 us (1.21)               5.0e-7 -> 4.3e-7
 //   d hidden, fp32 x fp32      1458 -> 1064 us (1.14)              3.2e-6 -> 1.4e-6
 //   d weight, fp32 x bf16      1448 -> 469 us (1.29)               1.1e-6 -> 7.0e-7
@@ -107,7 +107,7 @@ constexpr float SP_LOG2E = 1.4426950408889634f;
 // B's fragments per wave: 2 where B comes in three pieces.  1 x 3 pieces then
 // need 80 KB of LDS and 256 registers, so two work-groups share a CU and one's
 // epilogue runs beside the other's products: logits with the cross-entropy
-// epilogue 566 -> 481 us, with the gradient epilogue 850 -> 660 us (one
+// epilogue 566 -> 481 us, with the gradient epilogue 850 -> 660 us then (one
 // work-group of 256 columns before), the written logits unchanged (589 us).
 __host__ __device__ constexpr int sp_tnf(int nb) { return nb == 3 ? 2 : 4; }
 
@@ -400,7 +400,8 @@ __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split
         // LDS tile (rows padded by 16 bytes), so that every store instruction
         // covers whole rows of the wave's columns: with 8-byte stores into 32 rows
         // the kernel ran 897 us at 4096 x 32000 x 768, with the rows
-        // staged 850 us, and with two work-groups per CU (below) 660 us.
+        // staged 850 us, with two work-groups per CU (sp_tnf) 660 us, and with
+        // the arithmetic below (no test per element, no spills) 620 us.
         constexpr int CW = 32 * TNF;              // the wave's columns
         constexpr int RS = CW * 2 + 16;           // LDS row stride
         constexpr int LPR = CW / 8;               // lanes per row of 16-byte stores
@@ -418,25 +419,74 @@ __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split
             const bool skip = lab == p.ignore;
             const float bad = (!skip && (lab < 0 || lab >= p.nb_valid)) ? __builtin_nanf("") : 0.0f;
             const float lr = m < p.M ? p.lse[m] : 0.0f;
-            Pack<bf16_t, 4> pc[3][TNF * 4];
+            // the gradient replaces the logits; what concerns few rows or tiles (a
+            // label among the wave's columns, ignored rows, the vocabulary's end)
+            // under uniform branches
 #pragma unroll
             for (int j = 0; j < TNF; ++j)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int n = cw0 + 32 * j + 8 * q + 4 * hb;
+                for (int r = 0; r < 16; ++r) acc[j][i][r] = __builtin_amdgcn_exp2f((acc[j][i][r] - lr) * SP_LOG2E);
+            const int at = lab >= cw0 && lab < cw0 + CW ? static_cast<int>(lab) - cw0 - 4 * hb : -1;
+            if (__any(at >= 0)) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float pr = __builtin_amdgcn_exp2f((acc[j][i][4 * q + e] - lr) * SP_LOG2E) -
-                                         (n + e == lab ? 1.0f : 0.0f);
-                        const float v = (skip || n + e >= p.nb_valid) ? 0.0f : pr * sc + bad;
-                        bf16_pieces(v, pc[0][4 * j + q].v[e], pc[1][4 * j + q].v[e], pc[2][4 * j + q].v[e]);
+                for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[j][i][r] -= at == 32 * j + 8 * (r >> 2) + (r & 3) ? 1.0f : 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[j][i][r] = acc[j][i][r] * sc + bad;
+            if (__any(skip) || cw0 + CW > p.nb_valid) {
+#pragma unroll
+                for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int n = cw0 + 32 * j + 8 * (r >> 2) + 4 * hb + (r & 3);
+                        if (skip || n >= p.nb_valid) acc[j][i][r] = 0.0f;
                     }
-                }
+            }
+            // Pieces two at a time without the tests of bf16_pieces: an element
+            // that needs them (not finite, or rounded up to infinity) leaves a
+            // NaN as its last remainder
+            sp_u32x2 pc[3][TNF * 4];
+            float last = 0.0f;
+#pragma unroll
+            for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        float x0 = acc[j][i][4 * q + 2 * e], x1 = acc[j][i][4 * q + 2 * e + 1];
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((sp_f32x2{x0, x1}), sp_bf16x2));
+                            pc[k][4 * j + q][e] = w;
+                            if (k < 2) {
+                                x0 -= __uint_as_float(w << 16);
+                                x1 -= __uint_as_float(w & 0xffff0000u);
+                            }
+                        }
+                        last += x0;
+                        last += x1;
+                    }
+            if (__any(last != last)) {
+#pragma unroll
+                for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        Pack<bf16_t, 4> w[3];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) bf16_pieces(acc[j][i][4 * q + e], w[0].v[e], w[1].v[e], w[2].v[e]);
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) pc[k][4 * j + q] = __builtin_bit_cast(sp_u32x2, w[k]);
+                    }
+            }
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
 #pragma unroll
                 for (int t = 0; t < TNF * 4; ++t)
-                    *reinterpret_cast<Pack<bf16_t, 4>*>(tile + l32 * RS + (8 * t + 4 * hb) * 2) = pc[k][t];
+                    *reinterpret_cast<sp_u32x2*>(tile + l32 * RS + (8 * t + 4 * hb) * 2) = pc[k][t];
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 #pragma unroll
                 for (int t = 0; t < 32 * LPR / 64; ++t) {
