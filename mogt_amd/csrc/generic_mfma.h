@@ -20,12 +20,16 @@
 // of operands are in flight.
 //
 // What bounds it: a step's chain of MFMAs in a wave for R = 64 (128 MFMAs of 32
-// cycles at CW = 2), memory for R = 16 in float64.  The scalar kernel it
+// cycles at CW = 2; the counters show the matrix unit busy 69 % of LOCAL's cycles,
+// 4 % waiting for memory, at 2.1 GHz), memory for R = 16 in float64.  The scalar kernel it
 // replaces at these ranks (one dot product per thread over LDS) spent about
 // 2 us in every step on its barriers and LDS round trips.  Measured: float64 R =
 // 16, C = 48, L = 32768 1036 -> 190 us (LOCAL 52 us = 5.2 TB/s, OUTPUT 106, the
 // carries in three passes 31 instead of 82 in one); fp32 R = C = 64, 24 x 2048
-// steps 4360 -> 1140 us.
+// steps 4360 -> 1178 us, and with the memory instructions spread between the
+// MFMAs and a lane's two columns adjacent (P2: 8-byte loads and stores, whose
+// counter then never limits the operands in flight) 1112 us; with the prefix
+// written too 1795 -> 1560 us.  PD = 4 in place of 2: no gain, up to 8 % slower.
 #pragma once
 
 #include <math.h>
@@ -126,18 +130,22 @@ template <typename TS, int RT> constexpr int gm_depth() { return RT == 1 ? 8 : R
 // writes.  The general form (any io dtype) decides at run time.
 enum GmOut { GM_FINAL = 0, GM_EVERY_H = 1, GM_EVERY_HP = 2, GM_ANY = 3 };
 
+// P2 (two tiles per wave, both columns of a pair inside or outside every view,
+// 8-byte aligned): tile h of the wave holds columns 2 n + h of its 32.
 // IS: bytes of an input element (2: bf16 or fp16); VA: a lane's 4 values of a
 // row of U as 16-byte loads (R a multiple of 4, rows 16-byte aligned, not
 // reversed).  The native form issues the same loads and stores in every step
 // (padding steps of a ragged chunk have empty ranges), so no wait has to assume
 // that the operands in flight were never issued.
-template <typename TS, int RT, int CW, int IS, bool VA, int OUT>
+template <typename TS, int RT, int CW, int IS, bool VA, int OUT, bool P2>
 __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, int64_t waves) {
+    static_assert(!P2 || (CW == 2 && sizeof(TS) == 4 && IS == 4 && OUT != GM_ANY), "paired columns: two fp32 tiles");
     typedef GMma<TS> M;
     typedef typename M::vec vec;
     constexpr bool ANY = OUT == GM_ANY;
     constexpr int PD = gm_depth<TS, RT>();
     constexpr int SS = static_cast<int>(sizeof(TS));
+    constexpr bool SPREAD = !ANY && CW == 2;
     const int64_t wid = static_cast<int64_t>(blockIdx.x) * GM_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (wid >= waves) return;   // whole waves: nothing below is shared between them
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
@@ -156,7 +164,7 @@ __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, 
     auto trow = [&](int rt, int i) { return 16 * rt + 4 * g + i; };
     int col[CW];
 #pragma unroll
-    for (int h = 0; h < CW; ++h) col[h] = (ct * CW + h) * 16 + n;
+    for (int h = 0; h < CW; ++h) col[h] = P2 ? ct * 32 + 2 * n + h : (ct * CW + h) * 16 + n;
 
     // per-lane byte offsets inside a step's block
     uint32_t offA[RT][RT][VA ? 1 : 4];
@@ -230,26 +238,27 @@ __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, 
             }
         }
     };
+    // element e = (rt, i, tile) of the lane's state, with P2 both tiles' values
+    constexpr int HS = P2 ? 1 : CW;
+    auto store_piece = [&](__amdgpu_buffer_rsrc_t r, const uint32_t (&off)[CW], uint32_t row, int code, int e, bool stream) {
+        const int h = e % HS, i = e / HS % 4, rt = e / HS / 4;
+        if constexpr (P2) {
+            const gm_u32x2 w = {__float_as_uint(static_cast<float>(X[rt][0][i])), __float_as_uint(static_cast<float>(X[rt][1][i]))};
+            __builtin_amdgcn_raw_buffer_store_b64(w, r, off[0] + (16 * rt + i) * row, 0, 0);
+        } else {
+            st_one(r, off[h] + (16 * rt + i) * row, code, X[rt][h][i], stream);
+        }
+    };
     auto store_state = [&](char* ph, char* pp, bool valid, bool stream, auto wantH, auto wantP) {
         if constexpr (decltype(wantH)::value) {
             const auto rh = rsrc(ph, valid ? hBytes : 0u);
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int h = 0; h < CW; ++h)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        st_one(rh, offH[h] + (16 * rt + i) * hrow, p.out_h.code, X[rt][h][i], stream);
+            for (int e = 0; e < RT * 4 * HS; ++e) store_piece(rh, offH, hrow, p.out_h.code, e, stream);
         }
         if constexpr (decltype(wantP)::value) {
             const auto rp = rsrc(pp, valid ? pBytes : 0u);
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int h = 0; h < CW; ++h)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        st_one(rp, offP[h] + (16 * rt + i) * prow, p.out_p.code, X[rt][h][i], stream);
+            for (int e = 0; e < RT * 4 * HS; ++e) store_piece(rp, offP, prow, p.out_p.code, e, stream);
         }
     };
     constexpr std::true_type YES{};
@@ -278,50 +287,53 @@ __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, 
     // operands of the chunk's step s, which must be fetched in order; an empty
     // range past the chunk, and for the transition of reversed position 0 (the
     // state before it is zero)
+    auto rsrc_u = [&](int s) { return rsrc(fu, s < len && !(p.rev && q0 + s == 0) ? trBytes : 0u); };
+    auto rsrc_v = [&](int s) { return rsrc(fv, s < len ? inBytes : 0u); };
+    auto fetch_a = [&](__amdgpu_buffer_rsrc_t ru, Ops& o, int rt, int kt) {
+        if constexpr (VA && SS == 4) {
+            o.A[rt][kt] = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(ru, offA[rt][kt][0], 0, 0));
+        } else if constexpr (VA) {
+            struct Two { gm_u32x4 a, b; } w = {
+                __builtin_bit_cast(gm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, offA[rt][kt][0], 0, 0)),
+                __builtin_bit_cast(gm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, offA[rt][kt][0] + 16, 0, 0))};
+            o.A[rt][kt] = __builtin_bit_cast(vec, w);
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                if constexpr (SS == 4)
+                    o.A[rt][kt][kk] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ru, offA[rt][kt][kk], 0, 0));
+                else
+                    o.A[rt][kt][kk] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ru, offA[rt][kt][kk], 0, 0));
+            }
+        }
+    };
+    auto fetch_v = [&](__amdgpu_buffer_rsrc_t rv, Ops& o, int e) {
+        const int h = e % HS, i = e / HS % 4, rt = e / HS / 4;
+        const uint32_t off = offV[h] + (16 * rt + i) * vrow;
+        if constexpr (P2) {
+            const gm_u32x2 w = __builtin_bit_cast(gm_u32x2, __builtin_amdgcn_raw_buffer_load_b64(rv, off, 0, 0));
+            o.v[rt][0][i][0] = w[0];
+            o.v[rt][1][i][0] = w[1];
+        } else if constexpr (IS == 8) {
+            const gm_u32x2 w = __builtin_bit_cast(gm_u32x2, __builtin_amdgcn_raw_buffer_load_b64(rv, off, 0, 0));
+            o.v[rt][h][i][0] = w[0];
+            o.v[rt][h][i][1] = w[1];
+        } else if constexpr (IS == 4) {
+            o.v[rt][h][i][0] = __builtin_amdgcn_raw_buffer_load_b32(rv, off, 0, 0);
+        } else {
+            o.v[rt][h][i][0] = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(rv, off, 0, 0));
+        }
+    };
     auto fetch = [&](int s, Ops& o) {
-        const auto ru = rsrc(fu, s < len && !(p.rev && q0 + s == 0) ? trBytes : 0u);
-        const auto rv = rsrc(fv, s < len ? inBytes : 0u);
+        const auto ru = rsrc_u(s), rv = rsrc_v(s);
         fu += du;
         fv += dv;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-            for (int kt = 0; kt < RT; ++kt) {
-                if constexpr (VA && SS == 4) {
-                    o.A[rt][kt] = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(ru, offA[rt][kt][0], 0, 0));
-                } else if constexpr (VA) {
-                    struct Two { gm_u32x4 a, b; } w = {
-                        __builtin_bit_cast(gm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, offA[rt][kt][0], 0, 0)),
-                        __builtin_bit_cast(gm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, offA[rt][kt][0] + 16, 0, 0))};
-                    o.A[rt][kt] = __builtin_bit_cast(vec, w);
-                } else {
+            for (int kt = 0; kt < RT; ++kt) fetch_a(ru, o, rt, kt);
 #pragma unroll
-                    for (int kk = 0; kk < 4; ++kk) {
-                        if constexpr (SS == 4)
-                            o.A[rt][kt][kk] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ru, offA[rt][kt][kk], 0, 0));
-                        else
-                            o.A[rt][kt][kk] = __builtin_bit_cast(
-                                double, __builtin_amdgcn_raw_buffer_load_b64(ru, offA[rt][kt][kk], 0, 0));
-                    }
-                }
-            }
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int h = 0; h < CW; ++h)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t off = offV[h] + (16 * rt + i) * vrow;
-                    if constexpr (IS == 8) {
-                        const gm_u32x2 w = __builtin_bit_cast(gm_u32x2, __builtin_amdgcn_raw_buffer_load_b64(rv, off, 0, 0));
-                        o.v[rt][h][i][0] = w[0];
-                        o.v[rt][h][i][1] = w[1];
-                    } else if constexpr (IS == 4) {
-                        o.v[rt][h][i][0] = __builtin_amdgcn_raw_buffer_load_b32(rv, off, 0, 0);
-                    } else {
-                        o.v[rt][h][i][0] = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(rv, off, 0, 0));
-                    }
-                }
+        for (int e = 0; e < RT * 4 * HS; ++e) fetch_v(rv, o, e);
     };
     auto input = [&](const uint32_t (&w)[IS == 8 ? 2 : 1]) -> TS {
         if constexpr (IS == 8) {
@@ -339,6 +351,70 @@ __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, 
     Ops ring[PD];
 #pragma unroll
     for (int pp = 0; pp < PD; ++pp) fetch(pp, ring[pp]);
+    if constexpr (SPREAD) {
+        // Two tiles per wave: memory instructions between the MFMAs, which a burst
+        // of them after a step's last would leave idle.  While contraction tile kt
+        // runs, the inputs of step s + PD (kt = 0) or its transition's tile kt - 1,
+        // whose registers are free by then, and the stores of the state before this
+        // step.  With one tile per wave the memory bounds the pass where it fills
+        // the chip, and the order above it reads and writes in (R = C = 64, 64 x
+        // 512 steps: OUTPUT 437 us) was better than this one (467 us).
+        constexpr int NV = RT * 4 * HS, TM = 4 * RT * CW;              // input loads; MFMAs per contraction tile
+        constexpr int NS = OUT == GM_EVERY_HP ? 2 * NV : OUT == GM_EVERY_H ? NV : 0, SM = (RT - 1) * TM;
+        static_assert(NS <= SM && NV <= TM && RT <= TM, "one of each a slot");
+        int s0 = 0;
+        for (; s0 < len; s0 += PD) {
+#pragma unroll
+            for (int pp = 0; pp < PD; ++pp) {
+                const int s = s0 + pp;
+                Ops& o = ring[pp];
+                vec acc[RT][CW];
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int h = 0; h < CW; ++h)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[rt][h][i] = input(o.v[rt][h][i]);
+                const auto ru = rsrc_u(s + PD), rv = rsrc_v(s + PD);
+                fu += du;
+                fv += dv;
+                const bool st = s > 0 && s <= len;
+                const auto rh = rsrc(oh - dh, NS > 0 && st ? hBytes : 0u);
+                const auto rp = rsrc(op - dp, NS > NV && st ? pBytes : 0u);
+#pragma unroll
+                for (int kt = 0; kt < RT; ++kt)
+#pragma unroll
+                    for (int m = 0; m < TM; ++m) {
+                        const int kk = m / (RT * CW), rt = m / CW % RT, h = m % CW;
+                        acc[rt][h] = M::mma(o.A[rt][kt][kk], X[kt][h][kk], acc[rt][h]);
+                        if (kt == 0) {
+                            if ((m + 1) * NV / TM > m * NV / TM) fetch_v(rv, o, m * NV / TM);
+                        } else {
+                            if ((m + 1) * RT / TM > m * RT / TM) fetch_a(ru, o, m * RT / TM, kt - 1);
+                            const int q = (kt - 1) * TM + m, e = q * NS / SM;
+                            if (NS > 0 && (q + 1) * NS / SM > e) {
+                                if (e < NV) store_piece(rh, offH, hrow, MOGT_F32, e, true);
+                                else store_piece(rp, offP, prow, MOGT_F32, e - NV, true);
+                            }
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) fetch_a(ru, o, rt, RT - 1);
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int h = 0; h < CW; ++h) X[rt][h] = acc[rt][h];
+                oh += dh;
+                op += dp;
+            }
+        }
+        // the state after the last step (not a padding step's)
+        if constexpr (OUT == GM_EVERY_H) store_state(oh - dh, op - dp, s0 == len, true, YES, NO);
+        if constexpr (OUT == GM_EVERY_HP) store_state(oh - dh, op - dp, s0 == len, true, YES, YES);
+        if constexpr (OUT == GM_FINAL) store_any(out_at(p.out_h, j, ob_h), out_at(p.out_p, j, ob_p), false);
+        return;
+    }
     for (int s0 = 0; s0 < len; s0 += PD) {
 #pragma unroll
         for (int pp = 0; pp < PD; ++pp) {
@@ -412,10 +488,10 @@ inline int64_t gm_segment(int64_t B, int64_t L, int64_t R, int64_t C, int64_t Wo
 // Whether every step's blocks fit the kernel's 32-bit offsets.
 inline bool gm_fits(int64_t R, int64_t C) { return R <= GM_MAX_R && R * (C + R) * 8 <= GM_MAX_BLOCK; }
 
-template <typename TS, int RT, int CW, int IS, bool VA, int OUT>
+template <typename TS, int RT, int CW, int IS, bool VA, int OUT, bool P2 = false>
 int gm_launch_k(const GParams& p, int64_t waves, hipStream_t st) {
     const dim3 grid(static_cast<unsigned>((waves + GM_WAVES - 1) / GM_WAVES)), block(64 * GM_WAVES);
-    hipLaunchKernelGGL((generic_mfma_kernel<TS, RT, CW, IS, VA, OUT>), grid, block, 0, st, p, waves);
+    hipLaunchKernelGGL((generic_mfma_kernel<TS, RT, CW, IS, VA, OUT, P2>), grid, block, 0, st, p, waves);
     return check_launch("generic_mfma_kernel");
 }
 
@@ -440,6 +516,16 @@ int gm_launch(const GParams& p, int64_t waves, hipStream_t st) {
     const int64_t align = 16 / SS;
     const bool va = !p.rev && p.R % 4 == 0 && p.tr.rs % align == 0 && p.tr.ss % align == 0 && p.tr.bs % align == 0 &&
                     p.tr_c0 % align == 0 && reinterpret_cast<uintptr_t>(p.tr.p) % 16 == 0;
+    if constexpr (SS == 4 && CW == 2) {
+        auto even = [](const GView& v) {
+            return !v.p || ((v.rs | v.ss | v.bs) % 2 == 0 && reinterpret_cast<uintptr_t>(v.p) % 8 == 0);
+        };
+        if (va && (p.cin | p.csplit | p.W) % 2 == 0 && even(p.in) && even(p.out_h) && even(p.out_p)) {
+            if (!p.every) return gm_launch_k<TS, RT, CW, SS, true, GM_FINAL, true>(p, waves, st);
+            if (!p.out_p.p) return gm_launch_k<TS, RT, CW, SS, true, GM_EVERY_H, true>(p, waves, st);
+            return gm_launch_k<TS, RT, CW, SS, true, GM_EVERY_HP, true>(p, waves, st);
+        }
+    }
     if (!p.every) return va ? gm_launch_k<TS, RT, CW, SS, true, GM_FINAL>(p, waves, st) : gm_launch_k<TS, RT, CW, SS, false, GM_FINAL>(p, waves, st);
     if (!p.out_p.p) return va ? gm_launch_k<TS, RT, CW, SS, true, GM_EVERY_H>(p, waves, st) : gm_launch_k<TS, RT, CW, SS, false, GM_EVERY_H>(p, waves, st);
     return va ? gm_launch_k<TS, RT, CW, SS, true, GM_EVERY_HP>(p, waves, st) : gm_launch_k<TS, RT, CW, SS, false, GM_EVERY_HP>(p, waves, st);
@@ -447,8 +533,8 @@ int gm_launch(const GParams& p, int64_t waves, hipStream_t st) {
 
 // Tiles per wave: every wave of a chunk reads the whole of U_t, so for fp32 ranks
 // above 32 a wave takes two while that leaves each SIMD a wave (R = 64, C = 64, 24
-// x 2048 steps: LOCAL 880 -> 520 us, OUTPUT 648 -> 540 us; four tiles spill and
-// ran 550 and 900 us); else one (a shorter step, more waves).
+// x 2048 steps, before the spread memory instructions: LOCAL 880 -> 520 us, OUTPUT
+// 648 -> 540 us; four tiles spill and ran 550 and 900 us); else one (a shorter step, more waves).
 inline int gm_tiles_per_wave(int64_t chunks, int tiles) {
     return tiles > 1 && chunks * ((tiles + 1) / 2) >= 1024 ? 2 : 1;
 }

@@ -383,6 +383,26 @@ def test_matrix_core_ranks_match_the_loop(gpu, state, B, L, R, C):
     assert rel_err(G.double().cpu().numpy(), _loop64(Ug, Vg, rev=True)[1].numpy()) <= tol
 
 
+@pytest.mark.parametrize("B,L,R,C", [(40, 700, 36, 20), (20, 1100, 36, 33), (32, 601, 52, 18), (33, 300, 50, 14),
+                                     (64, 250, 64, 2)])
+def test_two_tiles_per_wave_match_the_loop(gpu, B, L, R, C):
+    """Enough chunks that a wave takes two column tiles: pairs of adjacent
+    columns (even C and offsets) and single ones (odd C, or rows of U that are not
+    16-byte aligned), ragged last chunks, with the prefix and without."""
+    announce(f"generic two tiles per wave {B} {L} {R} {C}")
+    g = np.random.default_rng(R * 100 + C)
+    U = torch.from_numpy((0.9 * np.eye(R) + 0.3 / R * g.standard_normal((B, L, R, R))).astype(np.float32))
+    V = torch.from_numpy(g.standard_normal((B, L, R, C)).astype(np.float32))
+    Pr, Hr = _loop64(U, V)
+    Ug, Vg = U.to(gpu), V.to(gpu)
+    P, H = torch.ops.mogt.affine_scan_generic(Ug, Vg, torch.float32, torch.float32, True, False)
+    H1 = torch.ops.mogt.affine_scan_generic(Ug, Vg, torch.float32, torch.float32, False, False)[1]
+    torch.cuda.synchronize()
+    assert rel_err(P.double().cpu().numpy(), Pr.numpy()) <= FP32_TOL
+    assert rel_err(H.double().cpu().numpy(), Hr.numpy()) <= FP32_TOL
+    assert rel_err(H1.double().cpu().numpy(), Hr.numpy()) <= FP32_TOL
+
+
 @pytest.mark.parametrize("state", [torch.float32, torch.float64])
 @pytest.mark.parametrize("vdt", [torch.float16, torch.bfloat16, torch.float32, torch.float64])
 @pytest.mark.parametrize("odt", [torch.float16, torch.bfloat16, torch.float32, torch.float64])
