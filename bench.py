@@ -894,7 +894,7 @@ def main():
                     "graph_nodes": rg_["graph_nodes"], "graph16_us": round(rg16["ms"] * 1e3, 2),
                     "graph16_nodes": rg16["graph_nodes"],
                     "note": "mogt_amd.diag_scan per call (eager: input checks, output allocation, C-ABI launch; "
-                            "the custom-op dispatch is taken only under autograd or tracing), the same call "
+                            "the custom-op dispatch is taken only under tracing and transforms), the same call "
                             "captured alone in a HIP graph and replayed (graph_nodes: nodes per captured graph; "
                             "the replay pays the runtime's graph launch), and 16 calls captured in one graph "
                             "(graph16_us: replay time per call)"}
