@@ -698,8 +698,9 @@ class MOGTForCausalLM(_WeightCacheOwner):
         cast of the whole table, 27 us at 32000 x 768) is kept until the weight
         changes, like the blocks' GEMM operands."""
         head = self.lm_head
-        plain = type(head) is nn.Linear and not (head._forward_hooks or head._forward_pre_hooks or
-                                                 head._backward_hooks or head._backward_pre_hooks)
+        plain = type(head) is nn.Linear and "forward" not in head.__dict__ and not (
+            head._forward_hooks or head._forward_pre_hooks or head._backward_hooks or head._backward_pre_hooks or
+            nn.modules.module._has_any_global_hook())
         if not plain or head.bias is not None or torch.is_grad_enabled() or _autocast_dtype() is None:
             return head(hidden)
         return F.linear(hidden, _gemm_weight(self, "lm_head", (head.weight,), lambda: head.weight))

@@ -355,3 +355,30 @@ def test_inference_weight_cache_follows_parameter_updates(gpu):
     for m in model.modules():
         m.__dict__.pop("_gemm_weight_cache", None)
     assert torch.equal(y4, run())
+
+
+def test_head_weight_cast_gives_way_to_module_hooks(gpu):
+    """Without gradients under autocast the head runs on a kept cast of its
+    weight, with the module's own result; a hook that would see the module's
+    call (its own or a global one) or a replaced ``forward`` still does."""
+    announce("head hooks")
+    from mogt_amd.model_mogt import MOGTForCausalLM
+
+    model = MOGTForCausalLM(vocab_size=97, d_model=64, num_layers=1, r=16).to(gpu).eval()
+    hidden = torch.randn(1, 8, 64, device=gpu)
+    seen = []
+
+    def hook(mod, *args):
+        if mod is model.lm_head:
+            seen.append(1)
+
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        want = model.lm_head(hidden)
+        assert torch.equal(model._lm_logits(hidden), want)
+        for register in (model.lm_head.register_forward_hook, torch.nn.modules.module.register_module_forward_hook):
+            handle = register(hook)
+            model._lm_logits(hidden)
+            handle.remove()
+        model.lm_head.forward = lambda x: seen.append(1) or want
+        model._lm_logits(hidden)
+    assert len(seen) == 3
