@@ -291,7 +291,11 @@ __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split
     auto pair_a = [](int q) { return NP == 6 ? (q < 3 ? 0 : q < 5 ? 1 : 2) : NB == 1 ? q : 0; };
     auto pair_b = [](int q) { return NP == 6 ? (q < 3 ? q : q < 5 ? q - 3 : 0) : NB == 1 ? 0 : q; };
     // One K-step's MFMAs on `cur`, with one fragment read of `next` (K-step kn of
-    // stage sn) and one load of stage sld every other MFMA.
+    // stage sn) and one load of stage sld every other MFMA; for 3 x 3 pieces, whose
+    // MFMAs leave room, the loads evenly over them (hidden gradient at 4096 x
+    // 32000 x 768 1012 -> 997 us; a load every MFMA 1052; the 1 x 3 forms were 1 -
+    // 3 % slower with even loads).
+    constexpr bool SPREAD = NP == 6;
     auto kstep = [&](const Frags& cur, Frags& next, int sn, int kn, int sld, auto reads, auto loads) {
         int t = 0;
 #pragma unroll
@@ -305,7 +309,8 @@ __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split
                     if constexpr (decltype(reads)::value)
                         if (t % 2 == 0 && t / 2 < NR) read(next, t / 2, sn, kn);
                     if constexpr (decltype(loads)::value)
-                        if (t % 2 == 1 && t / 2 < NL) load(t / 2, sld);
+                        if (SPREAD ? (t + 1) * NL / NM > t * NL / NM : t % 2 == 1 && t / 2 < NL)
+                            load(SPREAD ? t * NL / NM : t / 2, sld);
                     __builtin_amdgcn_sched_barrier(0);
                     ++t;
                 }
