@@ -694,16 +694,10 @@ class MOGTForCausalLM(_WeightCacheOwner):
             blk.ffn.w3.weight.zero_()
 
     def _lm_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        """``lm_head(hidden)``; without gradients the head's autocast weight (a
-        cast of the whole table, 27 us at 32000 x 768) is kept until the weight
-        changes, like the blocks' GEMM operands."""
-        head = self.lm_head
-        plain = type(head) is nn.Linear and "forward" not in head.__dict__ and not (
-            head._forward_hooks or head._forward_pre_hooks or head._backward_hooks or head._backward_pre_hooks or
-            nn.modules.module._has_any_global_hook())
-        if not plain or head.bias is not None or torch.is_grad_enabled() or _autocast_dtype() is None:
-            return head(hidden)
-        return F.linear(hidden, _gemm_weight(self, "lm_head", (head.weight,), lambda: head.weight))
+        """The module's own call, also under autocast: the head is the embedding
+        table, which every call reads anew, so a cast of it kept between calls
+        would part from the embedding after a write through ``weight.data``."""
+        return self.lm_head(hidden)
 
     def forward(self, input_ids, labels=None, *, return_logits=True, loss_chunk_size=0):
         """model_mogt.py:350-380.  Without labels: logits.  With labels and

@@ -358,9 +358,8 @@ def test_inference_weight_cache_follows_parameter_updates(gpu):
 
 
 def test_head_weight_cast_gives_way_to_module_hooks(gpu):
-    """Without gradients under autocast the head runs on a kept cast of its
-    weight, with the module's own result; a hook that would see the module's
-    call (its own or a global one) or a replaced ``forward`` still does."""
+    """Without gradients under autocast the head is the module's own call: a
+    hook (its own or a global one) or a replaced ``forward`` sees it."""
     announce("head hooks")
     from mogt_amd.model_mogt import MOGTForCausalLM
 

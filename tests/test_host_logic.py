@@ -60,6 +60,23 @@ def test_gemm_weight_cache_invalidation_paths():
         assert _gemm_weight(ffn, "w12", (ffn.w1.weight, ffn.w2.weight), build) is not w3
 
 
+def test_tied_head_follows_writes_through_weight_data(monkeypatch):
+    """The tied head and the embedding are one table: after a write through
+    ``weight.data`` (an EMA swap, a manual load), which moves no version counter,
+    a no-grad call under autocast takes both from the new values."""
+    from mogt_amd import model_mogt
+
+    model = model_mogt.MOGTForCausalLM(vocab_size=31, d_model=32, num_layers=1, r=4).eval()
+    hidden = torch.randn(1, 5, 32)
+    model.mogt.forward = lambda ids: hidden
+    monkeypatch.setattr(model_mogt, "_autocast_dtype", lambda: torch.bfloat16)
+    for mode in (torch.no_grad, torch.inference_mode):
+        with mode(), torch.autocast("cpu", dtype=torch.bfloat16):
+            model(None)
+            model.lm_head.weight.data.normal_()
+            assert torch.equal(model(None)[0], nn.functional.linear(hidden, model.lm_head.weight))
+
+
 def test_gemm_table_is_well_formed():
     """The tuned GEMM table: TunableOp's validator header for gfx950 and one
     solution per backbone GEMM shape (bf16, the d_model 768 projections)."""
