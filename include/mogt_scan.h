@@ -288,6 +288,15 @@ int mogt_affine_scan_generic_fwd(const void* U, const void* V, void* H, void* U_
                                  int64_t batch, int64_t length, int64_t rank, int64_t channels,
                                  int v_dtype, int state_dtype, int out_dtype, int reverse,
                                  void* workspace, size_t workspace_bytes, void* stream);
+/* Host-only self-check, no device work: walks the passes that
+ * mogt_affine_scan_generic_fwd would launch for these arguments and evaluates
+ * the 32-bit byte offsets of those that take the matrix-core kernel, padded
+ * rows included: valid elements at their place, all others past the step's
+ * range.  Returns 0, or MOGT_E_INVALID naming the first pass that fails.  No
+ * counterpart in the reference.                                             */
+int mogt_affine_scan_generic_check_offsets(int64_t batch, int64_t length, int64_t rank, int64_t channels,
+                                           int with_prefix, int v_dtype, int state_dtype, int out_dtype,
+                                           int reverse);
 
 /* Block-local scan on the generic kernel, for what mogt_affine_local_scan
  * does not take (R > 32, float64): per block of `block_size` steps, from the

@@ -121,6 +121,8 @@ SIGNATURES: dict[str, tuple] = {
         _c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_void_p,
                  _c_size, _c_void_p]),
     "mogt_affine_scan_generic_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int]),
+    "mogt_affine_scan_generic_check_offsets": (
+        _c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int]),
     "mogt_affine_scan_generic_fwd": (
         _c_int,
         [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int,

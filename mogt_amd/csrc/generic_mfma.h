@@ -121,7 +121,7 @@ template <> struct GMma<double> {
 constexpr int GM_MAX_R = 64;      // ranks of the matrix-core kernel
 constexpr int GM_WAVES = 4;       // waves (independent) per work-group
 constexpr uint32_t GM_OOB = 0x40000000u;   // past every range, also after a row offset
-constexpr int64_t GM_MAX_BLOCK = 0x3fffffff;   // bytes of one step's block of a view
+constexpr int64_t GM_MAX_BLOCK = 0x3fffffff;   // bytes of one step's block of a view, padded rows included
 
 // Steps of operands in flight: what fits the registers beside the state.
 template <typename TS, int RT> constexpr int gm_depth() { return RT == 1 ? 8 : RT == 2 ? 4 : 2; }
@@ -485,8 +485,13 @@ inline int64_t gm_segment(int64_t B, int64_t L, int64_t R, int64_t C, int64_t Wo
     return best;
 }
 
-// Whether every step's blocks fit the kernel's 32-bit offsets.
-inline bool gm_fits(int64_t R, int64_t C) { return R <= GM_MAX_R && R * (C + R) * 8 <= GM_MAX_BLOCK; }
+// Whether every step's blocks fit the kernel's 32-bit offsets; row: the longest
+// row of the views in elements.  A lane forms the offsets of all 16 RT padded
+// rows (and GM_OOB plus them), so it is their extent that must not wrap: a
+// wrapped offset of a padded row would lie inside the range again.
+inline bool gm_fits(int64_t R, int64_t row) {
+    return R <= GM_MAX_R && row <= GM_MAX_BLOCK && (R + 15) / 16 * 16 * row * 8 <= GM_MAX_BLOCK;
+}
 
 template <typename TS, int RT, int CW, int IS, bool VA, int OUT, bool P2 = false>
 int gm_launch_k(const GParams& p, int64_t waves, hipStream_t st) {

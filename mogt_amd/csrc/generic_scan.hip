@@ -187,7 +187,7 @@ GGeo generic_geometry(int64_t B, int64_t L, int64_t R, int64_t C, int with_prefi
     g.Wl = static_cast<int>(C + R);
     g.Wo = static_cast<int>(C + (with_prefix ? R : 0));
     const size_t ts = state_code == MOGT_F64 ? 8 : 4;
-    const bool mfma = gm_fits(R, C);
+    const bool mfma = gm_fits(R, C + R);
     g.bytes = WS_HDR_BYTES;
     int64_t len = L;
     for (int l = 0; l < GS_LEVELS; ++l) {
@@ -221,10 +221,16 @@ int tile_width(int R, int W) {
     return cb;
 }
 
+// Whether a pass takes the matrix-core kernel (rank <= 64).
+bool takes_mfma(const GParams& p) {
+    int64_t row = p.W;
+    for (const GView* v : {&p.tr, &p.in, &p.out_h, &p.out_p}) row = v->rs > row ? v->rs : row;
+    return gm_fits(p.R, row);
+}
+
 template <typename TS>
 int launch_generic(GParams p, int64_t batch, hipStream_t st, const char* what) {
-    if (gm_fits(p.R, p.W - p.R > 0 ? p.W - p.R : 0) && p.tr.rs * p.R * 8 <= GM_MAX_BLOCK)
-        return generic_mfma_launch<TS>(p, batch, st);   // rank <= 64
+    if (takes_mfma(p)) return generic_mfma_launch<TS>(p, batch, st);
     p.Cb = tile_width(p.R, p.W);
     p.ntile = (p.W + p.Cb - 1) / p.Cb;
     const int64_t blocks = batch * p.nseg * p.ntile;
@@ -240,11 +246,12 @@ bool io_code(int c) { return c == MOGT_F32 || c == MOGT_BF16 || c == MOGT_F64 ||
 // The scan `out` describes, at level l of the geometry: in one pass, or LOCAL
 // over its chunks (state [H | P], the summaries), the carries as the exclusive
 // scan of the summaries (one level up), then `out` from each chunk's carry.
-template <typename TS>
-int scan_level(GParams out, int64_t B, const GGeo& g, int l, unsigned char* base, int state_code, hipStream_t st) {
+// launch(pass, name): launches a pass, or checks it on the host.
+template <typename Launch>
+int scan_level(GParams out, const GGeo& g, int l, unsigned char* base, int state_code, const Launch& launch) {
     if (l >= g.levels) {
         out.seg = out.L; out.nseg = 1;
-        return launch_generic<TS>(out, B, st, "generic_scan output");
+        return launch(out, "generic_scan output");
     }
     const int64_t R = out.R, nch = g.nch[l];
     const GView vS{base + g.s_off[l], nch * R * g.Wl, R * g.Wl, g.Wl, state_code};   // [B][nch][R][C+R]
@@ -256,7 +263,7 @@ int scan_level(GParams out, int64_t B, const GGeo& g, int l, unsigned char* base
     loc.seg = g.seg[l]; loc.nseg = static_cast<int>(nch);
     loc.init = none; loc.out_h = vS; loc.out_p = none;
     loc.W = g.Wl; loc.csplit = g.Wl; loc.every = 0; loc.shift = 0; loc.stream = 0;
-    int rc = launch_generic<TS>(loc, B, st, "generic_scan local");
+    int rc = launch(loc, "generic_scan local");
     if (rc) return rc;
 
     GParams car{};
@@ -264,17 +271,17 @@ int scan_level(GParams out, int64_t B, const GGeo& g, int l, unsigned char* base
     car.L = nch - 1;
     car.R = out.R; car.W = g.Wo; car.tr_c0 = iC; car.cin = iC; car.cid = iC; car.csplit = g.Wo;
     car.every = 1; car.shift = 1; car.rev = 0;
-    rc = scan_level<TS>(car, B, g, l + 1, base, state_code, st);
+    rc = scan_level(car, g, l + 1, base, state_code, launch);
     if (rc) return rc;
 
     out.seg = g.seg[l]; out.nseg = static_cast<int>(nch);
     out.init = vM;
-    return launch_generic<TS>(out, B, st, "generic_scan output");
+    return launch(out, "generic_scan output");
 }
 
-template <typename TS>
-int run_generic(const void* U, const void* V, void* H, void* P, int64_t B, int64_t L, int64_t R, int64_t C,
-                int v_code, int state_code, int out_code, int reverse, void* ws, hipStream_t st) {
+template <typename Launch>
+int run_passes(const void* U, const void* V, void* H, void* P, int64_t B, int64_t L, int64_t R, int64_t C,
+               int v_code, int state_code, int out_code, int reverse, void* ws, const Launch& launch) {
     const GGeo g = generic_geometry(B, L, R, C, P != nullptr, state_code);
     const int iR = static_cast<int>(R), iC = static_cast<int>(C);
     // U / V / H / U_prefix views: [B][L][R][*]
@@ -289,7 +296,36 @@ int run_generic(const void* U, const void* V, void* H, void* P, int64_t B, int64
     out.tr = vU; out.in = vV; out.init = none; out.out_h = vH; out.out_p = vP;
     out.L = L; out.R = iR; out.W = g.Wo; out.tr_c0 = 0; out.cin = iC; out.cid = iC; out.csplit = iC;
     out.every = 1; out.shift = 0; out.rev = reverse; out.stream = 1;
-    return scan_level<TS>(out, B, g, 0, base, state_code, st);
+    return scan_level(out, g, 0, base, state_code, launch);
+}
+
+template <typename TS>
+int run_generic(const void* U, const void* V, void* H, void* P, int64_t B, int64_t L, int64_t R, int64_t C,
+                int v_code, int state_code, int out_code, int reverse, void* ws, hipStream_t st) {
+    return run_passes(U, V, H, P, B, L, R, C, v_code, state_code, out_code, reverse, ws,
+                      [&](const GParams& p, const char* what) { return launch_generic<TS>(p, B, st, what); });
+}
+
+int64_t code_size(int code) { return code == MOGT_F64 ? 8 : code == MOGT_F32 ? 4 : 2; }
+
+// The matrix-core kernel's offsets of one view's step block, as the kernel
+// forms them in 32 bits: rows below R and columns below `width` inside the
+// range, every other (padded row, or GM_OOB for a column) past it.  The offsets
+// rise with the column, so the ends of a row stand for it.
+bool offsets_ok(const GView& v, int R, int64_t c0, int64_t width) {
+    if (!v.p || width <= 0) return true;
+    const int64_t es = code_size(v.code), range = (v.rs * (R - 1) + c0 + width) * es;
+    if (range > GM_MAX_BLOCK) return false;
+    const uint32_t row = static_cast<uint32_t>(v.rs) * static_cast<uint32_t>(es);
+    for (int r = 0; r < (R + 15) / 16 * 16; ++r)
+        for (int k = 0; k < 3; ++k) {
+            const int64_t c = k == 0 ? c0 : c0 + width - 1;
+            const uint32_t off = k == 2 ? GM_OOB : static_cast<uint32_t>(c * es);
+            const uint32_t got = off + static_cast<uint32_t>(r) * row;
+            const bool inside = got < static_cast<uint32_t>(range);
+            if (inside != (k < 2 && r < R) || (inside && got != (r * v.rs + c) * es)) return false;
+        }
+    return true;
 }
 
 int check_generic(int64_t B, int64_t L, int64_t R, int64_t C, int v_code, int state_code, int out_code,
@@ -335,6 +371,24 @@ extern "C" int mogt_affine_scan_generic_fwd(const void* U, const void* V, void* 
                                      out_dtype, reverse, workspace, st)
                : run_generic<float>(U, V, H, U_prefix, batch, length, rank, channels, v_dtype, state_dtype,
                                     out_dtype, reverse, workspace, st);
+}
+
+extern "C" int mogt_affine_scan_generic_check_offsets(int64_t batch, int64_t length, int64_t rank, int64_t channels,
+                                                      int with_prefix, int v_dtype, int state_dtype, int out_dtype,
+                                                      int reverse) {
+    clear_error();
+    void* some = reinterpret_cast<void*>(uintptr_t(256));   // views are told from absent ones; nothing is read
+    void* P = with_prefix ? some : nullptr;
+    if (int rc = check_generic(batch, length, rank, channels, v_dtype, state_dtype, out_dtype, reverse, P)) return rc;
+    if (batch == 0 || length == 0 || (channels == 0 && !P)) return MOGT_OK;
+    return run_passes(some, some, some, P, batch, length, rank, channels, v_dtype, state_dtype, out_dtype, reverse,
+                      some, [](const GParams& p, const char* what) -> int {
+                          if (!takes_mfma(p)) return MOGT_OK;
+                          const bool ok = offsets_ok(p.tr, p.R, p.tr_c0, p.R) && offsets_ok(p.in, p.R, 0, p.cin) &&
+                                          offsets_ok(p.out_h, p.R, 0, p.csplit) &&
+                                          offsets_ok(p.out_p, p.R, 0, p.W - p.csplit);
+                          return ok ? MOGT_OK : set_error(MOGT_E_INVALID, "%s: a 32-bit offset wraps", what);
+                      });
 }
 
 extern "C" int mogt_affine_local_scan_generic(const void* U, const void* V, void* U_prefix, void* H_prefix,

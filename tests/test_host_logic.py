@@ -236,6 +236,25 @@ def test_rank1_buffer_ranges_stay_in_bounds():
     assert lib.mogt_rank1_check_ranges(0, 100, 1, 2) == -1
 
 
+def test_generic_scan_offsets_do_not_wrap():
+    """The matrix-core kernel of the generic scan forms 32-bit byte offsets of
+    whole 16-row tiles: at few ranks and very many channels the padded rows'
+    offsets must not come back into the range (such sizes take the scalar
+    kernel)."""
+    from mogt_amd import _lib
+
+    lib = _lib.load()
+    F32, BF16, F64, F16 = _lib.MOGT_F32, _lib.MOGT_BF16, _lib.MOGT_F64, _lib.MOGT_F16
+    forms = [(F32, F32, F32), (BF16, F32, BF16), (F16, F32, F16), (F64, F64, F64), (F16, F64, BF16)]
+    edges = [1 << k for k in range(18, 30)] + [36_000_000, 40_000_000, 72_000_000, 134_217_727, 0x3fffffff - 64]
+    for R in (1, 2, 3, 7, 16, 17, 33, 48, 63, 64, 65):
+        for C in [1, 5, 64] + [e // R + d for e in edges for d in (-1, 0, 1)]:
+            for v, state, out in forms:
+                for L, prefix, reverse in ((3, 0, 0), (100, 1, 0), (5000, 0, 1)):
+                    rc = lib.mogt_affine_scan_generic_check_offsets(1, L, R, C, prefix, v, state, out, reverse)
+                    assert rc == 0, (R, C, v, state, out, L, prefix, reverse, lib.mogt_last_error())
+
+
 def _fake_device_workspace(monkeypatch):
     """ops.workspace on host tensors: one fake stream, no capture."""
     from mogt_amd import ops
