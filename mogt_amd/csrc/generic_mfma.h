@@ -126,23 +126,29 @@ constexpr int64_t GM_MAX_BLOCK = 0x3fffffff;   // bytes of one step's block of a
 // Steps of operands in flight: what fits the registers beside the state.
 template <typename TS, int RT> constexpr int gm_depth() { return RT == 1 ? 8 : RT == 2 ? 4 : 2; }
 
+// How a lane loads its 4 values of a row of U: one by one, or as 16-byte loads
+// (R a multiple of 4, rows 16-byte aligned, not reversed); FULL: those, and the
+// rank fills its row tiles (no padded row to keep zero, 0.8 % of the R = 16,
+// C = 48, L = 32768 float64 scan).
+enum GmU { GM_U1 = 0, GM_U16 = 1, GM_U16_FULL = 2 };
+
 // OUT of the native form (inputs and outputs in the state's dtype): what a pass
 // writes.  The general form (any io dtype) decides at run time.
 enum GmOut { GM_FINAL = 0, GM_EVERY_H = 1, GM_EVERY_HP = 2, GM_ANY = 3 };
 
 // P2 (two tiles per wave, both columns of a pair inside or outside every view,
 // 8-byte aligned): tile h of the wave holds columns 2 n + h of its 32.
-// IS: bytes of an input element (2: bf16 or fp16); VA: a lane's 4 values of a
-// row of U as 16-byte loads (R a multiple of 4, rows 16-byte aligned, not
-// reversed).  The native form issues the same loads and stores in every step
-// (padding steps of a ragged chunk have empty ranges), so no wait has to assume
-// that the operands in flight were never issued.
-template <typename TS, int RT, int CW, int IS, bool VA, int OUT, bool P2>
+// IS: bytes of an input element (2: bf16 or fp16); UA: GmU.  The native form
+// issues the same loads and stores in every step (padding steps of a ragged
+// chunk have empty ranges), so no wait has to assume that the operands in flight
+// were never issued.
+template <typename TS, int RT, int CW, int IS, int UA, int OUT, bool P2>
 __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, int64_t waves) {
     static_assert(!P2 || (CW == 2 && sizeof(TS) == 4 && IS == 4 && OUT != GM_ANY), "paired columns: two fp32 tiles");
     typedef GMma<TS> M;
     typedef typename M::vec vec;
     constexpr bool ANY = OUT == GM_ANY;
+    constexpr bool VA = UA != GM_U1;
     constexpr int PD = gm_depth<TS, RT>();
     constexpr int SS = static_cast<int>(sizeof(TS));
     constexpr bool SPREAD = !ANY && CW == 2;
@@ -348,6 +354,19 @@ __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, 
         }
     };
 
+    // acc is the state after a step; the rows past R stay zero (an infinite state
+    // times the zeros of U's padding would leave NaN there, which the next step
+    // would multiply into every row)
+    auto take = [&](const vec (&acc)[RT][CW]) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int h = 0; h < CW; ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    X[rt][h][i] = UA == GM_U16_FULL || rt < RT - 1 || trow(rt, i) < R ? acc[rt][h][i] : TS(0);
+    };
+
     Ops ring[PD];
 #pragma unroll
     for (int pp = 0; pp < PD; ++pp) fetch(pp, ring[pp]);
@@ -401,10 +420,7 @@ __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, 
                     }
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) fetch_a(ru, o, rt, RT - 1);
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                    for (int h = 0; h < CW; ++h) X[rt][h] = acc[rt][h];
+                take(acc);
                 oh += dh;
                 op += dp;
             }
@@ -440,10 +456,7 @@ __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, 
             if constexpr (ANY) {
                 if (s >= len) break;   // uniform
             }
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int h = 0; h < CW; ++h) X[rt][h] = acc[rt][h];
+            take(acc);
             fetch(s + PD, o);
             if constexpr (ANY) {
                 if (p.every) store_any(oh, op, p.stream);
@@ -493,11 +506,20 @@ inline bool gm_fits(int64_t R, int64_t row) {
     return R <= GM_MAX_R && row <= GM_MAX_BLOCK && (R + 15) / 16 * 16 * row * 8 <= GM_MAX_BLOCK;
 }
 
-template <typename TS, int RT, int CW, int IS, bool VA, int OUT, bool P2 = false>
+template <typename TS, int RT, int CW, int IS, int UA, int OUT, bool P2 = false>
 int gm_launch_k(const GParams& p, int64_t waves, hipStream_t st) {
     const dim3 grid(static_cast<unsigned>((waves + GM_WAVES - 1) / GM_WAVES)), block(64 * GM_WAVES);
-    hipLaunchKernelGGL((generic_mfma_kernel<TS, RT, CW, IS, VA, OUT, P2>), grid, block, 0, st, p, waves);
+    hipLaunchKernelGGL((generic_mfma_kernel<TS, RT, CW, IS, UA, OUT, P2>), grid, block, 0, st, p, waves);
     return check_launch("generic_mfma_kernel");
+}
+
+// the native form
+template <typename TS, int RT, int CW, int UA, bool P2>
+int gm_launch_out(const GParams& p, int64_t waves, hipStream_t st) {
+    constexpr int SS = static_cast<int>(sizeof(TS));
+    if (!p.every) return gm_launch_k<TS, RT, CW, SS, UA, GM_FINAL, P2>(p, waves, st);
+    if (!p.out_p.p) return gm_launch_k<TS, RT, CW, SS, UA, GM_EVERY_H, P2>(p, waves, st);
+    return gm_launch_k<TS, RT, CW, SS, UA, GM_EVERY_HP, P2>(p, waves, st);
 }
 
 template <typename TS, int RT, int CW>
@@ -512,28 +534,27 @@ int gm_launch(const GParams& p, int64_t waves, hipStream_t st) {
             return set_error(MOGT_E_INVALID, "generic scan: form not built");   // not reached: generic_mfma_launch
         } else {
             switch (p.in.code) {
-                case MOGT_F64: return gm_launch_k<TS, RT, CW, 8, false, GM_ANY>(p, waves, st);
-                case MOGT_F32: return gm_launch_k<TS, RT, CW, 4, false, GM_ANY>(p, waves, st);
-                default: return gm_launch_k<TS, RT, CW, 2, false, GM_ANY>(p, waves, st);
+                case MOGT_F64: return gm_launch_k<TS, RT, CW, 8, GM_U1, GM_ANY>(p, waves, st);
+                case MOGT_F32: return gm_launch_k<TS, RT, CW, 4, GM_U1, GM_ANY>(p, waves, st);
+                default: return gm_launch_k<TS, RT, CW, 2, GM_U1, GM_ANY>(p, waves, st);
             }
         }
     }
     const int64_t align = 16 / SS;
     const bool va = !p.rev && p.R % 4 == 0 && p.tr.rs % align == 0 && p.tr.ss % align == 0 && p.tr.bs % align == 0 &&
                     p.tr_c0 % align == 0 && reinterpret_cast<uintptr_t>(p.tr.p) % 16 == 0;
+    const bool full = va && p.R == 16 * RT;
     if constexpr (SS == 4 && CW == 2) {
         auto even = [](const GView& v) {
             return !v.p || ((v.rs | v.ss | v.bs) % 2 == 0 && reinterpret_cast<uintptr_t>(v.p) % 8 == 0);
         };
-        if (va && (p.cin | p.csplit | p.W) % 2 == 0 && even(p.in) && even(p.out_h) && even(p.out_p)) {
-            if (!p.every) return gm_launch_k<TS, RT, CW, SS, true, GM_FINAL, true>(p, waves, st);
-            if (!p.out_p.p) return gm_launch_k<TS, RT, CW, SS, true, GM_EVERY_H, true>(p, waves, st);
-            return gm_launch_k<TS, RT, CW, SS, true, GM_EVERY_HP, true>(p, waves, st);
-        }
+        if (va && (p.cin | p.csplit | p.W) % 2 == 0 && even(p.in) && even(p.out_h) && even(p.out_p))
+            return full ? gm_launch_out<TS, RT, CW, GM_U16_FULL, true>(p, waves, st)
+                        : gm_launch_out<TS, RT, CW, GM_U16, true>(p, waves, st);
     }
-    if (!p.every) return va ? gm_launch_k<TS, RT, CW, SS, true, GM_FINAL>(p, waves, st) : gm_launch_k<TS, RT, CW, SS, false, GM_FINAL>(p, waves, st);
-    if (!p.out_p.p) return va ? gm_launch_k<TS, RT, CW, SS, true, GM_EVERY_H>(p, waves, st) : gm_launch_k<TS, RT, CW, SS, false, GM_EVERY_H>(p, waves, st);
-    return va ? gm_launch_k<TS, RT, CW, SS, true, GM_EVERY_HP>(p, waves, st) : gm_launch_k<TS, RT, CW, SS, false, GM_EVERY_HP>(p, waves, st);
+    if (full) return gm_launch_out<TS, RT, CW, GM_U16_FULL, false>(p, waves, st);
+    if (va) return gm_launch_out<TS, RT, CW, GM_U16, false>(p, waves, st);
+    return gm_launch_out<TS, RT, CW, GM_U1, false>(p, waves, st);
 }
 
 // Tiles per wave: every wave of a chunk reads the whole of U_t, so for fp32 ranks

@@ -437,3 +437,24 @@ def test_matrix_core_workspace_covers_both_levels():
     n = lib.mogt_affine_scan_generic_workspace_bytes(1, 32768, 16, 48, 0, 2)
     assert n > 256 + 8 * 16 * (64 + 48) * 128
     assert lib.mogt_affine_scan_generic_workspace_bytes(1, 32768, 16, 48, 1, 2) > n
+
+
+@pytest.mark.parametrize("state", [torch.float32, torch.float64])
+@pytest.mark.parametrize("B,L,R,C", [(1, 9, 1, 1), (2, 40, 5, 3), (1, 600, 20, 6), (40, 70, 40, 20), (2, 50, 64, 16)])
+def test_infinite_state_keeps_its_sign(gpu, state, B, L, R, C):
+    """An infinity entering one column of a rank that does not fill its row tiles
+    stays an infinity (positive transitions): the padded rows must not turn it
+    into NaN, and the other columns stay as they are."""
+    announce(f"generic infinite state {state} {B} {L} {R} {C}")
+    g = torch.Generator().manual_seed(R)
+    U = ((0.5 + torch.rand(B, L, R, R, generator=g, dtype=torch.float64)) / R).to(state)
+    V = torch.rand(B, L, R, C, generator=g, dtype=torch.float64).to(state)
+    V[:, L // 3, R // 2, 0] = float("inf")
+    for rev in (False, True):
+        ref = _loop64(U, V, rev=rev)[1]
+        _, H = torch.ops.mogt.affine_scan_generic(U.to(gpu), V.to(gpu), state, state, False, rev)
+        H = H.double().cpu()
+        inf = torch.isinf(ref)
+        assert inf.any() and not torch.isnan(ref).any()
+        assert torch.equal(torch.isinf(H), inf) and not torch.isnan(H).any()
+        assert bool((H[inf] > 0).all()) and rel_err(H[~inf].numpy(), ref[~inf].numpy()) <= FP32_TOL
