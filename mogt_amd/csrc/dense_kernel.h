@@ -487,7 +487,10 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
 #pragma unroll
                 for (int h = 0; h < CTW; ++h)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s_h[trow(rt, i)][16 * h + n] = X[rt][RT + h][i];
+                    for (int i = 0; i < 4; ++i)
+                        // columns past C (in the last tile) meet zeros of G, which an
+                        // infinite U's NaN there would turn into NaN
+                        s_h[trow(rt, i)][16 * h + n] = h < CTW - 1 || 16 * h + n < C ? X[rt][RT + h][i] : 0.0f;
             lds_order();
             f32x4 hb[RT][CTW];
 #pragma unroll

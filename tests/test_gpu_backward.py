@@ -350,3 +350,24 @@ def test_kept_carries_give_the_same_scan_and_gradient(gpu, vdt, odt, B, L, R, C)
     Vr = V.clone().requires_grad_()   # no gradient of U: no carries kept
     (gv,) = torch.autograd.grad(triton_scan.triton_affine_scan_hybrid(U, Vr, output_dtype=odt), Vr, G.to(odt))
     assert torch.equal(gv, rv)
+
+
+@pytest.mark.parametrize("C", [8, 24, 40, 48])
+def test_recomputed_grad_u_of_infinite_states(gpu, C):
+    """Infinite transitions leave the columns that pad the channels out of dU:
+    infinite where the sum over the C channels is, not NaN."""
+    announce(f"recomputed dU, infinite transition, C={C}")
+    g = torch.Generator().manual_seed(C)
+    L, R = 70, 16
+    U = (0.5 + torch.rand(1, L, R, R, generator=g)) / R
+    V, G = torch.rand(1, L, R, C, generator=g) + 0.1, torch.rand(1, L, R, C, generator=g) + 0.1
+    U[0, 40, 3, :] = float("inf")
+    H = torch.zeros(R, C, dtype=torch.float64)
+    ref = torch.empty(1, L, R, R, dtype=torch.float64)
+    for t in range(L):
+        ref[0, t] = G[0, t].double() @ H.t()
+        H = U[0, t].double() @ H + V[0, t].double()
+    assert torch.isinf(ref).any() and not torch.isnan(ref).any()
+    dU = torch.ops.mogt.affine_scan_recompute_grad_u(U.to(gpu), V.to(gpu), G.to(gpu)).double().cpu()
+    assert torch.equal(torch.isinf(dU), torch.isinf(ref)) and not torch.isnan(dU).any()
+    assert rel_err(to_np(dU[~torch.isinf(ref)]), to_np(ref[~torch.isinf(ref)])) <= FP32_TOL
