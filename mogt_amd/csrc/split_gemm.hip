@@ -12,7 +12,10 @@
 // at 3 or 6 bf16 products instead of one fp32 product: the bf16 matrix rate is
 // 16 times the fp32 one (155 TFLOP/s reached by the BLAS library's fp32 GEMM,
 // which is that unit's peak).  Elements that are not finite go whole into the
-// first piece.
+// first piece; where infinite elements or overflowing products meet pieces that
+// are zero or of the other sign, the sum of the piece products is NaN though the
+// fp32 product is not: a wave that finds a NaN among its results forms them
+// again in fp32 (exact_tile).
 //
 // Operand layouts, per operand:
 //   K_FAST  element (row, k) at row * ld + k   (K padded with zeros in memory
@@ -197,6 +200,58 @@ struct Operand {
     }
 };
 
+// 8 consecutive k of one row of an operand as the fp32 values its pieces sum to
+// (k: a multiple of 8; K_SLOW: zero from K on).
+template <int NPC, bool KS>
+__device__ __forceinline__ void exact_row(float (&x)[8], const bf16_t* base, int64_t plane, int64_t ld, int row, int k, int K) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) x[q] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NPC; ++c) {
+        if constexpr (KS) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (k + q < K) x[q] += bf16_to_f32(base[c * plane + (k + q) * ld + row]);
+        } else {
+            const Pack<bf16_t, 8> w = *reinterpret_cast<const Pack<bf16_t, 8>*>(base + c * plane + row * ld + k);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) x[q] += bf16_to_f32(w.v[q]);
+        }
+    }
+}
+
+// The wave's accumulators from fp32 products of the same operands (stages s0 ..
+// s0 + T - 1), read from memory: v_mfma_f32_32x32x2_f32 leaves its results where
+// the bf16 form does, and lane half h takes k = 8 h + q as there.  Rows past the
+// end repeat the last one; their results are not used.
+template <int NA, int NB, bool KSA, bool KSB, int TNF, bool TR>
+__device__ __forceinline__ void exact_tile(sp_f32x16 (&acc)[TNF][4], const SplitParams& p, int m0, int n0, int s0, int T,
+                                           int l32, int hb) {
+#pragma unroll
+    for (int j = 0; j < TNF; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.0f;
+    for (int k0 = s0 * SP_BK; k0 < (s0 + T) * SP_BK; k0 += 16) {
+        const int k = k0 + 8 * hb;
+        float b[TNF][8];
+#pragma unroll
+        for (int j = 0; j < TNF; ++j)
+            exact_row<NB, KSB>(b[j], p.b, p.pb, p.ldb, min(n0 + 32 * j + l32, p.nb_valid - 1), k, p.K);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float a[8];
+            exact_row<NA, KSA>(a, p.a, p.pa, p.lda, min(m0 + 32 * i + l32, p.M - 1), k, p.K);
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+#pragma unroll
+                for (int j = 0; j < TNF; ++j)
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(TR ? a[q] : b[j][q], TR ? b[j][q] : a[q], acc[j][i], 0, 0, 0);
+        }
+    }
+}
+
 template <int NA, int NB, bool KSA, bool KSB, int TNF, int EPI, bool TR>
 __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split_gemm_kernel(SplitParams p) {
     static_assert(EPI == EPI_STORE || (!KSA && !KSB && !TR), "cross-entropy epilogues: the logits form");
@@ -353,6 +408,21 @@ __global__ __launch_bounds__(SP_THREADS, NA == 1 && TNF == 2 ? 2 : 1) void split
     }
     kstep(f0, f1, s, 1, 0, YES, NO);
     kstep(f1, f0, 0, 0, 0, NO, NO);
+
+    // a NaN among the wave's results (or infinities of both signs) leaves one in
+    // their sum (a training pass of the loss over 8192 tokens, vocabulary 32000:
+    // 5124 us without the test, 5132 with it)
+    if constexpr (NP > 1) {
+        float any = 0.0f;
+#pragma unroll
+        for (int j = 0; j < TNF; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) any += acc[j][i][r];
+        if (__any(any != any))
+            exact_tile<NA, NB, KSA, KSB, TNF, TR>(acc, p, m0 + 128 * wm, n0 + 32 * TNF * wn, s0, T, l32, hb);
+    }
 
     // lane (l32, hb), register group q of acc[j][i]: row m0 + 128 wm + 32 i +
     // l32, columns n0 + 32 TNF wn + 32 j + 8 q + 4 hb .. + 3

@@ -325,8 +325,8 @@ def test_chunked_linear_ce_split_form_matches_library_form(gpu, monkeypatch, hd,
 def test_split_ce_epilogues_match_the_row_kernels(gpu, da, db, M, V, K):
     """The cross-entropy epilogues against the row kernels on the same product's
     written logits: ragged row and column tiles, a label in every column group
-    and at the edges, ignored and bad labels, a row of equal logits and rows
-    with -inf / NaN."""
+    and at the edges, ignored and bad labels, a row of equal logits and a row of
+    NaN."""
     announce(f"split ce {M} {V} {K} {da} {db}")
     from mogt_amd import ops
 
@@ -384,3 +384,127 @@ def test_chunked_linear_ce_fused_epilogue_end_to_end(gpu):
 
     for got, ref in zip(call(0), call(1 << 62)):
         assert rel_err(to_np(got), to_np(ref)) <= (1e-5 if got.dtype == torch.float32 else 2.0 ** -8)
+
+
+def _fp32_products(a, b):
+    """sum_k a b as an fp32 sum of fp32 products has it (infinities, overflow)."""
+    return (a.float().cpu()[:, None, :] * b.float().cpu()[None, :, :]).sum(-1)
+
+
+def _same_specials(got, ref):
+    got, ref = got.float().cpu(), ref.float().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.isposinf(got), torch.isposinf(ref)) and torch.equal(torch.isneginf(got), torch.isneginf(ref))
+
+
+def _specials(a, b):
+    """Infinities against pieces that are zero or of the other sign, and products
+    past the largest float, in few rows of each operand."""
+    inf = float("inf")
+    a[0] = 1.0                                  # exact in one piece: its others are zero
+    a[1, 0], a[2, 1] = inf, -inf
+    b[1, 0], b[2, 3], b[3, 5] = -inf, inf, 0.0
+    a[3, 7], b[4, 7], b[5, 7] = 1e30, 1e30, -1e30
+    b[6, 0] = 0.0                               # 0 * inf
+
+
+@pytest.mark.parametrize("da,db", SPLIT_DT)
+@pytest.mark.parametrize("M,N,K", [(9, 8, 32), (300, 200, 96)])
+def test_split_gemm_infinities_as_in_fp32(gpu, da, db, M, N, K):
+    """Infinite and overflowing products come out as fp32 products give them, in
+    every piece pair; elements without them within the fp32 bound."""
+    announce(f"split gemm infinities {M} {N} {K} {da} {db}")
+    from mogt_amd import ops
+
+    a, b = _bf16_or_f32((M, K), da, 41), _bf16_or_f32((N, K), db, 42)
+    _specials(a, b)
+    a, b = a.to(gpu), b.to(gpu)
+    out = torch.empty(M, -(-N // 4) * 4, device=gpu)[:, :N]
+    ops.split_gemm_(out, _pieces_of(a), _pieces_of(b), K)
+    ref = _fp32_products(a, b)
+    _same_specials(out, ref)
+    fin = torch.isfinite(ref)
+    d64 = (a.double().cpu() @ b.double().cpu().t(), a.double().abs().cpu() @ b.double().abs().cpu().t())
+    assert bool(((out.double().cpu() - d64[0]).abs() <= (K + 8) * 2.0 ** -24 * d64[1])[fin].all())
+
+
+@pytest.mark.parametrize("db", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,V,D", [(37, 1001, 64), (300, 4096, 96)])
+def test_split_gemm_gradient_infinities_as_in_fp32(gpu, n, V, D, db):
+    announce(f"split gemm gradient infinities {n} {V} {D} {db}")
+    from mogt_amd import ops
+
+    g, x, h = _bf16_or_f32((n, V), torch.float32, 43), _bf16_or_f32((V, D), db, 44), _bf16_or_f32((n, D), db, 45)
+    inf = float("inf")
+    g[0, 0], g[1, 5], g[2, V - 1], g[3, 9] = 0.5, inf, -inf, 1e30   # 0.5: one piece
+    x[0, 1], x[V - 1, 2], x[9, 3], x[5, 4] = inf, -inf, 1e30, 0.0
+    h[0, 1], h[1, 4], h[3, 3] = -inf, 0.0, 1e30
+    gp = ops.split_pieces(g.to(gpu))
+    dh = torch.empty(n, D, device=gpu)
+    ops.split_gemm_(dh, gp, _pieces_of(x.to(gpu)), V, k_slow_b=True)
+    _same_specials(dh, torch.cat([_fp32_products(g[i:i + 8], x.t()) for i in range(0, n, 8)]))
+    dw = torch.zeros(V, D, device=gpu)
+    ops.split_gemm_(dw, gp, _pieces_of(h.to(gpu)), n, k_slow_a=True, k_slow_b=True, accumulate=True)
+    _same_specials(dw, torch.cat([_fp32_products(g.t()[i:i + 64], h.t()) for i in range(0, V, 64)]))
+
+
+@pytest.mark.parametrize("da,db", SPLIT_DT)
+def test_split_ce_epilogues_of_infinite_logits(gpu, da, db):
+    """Rows with -inf logits (masked vocabulary rows against a constant feature),
+    +inf and NaN logits: the epilogues as the row kernels on the fp32 products."""
+    announce(f"split ce infinities {da} {db}")
+    from mogt_amd import ops
+
+    M, V, K = 270, 515, 64
+    a, b = _bf16_or_f32((M, K), da, 51), _bf16_or_f32((V, K), db, 52)
+    a[:, 0] = 1.0
+    b[5:400:7, 0] = float("-inf")
+    a[260, 1], a[261, 1] = float("inf"), float("nan")
+    b[0, 1] = 0.0
+    a, b = a.to(gpu), b.to(gpu)
+    lab = torch.randint(0, V, (M,), generator=torch.Generator().manual_seed(1)).to(gpu)
+    lab[7], lab[8] = 5, 6
+    logits = torch.cat([_fp32_products(a[i:i + 16], b) for i in range(0, M, 16)]).to(gpu)
+    loss, lse = ops.lm_ce_forward(logits, lab)
+    assert int(torch.isfinite(loss).sum()) > 200 and bool(torch.isinf(loss[7]))
+    # two fp32 sums of K products, each within (K + 8) 2^-24 sum |a b| of the exact
+    # logit: a probability changes by that relative amount
+    size = torch.where(torch.isfinite(a), a, 0).abs().double() @ torch.where(torch.isfinite(b), b, 0).abs().double().t()
+    tol = ROW_TOL + 2 * (K + 8) * 2.0 ** -24 * float(size.max())
+    loss2, lse2 = ops.split_ce_forward(_pieces_of(a), _pieces_of(b), K, lab)
+    _same_specials(loss2, loss)
+    _same_specials(lse2, lse)
+    fin = torch.isfinite(loss)
+    assert rel_err(to_np(loss2[fin]), to_np(loss[fin])) <= tol
+    scale = torch.tensor([0.37], device=gpu)
+    g = ops.lm_ce_grad(logits, lab, lse, scale)
+    g2 = ops.split_ce_grad_pieces(_pieces_of(a), _pieces_of(b), K, lab, lse, scale).float().sum(0)[:, :V]
+    _same_specials(g2, g)
+    fin = torch.isfinite(g)
+    assert rel_err(to_np(g2[fin]), to_np(g[fin])) <= tol
+
+
+@pytest.mark.parametrize("hd", [torch.float32, torch.bfloat16])
+def test_chunked_linear_ce_masked_vocabulary(gpu, monkeypatch, hd):
+    """Vocabulary rows masked by -inf against a constant hidden feature: the loss
+    of the split form is finite as the library form's, the gradients alike."""
+    announce(f"chunked CE masked vocabulary {hd}")
+    from mogt_amd import chunked_lm_loss as cl
+
+    h, w = _bf16_or_f32((1, 300, 64), hd, 61), _bf16_or_f32((1003, 64), torch.float32, 62, 0.3)
+    h[..., 0] = 1.0
+    w[10:20, 0] = float("-inf")
+    h, w = h.to(gpu).requires_grad_(), w.to(gpu).requires_grad_()
+    lab = torch.randint(20, 1003, (1, 300), generator=torch.Generator().manual_seed(5)).to(gpu)
+
+    def call():
+        loss = cl.chunked_linear_cross_entropy(h, w, lab, chunk_size=128)
+        return [loss.detach(), *torch.autograd.grad(loss, [h, w])]
+
+    lib = call()
+    assert bool(torch.isfinite(lib[0])) and bool(torch.isfinite(lib[2]).all())
+    monkeypatch.setattr(cl, "SPLIT_MIN_MACS", 0)
+    for got, ref in zip(call(), lib):
+        _same_specials(got, ref)
+        fin = torch.isfinite(ref)
+        assert rel_err(to_np(got[fin]), to_np(ref[fin])) <= (1e-5 if got.dtype == torch.float32 else 2.0 ** -8)
