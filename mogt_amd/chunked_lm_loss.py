@@ -176,6 +176,19 @@ class _Head:
         ops.split_gemm_(d_w32, g, rows, block.shape[0], k_slow_a=True, k_slow_b=True, accumulate=not first)
 
 
+class _NotTwiceDifferentiable(torch.autograd.Function):
+    """Gradients that a second differentiation refuses (through ``grads`` as well
+    as through ``inputs``) instead of taking them as constants."""
+
+    @staticmethod
+    def forward(ctx, n_inputs: int, *tensors):
+        return tuple(g.view_as(g) for g in tensors[n_inputs:])
+
+    @staticmethod
+    def backward(ctx, *grad_outputs):
+        raise RuntimeError("chunked_linear_cross_entropy has no second derivative")
+
+
 class _ChunkedLinearCrossEntropy(torch.autograd.Function):
     """chunked_lm_loss.py:5-72 on the HIP cross-entropy rows."""
 
@@ -216,10 +229,14 @@ class _ChunkedLinearCrossEntropy(torch.autograd.Function):
         head = _Head(rows, weight, ctx.chunk_size, ctx.autocast)
         d_rows = torch.empty_like(rows)
         d_w32 = head.new_weight_grad()
-        for i, sl in enumerate(_token_blocks(n_tok, ctx.chunk_size)):
-            with torch.autocast("cuda", enabled=False):
-                head.backward(targets[sl], lse[sl], scale, rows[sl], d_rows[sl], d_w32, first=i == 0)
-        return d_rows.view_as(hidden_states), d_w32.to(weight.dtype), None, None
+        with torch.no_grad():
+            for i, sl in enumerate(_token_blocks(n_tok, ctx.chunk_size)):
+                with torch.autocast("cuda", enabled=False):
+                    head.backward(targets[sl], lse[sl], scale, rows[sl], d_rows[sl], d_w32, first=i == 0)
+        d_hidden, d_weight = d_rows.view_as(hidden_states), d_w32.to(weight.dtype)
+        if torch.is_grad_enabled() and not torch.compiler.is_compiling():   # create_graph
+            d_hidden, d_weight = _NotTwiceDifferentiable.apply(3, hidden_states, weight, grad_output, d_hidden, d_weight)
+        return d_hidden, d_weight, None, None
 
 
 def chunked_linear_cross_entropy(hidden_states, weight, labels, *, chunk_size: int):

@@ -508,3 +508,21 @@ def test_chunked_linear_ce_masked_vocabulary(gpu, monkeypatch, hd):
         _same_specials(got, ref)
         fin = torch.isfinite(ref)
         assert rel_err(to_np(got[fin]), to_np(ref[fin])) <= (1e-5 if got.dtype == torch.float32 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_chunked_linear_ce_second_derivative_is_refused(gpu, monkeypatch, split):
+    """The gradients are not differentiable again: a second derivative raises
+    instead of taking them as constants."""
+    announce(f"chunked CE second derivative split={split}")
+    from mogt_amd import chunked_lm_loss as cl
+
+    monkeypatch.setattr(cl, "SPLIT_MIN_MACS", 0 if split else 1 << 62)
+    h = torch.randn(1, 40, 32, device=gpu, requires_grad=True)
+    w = torch.randn(65, 32, device=gpu, requires_grad=True)
+    lab = torch.randint(0, 65, (1, 40), device=gpu)
+    loss = cl.chunked_linear_cross_entropy(h, w, lab, chunk_size=32)
+    gh, gw = torch.autograd.grad(loss, [h, w], create_graph=True)
+    for penalty in (gh.square().sum(), gw.square().sum(), loss + gh.square().sum()):
+        with pytest.raises(RuntimeError):
+            torch.autograd.grad(penalty, [h, w], retain_graph=True)
