@@ -69,6 +69,14 @@ def _stream_handle(device: torch.device) -> int:
 LOOKBACK_FAMILIES = frozenset({"diag", "diag_rev", "diag_grad", "coupled", "coupled_rev", "rank1"})
 
 
+def scratch(nbytes: int, device: torch.device) -> torch.Tensor:
+    """Uninitialised memory for one call, read back by a later launch of the
+    same call: from the caching allocator, so that calls of several threads on
+    one stream, whose launches may interleave, do not share it (``workspace``
+    does)."""
+    return torch.empty(int(nbytes), dtype=torch.uint8, device=device)
+
+
 def workspace(nbytes: int, device: torch.device, family: str = "plain", layout: tuple | None = None
               ) -> torch.Tensor:
     """Zero-initialised scratch of at least ``nbytes`` for the current stream.
@@ -2250,7 +2258,7 @@ def _split_gemm_impl(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, k: int
     lib = _lib.load()
     M, N = out.shape
     nbytes = int(lib.mogt_split_gemm_workspace_bytes(M, N, k, a.shape[0], b.shape[0], 0, 0))
-    ws = workspace(nbytes, out.device)
+    ws = scratch(nbytes, out.device)
     rc = lib.mogt_split_gemm(a.data_ptr(), a.stride(1), a.stride(0), a.shape[0], int(k_slow_a), b.data_ptr(),
                              b.stride(1), b.stride(0), b.shape[0], int(k_slow_b), out.data_ptr(), out.stride(0), M, N,
                              k, int(accumulate), dtype_code(out.dtype, "split_gemm"), 0, ws.data_ptr(), ws.numel(),
@@ -2309,7 +2317,7 @@ def _split_ce_fwd_op(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Ten
     M, V = a.shape[1], b.shape[1]
     loss = torch.empty(M, dtype=torch.float32, device=a.device)
     lse = torch.empty(M, dtype=torch.float32, device=a.device)
-    ws = workspace(int(lib.mogt_split_ce_workspace_bytes(M, V, a.shape[0], b.shape[0])), a.device)
+    ws = scratch(lib.mogt_split_ce_workspace_bytes(M, V, a.shape[0], b.shape[0]), a.device)
     rc = lib.mogt_split_ce_fwd(a.data_ptr(), a.stride(1), a.stride(0), a.shape[0], b.data_ptr(), b.stride(1),
                                b.stride(0), b.shape[0], labels.data_ptr(), M, V, k, int(ignore_index),
                                loss.data_ptr(), lse.data_ptr(), ws.data_ptr(), ws.numel(), _stream_handle(a.device))

@@ -388,6 +388,47 @@ def test_checked_mode_reports_each_give_up_once(monkeypatch):
         ops._checked(ws, "scan")                  # one more
 
 
+def test_split_products_of_two_threads_keep_apart(monkeypatch):
+    """Two threads on one stream (a launch drops the interpreter lock) may each
+    be between the launch that writes the rows' pairs or the slices' partials
+    and the one that reads them: each call brings scratch memory of its own."""
+    import threading
+
+    ops, dev = _fake_device_workspace(monkeypatch)
+    both = threading.Barrier(2, timeout=60)
+    seen = {"ce": [], "gemm": []}
+
+    class Lib:
+        def mogt_split_ce_workspace_bytes(self, *args):
+            return 4096
+
+        def mogt_split_gemm_workspace_bytes(self, *args):
+            return 4096
+
+        def mogt_split_ce_fwd(self, *args):
+            seen["ce"].append((args[15], args[16]))
+            both.wait()   # both calls are between their launches
+            return 0
+
+        def mogt_split_gemm(self, *args):
+            seen["gemm"].append((args[18], args[19]))
+            both.wait()
+            return 0
+
+    monkeypatch.setattr(ops._lib, "load", lambda: Lib())
+    a, b = torch.zeros(1, 4, 32, dtype=torch.bfloat16), torch.zeros(1, 8, 32, dtype=torch.bfloat16)
+    labels = torch.zeros(4, dtype=torch.int64)
+    for name, call in (("ce", lambda: ops._split_ce_fwd_op.impl(a, b, 32, labels, -100)),
+                       ("gemm", lambda: ops._split_gemm_op.impl(torch.zeros(4, 8), a, b, 32, False, False, False))):
+        threads = [threading.Thread(target=call) for _ in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        (p0, n0), (p1, n1) = seen[name]
+        assert n0 >= 4096 and n1 >= 4096 and (p0 + n0 <= p1 or p1 + n1 <= p0)
+
+
 @pytest.mark.parametrize("source", ["swiglu_gemm.hip", "wgrad_gemm.hip", "rank1_scan.hip", "split_gemm.hip"])
 def test_gemm_m0_only_feeds_lds_dma(tmp_path, source):
     """The bf16 GEMMs (fused SwiGLU, split-K weight gradient) and the rank-1
