@@ -582,11 +582,12 @@ int mogt_lm_ce_bwd_pieces(const void* logits, int64_t ld, int logits_dtype, cons
  *   pieces); A k_slow 0 or 1 in 3 pieces with B k_slow 1.  C fp32 (accumulate
  *   adds to it) or bf16, row stride ldc >= N rounded up to 4 (those columns are
  *   written).  Workspace: fp32 partials of the K slices (splits <= 0: chosen),
- *   mogt_split_gemm_workspace_bytes(... cus <= 0: of the current device).    */
+ *   mogt_split_gemm_workspace_bytes(... cus <= 0: of the current device); 0,
+ *   and the workspace may be null, where one slice writes an fp32 C.         */
 int mogt_split_pieces(const void* src, int64_t ld_src, void* dst, int64_t ld_dst, int64_t rows, int64_t cols,
                       void* stream);
-size_t mogt_split_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int pieces_a, int pieces_b, int64_t splits,
-                                       int64_t cus);
+size_t mogt_split_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int pieces_a, int pieces_b, int k_slow_a,
+                                       int out_dtype, int64_t splits, int64_t cus);
 int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int pieces_a, int k_slow_a, const void* B,
                     int64_t ldb, int64_t plane_b, int pieces_b, int k_slow_b, void* C, int64_t ldc, int64_t M,
                     int64_t N, int64_t K, int accumulate, int out_dtype, int64_t splits, void* workspace,

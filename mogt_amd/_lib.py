@@ -185,7 +185,8 @@ SIGNATURES: dict[str, tuple] = {
         _c_int, [_c_void_p, _c_i64, _c_int, _c_void_p, _c_void_p, _c_i64, _c_i64, _c_i64, _c_void_p,
                  _c_void_p, _c_i64, _c_void_p]),
     "mogt_split_pieces": (_c_int, [_c_void_p, _c_i64, _c_void_p, _c_i64, _c_i64, _c_i64, _c_void_p]),
-    "mogt_split_gemm_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_i64, _c_i64]),
+    "mogt_split_gemm_workspace_bytes": (
+        _c_size, [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_i64, _c_i64]),
     "mogt_split_gemm": (
         _c_int, [_c_void_p, _c_i64, _c_i64, _c_int, _c_int, _c_void_p, _c_i64, _c_i64, _c_int, _c_int, _c_void_p,
                  _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_i64, _c_void_p, _c_size, _c_void_p]),

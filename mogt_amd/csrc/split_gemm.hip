@@ -749,6 +749,17 @@ void launch_split_pieces(const SplitParams& p, int na, int nb, int64_t blocks, h
 // 21; 16000 x 1024 over 4096 rows, where both fill their rounds, 305 in both.
 bool swap_operands(int na, int nb, bool k_slow_a) { return k_slow_a && na == 3 && nb == 1; }
 
+SplitPlan plan_launch(int64_t M, int64_t N, int64_t K, int na, int nb, bool k_slow_a, int64_t splits, int64_t cus) {
+    return swap_operands(na, nb, k_slow_a) ? plan_split(N, M, K, nb, na, splits, cus) : plan_split(M, N, K, na, nb, splits, cus);
+}
+
+// Bytes of the slices' fp32 partials (M x N, N rounded up to 4): none where one
+// slice writes fp32 straight to the output.
+size_t partials_bytes(const SplitPlan& pl, int64_t M, int64_t N, int out_dtype) {
+    if (pl.slices == 1 && out_dtype == MOGT_F32) return 0;
+    return static_cast<size_t>(pl.slices) * M * ((N + 3) / 4 * 4) * sizeof(float);
+}
+
 template <int EPI>
 void launch_split_ce(const SplitParams& p, int na, int nb, int64_t blocks, hipStream_t st) {
     if (na == 3 && nb == 3) launch_split<3, 3, false, false, EPI>(p, blocks, st);
@@ -786,21 +797,14 @@ extern "C" int mogt_split_pieces(const void* src, int64_t ld_src, void* dst, int
 }
 
 extern "C" size_t mogt_split_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int pieces_a, int pieces_b,
-                                                  int64_t splits, int64_t cus) {
+                                                  int k_slow_a, int out_dtype, int64_t splits, int64_t cus) {
     if (check_split_shape(M, N, K, pieces_a, pieces_b) != MOGT_OK || M == 0 || N == 0 || K == 0) return 0;
     if (cus <= 0) {
         int n = 0;
         if (device_cu_count(n) != MOGT_OK) return 0;
         cus = n;
     }
-    // at most this many bytes whatever the output type (a bf16 output always
-    // goes through the partials) and the layouts (swap_operands)
-    int64_t slices = plan_split(M, N, K, pieces_a, pieces_b, splits, cus).slices;
-    if (swap_operands(pieces_a, pieces_b, true)) {
-        const int64_t swapped = plan_split(N, M, K, pieces_b, pieces_a, splits, cus).slices;
-        if (swapped > slices) slices = swapped;
-    }
-    return static_cast<size_t>(slices) * M * ((N + 3) / 4 * 4) * sizeof(float);
+    return partials_bytes(plan_launch(M, N, K, pieces_a, pieces_b, k_slow_a, splits, cus), M, N, out_dtype);
 }
 
 extern "C" int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int pieces_a, int k_slow_a, const void* B,
@@ -828,13 +832,12 @@ extern "C" int mogt_split_gemm(const void* A, int64_t lda, int64_t plane_a, int 
     int cus = 0;
     if (int rc = device_cu_count(cus)) return rc;
     const bool swap = swap_operands(pieces_a, pieces_b, k_slow_a);
-    const SplitPlan pl = swap ? plan_split(N, M, K, pieces_b, pieces_a, splits, cus)
-                              : plan_split(M, N, K, pieces_a, pieces_b, splits, cus);
+    const SplitPlan pl = plan_launch(M, N, K, pieces_a, pieces_b, k_slow_a, splits, cus);
     const int64_t blocks = pl.n_mb * pl.n_nb * pl.slices;
     if (blocks > 0x7fffffff) return set_error(MOGT_E_INVALID, "split_gemm: too many tiles");
-    const bool parts = pl.slices > 1 || out_dtype == MOGT_BF16;
+    const size_t need = partials_bytes(pl, M, N, out_dtype);
+    const bool parts = need > 0;
     if (parts) {
-        const size_t need = static_cast<size_t>(pl.slices) * M * Np * sizeof(float);
         if (!workspace || workspace_bytes < need)
             return set_error(MOGT_E_WORKSPACE, "split_gemm: workspace of %zu bytes needed, %zu given", need,
                              workspace_bytes);

@@ -2257,11 +2257,12 @@ def _split_gemm_impl(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, k: int
                    accumulate: bool) -> None:
     lib = _lib.load()
     M, N = out.shape
-    nbytes = int(lib.mogt_split_gemm_workspace_bytes(M, N, k, a.shape[0], b.shape[0], 0, 0))
-    ws = scratch(nbytes, out.device)
+    code = dtype_code(out.dtype, "split_gemm")
+    nbytes = lib.mogt_split_gemm_workspace_bytes(M, N, k, a.shape[0], b.shape[0], int(k_slow_a), code, 0, 0)
+    ws = scratch(nbytes, out.device) if nbytes else None   # none: one slice writes straight to out
     rc = lib.mogt_split_gemm(a.data_ptr(), a.stride(1), a.stride(0), a.shape[0], int(k_slow_a), b.data_ptr(),
                              b.stride(1), b.stride(0), b.shape[0], int(k_slow_b), out.data_ptr(), out.stride(0), M, N,
-                             k, int(accumulate), dtype_code(out.dtype, "split_gemm"), 0, ws.data_ptr(), ws.numel(),
+                             k, int(accumulate), code, 0, ws.data_ptr() if nbytes else None, nbytes,
                              _stream_handle(out.device))
     _lib.check(rc, "mogt_split_gemm")
 

@@ -429,6 +429,32 @@ def test_split_products_of_two_threads_keep_apart(monkeypatch):
         assert n0 >= 4096 and n1 >= 4096 and (p0 + n0 <= p1 or p1 + n1 <= p0)
 
 
+def test_split_products_ask_for_partials_only():
+    """One K slice with an fp32 output writes straight to it and asks for no
+    scratch memory; otherwise the partials of the slices the launch takes, in the
+    layout it takes."""
+    from mogt_amd import _lib
+
+    lib = _lib.load()
+    F32, BF16, cus = _lib.MOGT_F32, _lib.MOGT_BF16, 256
+    size = lambda *a: lib.mogt_split_gemm_workspace_bytes(*a, cus)   # noqa: E731
+    # the weight gradient of a bf16 and an fp32 hidden state, the logits, in one slice
+    assert size(32000, 768, 4096, 3, 1, 1, F32, 0) == 0
+    assert size(128256, 4096, 4096, 3, 1, 1, F32, 0) == 0
+    assert size(32000, 768, 4096, 3, 3, 1, F32, 1) == 0
+    assert size(4096, 32000, 768, 1, 3, 0, F32, 0) == 0
+    # a bf16 output goes through the partials, also in one slice
+    assert size(4096, 770, 32000, 3, 3, 0, BF16, 1) == 4096 * 772 * 4
+    for M, N, K, pa, pb in ((4096, 768, 32000, 3, 3), (300, 129, 10007, 3, 1), (33, 50257, 768, 1, 3), (1, 1, 32, 1, 1)):
+        slices = lib.mogt_split_gemm_slices(M, N, K, pa, pb, cus)
+        want = slices * M * (-(-N // 4) * 4) * 4
+        assert size(M, N, K, pa, pb, 0, BF16, 0) == want
+        assert size(M, N, K, pa, pb, 0, F32, 0) == (want if slices > 1 else 0)
+    # 3 x 1 pieces with both operands K-slow swap places
+    swapped = lib.mogt_split_gemm_slices(256, 4000, 20000, 1, 3, cus)
+    assert swapped > 1 and size(4000, 256, 20000, 3, 1, 1, F32, 0) == swapped * 4000 * 256 * 4
+
+
 @pytest.mark.parametrize("source", ["swiglu_gemm.hip", "wgrad_gemm.hip", "rank1_scan.hip", "split_gemm.hip"])
 def test_gemm_m0_only_feeds_lds_dma(tmp_path, source):
     """The bf16 GEMMs (fused SwiGLU, split-K weight gradient) and the rank-1
