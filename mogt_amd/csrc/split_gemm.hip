@@ -200,54 +200,73 @@ struct Operand {
     }
 };
 
-// 8 consecutive k of one row of an operand as the fp32 values its pieces sum to
-// (k: a multiple of 8; K_SLOW: zero from K on).
-template <int NPC, bool KS>
-__device__ __forceinline__ void exact_row(float (&x)[8], const bf16_t* base, int64_t plane, int64_t ld, int row, int k, int K) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) x[q] = 0.0f;
-#pragma unroll
-    for (int c = 0; c < NPC; ++c) {
-        if constexpr (KS) {
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                if (k + q < K) x[q] += bf16_to_f32(base[c * plane + (k + q) * ld + row]);
-        } else {
-            const Pack<bf16_t, 8> w = *reinterpret_cast<const Pack<bf16_t, 8>*>(base + c * plane + row * ld + k);
-#pragma unroll
-            for (int q = 0; q < 8; ++q) x[q] += bf16_to_f32(w.v[q]);
-        }
+// Q consecutive k of one row of one piece, as loaded (k: a multiple of Q).
+template <bool KS, int Q> struct RawRow {
+    Pack<bf16_t, Q> w;
+    __device__ __forceinline__ void load(const bf16_t* base, int64_t ld, int row, int k, int) {
+        w = *reinterpret_cast<const Pack<bf16_t, Q>*>(base + row * ld + k);
     }
-}
+    __device__ __forceinline__ float at(int q, int, int) const { return bf16_to_f32(w.v[q]); }
+};
+template <int Q> struct RawRow<true, Q> {
+    bf16_t v[Q];
+    // rows past K repeat the last one: the loads carry no condition, which would
+    // make each wait for the one before
+    __device__ __forceinline__ void load(const bf16_t* base, int64_t ld, int row, int k, int K) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) v[q] = base[min(k + q, K - 1) * ld + row];
+    }
+    __device__ __forceinline__ float at(int q, int k, int K) const { return k + q < K ? bf16_to_f32(v[q]) : 0.0f; }
+};
 
 // The wave's accumulators from fp32 products of the same operands (stages s0 ..
-// s0 + T - 1), read from memory: v_mfma_f32_32x32x2_f32 leaves its results where
-// the bf16 form does, and lane half h takes k = 8 h + q as there.  Rows past the
-// end repeat the last one; their results are not used.
+// s0 + T - 1), read from memory and summed from their pieces:
+// v_mfma_f32_32x32x2_f32 leaves its results where the bf16 form does; lane half h
+// takes k = Q h + q of a step of 2 Q.  Rows past the end repeat the last one; their
+// results are not used.  (All inputs NaN, where every wave comes here: a training
+// pass over 8192 tokens, vocabulary 32000, 21 ms; the BLAS library's fp32 GEMMs 12.)
 template <int NA, int NB, bool KSA, bool KSB, int TNF, bool TR>
 __device__ __forceinline__ void exact_tile(sp_f32x16 (&acc)[TNF][4], const SplitParams& p, int m0, int n0, int s0, int T,
                                            int l32, int hb) {
+    constexpr int Q = NA == 1 && KSA ? 4 : 8;   // 8 would spill at that form's 256 registers
 #pragma unroll
     for (int j = 0; j < TNF; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.0f;
-    for (int k0 = s0 * SP_BK; k0 < (s0 + T) * SP_BK; k0 += 16) {
-        const int k = k0 + 8 * hb;
-        float b[TNF][8];
+    for (int k0 = s0 * SP_BK; k0 < (s0 + T) * SP_BK; k0 += 2 * Q) {
+        const int k = k0 + Q * hb;
+        RawRow<KSA, Q> a[4][NA];
+        RawRow<KSB, Q> b[TNF][NB];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < NA; ++c) a[i][c].load(p.a + c * p.pa, p.lda, min(m0 + 32 * i + l32, p.M - 1), k, p.K);
 #pragma unroll
         for (int j = 0; j < TNF; ++j)
-            exact_row<NB, KSB>(b[j], p.b, p.pb, p.ldb, min(n0 + 32 * j + l32, p.nb_valid - 1), k, p.K);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float a[8];
-            exact_row<NA, KSA>(a, p.a, p.pa, p.lda, min(m0 + 32 * i + l32, p.M - 1), k, p.K);
+            for (int c = 0; c < NB; ++c) b[j][c].load(p.b + c * p.pb, p.ldb, min(n0 + 32 * j + l32, p.nb_valid - 1), k, p.K);
 #pragma unroll
-            for (int q = 0; q < 8; ++q)
+        for (int q = 0; q < Q; ++q) {
+            float x[4], y[TNF];
 #pragma unroll
-                for (int j = 0; j < TNF; ++j)
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(TR ? a[q] : b[j][q], TR ? b[j][q] : a[q], acc[j][i], 0, 0, 0);
+            for (int i = 0; i < 4; ++i) {
+                x[i] = a[i][0].at(q, k, p.K);
+#pragma unroll
+                for (int c = 1; c < NA; ++c) x[i] += a[i][c].at(q, k, p.K);
+            }
+#pragma unroll
+            for (int j = 0; j < TNF; ++j) {
+                y[j] = b[j][0].at(q, k, p.K);
+#pragma unroll
+                for (int c = 1; c < NB; ++c) y[j] += b[j][c].at(q, k, p.K);
+            }
+#pragma unroll
+            for (int j = 0; j < TNF; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(TR ? x[i] : y[j], TR ? y[j] : x[i], acc[j][i], 0, 0, 0);
         }
     }
 }
