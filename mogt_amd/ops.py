@@ -247,8 +247,11 @@ _NO_RANGE = contextlib.nullcontext()
 
 def profiler_range(name: str):
     """A profiler range while a profiler runs (entering one costs about 5 us of
-    host time, several times per layer)."""
-    return torch.autograd.profiler.record_function(name) if torch.autograd._profiler_enabled() else _NO_RANGE
+    host time, several times per layer); none in a compiled graph, which cannot
+    hold the question."""
+    if torch.compiler.is_compiling() or not torch.autograd._profiler_enabled():
+        return _NO_RANGE
+    return torch.autograd.profiler.record_function(name)
 
 
 def require_cuda(what: str, *tensors: torch.Tensor) -> None:

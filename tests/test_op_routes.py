@@ -1,7 +1,8 @@
 """The two routes of an op (``ops._Op``): the direct call of plain eager tensors
 and the dispatcher.  On the CPU, with ops made of torch arithmetic: which calls
 take which route, and that both give the same results, gradients, saved-tensor
-hooks and version counts."""
+hooks and version counts.  The public functions and a layer are traced with fake
+GPU tensors into one graph (``torch.compile(fullgraph=True)``)."""
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -165,3 +166,49 @@ def test_written_arguments_count_a_version(monkeypatch):
     _fill(s, 2.0)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         z.backward()
+
+
+class _Traced(Exception):
+    pass
+
+
+def _trace(fn, *args):
+    """The one graph torch.compile makes of the call, traced and not run."""
+    graphs = []
+
+    def backend(gm, inputs):
+        graphs.append(gm)
+
+        def run(*a):
+            raise _Traced
+
+        return run
+
+    torch._dynamo.reset()
+    with pytest.raises(_Traced):
+        torch.compile(fn, fullgraph=True, backend=backend)(*args)
+    (graph,) = graphs
+    return "".join(m.code for m in graph.modules() if isinstance(m, torch.fx.GraphModule))
+
+
+def _fake(*shape, dtype=torch.float32, grad=False):
+    with _FAKE:
+        return torch.empty(*shape, dtype=dtype, device="cuda").requires_grad_(grad)
+
+
+_FAKE = FakeTensorMode()
+
+
+def test_profiled_functions_trace_into_one_graph():
+    """The hybrid scan with gradients and a layer in training, whose parts sit in
+    profiler ranges."""
+    from mogt_amd import model_mogt, triton_scan
+
+    code = _trace(triton_scan.triton_affine_scan_hybrid, _fake(1, 100, 16, 16, grad=True), _fake(1, 100, 16, 48, grad=True))
+    assert "affine_scan_carry" in code
+    for connection in ("identity", "matrix_exp"):
+        with _FAKE, torch.device("cuda"):
+            block = model_mogt.MOGTBlock(d_model=128, r=16, ffn_hidden=256)
+        block.connection_impl, block.scan_impl = connection, "triton_hybrid"
+        code = _trace(lambda x: block(x), _fake(1, 64, 128))
+        assert ("diag_scan" if connection == "identity" else "connection_map") in code
