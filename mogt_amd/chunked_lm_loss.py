@@ -92,10 +92,13 @@ def _split_ok(rows: torch.Tensor, weight: torch.Tensor, chunk: int, autocast: bo
 
 def _pieces(x: torch.Tensor) -> torch.Tensor:
     """``x [rows, D]`` as the bf16 pieces of its fp32 value (one where it is
-    bf16 already)."""
+    bf16 already, in place if the kernels can read it there; a traced call,
+    which has no pointer to look at, copies it)."""
     if x.dtype != torch.bfloat16:
         return ops.split_pieces(x.float())
-    if x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < x.shape[1] or x.data_ptr() % 16 != 0:
+    if not ops._plain((x,)):
+        x = x.clone(memory_format=torch.contiguous_format)
+    elif x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < x.shape[1] or x.data_ptr() % 16 != 0:
         x = x.contiguous()
     return x.unsqueeze(0)
 
@@ -123,25 +126,14 @@ class _Head:
         return self._pieces
 
     def logits(self, block: torch.Tensor) -> torch.Tensor:
-        if self.autocast.enabled or not self.split:
-            return _block_logits(block, self.w32)
-        V, D = self.weight.shape
-        out = torch.empty((block.shape[0], ops.split_pad(V)), dtype=torch.float32, device=block.device)[:, :V]
-        return ops.split_gemm_(out, _pieces(block), self.pieces, D)
-
-    def fused(self, block: torch.Tensor) -> bool:
-        """Whether the cross-entropy rows run in the logits product's epilogue:
-        the split form, where one K slice already fills the compute units."""
-        V, D = self.weight.shape
-        return (self.split and not self.autocast.enabled
-                and ops.split_logits_slices(block.shape[0], V, D, 1 if block.dtype == torch.bfloat16 else 3,
-                                            self.pieces.shape[0]) == 1)
+        """The block's logits from the library, under the caller's autocast."""
+        return _block_logits(block, self.w32)
 
     def loss_rows(self, block: torch.Tensor, targets: torch.Tensor):
         """The block's per-row loss and log-sum-exp."""
-        if self.fused(block):
-            return ops.split_ce_forward(_pieces(block), self.pieces, self.weight.shape[1], targets,
-                                        ignore_index=IGNORE_INDEX)
+        if self.split and not self.autocast.enabled:
+            return ops.split_head_loss(_pieces(block), self.pieces, self.weight.shape[1], targets,
+                                       ignore_index=IGNORE_INDEX)
         return ops.lm_ce_forward(self.logits(block), targets, ignore_index=IGNORE_INDEX)
 
     def new_weight_grad(self) -> torch.Tensor:
@@ -151,21 +143,24 @@ class _Head:
 
     def backward(self, targets, lse, scale, block, d_rows, d_w32, first: bool) -> None:
         """d_rows = g @ weight and d_w32 += g^T @ block in fp32, for the gradient
-        g of the block's logits, recomputed under the forward's autocast state."""
+        g of the block's logits, recomputed under the forward's autocast state.
+        Only library calls stand inside the autocast regions: a graph cannot be
+        traced with this library's functions there."""
         logits = None
-        if not self.fused(block):
+        if not self.split or self.autocast.enabled:
             with self.autocast():
                 logits = self.logits(block)
         if not self.split:
             # fp32 gradient block, whatever the logits' dtype
             g = ops.lm_ce_grad(logits, targets, lse, scale, ignore_index=IGNORE_INDEX)
-            d_rows.copy_(g.matmul(self.w32))
-            d_w32.addmm_(g.t(), block.float())
+            with torch.autocast("cuda", enabled=False):
+                d_rows.copy_(g.matmul(self.w32))
+                d_w32.addmm_(g.t(), block.float())
             return
         V, D = self.weight.shape
         rows = _pieces(block)
         if logits is None:
-            g = ops.split_ce_grad_pieces(rows, self.pieces, D, targets, lse, scale, ignore_index=IGNORE_INDEX)
+            g = ops.split_head_grad_pieces(rows, self.pieces, D, targets, lse, scale, ignore_index=IGNORE_INDEX)
         else:
             g = ops.lm_ce_grad_pieces(logits, targets, lse, scale, ignore_index=IGNORE_INDEX)
         direct = d_rows.dtype in (torch.float32, torch.bfloat16) and d_rows.is_contiguous()
@@ -231,8 +226,7 @@ class _ChunkedLinearCrossEntropy(torch.autograd.Function):
         d_w32 = head.new_weight_grad()
         with torch.no_grad():
             for i, sl in enumerate(_token_blocks(n_tok, ctx.chunk_size)):
-                with torch.autocast("cuda", enabled=False):
-                    head.backward(targets[sl], lse[sl], scale, rows[sl], d_rows[sl], d_w32, first=i == 0)
+                head.backward(targets[sl], lse[sl], scale, rows[sl], d_rows[sl], d_w32, first=i == 0)
         d_hidden, d_weight = d_rows.view_as(hidden_states), d_w32.to(weight.dtype)
         if torch.is_grad_enabled() and not torch.compiler.is_compiling():   # create_graph
             d_hidden, d_weight = _NotTwiceDifferentiable.apply(3, hidden_states, weight, grad_output, d_hidden, d_weight)

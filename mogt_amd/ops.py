@@ -2370,3 +2370,63 @@ def split_ce_grad_pieces(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch
     if scale.numel() != 1 or scale.dtype != torch.float32 or scale.device != a.device:
         raise ValueError("split_ce_grad_pieces: scale must be a one-element float32 tensor on the operands' device")
     return _split_ce_bwd_op(a, b, int(k), labels, lse, scale.reshape(1).contiguous(), int(ignore_index))
+
+
+# The head's two products with the choice between the epilogues and the written
+# logits inside an op: it is the library's (a host call), which a traced graph
+# cannot hold.
+def _split_logits(a: torch.Tensor, b: torch.Tensor, k: int) -> torch.Tensor:
+    out = torch.empty((a.shape[1], split_pad(b.shape[1])), dtype=torch.float32, device=a.device)[:, :b.shape[1]]
+    _split_gemm_op.impl(out, a, b, k, False, False, False)
+    return out
+
+
+def _one_slice(a: torch.Tensor, b: torch.Tensor, k: int) -> bool:
+    return split_logits_slices(a.shape[1], b.shape[1], k, a.shape[0], b.shape[0]) == 1
+
+
+@_op("mogt::split_head_loss")
+def _split_head_loss_op(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor,
+                        ignore_index: int) -> tuple[torch.Tensor, torch.Tensor]:
+    if _one_slice(a, b, k):
+        return _split_ce_fwd_op.impl(a, b, k, labels, ignore_index)
+    return _lm_ce_fwd_op.impl(_split_logits(a, b, k), labels, ignore_index)
+
+
+@_split_head_loss_op.register_fake
+def _(a, b, k, labels, ignore_index):
+    return a.new_empty(a.shape[1], dtype=torch.float32), a.new_empty(a.shape[1], dtype=torch.float32)
+
+
+def split_head_loss(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor, *, ignore_index: int = -100):
+    """``(loss_rows, lse_rows)`` of the logits ``a @ b^T`` (``split_gemm_``'s
+    operands): the cross-entropy rows in the product's epilogue
+    (``split_ce_forward``) where one K slice of it already fills the compute
+    units, else on the written logits."""
+    _check_split_ce(a, b, k, labels, "split_head_loss")
+    return _split_head_loss_op(a, b, int(k), labels, int(ignore_index))
+
+
+@_op("mogt::split_head_grad_pieces")
+def _split_head_grad_pieces_op(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor, lse: torch.Tensor,
+                               scale: torch.Tensor, ignore_index: int) -> torch.Tensor:
+    if _one_slice(a, b, k):
+        return _split_ce_bwd_op.impl(a, b, k, labels, lse, scale, ignore_index)
+    return _lm_ce_grad_pieces_op.impl(_split_logits(a, b, k), labels, lse, scale, ignore_index)
+
+
+@_split_head_grad_pieces_op.register_fake
+def _(a, b, k, labels, lse, scale, ignore_index):
+    return a.new_empty((3, a.shape[1], split_pad(b.shape[1])))
+
+
+def split_head_grad_pieces(a: torch.Tensor, b: torch.Tensor, k: int, labels: torch.Tensor, lse: torch.Tensor,
+                           scale: torch.Tensor, *, ignore_index: int = -100) -> torch.Tensor:
+    """``lm_ce_grad_pieces`` of the logits ``a @ b^T``, in the form
+    ``split_head_loss`` takes for them."""
+    _check_split_ce(a, b, k, labels, "split_head_grad_pieces")
+    if lse.shape != labels.shape or lse.dtype != torch.float32:
+        raise ValueError("split_head_grad_pieces: lse must be float32 [rows]")
+    if scale.numel() != 1 or scale.dtype != torch.float32 or scale.device != a.device:
+        raise ValueError("split_head_grad_pieces: scale must be a one-element float32 tensor on the operands' device")
+    return _split_head_grad_pieces_op(a, b, int(k), labels, lse, scale.reshape(1).contiguous(), int(ignore_index))

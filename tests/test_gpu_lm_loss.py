@@ -526,3 +526,31 @@ def test_chunked_linear_ce_second_derivative_is_refused(gpu, monkeypatch, split)
     for penalty in (gh.square().sum(), gw.square().sum(), loss + gh.square().sum()):
         with pytest.raises(RuntimeError):
             torch.autograd.grad(penalty, [h, w], retain_graph=True)
+
+
+@pytest.mark.parametrize("hd", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("autocast", [False, True])
+def test_chunked_linear_ce_compiled(gpu, monkeypatch, hd, autocast):
+    """The split form traced and functionalised into one graph gives the eager
+    call's loss and gradients."""
+    announce(f"chunked CE compiled {hd} {autocast}")
+    from mogt_amd import chunked_lm_loss as cl
+
+    monkeypatch.setattr(cl, "SPLIT_MIN_MACS", 0)
+    monkeypatch.setattr(cl, "SPLIT_MIN_MACS_AUTOCAST", 0)
+    h = _bf16_or_f32((2, 150, 64), hd, 81).to(gpu).requires_grad_()
+    w = _bf16_or_f32((1003, 64), torch.float32, 82, 0.3).to(gpu).requires_grad_()
+    lab = _labels(300, 1003, gpu, seed=83, ignore_every=7).view(2, 150)
+
+    def loss(h, w, lab):
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            return cl.chunked_linear_cross_entropy(h, w, lab, chunk_size=128)
+
+    def run(fn):
+        value = fn(h, w, lab)
+        return [value.detach(), *torch.autograd.grad(value, [h, w])]
+
+    eager = run(loss)
+    torch._dynamo.reset()
+    for got, ref in zip(run(torch.compile(loss, backend="aot_eager", fullgraph=True)), eager):
+        assert got.dtype == ref.dtype and torch.equal(got, ref)

@@ -212,3 +212,15 @@ def test_profiled_functions_trace_into_one_graph():
         block.connection_impl, block.scan_impl = connection, "triton_hybrid"
         code = _trace(lambda x: block(x), _fake(1, 64, 128))
         assert ("diag_scan" if connection == "identity" else "connection_map") in code
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_chunked_loss_traces_into_one_graph(dtype):
+    """The tied-head loss with gradients at a size whose products take the split
+    form."""
+    from mogt_amd import chunked_lm_loss as cl
+
+    code = _trace(lambda h, w, labels: cl.chunked_linear_cross_entropy(h, w, labels, chunk_size=1024),
+                  _fake(1, 2000, 768, dtype=dtype, grad=True), _fake(32000, 768, grad=True),
+                  _fake(1, 2000, dtype=torch.int64))
+    assert "split_head_loss" in code and "split_gemm_" in code
