@@ -96,10 +96,11 @@ def _pieces(x: torch.Tensor) -> torch.Tensor:
     which has no pointer to look at, copies it)."""
     if x.dtype != torch.bfloat16:
         return ops.split_pieces(x.float())
-    if not ops._plain((x,)):
+    if (x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < x.shape[1] or not ops._plain((x,))
+            or x.data_ptr() % 16 != 0):
+        # a clone, not contiguous(): that returns an x which is misaligned, or one
+        # row of any stride, as it is
         x = x.clone(memory_format=torch.contiguous_format)
-    elif x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < x.shape[1] or x.data_ptr() % 16 != 0:
-        x = x.contiguous()
     return x.unsqueeze(0)
 
 

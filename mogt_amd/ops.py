@@ -2230,8 +2230,9 @@ def split_pad(n: int) -> int:
 
 def _split_pieces_impl(x: torch.Tensor) -> torch.Tensor:
     lib = _lib.load()
-    x = x if x.stride(1) == 1 else x.contiguous()
     rows, cols = x.shape
+    if x.stride(1) != 1 or (rows > 1 and x.stride(0) < cols):   # rows that overlap: an expanded x
+        x = x.contiguous()
     out = torch.empty((3, rows, split_pad(cols)), dtype=torch.bfloat16, device=x.device)
     rc = lib.mogt_split_pieces(x.data_ptr(), x.stride(0) if rows > 1 else cols, out.data_ptr(), out.stride(1), rows,
                                cols, _stream_handle(x.device))

@@ -554,3 +554,48 @@ def test_chunked_linear_ce_compiled(gpu, monkeypatch, hd, autocast):
     torch._dynamo.reset()
     for got, ref in zip(run(torch.compile(loss, backend="aot_eager", fullgraph=True)), eager):
         assert got.dtype == ref.dtype and torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("hd", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [129, 200])
+def test_chunked_linear_ce_of_repeated_hidden_states(gpu, monkeypatch, n, hd):
+    """Hidden states expanded from one row (row stride 0), with a last chunk of
+    one row."""
+    announce(f"chunked CE expanded hidden states n={n} {hd}")
+    from mogt_amd import chunked_lm_loss as cl
+
+    base = _bf16_or_f32((1, 1, 64), hd, 71).to(gpu)
+    w = _bf16_or_f32((1003, 64), torch.float32, 72, 0.3).to(gpu).requires_grad_()
+    lab = torch.randint(0, 1003, (1, n), generator=torch.Generator().manual_seed(n)).to(gpu)
+
+    def call():
+        loss = cl.chunked_linear_cross_entropy(base.expand(1, n, 64), w, lab, chunk_size=128)
+        return [loss.detach(), *torch.autograd.grad(loss, [w])]
+
+    lib = call()
+    monkeypatch.setattr(cl, "SPLIT_MIN_MACS", 0)
+    for got, ref in zip(call(), lib):
+        assert rel_err(to_np(got), to_np(ref)) <= 1e-5
+
+
+@pytest.mark.parametrize("which", ["hidden", "weight"])
+def test_chunked_linear_ce_of_misaligned_bf16(gpu, monkeypatch, which):
+    """bf16 operands that start at an odd element."""
+    announce(f"chunked CE misaligned {which}")
+    from mogt_amd import chunked_lm_loss as cl
+
+    h, w = _bf16_or_f32((1, 200, 64), torch.bfloat16, 91).to(gpu), _bf16_or_f32((1003, 64), torch.bfloat16, 92, 0.3).to(gpu)
+    lab = torch.randint(0, 1003, (1, 200), generator=torch.Generator().manual_seed(9)).to(gpu)
+
+    def odd(x):
+        return torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(x.shape)
+
+    def call(h, w):
+        h, w = h.detach().requires_grad_(), w.detach().requires_grad_()
+        loss = cl.chunked_linear_cross_entropy(h, w, lab, chunk_size=128)
+        return [loss.detach(), *torch.autograd.grad(loss, [h, w])]
+
+    monkeypatch.setattr(cl, "SPLIT_MIN_MACS", 0)
+    ref = call(h, w)
+    for got, r in zip(call(odd(h) if which == "hidden" else h, odd(w) if which == "weight" else w), ref):
+        assert torch.equal(got, r)
