@@ -78,16 +78,28 @@ SPLIT_MIN_MACS = 1 << 30
 SPLIT_MIN_MACS_AUTOCAST = 6_000_000_000
 
 
+def _span_ok(rows: int, ld: int) -> bool:
+    """Whether an operand of ``rows`` rows of stride ``ld`` stays within the
+    kernels' 32-bit byte offsets, a block of 256 rows across the contraction and
+    all of it along (``mogt_split_gemm``'s limits)."""
+    return max(256, ops.split_pad(rows) + ops.SPLIT_K) * ld * 2 < 1 << 31
+
+
 def _split_ok(rows: torch.Tensor, weight: torch.Tensor, chunk: int, autocast: bool) -> bool:
     """Whether this head's fp32 GEMMs run from bf16 pieces: tensors on the GPU,
-    a contraction of whole stages, a first block large enough to gain and
-    gradient rows within the kernel's 32-bit offsets."""
+    a contraction of whole stages, a first block large enough to gain, and the
+    gradient block, weight and hidden rows within the kernels' offsets."""
     n, D = min(rows.shape[0], chunk), rows.shape[1]
     V = weight.shape[0]
     return (rows.is_cuda and weight.is_cuda and rows.device == weight.device and D % ops.SPLIT_K == 0
             and n * V * D >= (SPLIT_MIN_MACS_AUTOCAST if autocast else SPLIT_MIN_MACS)
-            and (ops.split_pad(n) + ops.SPLIT_K) * ops.split_pad(V) * 2 < 1 << 31
-            and (ops.split_pad(V) + ops.SPLIT_K) * D * 2 < 1 << 31)
+            and _span_ok(n, ops.split_pad(V)) and _span_ok(V, D) and _span_ok(n, D))
+
+
+def _in_place(x: torch.Tensor) -> bool:
+    """Whether the kernels can read bf16 rows where they are."""
+    return (x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]
+            and _span_ok(x.shape[0], x.stride(0)) and ops._plain((x,)) and x.data_ptr() % 16 == 0)
 
 
 def _pieces(x: torch.Tensor) -> torch.Tensor:
@@ -96,8 +108,7 @@ def _pieces(x: torch.Tensor) -> torch.Tensor:
     which has no pointer to look at, copies it)."""
     if x.dtype != torch.bfloat16:
         return ops.split_pieces(x.float())
-    if (x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < x.shape[1] or not ops._plain((x,))
-            or x.data_ptr() % 16 != 0):
+    if not _in_place(x):
         # a clone, not contiguous(): that returns an x which is misaligned, or one
         # row of any stride, as it is
         x = x.clone(memory_format=torch.contiguous_format)

@@ -455,6 +455,66 @@ def test_split_products_ask_for_partials_only():
     assert swapped > 1 and size(4000, 256, 20000, 3, 1, 1, F32, 0) == swapped * 4000 * 256 * 4
 
 
+def test_split_head_sizes_are_the_kernels():
+    """Sizes at which the tied-head loss takes the split products lie within what
+    their C entries take (operand blocks below 2 GiB), and sizes just past those
+    limits keep the library form.  The entries are called up to their first check
+    after the limits (no workspace, no result rows), so nothing is launched."""
+    from types import SimpleNamespace
+
+    from mogt_amd import _lib, ops
+    from mogt_amd import chunked_lm_loss as cl
+
+    lib = _lib.load()
+    some = 4096   # an aligned pointer that is never read
+
+    def takes(n, V, D, pieces):
+        """Whether the C entries take the head's four products."""
+        gp = ops.split_pad(V)
+        calls = [
+            lambda: lib.mogt_split_ce_fwd(some, D, n * D, pieces, some, D, V * D, 3, some, n, V, D, -100, None, None,
+                                          None, 0, None),
+            lambda: lib.mogt_split_gemm(some, D, n * D, pieces, 0, some, D, V * D, 3, 0, some, gp, n, V, D, 0,
+                                        _lib.MOGT_BF16, 0, None, 0, None),
+            lambda: lib.mogt_split_gemm(some, gp, n * gp, 3, 0, some, D, V * D, 3, 1, some, D, n, D, V, 0,
+                                        _lib.MOGT_BF16, 0, None, 0, None),
+            lambda: lib.mogt_split_gemm(some, gp, n * gp, 3, 1, some, D, n * D, pieces, 1, some, D, V, D, n, 0,
+                                        _lib.MOGT_BF16, 0, None, 0, None),
+        ]
+        for call in calls:
+            assert call() != 0
+            msg = lib.mogt_last_error().decode()
+            if "2 GiB" in msg or "row strides" in msg or "too many" in msg or "size" in msg:
+                return False
+        return True
+
+    def split(n, V, D):
+        tensor = lambda *shape: SimpleNamespace(shape=shape, is_cuda=True, device="cuda:0")   # noqa: E731
+        return cl._split_ok(tensor(n, D), tensor(V, D), n, False)
+
+    sizes = [(64, 5_000_000, 128), (192, 4_194_304, 32), (192, 4_194_240, 32), (1, 33_554_400, 32), (8192, 131_008, 64),
+             (8192, 130_496, 64), (65536, 16320, 16384), (65536, 16320, 16352), (200, 64, 5_000_000 // 32 * 32),
+             (4096, 32000, 768), (256, 4_194_240, 96), (32768, 32704, 32), (32, 128256, 8192), (64, 128256, 8320)]
+    taken = [split(*s) for s in sizes]
+    assert any(taken) and not all(taken)
+    for (n, V, D), yes in zip(sizes, taken):
+        for pieces in (1, 3):
+            if yes:
+                assert takes(n, V, D, pieces), (n, V, D, pieces, lib.mogt_last_error())
+    assert not split(64, 5_000_000, 128) and split(4096, 32000, 768)
+
+
+def test_wide_row_strides_are_copied():
+    """bf16 rows whose stride takes an operand block past the kernels' 2 GiB."""
+    from mogt_amd import chunked_lm_loss as cl
+
+    wide = torch.empty_strided((300, 64), (1 << 22, 1), dtype=torch.bfloat16, device="meta")
+    base = torch.zeros(1, dtype=torch.bfloat16)
+    near = torch.zeros(300, 72, dtype=torch.bfloat16)[:, :64]
+    assert cl._pieces(near).data_ptr() == near.data_ptr()
+    assert cl._in_place(near) and not cl._in_place(wide) and not cl._in_place(base.expand(300, 64))
+
+
 @pytest.mark.parametrize("source", ["swiglu_gemm.hip", "wgrad_gemm.hip", "rank1_scan.hip", "split_gemm.hip"])
 def test_gemm_m0_only_feeds_lds_dma(tmp_path, source):
     """The bf16 GEMMs (fused SwiGLU, split-K weight gradient) and the rank-1
