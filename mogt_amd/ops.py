@@ -83,7 +83,9 @@ def workspace(nbytes: int, device: torch.device, family: str = "plain", layout: 
 
     One buffer per (device, stream, family) keeps concurrent streams and the
     kernel families apart.  Look-back families (``LOOKBACK_FAMILIES``) pass the
-    launch's ``layout`` (its shape, dtypes and tile).  Kernels using the
+    launch's ``layout`` (its shape, dtypes and tile; the tile follows from the
+    inputs' alignment too, so their addresses modulo 16 stand for it, outputs
+    coming aligned from the allocator).  Kernels using the
     look-back protocol leave the buffer reusable after every launch, so
     launches of one layout never clear it; a launch of another layout first
     clears bytes ``[256, nbytes)`` with a fill kernel.  A buffer that a graph
@@ -274,14 +276,15 @@ def _diag_scan_launch(a: torch.Tensor, b: torch.Tensor, h: torch.Tensor,
         nbytes = lib.mogt_diag_scan_workspace_bytes(B, L, D, in_code)
     else:
         nbytes = lib.mogt_diag_scan_workspace_bytes_cfg(B, L, D, *cfg)
-    ws = workspace(nbytes, a.device, "diag", (B, L, D, in_code, cfg))
+    pa, pb = a.data_ptr(), b.data_ptr()
+    ws = workspace(nbytes, a.device, "diag", (B, L, D, in_code, cfg, pa & 15, pb & 15))
     pre = prefix.data_ptr() if prefix is not None else None
     stream = _stream_handle(a.device)
     if cfg is None:
-        rc = lib.mogt_diag_scan_fwd(a.data_ptr(), b.data_ptr(), h.data_ptr(), pre, B, L, D,
+        rc = lib.mogt_diag_scan_fwd(pa, pb, h.data_ptr(), pre, B, L, D,
                                     in_code, out_code, ws.data_ptr(), ws.numel(), stream)
     else:
-        rc = lib.mogt_diag_scan_fwd_cfg(a.data_ptr(), b.data_ptr(), h.data_ptr(), pre, B, L, D,
+        rc = lib.mogt_diag_scan_fwd_cfg(pa, pb, h.data_ptr(), pre, B, L, D,
                                         in_code, out_code, cfg[0], cfg[1], cfg[2], cfg[3],
                                         ws.data_ptr(), ws.numel(), stream)
     _lib.check(rc, "mogt_diag_scan_fwd")
@@ -344,9 +347,11 @@ def _diag_scan_rev_op(a: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     B, L, D = a.shape
     out = torch.empty(a.shape, dtype=torch.float32, device=a.device)
     code = _lib.MOGT_BF16 if bf16 else _lib.MOGT_F32
-    ws = workspace(lib.mogt_diag_scan_workspace_bytes(B, L, D, code), a.device, "diag_rev", (B, L, D, code))
+    pa, pg = a.data_ptr(), g.data_ptr()
+    ws = workspace(lib.mogt_diag_scan_workspace_bytes(B, L, D, code), a.device, "diag_rev",
+                   (B, L, D, code, pa & 15, pg & 15))
     run = lib.mogt_diag_scan_rev_bf16_fwd if bf16 else lib.mogt_diag_scan_rev_fwd
-    rc = run(a.data_ptr(), g.data_ptr(), out.data_ptr(), B, L, D, ws.data_ptr(), ws.numel(),
+    rc = run(pa, pg, out.data_ptr(), B, L, D, ws.data_ptr(), ws.numel(),
              _stream_handle(a.device))
     _lib.check(rc, "mogt_diag_scan_rev_fwd")
     _checked(ws, "mogt_diag_scan_rev_fwd")
@@ -369,8 +374,10 @@ def _diag_scan_grad_op(a: torch.Tensor, b: torch.Tensor, G: torch.Tensor) -> tup
     code = dtype_code(a.dtype, "diag_scan_grad")
     da = torch.empty(a.shape, dtype=a.dtype, device=a.device)
     db = torch.empty(a.shape if code == _lib.MOGT_BF16 else (0,), dtype=a.dtype, device=a.device)
-    ws = workspace(lib.mogt_diag_scan_workspace_bytes(B, L, D, code), a.device, "diag_grad", (B, L, D, code))
-    rc = lib.mogt_diag_scan_grad(a.data_ptr(), b.data_ptr(), G.data_ptr(), da.data_ptr(),
+    pa, pb, pg = a.data_ptr(), b.data_ptr(), G.data_ptr()
+    ws = workspace(lib.mogt_diag_scan_workspace_bytes(B, L, D, code), a.device, "diag_grad",
+                   (B, L, D, code, pa & 15, pb & 15, pg & 15))
+    rc = lib.mogt_diag_scan_grad(pa, pb, pg, da.data_ptr(),
                                  db.data_ptr() if code == _lib.MOGT_BF16 else None, B, L, D, code, ws.data_ptr(),
                                  ws.numel(), _stream_handle(a.device))
     _lib.check(rc, "mogt_diag_scan_grad")
@@ -449,7 +456,7 @@ def _coupled_rank_scan_impl(z: torch.Tensor, v: torch.Tensor, rank: int, damping
     vc = dtype_code(v.dtype, "coupled_rank_scan")
     oc = dtype_code(out_dtype, "coupled_rank_scan")
     nbytes = lib.mogt_coupled_rank_scan_workspace_bytes(B, L, rank, C, vc)
-    ws = workspace(nbytes, v.device, "coupled", ("plain", B, L, rank, C, vc))
+    ws = workspace(nbytes, v.device, "coupled", ("plain", B, L, rank, C, vc, v.data_ptr() & 15))
     rc = lib.mogt_coupled_rank_scan_fwd(z.data_ptr(), v.data_ptr(), h.data_ptr(), B, L, rank, C,
                                         float(damping), zc, vc, oc, ws.data_ptr(), ws.numel(),
                                         _stream_handle(v.device))
@@ -476,7 +483,7 @@ def _coupled_scan_rev_op(z: torch.Tensor, grad_h: torch.Tensor, rank: int, dampi
     B, L, D = g.shape
     out = torch.empty_like(g)
     nbytes = lib.mogt_coupled_rank_scan_rev_workspace_bytes(B, L, rank, D // rank)
-    ws = workspace(nbytes, g.device, "coupled_rev", (B, L, rank, D // rank))
+    ws = workspace(nbytes, g.device, "coupled_rev", (B, L, rank, D // rank, g.data_ptr() & 15))
     rc = lib.mogt_coupled_rank_scan_rev_fwd(z.data_ptr(), g.data_ptr(), out.data_ptr(), B, L, rank, D // rank,
                                             float(damping), dtype_code(z.dtype, "coupled_scan_rev"), ws.data_ptr(),
                                             ws.numel(), _stream_handle(g.device))
@@ -575,7 +582,7 @@ def _coupled_rank_scan_stats_op(z: torch.Tensor, v: torch.Tensor, rank: int, dam
     stats = torch.empty((B, L, -(-D // STAT_GROUP)), dtype=torch.float32, device=v.device)
     vc = dtype_code(v.dtype, "coupled_rank_scan_stats")
     ws = workspace(lib.mogt_coupled_rank_scan_workspace_bytes(B, L, rank, C, vc), v.device, "coupled",
-                   ("stats", B, L, rank, C, vc))
+                   ("stats", B, L, rank, C, vc, v.data_ptr() & 15))
     rc = lib.mogt_coupled_rank_scan_stats_fwd(z.data_ptr(), v.data_ptr(), h.data_ptr(), stats.data_ptr(), B, L,
                                               rank, C, float(damping), vc,
                                               dtype_code(out_dtype, "coupled_rank_scan_stats"), ws.data_ptr(),
@@ -621,7 +628,7 @@ def _coupled_rank_scan_proj_op(proj: torch.Tensor, features: int, gate_prev: boo
     if gate_const is not None:
         gc = gate_const.to(torch.float32).expand(B, rank).contiguous()
     ws = workspace(lib.mogt_coupled_rank_scan_workspace_bytes(B, L, rank, C, code), proj.device, "coupled",
-                   ("proj", B, L, rank, C, code, ld, int(bool(gate_prev))))
+                   ("proj", B, L, rank, C, code, ld, int(bool(gate_prev)), proj.data_ptr() & 15))
     rc = lib.mogt_coupled_rank_scan_proj_fwd(proj.data_ptr(), ld, D, int(bool(gate_prev)),
                                              gc.data_ptr() if gc is not None else None, h.data_ptr(),
                                              stats.data_ptr(), None, B, L, rank, C, float(damping), code, code,
@@ -672,7 +679,7 @@ def _coupled_proj_scan_op(proj: torch.Tensor, gate_const: torch.Tensor | None, f
     code = dtype_code(proj.dtype, "coupled_proj_scan")
     gc = gate_const.to(torch.float32).contiguous() if gate_const is not None else None
     ws = workspace(lib.mogt_coupled_rank_scan_workspace_bytes(B, L, rank, C, code), proj.device, "coupled",
-                   ("proj", B, L, rank, C, code, ld, int(bool(gate_prev))))
+                   ("proj", B, L, rank, C, code, ld, int(bool(gate_prev)), proj.data_ptr() & 15))
     rc = lib.mogt_coupled_rank_scan_proj_fwd(proj.data_ptr(), ld, D, int(bool(gate_prev)),
                                              gc.data_ptr() if gc is not None else None, h.data_ptr(), None,
                                              z.data_ptr(), B, L, rank, C, float(damping), code, _lib.MOGT_F32,

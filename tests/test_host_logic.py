@@ -308,6 +308,58 @@ def test_lookback_workspaces_are_kept_apart_and_cleared_on_layout_change(monkeyp
     assert c is not a and c.numel() >= 1 << 20 and int(c.max()) == 0 and a in ops._ws_retired
 
 
+def test_lookback_layouts_tell_alignments_apart(monkeypatch):
+    """A scan's tile, and with it the place of the look-back words, follows from
+    the alignment of its inputs as well: a call on an offset view names another
+    layout than the aligned call of the same shape."""
+    ops, dev = _fake_device_workspace(monkeypatch)
+    layouts = []
+
+    def spy(nbytes, device, family="plain", layout=None):
+        layouts.append((family, layout))
+        return torch.zeros(max(int(nbytes), 512), dtype=torch.uint8)
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *args: 4096 if "workspace_bytes" in name else 0
+
+    monkeypatch.setattr(ops, "workspace", spy)
+    monkeypatch.setattr(ops._lib, "load", lambda: Lib())
+
+    def tensor(offset, *shape, dtype=torch.float32):
+        n = 1
+        for k in shape:
+            n *= k
+        return torch.zeros(n + 8, dtype=dtype)[offset:offset + n].view(shape)
+
+    f32, bf16 = torch.float32, torch.bfloat16
+    calls = {
+        "diag": lambda x: ops._diag_scan_op.impl(x, tensor(0, 2, 9, 8, dtype=x.dtype), f32),
+        "diag b": lambda x: ops._diag_scan_op.impl(tensor(0, 2, 9, 8, dtype=x.dtype), x, f32),
+        "diag_rev": lambda x: ops._diag_scan_rev_op.impl(x, tensor(0, 2, 9, 8, dtype=x.dtype)),
+        "diag_rev g": lambda x: ops._diag_scan_rev_op.impl(tensor(0, 2, 9, 8, dtype=x.dtype), x),
+        "diag_grad": lambda x: ops._diag_scan_grad_op.impl(x, tensor(0, 2, 9, 8, dtype=x.dtype), tensor(0, 2, 9, 8)),
+        "diag_grad b": lambda x: ops._diag_scan_grad_op.impl(tensor(0, 2, 9, 8, dtype=x.dtype), x, tensor(0, 2, 9, 8)),
+        "diag_grad G": lambda x: ops._diag_scan_grad_op.impl(tensor(0, 2, 9, 8), tensor(0, 2, 9, 8), x.float()
+                                                             if x.dtype == bf16 else x),
+        "coupled": lambda x: ops._coupled_rank_scan_op.impl(tensor(0, 2, 9, 2), x, 2, 1.0, f32),
+        "coupled stats": lambda x: ops._coupled_rank_scan_stats_op.impl(tensor(0, 2, 9, 2), x, 2, 1.0, f32),
+        "coupled proj": lambda x: ops._coupled_rank_scan_proj_op.impl(x, 6, False, None, 2, 1.0),
+        "coupled training": lambda x: ops._coupled_proj_scan_op.impl(x, None, 6, 2, False, 1.0),
+        "coupled_rev": lambda x: ops._coupled_scan_rev_op.impl(tensor(0, 2, 9, 2), x, 2, 1.0),
+    }
+    for name, call in calls.items():
+        for dtype in (f32, bf16) if name not in ("diag_grad G", "coupled_rev") else (f32,):
+            layouts.clear()
+            for offset in (0, 0, 1, 2, 4):
+                call(tensor(offset, 2, 9, 8, dtype=dtype))
+            (first, again, *others) = layouts
+            assert first == again
+            # 4 elements of fp32 are 16 bytes: the alignment of the start
+            assert first not in others[:2 if dtype == f32 else 3], (name, dtype, layouts)
+            assert all(family == name.split()[0] for family, _ in layouts)
+
+
 def test_captured_workspace_is_pinned_to_its_layout(monkeypatch):
     """A look-back buffer used under graph capture keeps serving its layout
     (no clearing fill recorded when the capture repeats the warm-up's layout);
