@@ -167,11 +167,15 @@ def _gate_input_parts(mode: str) -> tuple[str, ...]:
 def _attr(block: nn.Module, name: str, default):
     """``getattr(block, name, default)`` without the exception nn.Module raises
     and getattr swallows for every attribute a block does not set."""
-    for table in (block.__dict__, block._modules, block._parameters, block._buffers):
-        if name in table:
-            return table[name]
-    if type(block).__getattr__ is nn.Module.__getattr__ and not hasattr(type(block), name):
-        return default
+    own = block.__dict__
+    if name in own and type(block) is MOGTBlock:   # no property that would go before it
+        return own[name]
+    if not hasattr(type(block), name):   # the class's own goes before what is registered
+        for table in (own, block._parameters, block._buffers, block._modules):
+            if name in table:
+                return table[name]
+        if type(block).__getattr__ is nn.Module.__getattr__:
+            return default
     return getattr(block, name, default)
 
 

@@ -77,6 +77,34 @@ def test_tied_head_follows_writes_through_weight_data(monkeypatch):
             assert torch.equal(model(None)[0], nn.functional.linear(hidden, model.lm_head.weight))
 
 
+def test_block_options_resolve_as_getattr_does():
+    """A block's options come from where getattr would take them: an attribute of
+    the class goes before a module or parameter registered under its name, a
+    property before the default."""
+    from mogt_amd.model_mogt import MixerSpec, MOGTBlock, _attr
+
+    class Sub(MOGTBlock):
+        phi_value_gate = None
+        scan_impl = "block_reference"
+
+        @property
+        def transport_gate_scale(self):
+            return 0.5
+
+    block, plain = Sub(d_model=32, r=4, ffn_hidden=64), MOGTBlock(d_model=32, r=4, ffn_hidden=64)
+    for b in (block, plain):
+        b.phi_value_gate = nn.Linear(32, 4)
+        b.phi_transport_gate = nn.Linear(32, 4)
+        b.mogt_residual_gate_logit = nn.Parameter(torch.zeros(1))
+        b.register_buffer("mogt_residual_scale", torch.tensor(0.25))
+        b.value_gate_input_mode = "current"
+        for name in ("phi_value_gate", "scan_impl", "transport_gate_scale", "phi_transport_gate", "training",
+                     "mogt_residual_gate_logit", "mogt_residual_scale", "value_gate_input_mode", "no_such_option"):
+            assert _attr(b, name, "default") is getattr(b, name, "default"), name
+    assert MixerSpec.of(block).value_gate is None and MixerSpec.of(plain).value_gate is plain.phi_value_gate
+    assert MixerSpec.of(block).scan == "block_reference" and MixerSpec.of(block).transport_scale == 0.5
+
+
 def test_gemm_table_is_well_formed():
     """The tuned GEMM table: TunableOp's validator header for gfx950 and one
     solution per backbone GEMM shape (bf16, the d_model 768 projections)."""
