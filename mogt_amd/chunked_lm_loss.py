@@ -77,6 +77,21 @@ def _block_logits(rows: torch.Tensor, w32: torch.Tensor) -> torch.Tensor:
 SPLIT_MIN_MACS = 1 << 30
 SPLIT_MIN_MACS_AUTOCAST = 6_000_000_000
 
+# Few rows against a weight that is split (not bf16) and past the caches: both
+# forms are bound by reading it, and the split form moves it as three pieces that
+# it first writes, forward and backward.  bf16 / fp32 hidden states, library over
+# split form: 128256 x 2048: 96 rows 0.82 / 0.69, 160 rows 1.32 / 1.07; 128256 x
+# 4096: 128 rows 0.92 / 0.74, 160 rows 1.07 / 0.83, 400 rows 1.96 / 1.41; 128000 x
+# 512: 48 rows 0.94 / 0.79, 96 rows 1.39 / 1.13.  At 32000 x 768 (2^24.6) 48 rows
+# gain already (1.73 / 1.34).
+SPLIT_CACHED_WEIGHT = 1 << 25   # elements
+
+
+def _split_min_rows(V: int, D: int, hidden: torch.dtype, weight: torch.dtype) -> int:
+    if weight == torch.bfloat16 or V * D <= SPLIT_CACHED_WEIGHT:
+        return 1
+    return max(64, D // 16) if hidden == torch.bfloat16 else max(96, D // 12)
+
 
 def _span_ok(rows: int, ld: int) -> bool:
     """Whether an operand of ``rows`` rows of stride ``ld`` stays within the
@@ -93,6 +108,7 @@ def _split_ok(rows: torch.Tensor, weight: torch.Tensor, chunk: int, autocast: bo
     V = weight.shape[0]
     return (rows.is_cuda and weight.is_cuda and rows.device == weight.device and D % ops.SPLIT_K == 0
             and n * V * D >= (SPLIT_MIN_MACS_AUTOCAST if autocast else SPLIT_MIN_MACS)
+            and n >= _split_min_rows(V, D, rows.dtype, weight.dtype)
             and _span_ok(n, ops.split_pad(V)) and _span_ok(V, D) and _span_ok(n, D))
 
 

@@ -535,15 +535,31 @@ def test_split_products_ask_for_partials_only():
     assert swapped > 1 and size(4000, 256, 20000, 3, 1, 1, F32, 0) == swapped * 4000 * 256 * 4
 
 
+def _split_ok_of(n, V, D, hidden, weight):
+    from types import SimpleNamespace
+
+    from mogt_amd import chunked_lm_loss as cl
+
+    make = lambda dtype, *shape: SimpleNamespace(shape=shape, dtype=dtype, is_cuda=True, device="cuda:0")   # noqa: E731
+    return cl._split_ok(make(hidden, n, D), make(weight, V, D), n, False)
+
+
+def test_split_head_leaves_few_rows_of_large_weights_to_the_library():
+    f32, bf16 = torch.float32, torch.bfloat16
+    for hidden, least in ((bf16, 128), (f32, 170)):
+        assert not _split_ok_of(least - 1, 128256, 2048, hidden, f32)
+        assert _split_ok_of(least, 128256, 2048, hidden, f32)
+        assert _split_ok_of(64, 32000, 768, hidden, f32)                # the weight stays in the caches
+        assert _split_ok_of(32, 128256, 2048, hidden, bf16)             # not split
+        assert not _split_ok_of(32, 128256, 2048, hidden, torch.float16)
+
+
 def test_split_head_sizes_are_the_kernels():
     """Sizes at which the tied-head loss takes the split products lie within what
     their C entries take (operand blocks below 2 GiB), and sizes just past those
     limits keep the library form.  The entries are called up to their first check
     after the limits (no workspace, no result rows), so nothing is launched."""
-    from types import SimpleNamespace
-
     from mogt_amd import _lib, ops
-    from mogt_amd import chunked_lm_loss as cl
 
     lib = _lib.load()
     some = 4096   # an aligned pointer that is never read
@@ -569,8 +585,7 @@ def test_split_head_sizes_are_the_kernels():
         return True
 
     def split(n, V, D):
-        tensor = lambda *shape: SimpleNamespace(shape=shape, is_cuda=True, device="cuda:0")   # noqa: E731
-        return cl._split_ok(tensor(n, D), tensor(V, D), n, False)
+        return _split_ok_of(n, V, D, torch.bfloat16, torch.bfloat16)
 
     sizes = [(64, 5_000_000, 128), (192, 4_194_304, 32), (192, 4_194_240, 32), (1, 33_554_400, 32), (8192, 131_008, 64),
              (8192, 130_496, 64), (65536, 16320, 16384), (65536, 16320, 16352), (200, 64, 5_000_000 // 32 * 32),
