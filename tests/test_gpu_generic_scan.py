@@ -426,6 +426,27 @@ def test_matrix_core_io_dtypes(gpu, state, vdt, odt):
     assert torch.equal(H, wide[1].float().to(odt) if odt != torch.float64 else wide[1].double())
 
 
+@pytest.mark.parametrize("vdt", [torch.float16, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("R", [36, 47, 48, 52, 64])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_wide_ranks_with_other_io_types(gpu, vdt, R, offset):
+    """The general form at three and four row tiles: 16-byte loads of U where the
+    rank and the pointer allow them (R = 47 and an offset U do not), forward with
+    prefix and reversed, over several chunks."""
+    announce(f"generic mfma wide io {vdt} R={R} offset {offset}")
+    g = torch.Generator().manual_seed(R)
+    B, L, C = 2, 75, 18
+    U = 0.9 * torch.eye(R) + 0.3 / R * torch.randn(B, L, R, R, generator=g)
+    V = torch.randn(B, L, R, C, generator=g).to(vdt)
+    flat = torch.zeros(U.numel() + 1, device=gpu)
+    Ug = flat[offset:offset + U.numel()].view(U.shape).copy_(U)
+    Pr, Hr = _loop64(U, V)
+    P, H = torch.ops.mogt.affine_scan_generic(Ug, V.to(gpu), torch.float32, torch.float32, True, False)
+    assert rel_err(H.double().cpu().numpy(), Hr.numpy()) <= 2e-6 and rel_err(P.double().cpu().numpy(), Pr.numpy()) <= 2e-6
+    _, G = torch.ops.mogt.affine_scan_generic(Ug, V.to(gpu), torch.float32, torch.float32, False, True)
+    assert rel_err(G.double().cpu().numpy(), _loop64(U, V, rev=True)[1].numpy()) <= 2e-6
+
+
 def test_matrix_core_workspace_covers_both_levels():
     """The workspace the C entry asks for grows with the chunks of both levels
     and is the header alone for one pass (host arithmetic only)."""
