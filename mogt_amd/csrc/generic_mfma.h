@@ -473,23 +473,35 @@ __global__ __launch_bounds__(64 * GM_WAVES) void generic_mfma_kernel(GParams p, 
 }
 
 // Steps of a chunk: the power of two (or the whole sequence, in one pass) that
-// makes the three passes' serial MFMA time the least.  A wave's step is its
-// MFMAs plus about 200 cycles of issue and waits; LOCAL carries C + R columns,
-// CARRY and OUTPUT Wo.
-inline int64_t gm_segment(int64_t B, int64_t L, int64_t R, int64_t C, int64_t Wo, bool f64) {
+// makes the three passes' serial time the least.  A wave's step is its MFMAs plus
+// about 200 cycles of issue and waits, counted per single 16-column tile and SIMD;
+// LOCAL carries C + R columns, CARRY and OUTPUT Wo.  In the general form (io types
+// other than the state's) a step of an unloaded SIMD does not go below its memory
+// latency, which that form exposes: 0.36 to 0.9 us for 1 to 4 row tiles.  Without
+// that floor many narrow sequences ran as one chunk each: R = 64, C = 1, 16 x 512
+// steps, bf16 io 723 us (scalar kernel 511), R = 1, C = 1000, 4 x 4000 steps, fp16
+// io 1060 -> 413 us; over 636 shapes the mean distance from the best length of
+// chunk fell from 4.8 to 1.0 %.
+inline int64_t gm_segment(int64_t B, int64_t L, int64_t R, int64_t C, int64_t Wo, bool f64, bool native) {
     const int64_t rt = (R + 15) / 16, simds = 1024;
     const double step = static_cast<double>(rt * rt * 4) * (f64 ? 64 : 32) + 200.0;
+    const double floors[4] = {750.0, 1160.0, 1640.0, 1920.0};   // cycles
+    const double floor = native ? 0.0 : floors[rt - 1];
     const int64_t tl = (C + R + 15) / 16, to = (Wo + 15) / 16;
     auto rounds = [&](int64_t waves) { return static_cast<double>((waves + simds - 1) / simds); };
+    auto pass = [&](int64_t waves, int64_t steps) {
+        const double busy = rounds(waves) * step;
+        return static_cast<double>(steps) * (busy > floor ? busy : floor);
+    };
     int64_t best = L;
-    double least = rounds(B * to) * static_cast<double>(L) * step;
+    double least = pass(B * to, L);
     for (int64_t seg = 16; seg < L && seg <= 1024; seg *= 2) {
         const int64_t nch = (L + seg - 1) / seg;
-        // the carries: one chain, or three of about sqrt(nch) steps
+        // the carries (always native): one chain, or three of about sqrt(nch) steps
         const double one = rounds(B * to) * static_cast<double>(nch) * step;
         const double nested = 3.0 * rounds(B * to) * sqrt(static_cast<double>(nch)) * step + 2.0e4;
-        const double t = (rounds(B * nch * tl) + rounds(B * nch * to)) * static_cast<double>(seg) * step +
-                         (one < nested ? one : nested) + 2.0e4;   // 2e4 cycles: two more launches
+        const double t = pass(B * nch * tl, seg) + pass(B * nch * to, seg) + (one < nested ? one : nested) +
+                         2.0e4;   // 2e4 cycles: two more launches
         if (t < least) {
             least = t;
             best = seg;

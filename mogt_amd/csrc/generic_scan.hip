@@ -182,17 +182,18 @@ struct GGeo {
 
 size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
-GGeo generic_geometry(int64_t B, int64_t L, int64_t R, int64_t C, int with_prefix, int state_code) {
+// native: inputs and outputs in the state's dtype
+GGeo geometry_of(int64_t B, int64_t L, int64_t R, int64_t C, int with_prefix, int state_code, bool native) {
     GGeo g{};
     g.Wl = static_cast<int>(C + R);
     g.Wo = static_cast<int>(C + (with_prefix ? R : 0));
     const size_t ts = state_code == MOGT_F64 ? 8 : 4;
     const bool mfma = gm_fits(R, C + R);
-    g.bytes = WS_HDR_BYTES;
+    size_t at = WS_HDR_BYTES;
     int64_t len = L;
     for (int l = 0; l < GS_LEVELS; ++l) {
         if (mfma) {
-            g.seg[l] = gm_segment(B, len, R, C, g.Wo, state_code == MOGT_F64);
+            g.seg[l] = gm_segment(B, len, R, C, g.Wo, state_code == MOGT_F64, native || l > 0);
         } else {
             if (l > 0) break;   // the scalar kernel's carries: one pass
             g.seg[l] = 16;
@@ -201,15 +202,31 @@ GGeo generic_geometry(int64_t B, int64_t L, int64_t R, int64_t C, int with_prefi
         g.nch[l] = (len + g.seg[l] - 1) / g.seg[l];
         if (g.nch[l] <= 1) break;
         g.levels = l + 1;
-        g.s_off[l] = g.bytes;
-        g.m_off[l] = g.s_off[l] + align256(static_cast<size_t>(B * g.nch[l] * R * g.Wl) * ts);
-        g.bytes = g.m_off[l] + align256(static_cast<size_t>(B * g.nch[l] * R * g.Wo) * ts);
+        g.s_off[l] = at;
+        g.m_off[l] = at + align256(static_cast<size_t>(B * g.nch[l] * R * g.Wl) * ts);
+        at = g.m_off[l] + align256(static_cast<size_t>(B * g.nch[l] * R * g.Wo) * ts);
         len = g.nch[l] - 1;   // the last chunk's summary is not needed
     }
+    return g;
+}
+
+// The geometry of a scan with these io types.  The workspace query knows the
+// state's type only, so `bytes` has room for either form's chunks; and for those
+// of a scan with and without the prefix, so that it grows with the prefix.
+GGeo generic_geometry(int64_t B, int64_t L, int64_t R, int64_t C, int with_prefix, int state_code, bool native) {
+    GGeo g = geometry_of(B, L, R, C, with_prefix, state_code, native);
+    const size_t ts = state_code == MOGT_F64 ? 8 : 4;
     // callers bring room for two chunks' summaries beyond 16 steps, also where
     // one pass is the shorter chain
-    if (g.levels == 0 && L > GS_ONE_CHUNK)
-        g.bytes += align256(static_cast<size_t>(B * 2 * R * g.Wl) * ts) + align256(static_cast<size_t>(B * 2 * R * g.Wo) * ts);
+    int64_t most[GS_LEVELS] = {L > GS_ONE_CHUNK ? 2 : 0, 0};
+    for (int form = 0; form < 4; ++form) {
+        const GGeo f = geometry_of(B, L, R, C, form & 1, state_code, form & 2);
+        for (int l = 0; l < f.levels; ++l) most[l] = f.nch[l] > most[l] ? f.nch[l] : most[l];
+    }
+    g.bytes = WS_HDR_BYTES;
+    for (int l = 0; l < GS_LEVELS; ++l)
+        g.bytes += align256(static_cast<size_t>(B * most[l] * R * g.Wl) * ts) +
+                   align256(static_cast<size_t>(B * most[l] * R * g.Wo) * ts);
     return g;
 }
 
@@ -239,6 +256,10 @@ int launch_generic(GParams p, int64_t batch, hipStream_t st, const char* what) {
     const size_t lds = 2 * static_cast<size_t>(p.Cb) * gs_ld<TS>(p.R) * sizeof(TS);
     hipLaunchKernelGGL((generic_scan_kernel<TS, 2>), dim3(static_cast<unsigned>(blocks)), dim3(GS_THREADS), lds, st, p);
     return check_launch(what);
+}
+
+bool io_native(int64_t C, int v_code, int state_code, int out_code) {
+    return (C == 0 || v_code == state_code) && out_code == state_code;
 }
 
 bool io_code(int c) { return c == MOGT_F32 || c == MOGT_BF16 || c == MOGT_F64 || c == MOGT_F16; }
@@ -282,7 +303,7 @@ int scan_level(GParams out, const GGeo& g, int l, unsigned char* base, int state
 template <typename Launch>
 int run_passes(const void* U, const void* V, void* H, void* P, int64_t B, int64_t L, int64_t R, int64_t C,
                int v_code, int state_code, int out_code, int reverse, void* ws, const Launch& launch) {
-    const GGeo g = generic_geometry(B, L, R, C, P != nullptr, state_code);
+    const GGeo g = generic_geometry(B, L, R, C, P != nullptr, state_code, io_native(C, v_code, state_code, out_code));
     const int iR = static_cast<int>(R), iC = static_cast<int>(C);
     // U / V / H / U_prefix views: [B][L][R][*]
     const GView vU{const_cast<void*>(U), L * R * R, R * R, R, state_code};
@@ -350,7 +371,7 @@ using namespace mogt;
 extern "C" size_t mogt_affine_scan_generic_workspace_bytes(int64_t batch, int64_t length, int64_t rank,
                                                           int64_t channels, int with_prefix, int state_dtype) {
     if (batch <= 0 || length <= 0 || rank <= 0 || rank > GS_MAX_R || channels < 0) return WS_HDR_BYTES;
-    return generic_geometry(batch, length, rank, channels, with_prefix != 0, state_dtype).bytes;
+    return generic_geometry(batch, length, rank, channels, with_prefix != 0, state_dtype, true).bytes;
 }
 
 extern "C" int mogt_affine_scan_generic_fwd(const void* U, const void* V, void* H, void* U_prefix, int64_t batch,
@@ -362,7 +383,7 @@ extern "C" int mogt_affine_scan_generic_fwd(const void* U, const void* V, void* 
     if (rc) return rc;
     if (batch == 0 || length == 0 || (channels == 0 && !U_prefix)) return MOGT_OK;
     if (!U || (channels > 0 && (!V || !H))) return set_error(MOGT_E_INVALID, "null tensor pointer");
-    const GGeo g = generic_geometry(batch, length, rank, channels, U_prefix != nullptr, state_dtype);
+    const GGeo g = generic_geometry(batch, length, rank, channels, U_prefix != nullptr, state_dtype, true);
     if (length > GS_ONE_CHUNK && (!workspace || workspace_bytes < g.bytes))
         return set_error(MOGT_E_WORKSPACE, "workspace of %zu bytes needed", g.bytes);
     hipStream_t st = static_cast<hipStream_t>(stream);
