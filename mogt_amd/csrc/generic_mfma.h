@@ -62,6 +62,7 @@ struct GParams {
     int shift;       // 1: step q is written at index q + 1 and the first chunk's initial state at index 0
     int rev;         // reverse, transposed transitions (generic_scan.hip's file comment)
     int stream;      // outputs are not read again by this scan
+    int scalar;      // host: take the scalar kernel (generic_scan.hip)
 };
 
 __device__ __forceinline__ int64_t at(const GView& v, int64_t b, int64_t s, int64_t r, int64_t c) {

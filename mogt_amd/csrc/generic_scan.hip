@@ -35,6 +35,7 @@ constexpr int GS_THREADS = 256;
 constexpr int GS_EPT = 4;                          // state elements per thread
 constexpr int GS_MAX_ELEMS = GS_THREADS * GS_EPT;  // R * column-tile width
 constexpr int GS_MAX_R = 1024;
+constexpr int GS_STAGED_R = 16;                    // transitions staged in LDS up to this rank
 constexpr int64_t GS_ONE_CHUNK = 16;               // steps up to which no workspace is asked for
 
 // Row length in LDS of the staged transition and of a state column: R rounded
@@ -45,17 +46,24 @@ __host__ __device__ constexpr int gs_ld(int R) {
                static_cast<int>(16 / sizeof(TS)) + static_cast<int>(16 / sizeof(TS));
 }
 
-// PD: steps of inputs in flight; the threads read their rows of U_t from memory.
-template <typename TS, int PD>
+// PD: steps of operands in flight.  RM = 0: the threads read their rows of U_t from
+// memory; else the rank is at most RM, U_t is staged through LDS (one value a
+// thread) and the contraction is unrolled, its LDS reads issued together.
+template <typename TS, int PD, int RM>
 __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_scan_kernel(GParams p) {
     extern __shared__ __align__(16) unsigned char gs_smem[];
-    // LDS: two state buffers stored column-major, [Cb][ld]; ld = R rounded up to
-    // 16 bytes plus 16 bytes of skew.  Padding columns / rows stay zero.
+    // LDS: the step's transition [R][ld] (staged form), then two state buffers
+    // stored column-major, [Cb][ld]; ld = R rounded up to 16 bytes plus 16 bytes
+    // of skew.  Padding columns / rows stay zero.
+    static_assert(RM * RM <= GS_THREADS, "one value of U a thread");
+    constexpr bool STAGED = RM > 0;
+    constexpr int VE = 16 / static_cast<int>(sizeof(TS));
     const int R = p.R, Cb = p.Cb, RCb = R * Cb;
     const int ld = gs_ld<TS>(R);
-    TS* sS = reinterpret_cast<TS*>(gs_smem);
-    const int lds_elems = 2 * Cb * ld;
-    for (int e = threadIdx.x; e < lds_elems; e += GS_THREADS) sS[e] = TS(0);
+    TS* sU = reinterpret_cast<TS*>(gs_smem);
+    TS* sS = sU + (STAGED ? R * ld : 0);
+    const int lds_elems = (STAGED ? R * ld : 0) + 2 * Cb * ld;
+    for (int e = threadIdx.x; e < lds_elems; e += GS_THREADS) sU[e] = TS(0);
     __syncthreads();
 
     const int tid = threadIdx.x;
@@ -96,8 +104,14 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
     // Operands of the next PD steps are in flight: slot pp of the ring holds
     // step s0 + pp of the current round and is refilled with step s0 + pp + PD
     // once its values have been consumed.
+    TS ureg[PD];
     TS vreg[PD][GS_EPT];
-    auto fetch = [&](int64_t q, TS (&v)[GS_EPT]) {
+    const int ur = tid / R, uc = tid - ur * R;   // the thread's value of U_t (staged form)
+    auto fetch = [&](int64_t q, TS& u, TS (&v)[GS_EPT]) {
+        // no transition enters the reversed position 0
+        if (STAGED && ur < R)
+            u = p.rev && q == 0 ? TS(0)
+                                : static_cast<const TS*>(p.tr.p)[at(p.tr, b, p.rev ? p.L - q : q, ur, p.tr_c0 + uc)];
         const int64_t ti = p.rev ? p.L - 1 - q : q;
 #pragma unroll
         for (int m = 0; m < GS_EPT; ++m)
@@ -107,16 +121,18 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
 
 #pragma unroll
     for (int pp = 0; pp < PD; ++pp)
-        if (pp < n) fetch(q0 + pp, vreg[pp]);
+        if (pp < n) fetch(q0 + pp, ureg[pp], vreg[pp]);
     __syncthreads();
     int cur = 0;
-    // one step: slot v holds step s; refilled with step s + PD
-    auto step = [&](int64_t s, TS (&v)[GS_EPT]) {
+    // one step: slot (u, v) holds step s; refilled with step s + PD
+    auto step = [&](int64_t s, TS& u, TS (&v)[GS_EPT]) {
         const int64_t q = q0 + s;
+        if (STAGED && ur < R) sU[p.rev ? uc * ld + ur : ur * ld + uc] = u;
         TS vin[GS_EPT];
 #pragma unroll
         for (int m = 0; m < GS_EPT; ++m) vin[m] = v[m];
-        if (s + PD < n) fetch(q + PD, v);   // later steps' loads overlap this step's arithmetic
+        if (s + PD < n) fetch(q + PD, u, v);   // later steps' loads overlap this step's arithmetic
+        if constexpr (STAGED) __syncthreads();
 
         const TS* Sc = sS + cur * Cb * ld;
         TS* Sn = sS + (cur ^ 1) * Cb * ld;
@@ -132,6 +148,19 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
         if (ident) {
 #pragma unroll
             for (int m = 0; m < GS_EPT; ++m) a[m] += scol[oi[m]];
+        } else if constexpr (STAGED) {
+            typedef TS vec_t __attribute__((ext_vector_type(VE)));
+#pragma unroll
+            for (int k = 0; k < RM; k += VE) {
+                if (k >= R) continue;
+                const vec_t sv = *reinterpret_cast<const vec_t*>(scol + k);
+#pragma unroll
+                for (int m = 0; m < GS_EPT; ++m) {
+                    const vec_t uv = *reinterpret_cast<const vec_t*>(sU + oi[m] * ld + k);
+#pragma unroll
+                    for (int e = 0; e < VE; ++e) a[m] += uv[e] * sv[e];
+                }
+            }
         } else {
             const TS* ut = static_cast<const TS*>(p.tr.p);
             for (int k = 0; k < R; ++k) {
@@ -158,7 +187,7 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
 #pragma unroll
         for (int pp = 0; pp < PD; ++pp) {
             if (s0 + pp >= n) break;   // uniform over the work-group
-            step(s0 + pp, vreg[pp]);
+            step(s0 + pp, ureg[pp], vreg[pp]);
         }
     }
     if (!p.every) {
@@ -173,9 +202,35 @@ __global__ __launch_bounds__(GS_THREADS, sizeof(TS) == 4 ? 3 : 2) void generic_s
 // chunk per sequence.
 constexpr int GS_LEVELS = 2;
 
+// Whether the scalar kernel is the faster one at ranks of which the matrix tiles
+// use few rows (a tile costs the same for 1 row as for 16): wide states over many
+// steps, where throughput counts; with fewer columns or steps its barriers and LDS
+// round trips do, and the matrix-core kernel is faster.  Matrix-core against
+// scalar kernel: R = 1, C = 1000, 4 x 4000 steps: float64 611 against 277 us, fp16 io
+// 414 against 197; R = 2, fp16 io, C = 500, 32 x 2000 955 against 442; R = 4, float64, C
+// = 1000, 4 x 4000 696 against 646, 64 x 128 152 against 252; R = 1, float64, C = 64, 32
+// x 2000 194 against 234; R = 2, fp16 io, C = 200, 4 x 4000 131 against 211.
+bool scalar_pays(int64_t B, int64_t L, int64_t R, int64_t C, bool f64, bool native) {
+    if (R < 1 || R > 4 || L <= GS_ONE_CHUNK) return false;
+    const double columns = static_cast<double>(B) * static_cast<double>(C);
+    const double values = columns * static_cast<double>(L);
+    const bool large = values >= 1.6e7;
+    if (f64 && native) {
+        if (L < 48 && (R > 2 || values < 3.0e6)) return false;
+        return values >= (R <= 2 ? 1.5e6 : 1.0e7) && (columns >= 2000.0 || large);
+    }
+    if (R == 1 && values >= 8.0e6 && L >= 48) return true;
+    if (columns < 3000.0 || values < 1.5e6) return false;
+    if (f64) return (R == 1 && L >= 48) || (R == 2 && L >= 100);
+    if (R == 1) return L >= 48 || (L >= 24 && values >= 3.0e6);
+    if (R == 2) return L >= 48 && (values >= 3.0e6 || (columns >= 6000.0 && L >= 100));
+    return large && L >= 48 && (R == 3 || values >= 3.0e7);
+}
+
 struct GGeo {
     int64_t seg[GS_LEVELS], nch[GS_LEVELS];   // steps per chunk, chunks
     int levels;                               // levels cut into more than one chunk
+    bool scalar;                              // every pass on the scalar kernel
     int Wl, Wo;          // LOCAL state width (C + R), OUTPUT / CARRY width (C + R if prefix)
     size_t s_off[GS_LEVELS], m_off[GS_LEVELS], bytes;
 };
@@ -188,7 +243,8 @@ GGeo geometry_of(int64_t B, int64_t L, int64_t R, int64_t C, int with_prefix, in
     g.Wl = static_cast<int>(C + R);
     g.Wo = static_cast<int>(C + (with_prefix ? R : 0));
     const size_t ts = state_code == MOGT_F64 ? 8 : 4;
-    const bool mfma = gm_fits(R, C + R);
+    g.scalar = scalar_pays(B, L, R, C, state_code == MOGT_F64, native);
+    const bool mfma = !g.scalar && gm_fits(R, C + R);
     size_t at = WS_HDR_BYTES;
     int64_t len = L;
     for (int l = 0; l < GS_LEVELS; ++l) {
@@ -242,7 +298,7 @@ int tile_width(int R, int W) {
 bool takes_mfma(const GParams& p) {
     int64_t row = p.W;
     for (const GView* v : {&p.tr, &p.in, &p.out_h, &p.out_p}) row = v->rs > row ? v->rs : row;
-    return gm_fits(p.R, row);
+    return !p.scalar && gm_fits(p.R, row);
 }
 
 template <typename TS>
@@ -253,8 +309,11 @@ int launch_generic(GParams p, int64_t batch, hipStream_t st, const char* what) {
     const int64_t blocks = batch * p.nseg * p.ntile;
     if (blocks <= 0) return MOGT_OK;
     if (blocks > 0x7fffffffLL) return set_error(MOGT_E_INVALID, "%s: problem too large for one launch", what);
-    const size_t lds = 2 * static_cast<size_t>(p.Cb) * gs_ld<TS>(p.R) * sizeof(TS);
-    hipLaunchKernelGGL((generic_scan_kernel<TS, 2>), dim3(static_cast<unsigned>(blocks)), dim3(GS_THREADS), lds, st, p);
+    const bool staged = p.R <= GS_STAGED_R;
+    const size_t lds = (2 * static_cast<size_t>(p.Cb) + (staged ? p.R : 0)) * gs_ld<TS>(p.R) * sizeof(TS);
+    const dim3 grid(static_cast<unsigned>(blocks)), block(GS_THREADS);
+    if (staged) hipLaunchKernelGGL((generic_scan_kernel<TS, 4, GS_STAGED_R>), grid, block, lds, st, p);
+    else hipLaunchKernelGGL((generic_scan_kernel<TS, 2, 0>), grid, block, lds, st, p);
     return check_launch(what);
 }
 
@@ -291,7 +350,7 @@ int scan_level(GParams out, const GGeo& g, int l, unsigned char* base, int state
     car.tr = vS; car.in = vS; car.init = none; car.out_h = vM; car.out_p = none;
     car.L = nch - 1;
     car.R = out.R; car.W = g.Wo; car.tr_c0 = iC; car.cin = iC; car.cid = iC; car.csplit = g.Wo;
-    car.every = 1; car.shift = 1; car.rev = 0;
+    car.every = 1; car.shift = 1; car.rev = 0; car.scalar = out.scalar;
     rc = scan_level(car, g, l + 1, base, state_code, launch);
     if (rc) return rc;
 
@@ -316,7 +375,7 @@ int run_passes(const void* U, const void* V, void* H, void* P, int64_t B, int64_
     GParams out{};   // the sequence's OUTPUT pass
     out.tr = vU; out.in = vV; out.init = none; out.out_h = vH; out.out_p = vP;
     out.L = L; out.R = iR; out.W = g.Wo; out.tr_c0 = 0; out.cin = iC; out.cid = iC; out.csplit = iC;
-    out.every = 1; out.shift = 0; out.rev = reverse; out.stream = 1;
+    out.every = 1; out.shift = 0; out.rev = reverse; out.stream = 1; out.scalar = g.scalar;
     return scan_level(out, g, 0, base, state_code, launch);
 }
 

@@ -447,6 +447,31 @@ def test_wide_ranks_with_other_io_types(gpu, vdt, R, offset):
     assert rel_err(G.double().cpu().numpy(), _loop64(U, V, rev=True)[1].numpy()) <= 2e-6
 
 
+@pytest.mark.parametrize("R,B,L,C,state,vdt", [(1, 16, 70, 1501, torch.float64, torch.float64),
+                                               (1, 3, 701, 1000, torch.float32, torch.float16),
+                                               (2, 40, 600, 130, torch.float32, torch.float64),
+                                               (2, 70, 150, 1000, torch.float64, torch.float32),
+                                               (3, 21, 300, 1600, torch.float64, torch.float64),
+                                               (4, 9, 1250, 900, torch.float64, torch.float64),
+                                               (4, 64, 500, 1000, torch.float32, torch.bfloat16)])
+def test_wide_states_of_few_ranks_match_the_loop(gpu, R, B, L, C, state, vdt):
+    """Wide states at ranks of 1 to 4 take the scalar kernel (transitions staged
+    in LDS): ragged chunks and column tiles, with the prefix, without, reversed."""
+    announce(f"generic wide low rank R={R} {B} {L} {C} {state} {vdt}")
+    g = torch.Generator().manual_seed(R * L)
+    U = (0.8 * torch.eye(R) + 0.2 / R * torch.randn(B, L, R, R, generator=g)).to(state)
+    V = torch.randn(B, L, R, C, generator=g).to(vdt)
+    Ug, Vg = U.to(gpu), V.to(gpu)
+    tol = 2e-6 if state == torch.float32 else 1e-13
+    Pr, Hr = _loop64(U, V)
+    P, H = torch.ops.mogt.affine_scan_generic(Ug, Vg, state, state, True, False)
+    one = torch.ops.mogt.affine_scan_generic(Ug, Vg, state, state, False, False)[1]
+    assert rel_err(H.double().cpu().numpy(), Hr.numpy()) <= tol and rel_err(P.double().cpu().numpy(), Pr.numpy()) <= tol
+    assert rel_err(one.double().cpu().numpy(), Hr.numpy()) <= tol
+    _, G = torch.ops.mogt.affine_scan_generic(Ug, Vg, state, state, False, True)
+    assert rel_err(G.double().cpu().numpy(), _loop64(U, V, rev=True)[1].numpy()) <= tol
+
+
 def test_matrix_core_workspace_covers_both_levels():
     """The workspace the C entry asks for grows with the chunks of both levels
     and is the header alone for one pass (host arithmetic only)."""
