@@ -279,9 +279,9 @@ int mogt_affine_scan_vk_fwd(const void* U, const void* v, const void* k, void* H
  * reverse = 1 runs the total-gradient recursion of the backward instead
  * (affine_scan_sequential_backward, affine_scan.py:110-118):
  * H_t = V_t + U_{t+1}^T H_{t+1}, H_{L-1} = V_{L-1}, with U_prefix NULL.
- * Up to three launches on `stream` (chunk summaries, carries, output); the
- * workspace (query with the same prefix flag and state dtype) needs no
- * clearing.                                                                 */
+ * Up to five launches on `stream` (chunk summaries, carries in one or three,
+ * output); the workspace (query with the same prefix flag and state dtype)
+ * needs no clearing.                                                        */
 size_t mogt_affine_scan_generic_workspace_bytes(int64_t batch, int64_t length, int64_t rank,
                                                 int64_t channels, int with_prefix, int state_dtype);
 int mogt_affine_scan_generic_fwd(const void* U, const void* V, void* H, void* U_prefix,

@@ -172,47 +172,47 @@ __device__ __forceinline__ int exp_doublings(float lam) {
 template <int RT>
 __device__ __forceinline__ Mat<RT> cayley_inverse(const Mat<RT>& X, const Mat<RT>& Mp, float (*sm)[33]) {
     const Mat<RT> zero = mat_scaled_identity<RT>(0.0f);
-            const Mat<RT> Z = mat_mul<RT>(X, X);                       // X^T X: (X^T)^T = X
-            // lam = ||Z||_inf >= lambda_max(Z): the spectrum of I + Z is in [1, 1 + lam]
-            float lam = 0.0f;
-            {
-                float rows[RT][4];
+    const Mat<RT> Z = mat_mul<RT>(X, X);                       // X^T X: (X^T)^T = X
+    // lam = ||Z||_inf >= lambda_max(Z): the spectrum of I + Z is in [1, 1 + lam]
+    float lam = 0.0f;
+    {
+        float rows[RT][4];
 #pragma unroll
-                for (int a = 0; a < RT; ++a)
+        for (int a = 0; a < RT; ++a)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float sum = 0.0f;
+            for (int i = 0; i < 4; ++i) {
+                float sum = 0.0f;
 #pragma unroll
-                        for (int b = 0; b < RT; ++b) sum += fabsf(Z.t[a][b][i]);
-                        rows[a][i] = sum;
-                    }
-                // sum over the 16 lanes of a row group (columns), then max over rows
-#pragma unroll
-                for (int off = 8; off >= 1; off >>= 1)
-#pragma unroll
-                    for (int a = 0; a < RT; ++a)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) rows[a][i] += __shfl_xor(rows[a][i], off, 64);
-#pragma unroll
-                for (int a = 0; a < RT; ++a)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) lam = fmaxf(lam, rows[a][i]);
-#pragma unroll
-                for (int off = 32; off >= 16; off >>= 1) lam = fmaxf(lam, __shfl_xor(lam, off, 64));
+                for (int b = 0; b < RT; ++b) sum += fabsf(Z.t[a][b][i]);
+                rows[a][i] = sum;
             }
-            // M^{-1} (M = I - X) by Newton-Schulz from Y_0 = c M^T, c = 2 / (2 + lam):
-            // the residual I - M Y_0 = I - c (I + Z) has norm <= lam / (2 + lam) < 1
-            // and squares every step.  Y is the left factor of its own update, so its
-            // exact transpose is formed (LDS) once per step.
-            const float c = 2.0f / (2.0f + lam);
-            const float w = lam / (2.0f + lam);
-            int K = 1;
-            if (w > 1e-8f) K = min(30, static_cast<int>(ceilf(log2f(fmaxf(-26.0f / log2f(w), 1.0f)))) + 1);
-                    Mat<RT> Y = mat_comb<RT>(c, Mp, 0.0f, zero, 0.0f);            // c M^T
-            for (int k = 0; k < K; ++k) {
-                const Mat<RT> T = mat_mul<RT>(Mp, Y);     // M Y   (M^T = I + X is M's transpose)
-                Y = mat_mul<RT>(mat_transpose<RT>(Y, sm), mat_comb<RT>(-1.0f, T, 0.0f, zero, 2.0f));
-            }
+        // sum over the 16 lanes of a row group (columns), then max over rows
+#pragma unroll
+        for (int off = 8; off >= 1; off >>= 1)
+#pragma unroll
+            for (int a = 0; a < RT; ++a)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) rows[a][i] += __shfl_xor(rows[a][i], off, 64);
+#pragma unroll
+        for (int a = 0; a < RT; ++a)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) lam = fmaxf(lam, rows[a][i]);
+#pragma unroll
+        for (int off = 32; off >= 16; off >>= 1) lam = fmaxf(lam, __shfl_xor(lam, off, 64));
+    }
+    // M^{-1} (M = I - X) by Newton-Schulz from Y_0 = c M^T, c = 2 / (2 + lam):
+    // the residual I - M Y_0 = I - c (I + Z) has norm <= lam / (2 + lam) < 1
+    // and squares every step.  Y is the left factor of its own update, so its
+    // exact transpose is formed (LDS) once per step.
+    const float c = 2.0f / (2.0f + lam);
+    const float w = lam / (2.0f + lam);
+    int K = 1;
+    if (w > 1e-8f) K = min(30, static_cast<int>(ceilf(log2f(fmaxf(-26.0f / log2f(w), 1.0f)))) + 1);
+    Mat<RT> Y = mat_comb<RT>(c, Mp, 0.0f, zero, 0.0f);            // c M^T
+    for (int k = 0; k < K; ++k) {
+        const Mat<RT> T = mat_mul<RT>(Mp, Y);     // M Y   (M^T = I + X is M's transpose)
+        Y = mat_mul<RT>(mat_transpose<RT>(Y, sm), mat_comb<RT>(-1.0f, T, 0.0f, zero, 2.0f));
+    }
     return Y;
 }
 

@@ -20,16 +20,17 @@
 // of operands are in flight.
 //
 // What bounds it: a step's chain of MFMAs in a wave for R = 64 (128 MFMAs of 32
-// cycles at CW = 2; the counters show the matrix unit busy 69 % of LOCAL's cycles,
-// 4 % waiting for memory, at 2.1 GHz), memory for R = 16 in float64.  The scalar kernel it
-// replaces at these ranks (one dot product per thread over LDS) spent about
-// 2 us in every step on its barriers and LDS round trips.  Measured: float64 R =
-// 16, C = 48, L = 32768 1036 -> 190 us (LOCAL 52 us = 5.2 TB/s, OUTPUT 106, the
+// cycles at CW = 2; counters over LOCAL of 24 x 2048 steps: matrix unit busy 69 % of
+// the cycles, 4 % of the waves' spent waiting), memory for R = 16 in float64.  The
+// scalar kernel it replaces at these ranks (one dot product per thread over LDS) spent
+// about 2 us in every step on its barriers and LDS round trips; it stays for wide
+// states of ranks up to 4 (generic_scan.hip, scalar_pays).  Measured: float64 R =
+// 16, C = 48, L = 32768 1036 -> 198 us (LOCAL 52 us = 5.2 TB/s, OUTPUT 106, the
 // carries in three passes 31 instead of 82 in one); fp32 R = C = 64, 24 x 2048
 // steps 4360 -> 1178 us, and with the memory instructions spread between the
 // MFMAs and a lane's two columns adjacent (P2: 8-byte loads and stores, whose
-// counter then never limits the operands in flight) 1112 us; with the prefix
-// written too 1795 -> 1560 us.  PD = 4 in place of 2: no gain, up to 8 % slower.
+// counter then never limits the operands in flight) 1110 us; with the prefix
+// written too 1795 -> 1548 us.  PD = 4 in place of 2: no gain, up to 8 % slower.
 #pragma once
 
 #include <math.h>

@@ -6,9 +6,10 @@
 // This file covers everything else the reference's functions accept: a float64 state
 // (the reference's own sanity check runs in float64, sanity_affine_scan.py:19-61), ranks
 // above 32, fp16 / fp64 inputs and outputs.  Ranks up to 64 run on the matrix-core chunk
-// kernel of generic_mfma.h; above (or where a step's block exceeds its 32-bit offsets) on
-// the scalar kernel below: every state element is one thread's running dot product over
-// the R rows of the previous state, with the state in LDS.
+// kernel of generic_mfma.h; above, for wide states of ranks up to 4 (scalar_pays) and where
+// a step's block exceeds its 32-bit offsets, on the scalar kernel below: every state element
+// is one thread's running dot product over the R rows of the previous state, with the state
+// in LDS.
 //
 // The prefix product U_prefix_t = U_t ... U_1 (return_prefix=True, affine_scan.py:43-55)
 // is the same recurrence applied to R extra state columns that start at the identity and

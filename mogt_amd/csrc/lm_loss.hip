@@ -7,7 +7,9 @@
 // (the forward of F.cross_entropy, whose default ignore_index is -100); any
 // other label outside [0, vocab) gives a NaN loss and a NaN gradient row.
 //
-// The logits GEMMs stay with the BLAS library.  These kernels replace the
+// The logits of large blocks come from split_gemm.hip, which also forms these rows
+// in its epilogue where one slice of the product fills the GPU; those of small
+// blocks, and all under autocast, from the BLAS library.  These kernels replace the
 // softmax / cross-entropy / one-hot / scale passes over each logits block: the
 // forward reads the block once (running maximum and rescaled sum of
 // exponentials per thread, merged across the work-group), the backward reads

@@ -5,7 +5,8 @@
 // Each fp32 operand comes as three bf16 pieces x = x1 + x2 + x3 (each the
 // rounded remainder of the ones before: 3 x 8 significant bits hold all 24 of
 // x), a bf16 operand as one.  A product of two bf16 pieces is exact in fp32
-// and the MFMA accumulates in fp32, so
+// and the MFMA accumulates in fp32, so (the splitting is Dekker's, "A floating-point
+// technique for extending the available precision", 1971, with bf16 pieces)
 //   1 x 3 pieces  x1 (y1 + y2 + y3)                              exact products
 //   3 x 3 pieces  x1 y1 + x1 y2 + x1 y3 + x2 y1 + x2 y2 + x3 y1  (the terms left
 //                 out are below 2^-26 of |x y|, under fp32's own rounding 2^-24)
@@ -50,13 +51,15 @@
 // kernel adds them in slice order, so results do not depend on scheduling.
 //
 // Measured (4096 rows, D = 768, vocabulary 32000; the library's fp32 GEMM before
-// -> here; error of the result against 64 bits, normwise):
+// -> here, one profiled run; figures beside the code are of pairs run back to back,
+// on cards whose clocks differ by some percent; error of the result against 64 bits,
+// normwise):
 //   logits, bf16 x fp32        1536 -> 589 us (1.02 PFLOP/s bf16)  5.0e-7 -> 3.0e-7
-//     with the loss rows       1650 -> 481 us (1.26)
-//     with the gradient block  1720 -> 620 us (786 MB of pieces written)
+//     with the loss rows       1650 -> 467 us (1.29)
+//     with the gradient block  1720 -> 577 us (1.05; 786 MB of pieces written)
 //   logits, fp32 x fp32        1518 -> 998 us (1.21)               5.0e-7 -> 4.3e-7
-//   d hidden, fp32 x fp32      1458 -> 1064 us (1.14)              3.2e-6 -> 1.4e-6
-//   d weight, fp32 x bf16      1448 -> 469 us (1.29)               1.1e-6 -> 7.0e-7
+//   d hidden, fp32 x fp32      1458 -> 997 us (1.21)               3.2e-6 -> 1.4e-6
+//   d weight, fp32 x bf16      1448 -> 449 us (1.34)               1.1e-6 -> 7.0e-7
 //   d weight, fp32 x fp32      1417 -> 957 us (1.26)               1.1e-6 -> 1.0e-6
 #include <math.h>
 
@@ -710,7 +713,9 @@ struct SplitPlan {
 };
 
 // Slices: the count that makes rounds of work-groups (one per CU) times their
-// length, in MFMA cycles, plus the partials' traffic the least.
+// length, plus the partials' traffic, the least.  A stage is taken for its MFMA
+// cycles at 1.9 GHz: 1.6 us for 3 x 3 pieces, which take 2.6 in the hidden
+// gradient, so the partials' traffic weighs more here than it does there.
 SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int na, int nb, int64_t splits, int64_t cus) {
     SplitPlan pl{};
     const int np = na == 3 && nb == 3 ? 6 : na * nb;

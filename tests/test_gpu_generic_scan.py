@@ -119,8 +119,8 @@ def test_fp64_state_multichunk(gpu, B, L, R, C):
 @pytest.mark.parametrize("R,L,C", [(33, 300, 4), (48, 257, 8), (64, 200, 3), (65, 150, 2), (100, 90, 5),
                                    (130, 40, 3)])
 def test_ranks_above_32(gpu, R, L, C):
-    """Ranks the matrix-core pipeline does not take: fp32 state (transitions
-    staged in LDS up to R = 64, read from memory above), through the hybrid
+    """Ranks the matrix-core pipeline does not take: fp32 state (the matrix-core
+    chunk kernel up to R = 64, the scalar kernel above), through the hybrid
     drop-in, with the prefix product; float64 state at the same shapes."""
     announce(f"generic scan R={R} L={L} C={C}")
     from mogt_amd import affine_scan as das
