@@ -274,7 +274,19 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
         }
     }
 
-    __shared__ __align__(16) float s_h[GRADU ? ROWS : 1][GRADU ? VS : 4];
+    // GRADU: the state of a step; its last row stays zero and stands for columns
+    // past C (C is a multiple of 8, in the last tile), which meet zeros of G that an
+    // infinite U's NaN there would turn into NaN
+    __shared__ __align__(16) float s_h[GRADU ? ROWS + 1 : 1][GRADU ? VS : 4];
+    const float* hlast[GRADU ? RT : 1];
+    if constexpr (GRADU) {
+        if (lane < 4) s_h[ROWS][lane] = 0.0f;
+#pragma unroll
+        for (int ct = 0; ct < RT; ++ct) {
+            const int c = 16 * (CTW - 1) + 4 * g;
+            hlast[ct] = c < C ? &s_h[16 * ct + n][c] : &s_h[ROWS][0];
+        }
+    }
     __shared__ __align__(16) float s_v[VBLOCK ? ROWS : 1][VBLOCK ? VS : 4];
     __shared__ __align__(16) float s_o[STAGE_OUT ? ROWS : 1][STAGE_OUT ? VS : 4];
     // Orders this wave's LDS writes before its reads of other lanes' data and
@@ -487,17 +499,14 @@ __global__ __launch_bounds__(64) void dense_chunk_kernel(ChunkParams p) {
 #pragma unroll
                 for (int h = 0; h < CTW; ++h)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        // columns past C (in the last tile) meet zeros of G, which an
-                        // infinite U's NaN there would turn into NaN
-                        s_h[trow(rt, i)][16 * h + n] = h < CTW - 1 || 16 * h + n < C ? X[rt][RT + h][i] : 0.0f;
+                    for (int i = 0; i < 4; ++i) s_h[trow(rt, i)][16 * h + n] = X[rt][RT + h][i];
             lds_order();
             f32x4 hb[RT][CTW];
 #pragma unroll
             for (int ct = 0; ct < RT; ++ct)
 #pragma unroll
                 for (int h = 0; h < CTW; ++h)
-                    hb[ct][h] = *reinterpret_cast<const f32x4*>(&s_h[16 * ct + n][16 * h + 4 * g]);
+                    hb[ct][h] = *reinterpret_cast<const f32x4*>(h < CTW - 1 ? &s_h[16 * ct + n][16 * h + 4 * g] : hlast[ct]);
             lds_order();
             f32x4 d[2][RT][RT];
 #pragma unroll
